@@ -17,9 +17,9 @@
 // another's epilogues; at 256 rows (106 KB) a CU held one.
 //
 // Backward: the max-pool sends each channel's gradient to one point, so the
-// per-point layers only need the <= 256 argmax rows per cloud (k_enc_rows
-// recomputes their activations).  Weight gradients are sums of outer products
-// over pairs / rows, done in two deterministic stages (fixed-order partials).
+// per-point layers only need the <= 256 argmax rows per cloud (k_enc_grad
+// recomputes their activations and keeps the weight gradients' partial sums in
+// registers).  Every sum is deterministic (fixed-order partials).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -30,6 +30,7 @@ namespace lcr {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kRows = 128;      // points per forward block (two blocks' LDS fit a CU)
@@ -229,209 +230,270 @@ __global__ void k_enc_head_back(const float* __restrict__ Z, const float* __rest
   const float* Hw1 = W + kEncHw1;
   for (int i = t; i < 512; i += 256) {
     float a = 0.f;
-    const float* row = Hw1 + i * 256;
-    for (int j = 0; j < 256; ++j) a = fmaf(dz[j], row[j], a);
+    const float4* row = reinterpret_cast<const float4*>(Hw1 + i * 256);
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {  // eight 16-byte loads in flight, one fmaf chain
+      const float4 v = row[j];
+      a = fmaf(dz[4 * j], v.x, a);
+      a = fmaf(dz[4 * j + 1], v.y, a);
+      a = fmaf(dz[4 * j + 2], v.z, a);
+      a = fmaf(dz[4 * j + 3], v.w, a);
+    }
     DG[b * 512 + i] = a;
   }
 }
 
-// C[i][j] = sum_{r < R} A[r * lda + i] * B[r * ldb + j] (+ bias sums of B when
-// i == M), one thread per output, rows in order: deterministic.  Used with R up to
-// a few thousand (pairs); larger R goes through the two-stage version.
-__global__ void k_outer_small(const float* __restrict__ A, int lda, const float* __restrict__ B,
-                              int ldb, int R, int M, int N, float* __restrict__ C,
-                              float* __restrict__ bias) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (M + 1) * N) return;
-  const int i = idx / N, j = idx % N;
-  float s = 0.f;
-  if (i < M) {
-    for (int r = 0; r < R; ++r) s = fmaf(A[(int64_t)r * lda + i], B[(int64_t)r * ldb + j], s);
-    C[i * N + j] = s;
-  } else {
-    for (int r = 0; r < R; ++r) s += B[(int64_t)r * ldb + j];
-    bias[j] = s;
-  }
-}
-
-// stage 1 of a large outer-product sum: block k sums rows [k*rows, (k+1)*rows)
-// into part[k][(M+1)*N] (last row = bias sums)
-__global__ void k_outer_part(const float* __restrict__ A, int lda, const float* __restrict__ B,
-                             int ldb, int R, int M, int N, int rows, float* __restrict__ part) {
-  const int k = blockIdx.y;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (M + 1) * N) return;
-  const int i = idx / N, j = idx % N;
-  const int r0 = k * rows, r1 = min(R, r0 + rows);
-  float s = 0.f;
-  // unrolled so that the loads of several rows are in flight; one accumulator,
-  // the rows in order
-  if (i < M) {
-#pragma unroll 8
-    for (int r = r0; r < r1; ++r) s = fmaf(A[(int64_t)r * lda + i], B[(int64_t)r * ldb + j], s);
-  } else {
-#pragma unroll 8
-    for (int r = r0; r < r1; ++r) s += B[(int64_t)r * ldb + j];
-  }
-  part[(int64_t)k * (M + 1) * N + idx] = s;
-}
-
-// k_outer_part with a 4 x 4 block of outputs per thread (M, N, lda, ldb multiples
-// of 4, A and B 16-byte aligned): per row one float4 of A and one of B feed 16
-// multiply-adds, where one output per thread read two values per multiply-add and
-// was bound by those loads.  Every output is the same fmaf chain over the rows in
-// order, so the sums are bitwise those of k_outer_part.  Threads past the 4 x 4
-// blocks sum the bias row, four columns each.
-__global__ void k_outer_part4(const float* __restrict__ A, int lda, const float* __restrict__ B,
-                              int ldb, int R, int M, int N, int rows, float* __restrict__ part) {
-  const int k = blockIdx.y;
-  const int nq = N >> 2, tiles = (M >> 2) * nq;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= tiles + nq) return;
-  const int r0 = k * rows, r1 = min(R, r0 + rows);
-  float* out = part + (int64_t)k * (M + 1) * N;
-  if (t < tiles) {
-    const int i0 = (t / nq) * 4, j0 = (t % nq) * 4;
-    float acc[4][4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[u][v] = 0.f;
-#pragma unroll 4
-    for (int r = r0; r < r1; ++r) {
-      const float4 a = *reinterpret_cast<const float4*>(A + (int64_t)r * lda + i0);
-      const float4 b = *reinterpret_cast<const float4*>(B + (int64_t)r * ldb + j0);
-      const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = fmaf(av[u], bv[v], acc[u][v]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) out[(i0 + u) * N + j0 + v] = acc[u][v];
-  } else {
-    const int j0 = (t - tiles) * 4;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int r = r0; r < r1; ++r) {
-      const float4 b = *reinterpret_cast<const float4*>(B + (int64_t)r * ldb + j0);
-      acc[0] += b.x;
-      acc[1] += b.y;
-      acc[2] += b.z;
-      acc[3] += b.w;
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) out[M * N + j0 + v] = acc[v];
-  }
-}
-
-__global__ void k_outer_fold(const float* __restrict__ part, int nparts, int M, int N,
-                             float* __restrict__ C, float* __restrict__ bias) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (M + 1) * N) return;
-  float s = 0.f;
-  for (int k = 0; k < nparts; ++k) s += part[(int64_t)k * (M + 1) * N + idx];
-  if (idx < M * N)
-    C[idx] = s;
-  else
-    bias[idx - M * N] = s;
-}
-
-// Per (cloud, channel) row of the max-pool backward: recompute h1, h2 at the
-// channel's argmax point and push the channel's gradient down to layer 1.
-// One block = 64 channels of one cloud.  Writes per row: x (3), h1 (64), da1 (64),
-// h2 (128), da2 (128) and the row's df (used by the W3 gradient).
+// C[i][j] = sum_{r < R} A[r * lda + i] * B[r * ldb + j], and the column sums of B
+// into bias[j] (a row of ones under A), on FP32 matrix instructions.  A block
+// computes one 16 x 16 tile: each of its 4 wavefronts runs a quarter of the rows
+// straight from memory (four rows per instruction, 64-byte row segments, eight
+// steps of loads in flight), and their tiles are added in wavefront order.  The
+// head's gradients at 256 pairs: 126 -> 9 us (one thread per output walked the
+// rows one after the other).
 __global__ void __launch_bounds__(256)
-k_enc_rows(const float4* __restrict__ X, int npts, const float* __restrict__ F,
-           const int* __restrict__ ARG, const float* __restrict__ DG, const float* __restrict__ W,
-           const __bf16* __restrict__ W2t, const __bf16* __restrict__ W3t, float* __restrict__ XA,
-           float* __restrict__ H1A, float* __restrict__ DA1, float* __restrict__ H2A,
-           float* __restrict__ DA2, float* __restrict__ DF) {
-  __shared__ float h1[64][65];
-  __shared__ float m1[64][64];
-  __shared__ float da2s[64][129];
-  __shared__ float xs[64][3];
-  __shared__ float dfs[64];
-  const int cloud = blockIdx.y, c0 = blockIdx.x * 64, t = threadIdx.x;
-  const int pair = cloud >> 1, side = cloud & 1;
-  const int64_t rbase = (int64_t)cloud * 256 + c0;
-  if (t < 64) {
-    const int c = c0 + t;
-    const float f = F[cloud * 256 + c];
-    const float df = f > 0.f ? DG[pair * 512 + side * 256 + c] : 0.f;
-    dfs[t] = df;
-    const float4 x = X[(int64_t)cloud * npts + ARG[cloud * 256 + c]];
-    xs[t][0] = x.x;
-    xs[t][1] = x.y;
-    xs[t][2] = x.z;
-    DF[rbase + t] = df;
-    XA[(rbase + t) * 3 + 0] = x.x;
-    XA[(rbase + t) * 3 + 1] = x.y;
-    XA[(rbase + t) * 3 + 2] = x.z;
-  }
-  __syncthreads();
-  // layer 1 for the 64 rows: thread -> (row r = t / 4, 16 columns)
-  {
-    const int r = t >> 2, j0 = (t & 3) * 16;
-    for (int j = j0; j < j0 + 16; ++j) {
-      float a = W[kEncB1 + j];
-      a = fmaf(xs[r][0], W[kEncW1 + j], a);
-      a = fmaf(xs[r][1], W[kEncW1 + 64 + j], a);
-      a = fmaf(xs[r][2], W[kEncW1 + 128 + j], a);
-      h1[r][j] = a > 0.f ? (float)(__bf16)a : 0.f;
-      m1[r][j] = a > 0.f ? 1.f : 0.f;
-      H1A[(rbase + r) * 64 + j] = h1[r][j];
-    }
-  }
-  __syncthreads();
-  // layer 2: thread -> column j = t % 128, rows r = t / 128 + 2m
-  {
-    const int j = t & 127;
-    float w2[64];
+k_outer_mfma(const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb, int R, int M,
+             int N, float* __restrict__ C, float* __restrict__ bias) {
+  __shared__ float red[4][256];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l16 = lane & 15, q = lane >> 4;
+  const int i = blockIdx.x * 16 + l16, j = blockIdx.y * 16 + l16;
+  const int per = ((R + 15) / 16) * 4;
+  const int r0 = w * per, r1 = min(R, r0 + per);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  // every load at an address inside the arrays; what lies past M, N or the rows is
+  // replaced afterwards
+  const float* pa = A + min(i, M - 1);
+  const float* pb = B + min(j, N - 1);
+  for (int rb = r0; rb < r1; rb += 32) {
+    float a[8], b[8];
 #pragma unroll
-    for (int i = 0; i < 64; ++i) w2[i] = (float)W2t[j * 64 + i];
-    const float b2 = W[kEncB2 + j];
-    for (int r = t >> 7; r < 64; r += 2) {
-      float a = b2;
+    for (int u = 0; u < 8; ++u) {
+      const int64_t rr = min(rb + 4 * u + q, R - 1);
+      a[u] = pa[rr * lda];
+      b[u] = pb[rr * ldb];
+    }
 #pragma unroll
-      for (int i = 0; i < 64; ++i) a = fmaf(h1[r][i], w2[i], a);
-      const float h2 = a > 0.f ? (float)(__bf16)a : 0.f;
-      const float g = a > 0.f ? dfs[r] * (float)W3t[(c0 + r) * 128 + j] : 0.f;
-      da2s[r][j] = g;
-      H2A[(rbase + r) * 128 + j] = h2;
-      DA2[(rbase + r) * 128 + j] = g;
+    for (int u = 0; u < 8; ++u) {
+      const bool ok = rb + 4 * u + q < r1;
+      const float x = i < M ? a[u] : (i == M ? 1.f : 0.f);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ok ? x : 0.f, ok && j < N ? b[u] : 0.f, acc, 0, 0, 0);
     }
   }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) red[w][(4 * q + e) * 16 + l16] = acc[e];
   __syncthreads();
-  // dh1 = da2 W2^T, masked: thread -> (row r = t / 4, 16 columns)
-  {
-    const int r = t >> 2, i0 = (t & 3) * 16;
-    for (int i = i0; i < i0 + 16; ++i) {
-      float s = 0.f;
-      for (int j = 0; j < 128; ++j) s = fmaf(da2s[r][j], (float)W2t[j * 64 + i], s);
-      DA1[(rbase + r) * 64 + i] = s * m1[r][i];
-    }
-  }
+  const int t = threadIdx.x, oi = blockIdx.x * 16 + t / 16, oj = blockIdx.y * 16 + t % 16;
+  if (oi > M || oj >= N) return;
+  const float s = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
+  if (oi < M)
+    C[oi * N + oj] = s;
+  else
+    bias[oj] = s;
 }
 
-// dW3[k][c] = sum_clouds H2A[(cloud, c)][k] * DF[(cloud, c)]; db3[c] = sum DF
-__global__ void k_enc_dw3(const float* __restrict__ H2A, const float* __restrict__ DF, int nclouds,
-                          float* __restrict__ G) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= 129 * 256) return;
-  const int k = idx / 256, c = idx % 256;
-  float s = 0.f;
-  if (k < 128) {
-    for (int cl = 0; cl < nclouds; ++cl) {
-      const int64_t r = (int64_t)cl * 256 + c;
-      s = fmaf(H2A[r * 128 + k], DF[r], s);
+// Backward through the per-point layers.  The max-pool sends each channel's
+// gradient to one point, so a cloud contributes 256 rows (channels).  A block
+// takes 64 channels (blockIdx.x) of the clouds blockIdx.y, + gridDim.y, ... and
+// keeps its share of every weight gradient in registers over all of them; only
+// that share leaves the chip (part_w, part_w3, added in a fixed order by
+// k_enc_grad_fold).  Per cloud:
+//   layer 1 recomputed for the 64 argmax points (FP32), h1 as bf16 in LDS;
+//   layer 2 on BF16 MFMA exactly as the forward computes it, transposed (columns
+//   = rows of the batch), so a lane holds four consecutive channels of one point:
+//   h2 df joins the W3 gradient, and m = (a2 > 0) W3 goes to LDS (bf16, exact);
+//   dh1 = df (m W2^T): both factors are bf16, the products exact, df applied after
+//   the FP32 sum; with h1's mask it joins the W1 gradient;
+//   the W2 gradient h1^T (df m) on FP32 MFMA, operands widened from LDS.
+// Bound by latency and the LDS and vector work around the MFMAs (about 6.5 GFLOP
+// in all).  256 pairs (512 clouds): 1238 -> 57 us with the fold; before, the rows'
+// activations and gradients (384 floats each) went through memory to four vector
+// kernels.
+constexpr int kGradW = kEncW3;                     // W1, b1, W2, b2: first in the flat layout
+constexpr int kGradW3 = kEncB3 + 256 - kEncW3;     // W3, b3: next
+constexpr int kGradGroups = 128;                   // cloud groups: 512 blocks, two per CU
+constexpr int kGradMS = 128 + 8;                   // LDS row stride of m (bf16)
+
+__global__ void __launch_bounds__(256, 2)
+k_enc_grad(const float4* __restrict__ X, int npts, const float* __restrict__ F,
+           const int* __restrict__ ARG, const float* __restrict__ DG, const float* __restrict__ W,
+           const __bf16* __restrict__ W2t, const __bf16* __restrict__ W3t, int nclouds,
+           float* __restrict__ part_w, float* __restrict__ part_w3) {
+  __shared__ __attribute__((aligned(16))) __bf16 H1[64 * kH1S];
+  __shared__ __attribute__((aligned(16))) __bf16 Mk[64 * kGradMS];
+  __shared__ float4 xs[64];
+  __shared__ float dfs[64];
+  __shared__ float4 w1[64];  // (b1, W1) per output of layer 1: kept out of the registers
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, l16 = lane & 15, q = lane >> 4, kq = q * 8;
+  const int c0 = blockIdx.x * 64;
+  bf16x8 A2[2][2], B1[4];
+  bf16x4 w3[4][2];
+  f32x4 b2[2], acc3[4][2], accb2[2], acc2[4][2];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int jt = 0; jt < 2; ++jt) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      A2[jt][ks] = *(const bf16x8*)(W2t + (32 * w + 16 * jt + l16) * 64 + 32 * ks + kq);
+    b2[jt] = *(const f32x4*)(W + kEncB2 + 32 * w + 16 * jt + 4 * q);
+    accb2[jt] = zero;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      w3[rt][jt] = *(const bf16x4*)(W3t + (c0 + 16 * rt + l16) * 128 + 32 * w + 16 * jt + 4 * q);
+      acc3[rt][jt] = zero;
+      acc2[rt][jt] = zero;
     }
-    G[kEncW3 + k * 256 + c] = s;
-  } else {
-    for (int cl = 0; cl < nclouds; ++cl) s += DF[(int64_t)cl * 256 + c];
-    G[kEncB3 + c] = s;
   }
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+      B1[ks][v] = (__bf16)W[kEncW2 + (16 * w + l16) * 128 + 32 * ks + kq + v];
+  float acc1[4] = {0.f, 0.f, 0.f, 0.f}, accb3 = 0.f;
+  if (t < 64)
+    w1[t] = make_float4(W[kEncB1 + t], W[kEncW1 + t], W[kEncW1 + 64 + t], W[kEncW1 + 128 + t]);
+  for (int cloud = blockIdx.y; cloud < nclouds; cloud += gridDim.y) {
+    if (t < 64) {
+      const int c = cloud * 256 + c0 + t;
+      const float df = F[c] > 0.f ? DG[c] : 0.f;
+      xs[t] = X[(int64_t)cloud * npts + ARG[c]];
+      dfs[t] = df;
+      accb3 += df;
+    }
+    __syncthreads();
+    {
+      const int r = t >> 2, j0 = (t & 3) * 16;
+      const float4 x = xs[r];
+      bf16x8 h[2];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const float4 v = w1[j0 + u];
+        float a = v.x;
+        a = fmaf(x.x, v.y, a);
+        a = fmaf(x.y, v.z, a);
+        a = fmaf(x.z, v.w, a);
+        h[u >> 3][u & 7] = (__bf16)relu(a);
+      }
+      *(bf16x8*)(H1 + r * kH1S + j0) = h[0];
+      *(bf16x8*)(H1 + r * kH1S + j0 + 8) = h[1];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) {
+      const int r = 16 * rt + l16;
+      const float df = dfs[r];
+      bf16x8 hf[2];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) hf[ks] = *(const bf16x8*)(H1 + r * kH1S + 32 * ks + kq);
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt) {
+        f32x4 acc = zero;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A2[jt][ks], hf[ks], acc, 0, 0, 0);
+        bf16x4 m;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float a = acc[e] + b2[jt][e];
+          const bool pos = a > 0.f;
+          const float h2 = pos ? (float)(__bf16)a : 0.f;
+          acc3[rt][jt][e] = fmaf(h2, df, acc3[rt][jt][e]);
+          m[e] = pos ? w3[rt][jt][e] : (__bf16)0.f;
+          accb2[jt][e] += df * (float)m[e];
+        }
+        *(bf16x4*)(Mk + r * kGradMS + 32 * w + 16 * jt + 4 * q) = m;
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one row tile's operands live at a time
+    }
+    __syncthreads();
+    // dh1 at columns i = 16 w + l16, and layer 1's gradient
+#pragma unroll 1
+    for (int rt = 0; rt < 4; ++rt) {
+      f32x4 acc = zero;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const bf16x8 mf = *(const bf16x8*)(Mk + (16 * rt + l16) * kGradMS + 32 * ks + kq);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mf, B1[ks], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 16 * rt + 4 * q + e;
+        const float4 x = xs[r];
+        const float d = (float)H1[r * kH1S + 16 * w + l16] > 0.f ? acc[e] * dfs[r] : 0.f;
+        acc1[0] = fmaf(x.x, d, acc1[0]);
+        acc1[1] = fmaf(x.y, d, acc1[1]);
+        acc1[2] = fmaf(x.z, d, acc1[2]);
+        acc1[3] += d;
+      }
+    }
+    // W2 gradient: columns j = 32 w + 16 jt + l16, rows of the batch four at a time
+#pragma unroll 2
+    for (int ks = 0; ks < 16; ++ks) {
+      const int r = 4 * ks + q;
+      const float df = dfs[r];
+      float bv[2];
+#pragma unroll
+      for (int jt = 0; jt < 2; ++jt) bv[jt] = df * (float)Mk[r * kGradMS + 32 * w + 16 * jt + l16];
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const float av = (float)H1[r * kH1S + 16 * it + l16];
+#pragma unroll
+        for (int jt = 0; jt < 2; ++jt)
+          acc2[it][jt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[jt], acc2[it][jt], 0, 0, 0);
+      }
+    }
+    __syncthreads();  // xs, dfs, H1 and Mk are rewritten for the next cloud
+  }
+  float* pw = part_w + (int64_t)(blockIdx.y * gridDim.x + blockIdx.x) * kGradW;
+  float* p3 = part_w3 + (int64_t)blockIdx.y * kGradW3;
+#pragma unroll
+  for (int it = 0; it < 4; ++it)
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        pw[kEncW2 + (16 * it + 4 * q + e) * 128 + 32 * w + 16 * jt + l16] = acc2[it][jt][e];
+        p3[(32 * w + 16 * jt + 4 * q + e) * 256 + c0 + 16 * it + l16] = acc3[it][jt][e];
+      }
+#pragma unroll
+  for (int jt = 0; jt < 2; ++jt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = accb2[jt][e];
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+      if (l16 == 0) pw[kEncB2 + 32 * w + 16 * jt + 4 * q + e] = v;
+    }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    float v = acc1[c];
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    if (q == 0) pw[kEncW1 + c * 64 + 16 * w + l16] = v;  // W1's three rows, then b1
+  }
+  if (t < 64) p3[kEncB3 - kEncW3 + c0 + t] = accb3;
+}
+
+// The blocks' shares added in a fixed order: 64 outputs per block, eight slices of
+// the shares each.  part_w has 4 * groups shares, part_w3 one per group.
+constexpr int kFoldSlices = 8;
+
+__global__ void __launch_bounds__(64 * kFoldSlices)
+k_enc_grad_fold(const float* __restrict__ part_w, const float* __restrict__ part_w3, int groups,
+                float* __restrict__ G) {
+  static_assert(kGradW % 64 == 0 && kGradW3 % 64 == 0, "a block's outputs lie in one part");
+  __shared__ float red[kFoldSlices][64];
+  const int o = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
+  const bool w3 = o >= kGradW;
+  const int n = w3 ? groups : 4 * groups, stride = w3 ? kGradW3 : kGradW;
+  const float* p = w3 ? part_w3 + (o - kGradW) : part_w + o;
+  float s = 0.f;
+#pragma unroll 8
+  for (int k = slice; k < n; k += kFoldSlices) s += p[(int64_t)k * stride];
+  red[slice][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (slice != 0) return;
+#pragma unroll
+  for (int k = 1; k < kFoldSlices; ++k) s += red[k][threadIdx.x];
+  G[o] = s;
 }
 
 // Adam (FP32 master weights), then refresh the BF16 transposed copies of W2, W3
@@ -461,6 +523,9 @@ __global__ void k_enc_bf16_weights(const float* __restrict__ W, __bf16* __restri
   }
 }
 
+// Cloud groups of the per-point backward: one per cloud up to kGradGroups.
+inline int enc_grad_groups(int nclouds) { return nclouds < kGradGroups ? nclouds : kGradGroups; }
+
 inline unsigned nb(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 }  // namespace
@@ -488,25 +553,17 @@ void launch_enc_backward(const EncBuffers& e, int npairs, int npts, hipStream_t 
   float* G = e.G;
   hipLaunchKernelGGL(k_enc_head_back, dim3(npairs), dim3(256), 0, s, e.Z, e.DOUT, e.W, e.DZ, e.DG);
   // head weights: dHw2 = Z^T dOut, dHw1 = G^T dZ (G = pooled features)
-  hipLaunchKernelGGL(k_outer_small, dim3(nb(257 * 6, 256)), dim3(256), 0, s, e.Z, 256, e.DOUT, 6,
-                     npairs, 256, 6, G + kEncHw2, G + kEncHb2);
-  hipLaunchKernelGGL(k_outer_small, dim3(nb(513 * 256, 256)), dim3(256), 0, s, e.F, 512, e.DZ, 256,
-                     npairs, 512, 256, G + kEncHw1, G + kEncHb1);
-  // per (cloud, channel) rows
-  hipLaunchKernelGGL(k_enc_rows, dim3(4, nclouds), dim3(256), 0, s, e.X, npts, e.F, e.ARG, e.DG,
-                     e.W, e.W2t, e.W3t, e.XA, e.H1A, e.DA1, e.H2A, e.DA2, e.DF);
-  hipLaunchKernelGGL(k_enc_dw3, dim3(nb(129 * 256, 256)), dim3(256), 0, s, e.H2A, e.DF, nclouds, G);
-  const int R = nclouds * 256;
-  const int rows = 1024;
-  const int parts = (R + rows - 1) / rows;
-  hipLaunchKernelGGL(k_outer_part4, dim3(nb(16 * 32 + 32, 256), parts), dim3(256), 0, s, e.H1A, 64,
-                     e.DA2, 128, R, 64, 128, rows, e.part_grad);
-  hipLaunchKernelGGL(k_outer_fold, dim3(nb(65 * 128, 256)), dim3(256), 0, s, e.part_grad, parts, 64,
-                     128, G + kEncW2, G + kEncB2);
-  hipLaunchKernelGGL(k_outer_part, dim3(nb(4 * 64, 256), parts), dim3(256), 0, s, e.XA, 3, e.DA1,
-                     64, R, 3, 64, rows, e.part_grad);
-  hipLaunchKernelGGL(k_outer_fold, dim3(nb(4 * 64, 256)), dim3(256), 0, s, e.part_grad, parts, 3, 64,
-                     G + kEncW1, G + kEncB1);
+  hipLaunchKernelGGL(k_outer_mfma, dim3(17, 1), dim3(256), 0, s, e.Z, 256, e.DOUT, 6, npairs, 256, 6,
+                     G + kEncHw2, G + kEncHb2);
+  hipLaunchKernelGGL(k_outer_mfma, dim3(33, 16), dim3(256), 0, s, e.F, 512, e.DZ, 256, npairs, 512,
+                     256, G + kEncHw1, G + kEncHb1);
+  // per-point layers
+  const int groups = enc_grad_groups(nclouds);
+  float* part_w3 = e.part_grad + (int64_t)4 * groups * kGradW;
+  hipLaunchKernelGGL(k_enc_grad, dim3(4, groups), dim3(256), 0, s, e.X, npts, e.F, e.ARG, e.DG, e.W,
+                     e.W2t, e.W3t, nclouds, e.part_grad, part_w3);
+  hipLaunchKernelGGL(k_enc_grad_fold, dim3((kGradW + kGradW3) / 64), dim3(64 * kFoldSlices), 0, s,
+                     e.part_grad, part_w3, groups, G);
 }
 
 void launch_adam(float* W, const float* G, float* M, float* V, int n, float lr, int step,
@@ -518,9 +575,7 @@ void launch_adam(float* W, const float* G, float* M, float* V, int n, float lr, 
 }
 
 int64_t enc_part_grad_floats(int npairs) {
-  const int R = 2 * npairs * 256;
-  const int parts = (R + 1023) / 1024;
-  return (int64_t)parts * 65 * 128;
+  return (int64_t)enc_grad_groups(2 * npairs) * (4 * kGradW + kGradW3);
 }
 
 }  // namespace lcr

@@ -222,13 +222,7 @@ struct EncBuffers {
   float* loss_part;      // [pair][6]
   float* DZ;             // [pair][256]
   float* DG;             // [pair][512]
-  float* XA;             // rows [cloud*256 + c]: x (3), h1 (64), da1 (64), h2 (128), da2 (128)
-  float* H1A;
-  float* DA1;
-  float* H2A;
-  float* DA2;
-  float* DF;
-  float* part_grad;
+  float* part_grad;      // the backward blocks' shares of the per-point layers' gradients
   float* G;              // gradient (kEncNParam)
 };
 void launch_enc_bf16_weights(const float* W, __bf16* W2t, __bf16* W3t, hipStream_t s);

@@ -188,8 +188,8 @@ struct ProposalImpl {
   int cap_pairs = 0, cap_pts = 0;
   int step = 0;
   DevBuf W, M, V, G, W2t, W3t;
-  DevBuf X, part_max, part_arg, F, ARG, Z, OUT, DOUT, loss_part, DZ, DG, XA, H1A, DA1, H2A, DA2,
-      DF, part_grad, lab, idx, losses, frame;
+  DevBuf X, part_max, part_arg, F, ARG, Z, OUT, DOUT, loss_part, DZ, DG, part_grad, lab, idx, losses,
+      frame;
   DevBuf ds_X, ds_lab;
   int ds_pairs = 0, ds_pts = 0;
   HostBuf h_io;
@@ -232,12 +232,6 @@ struct ProposalImpl {
     loss_part.reserve(P * 6 * sizeof(float));
     DZ.reserve(P * 256 * sizeof(float));
     DG.reserve(P * 512 * sizeof(float));
-    XA.reserve(C * 256 * 3 * sizeof(float));
-    H1A.reserve(C * 256 * 64 * sizeof(float));
-    DA1.reserve(C * 256 * 64 * sizeof(float));
-    H2A.reserve(C * 256 * 128 * sizeof(float));
-    DA2.reserve(C * 256 * 128 * sizeof(float));
-    DF.reserve(C * 256 * sizeof(float));
     part_grad.reserve(enc_part_grad_floats((int)P) * sizeof(float));
     lab.reserve(P * 6 * sizeof(float));
     idx.reserve(P * sizeof(int));
@@ -258,12 +252,6 @@ struct ProposalImpl {
     e.loss_part = loss_part.as<float>();
     e.DZ = DZ.as<float>();
     e.DG = DG.as<float>();
-    e.XA = XA.as<float>();
-    e.H1A = H1A.as<float>();
-    e.DA1 = DA1.as<float>();
-    e.H2A = H2A.as<float>();
-    e.DA2 = DA2.as<float>();
-    e.DF = DF.as<float>();
     e.part_grad = part_grad.as<float>();
     e.G = G.as<float>();
     return e;

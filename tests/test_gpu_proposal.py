@@ -74,6 +74,28 @@ def test_gradient_matches_oracle(lcr):
         assert err <= tol, (name, err)
 
 
+@pytest.mark.parametrize("B,n", [(1, 1), (3, 17), (65, 33)])
+def test_gradient_sizes_match_oracle(lcr, B, n):
+    """Batches at the edges of the backward's blocks: one cloud per group and fewer
+    clouds than groups, more clouds than groups (130 against 128), one point per
+    cloud, row counts that are no multiple of the head gradients' 16 and 4 rows.
+    Same bars as above, for the same reasons."""
+    rng = np.random.default_rng(100 * B + n)
+    w = init_weights(rng)
+    src = rng.normal(size=(B, n, 3)).astype(np.float32)
+    tgt = rng.normal(size=(B, n, 3)).astype(np.float32)
+    lab = rng.normal(size=(B, 6)).astype(np.float32)
+    print_case(test="proposal_grad_sizes", B=B, n=n)
+    loss, g = lcr.Proposal(w).loss_grad(src, tgt, lab)
+    rloss, rg = oracle.enc_loss_grad(w.astype(np.float64), src, tgt, lab, quantize=True)
+    assert abs(loss - rloss) <= 1e-2 * max(1.0, rloss)
+    gb, rb = blocks(g.astype(np.float64)), blocks(rg)
+    for name in rb:
+        err = np.linalg.norm(gb[name] - rb[name]) / max(np.linalg.norm(rb[name]), 1e-12)
+        tol = 1e-3 if name in ("Hw1", "hb1", "Hw2", "hb2") else 3e-2
+        assert err <= tol, (name, err)
+
+
 def test_training_reduces_loss(lcr):
     """A small regression task (recover a random rotation's axis-angle from a cloud
     and its rotated copy): the device's Adam steps lower the loss."""
