@@ -7,14 +7,18 @@
 // on BF16 MFMA (v_mfma_f32_16x16x32_bf16) with FP32 accumulation, from BF16 copies
 // of W2/W3 and BF16 activations h1/h2.
 //
-// Forward (k_enc_points): one block per kRows (128) points of one cloud.  Layer 1
-// writes h1 (bf16) to LDS; each of the 4 waves computes a 32-column slab of layer
-// 2 for all rows (its B fragments stay in registers) and writes h2 (bf16) to LDS;
-// each wave then computes a 64-column slab of layer 3 and folds bias, ReLU and
-// the max-pool (with the lowest point index on ties) into registers, so only 256
-// (max, argmax) pairs per block leave the chip.  At 128 rows a block holds 53 KB
-// of LDS and two or three blocks share a CU, so one block's MFMA work overlaps
-// another's epilogues; at 256 rows (106 KB) a CU held one.
+// Forward (k_enc_points): one block per cloud and up to kMaxPasses passes of kRows
+// (128) points.  Layer 1 writes h1 (bf16) to LDS; each of the 4 waves computes 32
+// channels of layer 2 for all rows (its weight fragments stay in registers) and
+// writes h2 (bf16) to LDS, four channels per store; each wave then computes 64
+// channels of layer 3 and folds bias, ReLU and the max-pool (with the lowest point
+// index on ties) into registers, so only 256 (max, argmax) pairs per block leave
+// the chip.  At 128 rows a block holds 53 KB of LDS and three blocks share a CU, so
+// one block's MFMA work overlaps another's vector work.  Bound by the vector
+// instructions around the MFMAs (per value of layer 3: bias, compare, select, max).
+// 256 pairs x 8192 points: 682 -> 342 us (1.01 PFLOP/s; a large bf16 matrix product
+// reaches 1.18 here) from one pass per block, weights loaded each time, two-byte
+// stores of h2 and a bounds test per value.
 //
 // Backward: the max-pool sends each channel's gradient to one point, so the
 // per-point layers only need the <= 256 argmax rows per cloud (k_enc_grad
@@ -22,6 +26,8 @@
 // registers).  Every sum is deterministic (fixed-order partials).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "lcr_kernels.hpp"
 
@@ -33,7 +39,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kRows = 128;      // points per forward block (two blocks' LDS fit a CU)
+constexpr int kRows = 128;      // points per forward pass (three blocks' LDS fit a CU)
+constexpr int kMaxPasses = 8;   // passes per forward block at most
 constexpr int kH1S = 64 + 8;    // LDS row strides (bf16), padded
 constexpr int kH2S = 128 + 8;
 
@@ -41,127 +48,131 @@ __device__ __forceinline__ float relu(float v) { return v > 0.f ? v : 0.f; }
 
 // ------------------------------------------------------------------ forward
 
-__global__ void __launch_bounds__(256)
-k_enc_points(const float4* __restrict__ X, int npts, const float* __restrict__ W,
+// A block's points per pass; it runs `iters` passes over consecutive points, so the
+// weight fragments are loaded once and one (max, argmax) pair per channel leaves
+// per kRows * iters points.
+__global__ void __launch_bounds__(256, 3)
+k_enc_points(const float4* __restrict__ X, int npts, int iters, const float* __restrict__ W,
              const __bf16* __restrict__ W2t, const __bf16* __restrict__ W3t,
              float* __restrict__ part_max, int* __restrict__ part_arg) {
   __shared__ __attribute__((aligned(16))) __bf16 H1[kRows * kH1S];
   __shared__ __attribute__((aligned(16))) __bf16 H2[kRows * kH2S];
+  static_assert(kRows == 128, "row and argmax arithmetic below");
   const int cloud = blockIdx.y, chunk = blockIdx.x, nchunks = gridDim.x;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int p0 = chunk * kRows;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int l16 = lane & 15, q = lane >> 4, kq = q * 8;  // fragment row/col and k offset
   const float* W1 = W + kEncW1;
   const float* b1 = W + kEncB1;
-  const float* b2 = W + kEncB2;
-  const float* b3 = W + kEncB3;
-  // layer 1 (FP32), kL1Threads threads per point, each a slice of the 64 outputs
-  {
-    constexpr int kL1Threads = 256 / kRows, kL1Cols = 64 / kL1Threads;
-    const int row = t % kRows, j0 = (t / kRows) * kL1Cols;
-    const int p = p0 + row;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    const bool ok = p < npts;
-    if (ok) x = X[(int64_t)cloud * npts + p];
-#pragma unroll 8
-    for (int jj = 0; jj < kL1Cols; ++jj) {
-      const int j = j0 + jj;
-      float a = b1[j];
-      a = fmaf(x.x, W1[j], a);
-      a = fmaf(x.y, W1[64 + j], a);
-      a = fmaf(x.z, W1[128 + j], a);
-      H1[row * kH1S + j] = (__bf16)(ok ? relu(a) : 0.f);
-    }
+  const int first = chunk * iters * kRows;
+  const float4* Xc = X + (int64_t)cloud * npts;
+  bf16x8 w2[2][2], w3[4][4];
+  f32x4 b2[2];
+  float b3[4], best[4];
+  int bidx[4];
+#pragma unroll
+  for (int jt = 0; jt < 2; ++jt) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      w2[jt][ks] = *(const bf16x8*)(W2t + (32 * w + 16 * jt + l16) * 64 + 32 * ks + kq);
+    b2[jt] = *(const f32x4*)(W + kEncB2 + 32 * w + 16 * jt + 4 * q);
   }
-  __syncthreads();
-  const int r16 = lane & 15, kq = (lane >> 4) * 8;  // fragment row/col and k offset
-  // layer 2: wave w -> columns [32w, 32w + 32)
-  {
-    bf16x8 bf[2][2];
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
+  for (int ct = 0; ct < 4; ++ct) {
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        bf[ct][ks] = *(const bf16x8*)(W2t + (32 * w + 16 * ct + r16) * 64 + 32 * ks + kq);
-    float bias[2][1];
+    for (int ks = 0; ks < 4; ++ks)
+      w3[ct][ks] = *(const bf16x8*)(W3t + (64 * w + 16 * ct + l16) * 128 + 32 * ks + kq);
+    b3[ct] = W[kEncB3 + 64 * w + 16 * ct + l16];
+    // a maximum of at most 0 pools to 0 (ReLU) at no point, so only v > 0 matters
+    best[ct] = 0.f;
+    bidx[ct] = -1;
+  }
+  // points past the end repeat the last one: a repeat never beats its original,
+  // which has the lower index
+  const int row = t & (kRows - 1), j0 = (w >> 1) * 32;
+  float4 x = Xc[min(first + row, npts - 1)];
+  for (int it = 0; it < iters && first + it * kRows < npts; ++it) {
+    // layer 1 (FP32), two threads per point, 32 outputs each
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) bias[ct][0] = b2[32 * w + 16 * ct + r16];
+    for (int g = 0; g < 4; ++g) {
+      bf16x8 h;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int j = j0 + 8 * g + u;
+        float a = b1[j];
+        a = fmaf(x.x, W1[j], a);
+        a = fmaf(x.y, W1[64 + j], a);
+        a = fmaf(x.z, W1[128 + j], a);
+        h[u] = (__bf16)fmaxf(a, 0.f);
+      }
+      *(bf16x8*)(H1 + row * kH1S + j0 + 8 * g) = h;
+    }
+    x = Xc[min(first + (it + 1) * kRows + row, npts - 1)];  // the next pass's point
+    __syncthreads();
+    // layer 2, transposed: wave w -> channels [32w, 32w + 32), a lane holds four
+    // consecutive channels of one point and writes them together
+#pragma unroll 2
     for (int rt = 0; rt < kRows / 16; ++rt) {
       f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const bf16x8 af = *(const bf16x8*)(H1 + (16 * rt + r16) * kH1S + 32 * ks + kq);
+        const bf16x8 hf = *(const bf16x8*)(H1 + (16 * rt + l16) * kH1S + 32 * ks + kq);
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bf[ct][ks], acc[ct], 0, 0, 0);
+        for (int jt = 0; jt < 2; ++jt)
+          acc[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w2[jt][ks], hf, acc[jt], 0, 0, 0);
       }
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct)
+      for (int jt = 0; jt < 2; ++jt) {
+        bf16x4 h;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = 16 * rt + (lane >> 4) * 4 + e;
-          const int col = 32 * w + 16 * ct + r16;
-          H2[row * kH2S + col] = (__bf16)relu(acc[ct][e] + bias[ct][0]);
-        }
+        for (int e = 0; e < 4; ++e) h[e] = (__bf16)fmaxf(acc[jt][e] + b2[jt][e], 0.f);
+        *(bf16x4*)(H2 + (16 * rt + l16) * kH2S + 32 * w + 16 * jt + 4 * q) = h;
+      }
     }
-  }
-  __syncthreads();
-  // layer 3 + bias + ReLU + max-pool: wave w -> columns [64w, 64w + 64)
-  {
-    bf16x8 bf[4][4];
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-        bf[ct][ks] = *(const bf16x8*)(W3t + (64 * w + 16 * ct + r16) * 128 + 32 * ks + kq);
-    float bias[4], best[4];
-    int brow[4];
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-      bias[ct] = b3[64 * w + 16 * ct + r16];
-      best[ct] = -1.f;
-      brow[ct] = 0x7fffffff;
-    }
-    const int valid = min(kRows, npts - p0);
+    __syncthreads();
+    // layer 3 + bias + ReLU + max-pool: wave w -> channels [64w, 64w + 64)
+#pragma unroll 2
     for (int rt = 0; rt < kRows / 16; ++rt) {
       f32x4 acc[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f},
                       {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const bf16x8 af = *(const bf16x8*)(H2 + (16 * rt + r16) * kH2S + 32 * ks + kq);
+        const bf16x8 af = *(const bf16x8*)(H2 + (16 * rt + l16) * kH2S + 32 * ks + kq);
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct)
-          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bf[ct][ks], acc[ct], 0, 0, 0);
+          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, w3[ct][ks], acc[ct], 0, 0, 0);
       }
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct)
+      for (int e = 0; e < 4; ++e) {
+        const int idx = (it * (kRows / 16) + rt) * 4 + e;  // wave-uniform
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = 16 * rt + (lane >> 4) * 4 + e;
-          const float v = relu(acc[ct][e] + bias[ct]);
-          if (row < valid && v > best[ct]) {
-            best[ct] = v;
-            brow[ct] = row;
-          }
+        for (int ct = 0; ct < 4; ++ct) {
+          const float v = acc[ct][e] + b3[ct];
+          bidx[ct] = v > best[ct] ? idx : bidx[ct];
+          best[ct] = fmaxf(best[ct], v);
         }
+      }
     }
-    // combine the 4 lane groups holding the same column (lanes l, l^16, l^32, l^48)
+  }
+  // combine the 4 lane groups holding the same column (lanes l, l^16, l^32, l^48)
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
+  for (int ct = 0; ct < 4; ++ct) {
+    // point = 128 * pass + 16 * rt + 4 * q + e
+    int p = bidx[ct] < 0 ? 0x7fffffff
+                         : first + (bidx[ct] >> 5) * kRows + ((bidx[ct] >> 2) & 7) * 16 + 4 * q +
+                               (bidx[ct] & 3);
 #pragma unroll
-      for (int off = 16; off <= 32; off <<= 1) {
-        const float ov = __shfl_xor(best[ct], off, 64);
-        const int orow = __shfl_xor(brow[ct], off, 64);
-        if (ov > best[ct] || (ov == best[ct] && orow < brow[ct])) {
-          best[ct] = ov;
-          brow[ct] = orow;
-        }
+    for (int off = 16; off <= 32; off <<= 1) {
+      const float ov = __shfl_xor(best[ct], off, 64);
+      const int op = __shfl_xor(p, off, 64);
+      if (ov > best[ct] || (ov == best[ct] && op < p)) {
+        best[ct] = ov;
+        p = op;
       }
-      if (lane < 16) {
-        const int col = 64 * w + 16 * ct + lane;
-        const int64_t o = ((int64_t)cloud * nchunks + chunk) * 256 + col;
-        part_max[o] = best[ct];
-        part_arg[o] = brow[ct] == 0x7fffffff ? 0x7fffffff : p0 + brow[ct];
-      }
+    }
+    if (lane < 16) {
+      const int64_t o = ((int64_t)cloud * nchunks + chunk) * 256 + 64 * w + 16 * ct + lane;
+      part_max[o] = best[ct];
+      part_arg[o] = p;
     }
   }
 }
@@ -539,9 +550,14 @@ void launch_enc_bf16_weights(const float* W, __bf16* W2t, __bf16* W3t, hipStream
 void launch_enc_forward(const EncBuffers& e, int npairs, int npts, const float* labels,
                         hipStream_t s) {
   const int nclouds = 2 * npairs;
-  const int nchunks = enc_forward_chunks(npts);
-  hipLaunchKernelGGL(k_enc_points, dim3(nchunks, nclouds), dim3(256), 0, s, e.X, npts, e.W, e.W2t,
-                     e.W3t, e.part_max, e.part_arg);
+  // Passes per block: up to kMaxPasses, as long as the blocks still fill the chip
+  // four times over at three per CU (more passes load the weights less often and
+  // leave fewer partials to fold; fewer blocks leave an emptier last round).
+  const int64_t units = (int64_t)enc_forward_chunks(npts) * nclouds;
+  const int iters = (int)std::min<int64_t>(std::max<int64_t>(units / (256 * 3 * 4), 1), kMaxPasses);
+  const int nchunks = (enc_forward_chunks(npts) + iters - 1) / iters;
+  hipLaunchKernelGGL(k_enc_points, dim3(nchunks, nclouds), dim3(256), 0, s, e.X, npts, iters, e.W,
+                     e.W2t, e.W3t, e.part_max, e.part_arg);
   hipLaunchKernelGGL(k_enc_pool, dim3(nclouds), dim3(256), 0, s, e.part_max, e.part_arg, nchunks,
                      e.F, e.ARG);
   hipLaunchKernelGGL(k_enc_head, dim3(npairs), dim3(256), 0, s, e.F, e.W, labels, npairs, e.Z,

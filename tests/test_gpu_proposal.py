@@ -54,6 +54,21 @@ def test_forward_matches_oracle(lcr, npts):
         assert np.max(np.abs(out[b] - ref)) <= 1e-2 * max(1.0, np.max(np.abs(ref))), (out[b], ref)
 
 
+@pytest.mark.parametrize("B,npts", [(60, 8000), (200, 8100)])
+def test_forward_passes_per_block_equal_one(lcr, B, npts):
+    """Large batches run several 128-point passes per block (two at 60 pairs of 8000
+    points, eight at 200 of 8100, the last block and the last pass of a cloud
+    ragged); a pair alone runs one.  The same sums and maxima: bitwise equal."""
+    rng = np.random.default_rng(npts)
+    p = lcr.Proposal(init_weights(rng))
+    src = rng.normal(size=(B, npts, 3)).astype(np.float32)
+    tgt = rng.normal(size=(B, npts, 3)).astype(np.float32)
+    print_case(test="proposal_forward_passes", B=B, npts=npts)
+    out = p.forward(src, tgt)
+    for b in (0, B // 2, B - 1):
+        np.testing.assert_array_equal(out[b], p.forward(src[b:b + 1], tgt[b:b + 1])[0])
+
+
 def test_gradient_matches_oracle(lcr):
     rng = np.random.default_rng(7)
     w = init_weights(rng)
