@@ -46,13 +46,22 @@ constexpr int kH2S = 128 + 8;
 
 __device__ __forceinline__ float relu(float v) { return v > 0.f ? v : 0.f; }
 
+// The points of the batch's cloud c: clouds lie in X in batch order, or (sel: the
+// pairs of a resident set that make up the batch) at their pair's place in the set.
+__device__ __forceinline__ const float4* cloud_points(const float4* X, const int* sel, int cloud,
+                                                      int npts) {
+  const int64_t c = sel ? 2 * (int64_t)sel[cloud >> 1] + (cloud & 1) : cloud;
+  return X + c * npts;
+}
+
 // ------------------------------------------------------------------ forward
 
 // A block's points per pass; it runs `iters` passes over consecutive points, so the
 // weight fragments are loaded once and one (max, argmax) pair per channel leaves
 // per kRows * iters points.
 __global__ void __launch_bounds__(256, 3)
-k_enc_points(const float4* __restrict__ X, int npts, int iters, const float* __restrict__ W,
+k_enc_points(const float4* __restrict__ X, const int* __restrict__ sel, int npts, int iters,
+             const float* __restrict__ W,
              const __bf16* __restrict__ W2t, const __bf16* __restrict__ W3t,
              float* __restrict__ part_max, int* __restrict__ part_arg) {
   __shared__ __attribute__((aligned(16))) __bf16 H1[kRows * kH1S];
@@ -64,7 +73,7 @@ k_enc_points(const float4* __restrict__ X, int npts, int iters, const float* __r
   const float* W1 = W + kEncW1;
   const float* b1 = W + kEncB1;
   const int first = chunk * iters * kRows;
-  const float4* Xc = X + (int64_t)cloud * npts;
+  const float4* Xc = cloud_points(X, sel, cloud, npts);
   bf16x8 w2[2][2], w3[4][4];
   f32x4 b2[2];
   float b3[4], best[4];
@@ -195,63 +204,95 @@ __global__ void k_enc_pool(const float* __restrict__ part_max, const int* __rest
   ARG[cloud * 256 + c] = arg == 0x7fffffff ? 0 : arg;
 }
 
-// head: one block (256 threads) per pair
+// head: one block (256 threads) per pair; with labels (of pair sel[b] when given)
+// also the loss and its gradient down to the hidden layer: dOut, dZ[j] = relu'(z)
+// sum_o dOut[o] Hw2[j][o].  Each sum is one fmaf chain in order, its weights loaded
+// 32 rows ahead (or from LDS): latency-bound, 256 pairs 26 -> 14 us with dZ.
 __global__ void __launch_bounds__(256)
 k_enc_head(const float* __restrict__ F, const float* __restrict__ W, const float* __restrict__ labels,
-           int npairs, float* __restrict__ Z, float* __restrict__ OUT, float* __restrict__ DOUT,
-           float* __restrict__ loss_part) {
+           const int* __restrict__ sel, int npairs, float* __restrict__ Z, float* __restrict__ OUT,
+           float* __restrict__ DOUT, float* __restrict__ loss_part, float* __restrict__ DZ) {
   __shared__ float g[512];
   __shared__ float z[256];
+  __shared__ float hw2[1536];
+  __shared__ float dout[6];
+  constexpr int kAhead = 32;
   const int b = blockIdx.x, t = threadIdx.x;
+  const float* Hw1 = W + kEncHw1 + t;
+  float next[kAhead];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) next[u] = Hw1[u * 256];
   g[t] = F[(2 * b) * 256 + t];
   g[256 + t] = F[(2 * b + 1) * 256 + t];
+#pragma unroll
+  for (int u = 0; u < 6; ++u) hw2[u * 256 + t] = W[kEncHw2 + u * 256 + t];
   __syncthreads();
-  const float* Hw1 = W + kEncHw1;
   float s = W[kEncHb1 + t];
-  for (int i = 0; i < 512; ++i) s = fmaf(g[i], Hw1[i * 256 + t], s);
+  for (int i = 0; i < 512; i += kAhead) {
+    float cur[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) cur[u] = next[u];
+    const int n = min(i + kAhead, 512 - kAhead);  // past the end: the last rows again, unused
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) next[u] = Hw1[(n + u) * 256];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) s = fmaf(g[i + u], cur[u], s);
+  }
   z[t] = relu(s);
   Z[b * 256 + t] = z[t];
   __syncthreads();
   if (t < 6) {
-    const float* Hw2 = W + kEncHw2;
     float o = W[kEncHb2 + t];
-    for (int i = 0; i < 256; ++i) o = fmaf(z[i], Hw2[i * 6 + t], o);
+#pragma unroll 16
+    for (int i = 0; i < 256; ++i) o = fmaf(z[i], hw2[i * 6 + t], o);
     OUT[b * 6 + t] = o;
     if (labels) {
-      const float d = o - labels[b * 6 + t];
-      DOUT[b * 6 + t] = 2.f * d / (float)npairs;
+      const float d = o - labels[(int64_t)(sel ? sel[b] : b) * 6 + t];
+      dout[t] = 2.f * d / (float)npairs;
+      DOUT[b * 6 + t] = dout[t];
       loss_part[b * 6 + t] = d * d / (float)npairs;
     }
   }
+  if (!labels) return;
+  __syncthreads();
+  float dz = 0.f;
+#pragma unroll
+  for (int o = 0; o < 6; ++o) dz = fmaf(dout[o], hw2[t * 6 + o], dz);
+  DZ[b * 256 + t] = z[t] > 0.f ? dz : 0.f;
 }
 
-// dZ[b][j] = relu'(z) * sum_o dOut[b][o] Hw2[j][o];  dG[b][i] = sum_j dZ[b][j] Hw1[i][j]
-__global__ void k_enc_head_back(const float* __restrict__ Z, const float* __restrict__ DOUT,
-                                const float* __restrict__ W, float* __restrict__ DZ,
-                                float* __restrict__ DG) {
-  __shared__ float dz[256];
-  const int b = blockIdx.x, t = threadIdx.x;
-  const float* Hw2 = W + kEncHw2;
-  float s = 0.f;
+// dG[b][i] = sum_j dZ[b][j] Hw1[i][j] on FP32 matrix instructions: a block computes
+// 16 pairs x 16 features, a wavefront 64 of the 256 terms (16-byte loads along
+// them; component c of the four feeds instruction c on both sides), the four
+// tiles added in wavefront order.
+__global__ void __launch_bounds__(256)
+k_enc_head_back(const float* __restrict__ DZ, const float* __restrict__ W, int npairs,
+                float* __restrict__ DG) {
+  __shared__ float red[4][256];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, l16 = lane & 15, q = lane >> 4;
+  const int b = blockIdx.x * 16 + l16, i = blockIdx.y * 16 + l16;
+  const float4* pa = reinterpret_cast<const float4*>(DZ + (int64_t)min(b, npairs - 1) * 256 + 64 * w + 4 * q);
+  const float4* pb = reinterpret_cast<const float4*>(W + kEncHw1 + i * 256 + 64 * w + 4 * q);
+  float4 a[4], v[4];
 #pragma unroll
-  for (int o = 0; o < 6; ++o) s = fmaf(DOUT[b * 6 + o], Hw2[t * 6 + o], s);
-  dz[t] = Z[b * 256 + t] > 0.f ? s : 0.f;
-  DZ[b * 256 + t] = dz[t];
-  __syncthreads();
-  const float* Hw1 = W + kEncHw1;
-  for (int i = t; i < 512; i += 256) {
-    float a = 0.f;
-    const float4* row = reinterpret_cast<const float4*>(Hw1 + i * 256);
-#pragma unroll 8
-    for (int j = 0; j < 64; ++j) {  // eight 16-byte loads in flight, one fmaf chain
-      const float4 v = row[j];
-      a = fmaf(dz[4 * j], v.x, a);
-      a = fmaf(dz[4 * j + 1], v.y, a);
-      a = fmaf(dz[4 * j + 2], v.z, a);
-      a = fmaf(dz[4 * j + 3], v.w, a);
-    }
-    DG[b * 512 + i] = a;
+  for (int u = 0; u < 4; ++u) {
+    a[u] = pa[4 * u];
+    v[u] = pb[4 * u];
   }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, v[u].x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, v[u].y, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].z, v[u].z, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].w, v[u].w, acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) red[w][(4 * q + e) * 16 + l16] = acc[e];
+  __syncthreads();
+  const int ob = blockIdx.x * 16 + t / 16;
+  if (ob < npairs)
+    DG[(int64_t)ob * 512 + blockIdx.y * 16 + t % 16] = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
 }
 
 // C[i][j] = sum_{r < R} A[r * lda + i] * B[r * ldb + j], and the column sums of B
@@ -324,7 +365,8 @@ constexpr int kGradGroups = 128;                   // cloud groups: 512 blocks, 
 constexpr int kGradMS = 128 + 8;                   // LDS row stride of m (bf16)
 
 __global__ void __launch_bounds__(256, 2)
-k_enc_grad(const float4* __restrict__ X, int npts, const float* __restrict__ F,
+k_enc_grad(const float4* __restrict__ X, const int* __restrict__ sel, int npts,
+           const float* __restrict__ F,
            const int* __restrict__ ARG, const float* __restrict__ DG, const float* __restrict__ W,
            const __bf16* __restrict__ W2t, const __bf16* __restrict__ W3t, int nclouds,
            float* __restrict__ part_w, float* __restrict__ part_w3) {
@@ -365,7 +407,7 @@ k_enc_grad(const float4* __restrict__ X, int npts, const float* __restrict__ F,
     if (t < 64) {
       const int c = cloud * 256 + c0 + t;
       const float df = F[c] > 0.f ? DG[c] : 0.f;
-      xs[t] = X[(int64_t)cloud * npts + ARG[c]];
+      xs[t] = cloud_points(X, sel, cloud, npts)[ARG[c]];
       dfs[t] = df;
       accb3 += df;
     }
@@ -507,10 +549,26 @@ k_enc_grad_fold(const float* __restrict__ part_w, const float* __restrict__ part
   G[o] = s;
 }
 
-// Adam (FP32 master weights), then refresh the BF16 transposed copies of W2, W3
-__global__ void k_adam(float* __restrict__ W, const float* __restrict__ G, float* __restrict__ M,
-                       float* __restrict__ V, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
+// Adam (FP32 master weights, and the BF16 transposed copies of W2 and W3 with them);
+// the block past the parameters sums the step's loss terms in a fixed order.
+__global__ void __launch_bounds__(256)
+k_adam(float* __restrict__ W, const float* __restrict__ G, float* __restrict__ M,
+       float* __restrict__ V, int n, float lr, float b1, float b2, float eps, float c1, float c2,
+       __bf16* __restrict__ W2t, __bf16* __restrict__ W3t, const float* __restrict__ loss_part,
+       int nloss, float* __restrict__ loss) {
+  if (blockIdx.x == gridDim.x - 1) {
+    __shared__ float s[256];
+    float a = 0.f;
+    for (int i = threadIdx.x; i < nloss; i += 256) a += loss_part[i];
+    s[threadIdx.x] = a;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+      if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss = s[0];
+    return;
+  }
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float g = G[i];
@@ -518,7 +576,15 @@ __global__ void k_adam(float* __restrict__ W, const float* __restrict__ G, float
   const float v = b2 * V[i] + (1.f - b2) * g * g;
   M[i] = m;
   V[i] = v;
-  W[i] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
+  const float x = W[i] - lr * (m / c1) / (sqrtf(v / c2) + eps);
+  W[i] = x;
+  if (i >= kEncW2 && i < kEncB2) {
+    const int k = i - kEncW2;  // W2[i][j] -> W2t[j][i]
+    W2t[(k & 127) * 64 + (k >> 7)] = (__bf16)x;
+  } else if (i >= kEncW3 && i < kEncB3) {
+    const int k = i - kEncW3;  // W3[k][c] -> W3t[c][k]
+    W3t[(k & 255) * 128 + (k >> 8)] = (__bf16)x;
+  }
 }
 
 __global__ void k_enc_bf16_weights(const float* __restrict__ W, __bf16* __restrict__ W2t,
@@ -556,18 +622,18 @@ void launch_enc_forward(const EncBuffers& e, int npairs, int npts, const float* 
   const int64_t units = (int64_t)enc_forward_chunks(npts) * nclouds;
   const int iters = (int)std::min<int64_t>(std::max<int64_t>(units / (256 * 3 * 4), 1), kMaxPasses);
   const int nchunks = (enc_forward_chunks(npts) + iters - 1) / iters;
-  hipLaunchKernelGGL(k_enc_points, dim3(nchunks, nclouds), dim3(256), 0, s, e.X, npts, iters, e.W,
-                     e.W2t, e.W3t, e.part_max, e.part_arg);
+  hipLaunchKernelGGL(k_enc_points, dim3(nchunks, nclouds), dim3(256), 0, s, e.X, e.sel, npts, iters,
+                     e.W, e.W2t, e.W3t, e.part_max, e.part_arg);
   hipLaunchKernelGGL(k_enc_pool, dim3(nclouds), dim3(256), 0, s, e.part_max, e.part_arg, nchunks,
                      e.F, e.ARG);
-  hipLaunchKernelGGL(k_enc_head, dim3(npairs), dim3(256), 0, s, e.F, e.W, labels, npairs, e.Z,
-                     e.OUT, e.DOUT, e.loss_part);
+  hipLaunchKernelGGL(k_enc_head, dim3(npairs), dim3(256), 0, s, e.F, e.W, labels, e.sel, npairs,
+                     e.Z, e.OUT, e.DOUT, e.loss_part, e.DZ);
 }
 
 void launch_enc_backward(const EncBuffers& e, int npairs, int npts, hipStream_t s) {
   const int nclouds = 2 * npairs;
   float* G = e.G;
-  hipLaunchKernelGGL(k_enc_head_back, dim3(npairs), dim3(256), 0, s, e.Z, e.DOUT, e.W, e.DZ, e.DG);
+  hipLaunchKernelGGL(k_enc_head_back, dim3(nb(npairs, 16), 32), dim3(256), 0, s, e.DZ, e.W, npairs, e.DG);
   // head weights: dHw2 = Z^T dOut, dHw1 = G^T dZ (G = pooled features)
   hipLaunchKernelGGL(k_outer_mfma, dim3(17, 1), dim3(256), 0, s, e.Z, 256, e.DOUT, 6, npairs, 256, 6,
                      G + kEncHw2, G + kEncHb2);
@@ -576,18 +642,18 @@ void launch_enc_backward(const EncBuffers& e, int npairs, int npts, hipStream_t 
   // per-point layers
   const int groups = enc_grad_groups(nclouds);
   float* part_w3 = e.part_grad + (int64_t)4 * groups * kGradW;
-  hipLaunchKernelGGL(k_enc_grad, dim3(4, groups), dim3(256), 0, s, e.X, npts, e.F, e.ARG, e.DG, e.W,
-                     e.W2t, e.W3t, nclouds, e.part_grad, part_w3);
+  hipLaunchKernelGGL(k_enc_grad, dim3(4, groups), dim3(256), 0, s, e.X, e.sel, npts, e.F, e.ARG, e.DG,
+                     e.W, e.W2t, e.W3t, nclouds, e.part_grad, part_w3);
   hipLaunchKernelGGL(k_enc_grad_fold, dim3((kGradW + kGradW3) / 64), dim3(64 * kFoldSlices), 0, s,
                      e.part_grad, part_w3, groups, G);
 }
 
-void launch_adam(float* W, const float* G, float* M, float* V, int n, float lr, int step,
+void launch_adam(const EncBuffers& e, float* M, float* V, int npairs, float lr, int step, float* loss,
                  hipStream_t s) {
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-  hipLaunchKernelGGL(k_adam, dim3(nb(n, 256)), dim3(256), 0, s, W, G, M, V, n, lr, b1, b2, eps, c1,
-                     c2);
+  hipLaunchKernelGGL(k_adam, dim3(nb(kEncNParam, 256) + 1), dim3(256), 0, s, e.W, e.G, M, V, kEncNParam,
+                     lr, b1, b2, eps, c1, c2, e.W2t, e.W3t, e.loss_part, npairs * 6, loss);
 }
 
 int64_t enc_part_grad_floats(int npairs) {

@@ -209,6 +209,8 @@ void launch_sor_distances(const GridDesc* grids, const int* cell_start, const fl
 // ---- K9 pose-proposal network (encoder.hip)
 struct EncBuffers {
   const float4* X;       // 2 * npairs clouds of npts normalised points (src, tgt, ...)
+  const int* sel;        // null, or per pair of the batch its place in a resident set (X
+                         // and the labels then hold the set)
   float* W;              // FP32 master weights (kEncNParam)
   __bf16* W2t;           // bf16 W2 transposed [128][64]
   __bf16* W3t;           // bf16 W3 transposed [256][128]
@@ -231,7 +233,8 @@ int enc_forward_chunks(int npts);
 void launch_enc_forward(const EncBuffers& e, int npairs, int npts, const float* labels,
                         hipStream_t s);
 void launch_enc_backward(const EncBuffers& e, int npairs, int npts, hipStream_t s);
-void launch_adam(float* W, const float* G, float* M, float* V, int n, float lr, int step,
+// One Adam step of every weight (and the BF16 copies) and the step's loss.
+void launch_adam(const EncBuffers& e, float* M, float* V, int npairs, float lr, int step, float* loss,
                  hipStream_t s);
 int64_t enc_part_grad_floats(int npairs);
 // training pairs generated on the device (synth.hip)

@@ -20,32 +20,6 @@ namespace {
 
 // ---- device helpers local to the proposal
 
-__global__ void k_gather_batch(const float4* __restrict__ ds, const float* __restrict__ ds_lab,
-                               const int* __restrict__ idx, int npts, int batch,
-                               float4* __restrict__ X, float* __restrict__ lab) {
-  const int64_t per_pair = 2 * (int64_t)npts;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < (int64_t)batch * per_pair) {
-    const int b = (int)(i / per_pair);
-    const int64_t o = i % per_pair;
-    X[i] = ds[(int64_t)idx[b] * per_pair + o];
-  }
-  if (i < (int64_t)batch * 6) lab[i] = ds_lab[(int64_t)idx[i / 6] * 6 + i % 6];
-}
-
-__global__ void k_sum_loss(const float* __restrict__ part, int n, float* __restrict__ out) {
-  __shared__ float s[256];
-  float a = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) a += part[i];
-  s[threadIdx.x] = a;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = s[0];
-}
-
 // Inputs of the network for every pair of a cycle: n_out points subsampled evenly
 // from each raw cloud, the source moved by the pair's seed T0, both normalised by
 // the target sample's centroid and RMS radius.  One block per pair; the sums are
@@ -188,8 +162,7 @@ struct ProposalImpl {
   int cap_pairs = 0, cap_pts = 0;
   int step = 0;
   DevBuf W, M, V, G, W2t, W3t;
-  DevBuf X, part_max, part_arg, F, ARG, Z, OUT, DOUT, loss_part, DZ, DG, part_grad, lab, idx, losses,
-      frame;
+  DevBuf X, part_max, part_arg, F, ARG, Z, OUT, DOUT, loss_part, DZ, DG, part_grad, lab, losses, frame;
   DevBuf ds_X, ds_lab;
   int ds_pairs = 0, ds_pts = 0;
   HostBuf h_io;
@@ -221,7 +194,6 @@ struct ProposalImpl {
     cap_pts = std::max(cap_pts, npts);
     const int64_t P = cap_pairs, C = 2 * P, N = cap_pts;
     const int64_t chunks = enc_forward_chunks((int)N);
-    X.reserve(C * N * sizeof(float4));
     part_max.reserve(C * chunks * 256 * sizeof(float));
     part_arg.reserve(C * chunks * 256 * sizeof(int));
     F.reserve(C * 256 * sizeof(float));
@@ -234,11 +206,15 @@ struct ProposalImpl {
     DG.reserve(P * 512 * sizeof(float));
     part_grad.reserve(enc_part_grad_floats((int)P) * sizeof(float));
     lab.reserve(P * 6 * sizeof(float));
-    idx.reserve(P * sizeof(int));
+  }
+  // the batch's own points (training and prediction read the resident set in place)
+  void reserve_points(int npairs, int npts) {
+    X.reserve((size_t)2 * npairs * npts * sizeof(float4));
   }
   EncBuffers bufs() const {
     EncBuffers e;
     e.X = X.as<float4>();
+    e.sel = nullptr;
     e.W = W.as<float>();
     e.W2t = W2t.as<__bf16>();
     e.W3t = W3t.as<__bf16>();
@@ -259,6 +235,7 @@ struct ProposalImpl {
   // host clouds (npairs * npts * 3 floats each) -> X as (src0, tgt0, src1, tgt1, ...)
   void upload_pairs(const float* src, const float* tgt, int npairs, int npts) {
     reserve(npairs, npts);
+    reserve_points(npairs, npts);
     const int64_t n = (int64_t)npairs * 2 * npts;
     h_io.reserve((size_t)n * sizeof(float4));
     float4* h = h_io.as<float4>();
@@ -279,6 +256,7 @@ struct ProposalImpl {
 void proposal_guesses(ProposalImpl& P, hipStream_t s, const CloudSet& cs, const int* d_src,
                       const int* d_tgt, int npairs, int npts, double* d_guess, int stride, int slot) {
   P.reserve(npairs, npts);
+  P.reserve_points(npairs, npts);
   P.frame.reserve((size_t)npairs * 4 * sizeof(float));
   hipLaunchKernelGGL(k_prop_prepare, dim3(npairs), dim3(kPrepThreads), 0, s, cs.d_raw.as<float4>(),
                      cs.d_cloud_off.as<int64_t>(), d_src, d_tgt, d_guess, stride, npts,
@@ -492,18 +470,13 @@ int lcr_proposal_predict(lcr_proposal* p, int32_t first, int32_t count, float* o
     for (int b0 = 0; b0 < count; b0 += chunk) {
       const int nb = std::min(chunk, count - b0);
       P.reserve(nb, P.ds_pts);
-      std::vector<int> ids(nb);
-      for (int i = 0; i < nb; ++i) ids[i] = first + b0 + i;
-      LCR_HIP(hipMemcpyAsync(P.idx.p, ids.data(), nb * sizeof(int), hipMemcpyHostToDevice, P.s));
-      const int64_t nx = (int64_t)nb * 2 * P.ds_pts;
-      hipLaunchKernelGGL(k_gather_batch, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, P.s,
-                         P.ds_X.as<float4>(), P.ds_lab.as<float>(), P.idx.as<int>(), P.ds_pts, nb,
-                         P.X.as<float4>(), P.lab.as<float>());
-      launch_enc_forward(P.bufs(), nb, P.ds_pts, nullptr, P.s);
+      EncBuffers e = P.bufs();
+      e.X = P.ds_X.as<float4>() + (int64_t)(first + b0) * 2 * P.ds_pts;
+      launch_enc_forward(e, nb, P.ds_pts, nullptr, P.s);
       LCR_HIP(hipMemcpyAsync(out + (int64_t)b0 * 6, P.OUT.p, (size_t)nb * 6 * 4, hipMemcpyDeviceToHost, P.s));
       if (labels)
-        LCR_HIP(hipMemcpyAsync(labels + (int64_t)b0 * 6, P.lab.p, (size_t)nb * 6 * 4,
-                               hipMemcpyDeviceToHost, P.s));
+        LCR_HIP(hipMemcpyAsync(labels + (int64_t)b0 * 6, P.ds_lab.as<float>() + (int64_t)(first + b0) * 6,
+                               (size_t)nb * 6 * 4, hipMemcpyDeviceToHost, P.s));
       LCR_HIP(hipStreamSynchronize(P.s));
     }
     return LCR_OK;
@@ -536,20 +509,14 @@ int lcr_proposal_train(lcr_proposal* p, int32_t steps, int32_t batch, float lr, 
     d_all.reserve(all.size() * sizeof(int));
     LCR_HIP(hipMemcpyAsync(d_all.p, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice,
                            P.s));
-    const EncBuffers e = P.bufs();
-    const int64_t nx = (int64_t)batch * 2 * P.ds_pts;
+    EncBuffers e = P.bufs();
+    e.X = P.ds_X.as<float4>();
     for (int st = 0; st < steps; ++st) {
-      hipLaunchKernelGGL(k_gather_batch, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, P.s,
-                         P.ds_X.as<float4>(), P.ds_lab.as<float>(), d_all.as<int>() + (int64_t)st * batch,
-                         P.ds_pts, batch, P.X.as<float4>(), P.lab.as<float>());
-      launch_enc_forward(e, batch, P.ds_pts, P.lab.as<float>(), P.s);
-      hipLaunchKernelGGL(k_sum_loss, dim3(1), dim3(256), 0, P.s, P.loss_part.as<float>(), batch * 6,
-                         P.losses.as<float>() + st);
+      e.sel = d_all.as<int>() + (int64_t)st * batch;
+      launch_enc_forward(e, batch, P.ds_pts, P.ds_lab.as<float>(), P.s);
       launch_enc_backward(e, batch, P.ds_pts, P.s);
       P.step += 1;
-      launch_adam(P.W.as<float>(), P.G.as<float>(), P.M.as<float>(), P.V.as<float>(), kEncNParam, lr,
-                  P.step, P.s);
-      launch_enc_bf16_weights(P.W.as<float>(), P.W2t.as<__bf16>(), P.W3t.as<__bf16>(), P.s);
+      launch_adam(e, P.M.as<float>(), P.V.as<float>(), batch, lr, P.step, P.losses.as<float>() + st, P.s);
     }
     if (losses)
       LCR_HIP(hipMemcpyAsync(losses, P.losses.p, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost,

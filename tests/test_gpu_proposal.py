@@ -111,6 +111,34 @@ def test_gradient_sizes_match_oracle(lcr, B, n):
         assert err <= tol, (name, err)
 
 
+@pytest.mark.parametrize("B,n", [(1, 5), (17, 130)])
+def test_training_step_equals_adam_on_the_batch_gradient(lcr, B, n):
+    """One step over a whole resident set (its pairs in a shuffled order, read in
+    place) moves every weight by Adam's first step, lr g / (|g| + eps), g the gradient
+    of the same pairs handed in.  Where |g| >= 1e-4 the step's sensitivity to g is at
+    most lr per unit, and the two gradients differ by the order of FP32 sums only."""
+    rng = np.random.default_rng(10 * B + n)
+    w = init_weights(rng)
+    src = rng.normal(size=(B, n, 3)).astype(np.float32)
+    tgt = rng.normal(size=(B, n, 3)).astype(np.float32)
+    lab = rng.normal(size=(B, 6)).astype(np.float32)
+    print_case(test="proposal_step", B=B, n=n)
+    loss, g = lcr.Proposal(w).loss_grad(src, tgt, lab)
+    p = lcr.Proposal(w)
+    p.dataset(src, tgt, lab)
+    lr = 1e-3
+    losses = p.train(1, B, lr=lr, seed=3)
+    assert abs(losses[0] - loss) <= 1e-5 * loss
+    big = np.abs(g) >= 1e-4
+    assert big.sum() > 1000
+    step = (w - p.get_weights())[big]
+    want = lr * g[big] / (np.abs(g[big]) + 1e-8)
+    assert np.max(np.abs(step - want)) <= 2e-3 * lr
+    out, got_lab = p.predict(0, B)
+    np.testing.assert_array_equal(got_lab, lab)
+    np.testing.assert_array_equal(out, p.forward(src, tgt))
+
+
 def test_training_reduces_loss(lcr):
     """A small regression task (recover a random rotation's axis-angle from a cloud
     and its rotated copy): the device's Adam steps lower the loss."""
