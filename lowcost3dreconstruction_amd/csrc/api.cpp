@@ -806,13 +806,12 @@ int lcr_outlier_removal(const float* xyz, int64_t n, int32_t mean_k, double stdd
     CloudSet cs;
     cs.upload(st.s, {xyz}, {nullptr}, {n}, 3 * sizeof(float));
     cs.build(st.s, std::max(2.5, 0.70 * sqrt((double)mean_k + 1.0)), nullptr, false);
-    DevBuf dist, fin, sums, nsel, defer, part, dstats, dkeep;
+    DevBuf dist, fin, sums, work, part, dstats, dkeep;
     dist.reserve((size_t)n * sizeof(float));
     fin.reserve((size_t)n);
     const size_t np = (size_t)std::max<int64_t>(cs.total_pts, 1);
     sums.reserve(np * sizeof(double));
-    nsel.reserve(np * sizeof(int));
-    defer.reserve((np + 1) * sizeof(int));
+    work.reserve((size_t)normals_work_ints((int64_t)np) * sizeof(int));
     part.reserve((size_t)sor_stat_blocks(n) * 3 * sizeof(double));
     dstats.reserve(3 * sizeof(double));
     dkeep.reserve((size_t)n);
@@ -820,7 +819,7 @@ int lcr_outlier_removal(const float* xyz, int64_t n, int32_t mean_k, double stdd
     LCR_HIP(hipMemsetAsync(fin.p, 0, (size_t)n, st.s));
     launch_sor_distances(cs.d_grids.as<GridDesc>(), cs.d_cell_start.as<int>(), cs.d_pts.as<float4>(),
                          cs.d_cloud_of_sorted.as<int>(), cs.d_cloud_off.as<int64_t>(), cs.total_pts,
-                         mean_k, sums.as<double>(), nsel.as<int>(), defer.as<int>(),
+                         mean_k, sums.as<double>(), work.as<int>(),
                          dist.as<float>(), fin.as<uint8_t>(), st.s);
     launch_sor_stats(dist.as<float>(), fin.as<uint8_t>(), n, stddev_mult, part.as<double>(),
                      dstats.as<double>(), dkeep.as<uint8_t>(), st.s);

@@ -156,15 +156,24 @@ k_sor_partials(const float* __restrict__ dist, const uint8_t* __restrict__ finit
   }
 }
 
-// one thread: fold the partials in block order; stats = mean, stddev, threshold
-__global__ void k_sor_stats(const double* __restrict__ part, int nparts, double mul,
-                            double* __restrict__ stats) {
-  double sum = 0.0, sq = 0.0, valid = 0.0;
-  for (int k = 0; k < nparts; ++k) {
-    sum += part[3 * k];
-    sq += part[3 * k + 1];
-    valid += part[3 * k + 2];
+// One block: fold the partials in a fixed order; stats = mean, stddev, threshold.
+// (One thread adding 391 partials took 50 us of a 100k-point call; this 4.5.)
+__global__ void __launch_bounds__(kSorThreads)
+k_sor_stats(const double* __restrict__ part, int nparts, double mul, double* __restrict__ stats) {
+  __shared__ double s[3][kSorThreads];
+  const int t = threadIdx.x;
+  double v[3] = {0.0, 0.0, 0.0};
+  for (int k = t; k < nparts; k += kSorThreads)
+    for (int a = 0; a < 3; ++a) v[a] += part[3 * k + a];
+  for (int a = 0; a < 3; ++a) s[a][t] = v[a];
+  __syncthreads();
+  for (int o = kSorThreads / 2; o > 0; o >>= 1) {
+    if (t < o)
+      for (int a = 0; a < 3; ++a) s[a][t] += s[a][t + o];
+    __syncthreads();
   }
+  if (t != 0) return;
+  const double sum = s[0][0], sq = s[1][0], valid = s[2][0];
   const double mean = valid > 0.0 ? sum / valid : 0.0;
   const double var = valid > 1.0 ? (sq - sum * sum / valid) / (valid - 1.0) : 0.0;
   const double sd = sqrt(var);
@@ -291,7 +300,7 @@ void launch_sor_stats(const float* dist, const uint8_t* finite, int64_t n, doubl
                       double* stats, uint8_t* keep, hipStream_t s) {
   const int nb = sor_stat_blocks(n);
   hipLaunchKernelGGL(k_sor_partials, dim3(nb), dim3(kSorThreads), 0, s, dist, finite, n, part);
-  hipLaunchKernelGGL(k_sor_stats, dim3(1), dim3(1), 0, s, part, nb, mul, stats);
+  hipLaunchKernelGGL(k_sor_stats, dim3(1), dim3(kSorThreads), 0, s, part, nb, mul, stats);
   if (n > 0)
     hipLaunchKernelGGL(k_sor_keep, dim3(blocks_of(n, 256)), dim3(256), 0, s, dist, n, stats, keep);
 }

@@ -200,11 +200,11 @@ void launch_depth_count(const int* pos, const int* flags, int64_t n, int64_t* ou
 
 // StatisticalOutlierRemoval distances (normals.hip's selection with mean_k + 1
 // neighbours): dist / finite per input point (the caller zeroes both first);
-// sums holds one double per sorted point, deferred npts_total + 1 ints.
+// sums holds one double per sorted point, work normals_work_ints(npts_total) ints.
 void launch_sor_distances(const GridDesc* grids, const int* cell_start, const float4* pts,
                           const int* cloud_of_sorted, const int64_t* cloud_off, int64_t npts_total,
-                          int mean_k, double* sums, int* nsel, int* deferred, float* dist,
-                          uint8_t* finite, hipStream_t s);
+                          int mean_k, double* sums, int* work, float* dist, uint8_t* finite,
+                          hipStream_t s);
 
 // ---- K9 pose-proposal network (encoder.hip)
 struct EncBuffers {

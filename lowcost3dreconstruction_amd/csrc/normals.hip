@@ -7,27 +7,12 @@
 // when (vp - p) . n < 0, then negated when the CLI's flip rule asks
 // (normal_estimation.cpp:112-118).  Fewer than 3 neighbours -> NaN normal.
 //
-// One wavefront per query, 64 consecutive cell-sorted queries per wavefront:
-//   1. stage every point of the 3x3x3 cells around the query's cell in LDS (one
-//      lane per row of cells finds the runs, then a flat coalesced copy); the
-//      next query in the same cell reuses the staged block.  A block larger than
-//      LDS is staged as an evenly strided subsample, whose K-th smallest d2 bounds
-//      the block's from above, and then restaged keeping only the points under
-//      that bound;
-//   2. find the exact K-th smallest FLANN-form d2: the K-th smallest of the 64
-//      per-lane minima bounds it; the points under that bound are compacted to
-//      one per lane and a bisection over the float bit pattern (counts by wave
-//      ballot) finds it there; equal distances are resolved by original index;
-//   3. certify: the K-th distance must be below the distance to the staged
-//      block's boundary, else stage the next larger block, keeping only the points
-//      within the K-th distance found so far, and repeat;
-//   4. list the selected points' original indices (ballot positions, fixed order).
-// A second pass, one point per lane, sums the FP64 moments of its listed
-// neighbours relative to it and solves the FP64 3x3 eigenproblem (keeping the
-// nine cross-lane FP64 sums and the solver's registers out of the search).  Queries the staged
-// search gives up on (very many equal distances, K above half the LDS capacity)
-// are listed and finished by a rescan pass that reads the block from memory for
-// every count.
+// Three selection passes find each point's exact K nearest neighbours by (FLANN
+// d2, original index): one lane per query over the 3x3x3 cells around it, one
+// wavefront per query that pass leaves over a growing block, and a rescan pass
+// with a bisection for what remains.  They sum what the caller needs (FP64 moments
+// for the normals, FP64 distances for outlier removal); the solve pass turns the
+// moments into normals, one point per lane.
 #include <hip/hip_runtime.h>
 
 #include "lcr_common.hpp"
@@ -40,15 +25,6 @@ namespace lcr {
 #pragma clang fp contract(off)
 
 namespace {
-
-constexpr int kWaves = 4;
-// staged points per wave: 4 x (576 x 16 + 64 x 4) B = 37 KiB per block, nine slots
-// of 64.  576 keeps the dense regions of Kinect-v2 captures (1.5 mm voxels, 74
-// clouds of 25k-88k points) mostly inside LDS -- 20.0 against 21.5 ms per cycle
-// step at 496 -- at no cost on Kinect-v1 captures (2 mm voxels, 36 clouds of
-// 37k-113k points); 600 and 624 (ten slots) cost those 1 %.
-constexpr int kCap = 576;
-constexpr int kSlots = (kCap + 63) / 64;
 
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -101,6 +77,13 @@ __device__ __forceinline__ void take(Moments& m, const float4& q, const float4& 
     add_moment(m, q, p);
   else
     m.v[0] += sqrt((double)d2);
+}
+
+// A query's sums: nine arrays of n, or one (kSqrtDist).
+template <int MODE>
+__device__ __forceinline__ void store_sums(const Moments& m, int64_t n, int64_t j, double* mom) {
+#pragma unroll
+  for (int c = 0; c < (MODE == kMoments ? 9 : 1); ++c) mom[c * n + j] = m.v[c];
 }
 
 // One selected point per lane where sel: kMoments writes its original index to
@@ -215,379 +198,6 @@ __device__ void select_rescan(const GridDesc& g, const int* cs, const float4* pt
       }
     });
   }
-}
-
-// The wave's staged candidate block in LDS.  When the (2K+1)^3 cells around the
-// query's cell hold at most kCap points it holds all of them, and the following
-// cell-sorted queries in the same cell reuse it.  A larger block is held filtered
-// -- the points whose FLANN d2 to the query is <= filt (the first kCap of them
-// when more qualify) -- or, without a bound to filter by, as an evenly strided
-// subsample; both serve that query only.
-struct Staged {
-  int64_t cell;   // cell whose complete unfiltered block is staged, else -1
-  int K;          // block radius in cells
-  int cnt;        // points in LDS
-  int total;      // points that qualified (more than kCap: LDS holds a subset)
-  unsigned filt;  // d2 filter as a bit pattern; 0xffffffff: none
-  unsigned lastT; // the previous query's k-th smallest d2 (bit pattern), 0: none
-};
-
-constexpr unsigned kNoFilter = 0xffffffffu;
-constexpr unsigned kInfBits = 0x7f800000u;
-
-// Sorted-index start and length of row r (z-major, then y) of block K.
-__device__ __forceinline__ void block_row(const GridDesc& g, const int* cs, int x0, int x1, int y0,
-                                          int z0, int nyb, int r, int& s, int& len) {
-  const int z = z0 + r / nyb, y = y0 + r % nyb;
-  const int row = (z * g.ny + y) * g.nx;
-  s = cs[row + x0];
-  len = cs[row + x1 + 1] - s;
-}
-
-// Stages block K around cp into sp (see Staged): the whole block when it fits
-// LDS, else the points with d2 <= U when a bound U is given, else an evenly
-// strided subsample.  Each lane looks up one x-contiguous row of cells, a wave
-// prefix sum places the rows, then the points are loaded four per lane at a time;
-// the filtered form keeps the qualifying ones in block order through ballots.
-__device__ __forceinline__ void stage_block(const GridDesc& g, const int* cs,
-                                            const float4* __restrict__ pts, const CellPos& cp, int K,
-                                            const float4& q, unsigned U, float4* sp, Staged& st) {
-  const int lane = threadIdx.x & 63;
-  wave_lds_sync();  // the previous block's reads come before these writes
-  st.K = K;
-  st.cnt = 0;
-  st.total = 0;
-  st.filt = kNoFilter;
-  const int z0 = max(cp.cz - K, 0), z1 = min(cp.cz + K, g.nz - 1);
-  const int y0 = max(cp.cy - K, 0), y1 = min(cp.cy + K, g.ny - 1);
-  const int x0 = max(cp.cx - K, 0), x1 = min(cp.cx + K, g.nx - 1);
-  if (z0 > z1 || y0 > y1 || x0 > x1) return;
-  const int nyb = y1 - y0 + 1, nrows = (z1 - z0 + 1) * nyb;
-  int tot = 0;
-  for (int rb = 0; rb < nrows; rb += 64) {
-    int s = 0, len = 0;
-    if (rb + lane < nrows) block_row(g, cs, x0, x1, y0, z0, nyb, rb + lane, s, len);
-    tot += wave_sum_i(len);
-  }
-  const bool filter = tot > kCap && U != kNoFilter;
-  // otherwise block positions i * stride are kept
-  const int stride = tot > kCap ? (tot + kCap - 1) / kCap : 1;
-  int pos = 0;  // filter: points kept so far; else block position of the group's first point
-  for (int rb = 0; rb < nrows; rb += 64) {
-    int s = 0, len = 0;
-    if (rb + lane < nrows) block_row(g, cs, x0, x1, y0, z0, nyb, rb + lane, s, len);
-    int inc = len;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int t = __shfl_up(inc, off, 64);
-      if (lane >= off) inc += t;
-    }
-    const int total = __shfl(inc, 63, 64);
-    const int excl = inc - len;
-    const int nr = min(64, nrows - rb);
-    // filter: group positions; else kept indices i with block position i * stride
-    // inside this group
-    const int i0 = filter ? 0 : (pos + stride - 1) / stride;
-    const int i1 = filter ? total : (pos + total + stride - 1) / stride;
-    for (int ib = i0; ib < i1; ib += 256) {
-      // positions past the end are clamped to the last one (loaded, not stored)
-      int tt[4], jb[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = min(ib + lane + 64 * u, i1 - 1);
-        tt[u] = filter ? i : i * stride - pos;
-      }
-      // row of position t: the last row whose first position is <= t
-      for (int rr = 0; rr < nr; ++rr) {
-        const int ex = __builtin_amdgcn_readlane(excl, rr);
-        const int sr = __builtin_amdgcn_readlane(s, rr);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (ex <= tt[u]) jb[u] = sr - ex;
-      }
-      float4 v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = pts[jb[u] + tt[u]];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = ib + lane + 64 * u;
-        if (filter) {
-          const bool keep = i < i1 && __float_as_uint(flann_d2(q.x, q.y, q.z, v[u])) <= U;
-          const uint64_t b = __ballot(keep);
-          const int at = pos + lane_prefix(b);
-          if (keep && at < kCap) sp[at] = v[u];
-          pos += __popcll(b);
-        } else if (i < i1) {
-          sp[i] = v[u];
-        }
-      }
-    }
-    if (!filter) pos += total;
-  }
-  if (filter) {
-    st.filt = U;
-    st.total = pos;
-    st.cnt = min(pos, kCap);
-  } else {
-    st.total = tot;
-    st.cnt = (tot + stride - 1) / stride;
-  }
-  wave_lds_sync();
-}
-
-// A complete unfiltered block can serve the following queries of its cell.
-__device__ __forceinline__ bool reusable(const Staged& st) {
-  return st.filt == kNoFilter && st.total <= kCap;
-}
-
-// FLANN d2 bit patterns of the staged points, point lane + 64 m in slot m
-// (0xffffffff past the end).
-__device__ __forceinline__ void fill_slots(const float4* sp, int cnt, const float4& q,
-                                           unsigned (&slot)[kSlots]) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int m = 0; m < kSlots; ++m) {
-    const int i = lane + 64 * m;
-    slot[m] = i < cnt ? __float_as_uint(flann_d2(q.x, q.y, q.z, sp[i])) : 0xffffffffu;
-  }
-}
-
-// Smallest t <= hi0 with at least kk values <= t: the kk-th smallest when at least
-// kk of the values are <= hi0.  Bisection over the bit pattern, counts by ballot.
-template <int NS>
-__device__ __forceinline__ unsigned kth_slots(const unsigned (&d)[NS], int ns, int kk, unsigned hi0) {
-  unsigned lo = 0u, hi = hi0;
-  while (lo < hi) {
-    const unsigned mid = lo + ((hi - lo) >> 1);
-    int c = 0;
-#pragma unroll
-    for (int m = 0; m < NS; ++m)
-      if (m < ns) c += popc_ballot(d[m] <= mid);
-    if (c >= kk)
-      hi = mid;
-    else
-      lo = mid + 1;
-  }
-  return lo;
-}
-
-// Maximum over the 64 lanes (every lane active): DPP inside each row of 16 lanes,
-// then the four row maxima.
-__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xF, 0xF, true));  // row_ror:4
-  v = max(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true));  // row_ror:8
-  return max(max((unsigned)__builtin_amdgcn_readlane((int)v, 0), (unsigned)__builtin_amdgcn_readlane((int)v, 16)),
-             max((unsigned)__builtin_amdgcn_readlane((int)v, 32), (unsigned)__builtin_amdgcn_readlane((int)v, 48)));
-}
-
-// The kk-th smallest of one value per lane (d: a bit pattern <= 0x7f800000, or
-// 0xffffffff for none), given c = count(d <= hi) >= kk.  Bisection over the bit
-// pattern keeping count(d <= lo - 1) < kk <= count(d <= hi); it stops as soon as
-// exactly kk values lie at or under hi -- the kk-th smallest is then the largest
-// of them -- which takes about log2 of the values' spread instead of all 31 bits.
-__device__ __forceinline__ unsigned kth_one(unsigned d, int kk, unsigned hi, int c) {
-  unsigned lo = 0u;
-  while (c > kk && lo < hi) {
-    const unsigned mid = lo + ((hi - lo) >> 1);
-    const int m = popc_ballot(d <= mid);
-    if (m >= kk) {
-      hi = mid;
-      c = m;
-    } else {
-      lo = mid + 1;
-    }
-  }
-  if (c == kk) return wave_max_u32(d <= hi ? d : 0u);
-  return lo;  // lo == hi: equal values at the kk-th place
-}
-
-// The kk-th smallest d2 of the cnt staged points (cnt >= kk).  With more than 64
-// points and kk <= 64 the points are filtered by a bound U with at least kk and
-// at most 64 staged points under it -- then the kk-th smallest lies under U --
-// and compacted to one per lane (cd, ci: d2 bits and staged index, through cb);
-// the bisection runs over that single slot.  U is the guess (a nearby query's
-// k-th d2, grown by 1.44) when its count qualifies, possibly after one doubling
-// or halving; else the kk-th smallest of the 64 per-lane minima, which are kk
-// distinct staged points.  comp tells whether the compacted slot was used.
-__device__ __forceinline__ unsigned kth_staged(const unsigned (&slot)[kSlots], int cnt, int kk,
-                                               unsigned guess, const float4* sp, const float4& q,
-                                               int* cb, unsigned& cd, int& ci, bool& comp) {
-  const int lane = threadIdx.x & 63;
-  const int nslots = (cnt + 63) >> 6;
-  comp = false;
-  if (nslots > 1 && kk <= 64) {
-    unsigned U = kInfBits;
-    int c = 65;  // > 64: no qualifying bound yet
-    if (guess != 0u) {
-      float gf = __uint_as_float(guess) * 1.44f;
-      for (int t = 0; t < 2; ++t) {
-        const unsigned gb = __float_as_uint(gf);
-        int n = 0;
-#pragma unroll
-        for (int m = 0; m < kSlots; ++m)
-          if (m < nslots) n += popc_ballot(slot[m] <= gb);
-        if (n >= kk && n <= 64) {
-          U = gb;
-          c = n;
-          break;
-        }
-        gf = n < kk ? gf * 2.0f : gf * 0.5f;
-      }
-    }
-    if (c > 64) {
-      unsigned mn = slot[0];
-#pragma unroll
-      for (int m = 1; m < kSlots; ++m) mn = min(mn, slot[m]);
-      U = kth_one(mn, kk, kInfBits, 64);  // more than 64 staged points: every lane has one
-      c = 0;
-#pragma unroll
-      for (int m = 0; m < kSlots; ++m)
-        if (m < nslots) c += popc_ballot(slot[m] <= U);
-    }
-    if (c <= 64) {
-      wave_lds_sync();
-      int base = 0;
-#pragma unroll
-      for (int m = 0; m < kSlots; ++m)
-        if (m < nslots) {
-          const bool keep = slot[m] <= U;
-          const uint64_t b = __ballot(keep);
-          if (keep) cb[base + lane_prefix(b)] = lane + 64 * m;
-          base += __popcll(b);
-        }
-      wave_lds_sync();
-      ci = lane < c ? cb[lane] : 0;
-      cd = lane < c ? __float_as_uint(flann_d2(q.x, q.y, q.z, sp[ci])) : 0xffffffffu;
-      comp = true;
-      return kth_one(cd, kk, U, c);
-    }
-  }
-  return kth_slots<kSlots>(slot, nslots, kk, kInfBits);
-}
-
-// Accumulates the kk points with the smallest (d2, original index) among
-// candidates (d bits, staged index ix) that hold every point with d2 <= T, T the
-// kk-th smallest d2: all points below T and the smallest indices at T.
-template <int MODE, int NS>
-__device__ __forceinline__ void take_kth(const unsigned (&d)[NS], const int (&ix)[NS], int ns, int kk,
-                                         unsigned T, const float4* sp, const float4& q, Moments& acc,
-                                         int* nbr) {
-  int clt = 0, cle = 0;
-#pragma unroll
-  for (int m = 0; m < NS; ++m)
-    if (m < ns) {
-      clt += popc_ballot(d[m] < T);
-      cle += popc_ballot(d[m] <= T);
-    }
-  int idcut = 0x7fffffff;
-  if (cle > kk) {
-    const int need = kk - clt;
-    int ids[NS];
-#pragma unroll
-    for (int m = 0; m < NS; ++m) ids[m] = d[m] == T ? __float_as_int(sp[ix[m]].w) : 0x7fffffff;
-    unsigned lo = 0u, hi = 0x7fffffffu;
-    while (lo < hi) {
-      const unsigned mid = lo + ((hi - lo) >> 1);
-      int c = 0;
-#pragma unroll
-      for (int m = 0; m < NS; ++m)
-        if (m < ns) c += popc_ballot(d[m] == T && (unsigned)ids[m] <= mid);
-      if (c >= need)
-        hi = mid;
-      else
-        lo = mid + 1;
-    }
-    idcut = (int)lo;
-  }
-  int base = 0;
-#pragma unroll
-  for (int m = 0; m < NS; ++m)
-    if (m < ns) {
-      bool sel = false;
-      float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (d[m] <= T) {
-        p = sp[ix[m]];
-        sel = d[m] < T || __float_as_int(p.w) <= idcut;
-      }
-      base += select_out<MODE>(sel, p, d[m], q, acc, nbr, base);
-    }
-}
-
-// Tightens an overflowing block's bound at most this many times before leaving
-// the query to the rescan pass.
-constexpr int kMaxTighten = 8;
-
-// Exact K-nearest selection for query q from LDS-staged blocks.  Block K grows
-// until the kk-th smallest d2 is certified below the distance to the block's
-// boundary.  A block larger than LDS is staged filtered by a proven upper bound
-// of its kk-th smallest d2 (the previous block's kk-th smallest, or that of a
-// staged subset of the block), so it fits LDS unless very many points tie.
-// Returns false (acc untouched) when it gives up; the query is then left to the
-// rescan pass.
-template <int MODE>
-__device__ __forceinline__ bool select_staged(const GridDesc& g, const int* cs, const float4* pts,
-                                              const float4& q, int kk, float4* sp, int* cb, Staged& st,
-                                              Moments& acc, int* nbr) {
-  const int lane = threadIdx.x & 63;
-  const CellPos cp = cell_pos(g, q.x, q.y, q.z);
-  const int64_t cell = (int64_t)g.cell_off + ((int64_t)cp.cz * g.ny + cp.cy) * g.nx + cp.cx;
-  if (st.cell != cell) {
-    stage_block(g, cs, pts, cp, 1, q, kNoFilter, sp, st);
-    st.cell = reusable(st) ? cell : -1;
-  }
-  int K = st.K;
-  unsigned slot[kSlots];
-  unsigned T = 0, cd = 0xffffffffu;
-  int ci = 0;
-  bool comp = false;
-  // Every pass grows K (until the block covers the grid) or tightens a bound, at
-  // most kMaxTighten times: the loop ends.
-  for (int tighten = 0;;) {
-    if (st.total > kCap) {
-      // LDS holds a subset of the qualifying points of block K: the kk-th smallest
-      // d2 among them bounds the block's kk-th smallest from above
-      if (st.cnt < kk || ++tighten > kMaxTighten) return false;
-      fill_slots(sp, st.cnt, q, slot);
-      const unsigned U = kth_slots<kSlots>(slot, (st.cnt + 63) >> 6, kk, kInfBits);
-      if (U >= st.filt) return false;  // no progress: very many equal distances
-      stage_block(g, cs, pts, cp, K, q, U, sp, st);
-      st.cell = -1;
-      continue;
-    }
-    const float Lc = block_gap(g, cp, K);
-    const bool covers = (Lc == INFINITY);
-    if (st.cnt >= kk) {
-      fill_slots(sp, st.cnt, q, slot);
-      T = kth_staged(slot, st.cnt, kk, st.lastT, sp, q, cb, cd, ci, comp);
-      const float L = (Lc - cp.slack) * g.h;
-      if (covers || (L > 0.0f && __uint_as_float(T) < L * L * 0.99998f)) break;
-      // the next block's kk-th smallest d2 is at most T
-      ++K;
-      stage_block(g, cs, pts, cp, K, q, T, sp, st);
-      st.cell = reusable(st) ? cell : -1;
-      continue;
-    }
-    // fewer than kk points: only an unfiltered block that does not cover the grid;
-    // an isolated point's block grows by half its radius at a time
-    if (st.filt != kNoFilter || covers) return false;
-    K += max(1, K >> 1);
-    stage_block(g, cs, pts, cp, K, q, kNoFilter, sp, st);
-    st.cell = reusable(st) ? cell : -1;
-  }
-  st.lastT = T;
-  if (comp) {
-    const unsigned d1[1] = {cd};
-    const int i1[1] = {ci};
-    take_kth<MODE, 1>(d1, i1, 1, kk, T, sp, q, acc, nbr);
-  } else {
-    int ix[kSlots];
-#pragma unroll
-    for (int m = 0; m < kSlots; ++m) ix[m] = lane + 64 * m;
-    take_kth<MODE, kSlots>(slot, ix, (st.cnt + 63) >> 6, kk, T, sp, q, acc, nbr);
-  }
-  return true;
 }
 
 // ---------------------------------------------------------------- lane path
@@ -788,7 +398,7 @@ constexpr int kNselOrig = 1 << 30;
 // when this block held too few points or no certificate, K otherwise; when
 // bucket B overflowed, B + 1 in bits 8 and up (at least kk points lie below
 // (B + 1) D2 / NB, up to the rounding of d2 * scale).
-template <int K, int NB, int NL>
+template <int MODE, int K, int NB, int NL>
 __device__ __forceinline__ int lane_query(const GridDesc* __restrict__ grids,
                                           const int* __restrict__ cell_start,
                                           const float4* __restrict__ pts,
@@ -799,7 +409,7 @@ __device__ __forceinline__ int lane_query(const GridDesc* __restrict__ grids,
   const float4 q = pts[j];
   const GridDesc g = grids[cloud_of_sorted[j]];
   const int kk = min(k, g.npts);
-  if (kk < 3) {
+  if (MODE == kMoments && kk < 3) {
     nsel[j] = kk;
     return 0;
   }
@@ -860,7 +470,7 @@ __device__ __forceinline__ int lane_query(const GridDesc* __restrict__ grids,
     if (valid && d < D2) {
       const int b = min((int)(d * scale), NB - 1);
       if (b < B) {
-        add_moment(acc, q, p);
+        take<MODE>(acc, q, p, d);
       } else if (b == B && nl < NL) {
         buf[3 * nl][lane] = __float_as_uint(d);
         buf[3 * nl + 1][lane] = (uint32_t)__float_as_int(p.w);
@@ -880,10 +490,14 @@ __device__ __forceinline__ int lane_query(const GridDesc* __restrict__ grids,
   const int need = kk - below;
 #pragma unroll
   for (int t = 0; t < NL; ++t)
-    if (t < need) add_moment(acc, q, load_point(rs, ei[t]));
-#pragma unroll
-  for (int c = 0; c < 9; ++c) mom[c * n + j] = acc.v[c];
-  nsel[j] = kk;
+    if (t < need) {
+      if constexpr (MODE == kMoments)
+        add_moment(acc, q, load_point(rs, ei[t]));
+      else
+        take<MODE>(acc, q, q, __uint_as_float((uint32_t)(e[t] >> 32)));
+    }
+  store_sums<MODE>(acc, n, j, mom);
+  if constexpr (MODE == kMoments) nsel[j] = kk;
   return 0;
 }
 
@@ -905,7 +519,7 @@ __device__ __forceinline__ void wave_append(bool take, int64_t j, int start_k,
 // The lane pass over every point: one lane per point, blocks mapped
 // XCD-contiguous; the points it leaves are appended to list.  No barrier: each
 // lane uses only its own LDS column.
-template <int K, int NB, int NL>
+template <int MODE, int K, int NB, int NL>
 __global__ void __launch_bounds__(kLaneThreads)
 k_normal_lane(const GridDesc* __restrict__ grids, const int* __restrict__ cell_start,
               const float4* __restrict__ pts, const int* __restrict__ cloud_of_sorted,
@@ -916,7 +530,7 @@ k_normal_lane(const GridDesc* __restrict__ grids, const int* __restrict__ cell_s
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t j = (int64_t)xcd_block(blockIdx.x, gridDim.x) * kLaneThreads + threadIdx.x;
   const __amdgpu_buffer_rsrc_t rs = points_rsrc(pts, total);
-  const int start_k = j < total ? lane_query<K, NB, NL>(grids, cell_start, pts, rs, cloud_of_sorted,
+  const int start_k = j < total ? lane_query<MODE, K, NB, NL>(grids, cell_start, pts, rs, cloud_of_sorted,
                                                         k, j, s_buf[w], lane, mom, total, nsel)
                                 : 0;
   wave_append(start_k > 0, j, start_k, list, count);
@@ -1081,6 +695,12 @@ __device__ __forceinline__ bool wave_find_bucket(const WaveLds& L, int kk, int& 
   return true;
 }
 
+// An upper bound of the distance from a query inside the grid to any of its points.
+__device__ __forceinline__ float grid_extent(const GridDesc& g) {
+  return ((float)g.nx + (float)g.ny + (float)g.nz + 3.0f) * g.h;
+}
+
+template <int MODE>
 __global__ void __launch_bounds__(kWaveThreads, 5)
 k_normal_wave(const GridDesc* __restrict__ grids, const int* __restrict__ cell_start,
               const float4* __restrict__ pts, const int* __restrict__ cloud_of_sorted, int k,
@@ -1098,7 +718,7 @@ k_normal_wave(const GridDesc* __restrict__ grids, const int* __restrict__ cell_s
     const int64_t j = __builtin_amdgcn_readfirstlane(e.x);
     const float4 q = pts[j];
     const GridDesc g = grids[cloud_of_sorted[j]];
-    const int kk = min(k, g.npts);  // at least 3: the lane pass serves the others
+    const int kk = min(k, g.npts);  // kMoments: at least 3, the lane pass serves the others
     const int* cs = cell_start + g.cell_off;
     const CellPos cp = cell_pos(g, q.x, q.y, q.z);
     bool done = false;
@@ -1108,8 +728,9 @@ k_normal_wave(const GridDesc* __restrict__ grids, const int* __restrict__ cell_s
     float U = INFINITY;
     for (int attempt = 0; attempt < 8 && !done && K <= kWaveMaxK; ++attempt) {
       const float Lc = block_gap(g, cp, K);
-      if (Lc == INFINITY) break;  // covers the grid: the rescan pass
-      const float Lm = (Lc - cp.slack) * g.h;
+      // A block that covers the grid holds every point and needs no certificate: its
+      // range is the grid's extent
+      const float Lm = Lc == INFINITY ? grid_extent(g) : (Lc - cp.slack) * g.h;
       const float D2 = Lm * Lm * 0.99998f;
       // the lane pass's bucket bound (same block, same D2), widened for rounding
       if (attempt == 0 && (code >> 8) > 0)
@@ -1200,7 +821,7 @@ k_normal_wave(const GridDesc* __restrict__ grids, const int* __restrict__ cell_s
         const bool lt = b < B || (b == B && sb < SB);
         const bool eq = b == B && sb == SB;
         const uint64_t beq = __ballot(eq);
-        if (lt) add_moment(acc, q, p);
+        if (lt) take<MODE>(acc, q, p, d);
         if (eq) {
           const int slot = nl + lane_prefix(beq);
           L.key[slot] = __float_as_uint(d);
@@ -1215,80 +836,31 @@ k_normal_wave(const GridDesc* __restrict__ grids, const int* __restrict__ cell_s
         const uint64_t mine = ((uint64_t)L.key[lane] << 32) | L.idx[lane];
         int rank = 0;
         for (int u = 0; u < nl; ++u) rank += (((uint64_t)L.key[u] << 32) | L.idx[u]) < mine ? 1 : 0;
-        if (rank < kk - below) add_moment(acc, q, load_point(rs, L.pos[lane]));
+        if (rank < kk - below) {
+          if constexpr (MODE == kMoments)
+            add_moment(acc, q, load_point(rs, L.pos[lane]));
+          else
+            take<MODE>(acc, q, q, __uint_as_float(L.key[lane]));
+        }
       }
 #pragma unroll
-      for (int c = 0; c < 9; ++c) {
-        const double v = wave_sum_dpp(acc.v[c]);
-        if (lane == 0) mom[c * total + j] = v;
+      for (int c = 0; c < (MODE == kMoments ? 9 : 1); ++c) acc.v[c] = wave_sum_dpp(acc.v[c]);
+      if (lane == 0) {
+        store_sums<MODE>(acc, total, j, mom);
+        if constexpr (MODE == kMoments) nsel[j] = kk;
       }
-      if (lane == 0) nsel[j] = kk;
       done = true;
     }
     if (!done && lane == 0) {
       // deferred[0] counts the list deferred[1..]
-      nsel[j] = kk | kNselOrig;
+      if constexpr (MODE == kMoments) nsel[j] = kk | kNselOrig;
       deferred[1 + atomicAdd(deferred, 1)] = (int)j;
     }
     wave_lds_sync();  // L is reused by the next query
   }
 }
 
-// Search pass, per point in cell-sorted order: the neighbour count and either
-// the original indices of its K nearest neighbours (kMoments: nbr holds k per
-// point, the moments are summed by the solve pass) or the FP64 sum of their
-// distances (kSqrtDist: mom holds 1 per point).
-template <int MODE>
-__global__ void __launch_bounds__(kWaves * 64)
-k_normal_moments(const GridDesc* __restrict__ grids, const int* __restrict__ cell_start,
-                 const float4* __restrict__ pts, const int* __restrict__ cloud_of_sorted,
-                 int64_t total, int k, double* __restrict__ mom, int* __restrict__ nbr,
-                 int* __restrict__ nsel, int* __restrict__ deferred) {
-  __shared__ float4 s_p[kWaves][kCap];
-  __shared__ int s_cb[kWaves][64];
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t base = ((int64_t)xcd_block(blockIdx.x, gridDim.x) * kWaves + w) * 64;
-  if (base >= total) return;
-  const int64_t jq = base + lane;
-  const bool own = jq < total;
-  const int nq = (int)min<int64_t>(64, total - base);
-  Staged st;
-  st.cell = -1;
-  st.K = 0;
-  st.cnt = 0;
-  st.total = 0;
-  st.filt = kNoFilter;
-  st.lastT = 0u;
-  int mine_n = 0;
-  for (int qi = 0; qi < nq; ++qi) {
-    // wave-uniform addresses: scalar loads, so no vector load issued before the
-    // loop stays pending into it (a pending one makes every iteration wait for
-    // the previous iteration's stores)
-    const float4 q = pts[base + qi];
-    const GridDesc g = grids[cloud_of_sorted[base + qi]];
-    const int kk = min(k, g.npts);
-    Moments acc;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) acc.v[i] = 0.0;
-    int* out = MODE == kMoments ? nbr + (base + qi) * k : nullptr;
-    if (kk >= (MODE == kMoments ? 3 : 1) &&
-        !select_staged<MODE>(g, cell_start + g.cell_off, pts, q, kk, s_p[w], s_cb[w], st, acc, out)) {
-      // deferred[0] counts the list deferred[1..]
-      if (lane == 0) deferred[1 + atomicAdd(deferred, 1)] = (int)(base + qi);
-      if (lane == qi) mine_n = kk;
-      continue;
-    }
-    if constexpr (MODE == kSqrtDist) {
-      const double s = wave_sum_dpp(acc.v[0]);
-      if (lane == 0) mom[base + qi] = s;
-    }
-    if (lane == qi) mine_n = kk;
-  }
-  if (own) nsel[jq] = mine_n;
-}
-
-// Rescan pass for the deferred queries (candidate blocks too large for LDS), one
+// Rescan pass for the deferred queries (see the wavefront pass), one
 // wavefront per query, reading the block from memory for every count.
 template <int MODE>
 __global__ void __launch_bounds__(256)
@@ -1395,24 +967,46 @@ __global__ void k_sor_dist(const float4* __restrict__ pts, const int* __restrict
 
 }  // namespace
 
+int64_t normals_work_ints(int64_t n) { return 4 * n + 3; }
+
+// The selection passes over every point: sums (and, kMoments, nsel and the rescan
+// pass's neighbour lists).  work (normals_work_ints(n)): [0] the lane pass's list
+// count, [1] the rescan count with its list at [2, 2 + n), the lane pass's list of
+// (point, start radius) at [2 + n, 2 + 3n).
+template <int MODE>
+static void launch_selection(const GridDesc* grids, const int* cell_start, const float4* pts,
+                             const int* cloud_of_sorted, int64_t n, int k, int* nbr, double* mom,
+                             int* nsel, int* work, hipStream_t s) {
+  int* count = work;
+  int* deferred = work + 1;
+  int2* list = reinterpret_cast<int2*>(work + 2 + n + (n & 1));
+  launch_fill_i32(work, 2, 0, s);
+  hipLaunchKernelGGL((k_normal_lane<MODE, 1, kLaneBuckets, 8>),
+                     dim3((unsigned)((n + kLaneThreads - 1) / kLaneThreads)), dim3(kLaneThreads), 0, s,
+                     grids, cell_start, pts, cloud_of_sorted, n, k, mom, nsel, list, count);
+  // persistent over the list (a few percent of the points): at most eight blocks
+  // of four wavefronts per CU
+  const int64_t wave_blocks = (n + kWaveThreads / 64 - 1) / (kWaveThreads / 64);
+  hipLaunchKernelGGL(k_normal_wave<MODE>, dim3((unsigned)(wave_blocks < 2048 ? wave_blocks : 2048)),
+                     dim3(kWaveThreads), 0, s, grids, cell_start, pts, cloud_of_sorted, k,
+                     (const int2*)list, (const int*)count, n, mom, nsel, deferred);
+  hipLaunchKernelGGL(k_normal_rescan<MODE>, dim3(1024), dim3(256), 0, s, grids, cell_start, pts,
+                     cloud_of_sorted, k, deferred, mom, nbr);
+}
+
+// Outlier removal runs the same selection as the normals, summing distances: 100k
+// points, 50 neighbours: 1477 -> 249 us against one wavefront per query over a
+// block staged in LDS.
 void launch_sor_distances(const GridDesc* grids, const int* cell_start, const float4* pts,
                           const int* cloud_of_sorted, const int64_t* cloud_off, int64_t npts_total,
-                          int mean_k, double* sums, int* nsel, int* deferred, float* dist,
-                          uint8_t* finite, hipStream_t s) {
+                          int mean_k, double* sums, int* work, float* dist, uint8_t* finite,
+                          hipStream_t s) {
   if (npts_total <= 0) return;
-  const int64_t per_block = (int64_t)kWaves * 64;
-  const unsigned blocks = (unsigned)((npts_total + per_block - 1) / per_block);
-  launch_fill_i32(deferred, 1, 0, s);
-  hipLaunchKernelGGL(k_normal_moments<kSqrtDist>, dim3(blocks), dim3(kWaves * 64), 0, s, grids,
-                     cell_start, pts, cloud_of_sorted, npts_total, mean_k + 1, sums, (int*)nullptr, nsel,
-                     deferred);
-  hipLaunchKernelGGL(k_normal_rescan<kSqrtDist>, dim3(1024), dim3(256), 0, s, grids, cell_start,
-                     pts, cloud_of_sorted, mean_k + 1, deferred, sums, (int*)nullptr);
+  launch_selection<kSqrtDist>(grids, cell_start, pts, cloud_of_sorted, npts_total, mean_k + 1, nullptr,
+                              sums, nullptr, work, s);
   hipLaunchKernelGGL(k_sor_dist, dim3((unsigned)((npts_total + 255) / 256)), dim3(256), 0, s, pts,
                      cloud_of_sorted, cloud_off, sums, npts_total, mean_k, dist, finite);
 }
-
-int64_t normals_work_ints(int64_t n) { return 4 * n + 3; }
 
 void launch_normals(const GridDesc* grids, const int* cell_start, const float4* pts,
                     const int* cloud_of_sorted, int64_t npts_total, int k, const float* vp,
@@ -1420,23 +1014,7 @@ void launch_normals(const GridDesc* grids, const int* cell_start, const float4* 
                     int* nsel, int* work, float4* nrm_sorted, hipStream_t s) {
   if (npts_total <= 0) return;
   const int64_t n = npts_total;
-  // work: [0] the lane pass's list count, [1] the rescan count with its list at
-  // [2, 2 + n), the lane pass's list of (point, start radius) at [2 + n, 2 + 3n)
-  int* count = work;
-  int* deferred = work + 1;
-  int2* list = reinterpret_cast<int2*>(work + 2 + n + (n & 1));
-  launch_fill_i32(work, 2, 0, s);
-  hipLaunchKernelGGL((k_normal_lane<1, kLaneBuckets, 8>), dim3((unsigned)((n + kLaneThreads - 1) / kLaneThreads)),
-                     dim3(kLaneThreads), 0, s, grids, cell_start, pts, cloud_of_sorted, n, k, mom,
-                     nsel, list, count);
-  // persistent over the list (a few percent of the points): at most eight blocks
-  // of four wavefronts per CU
-  const int64_t wave_blocks = (n + kWaveThreads / 64 - 1) / (kWaveThreads / 64);
-  hipLaunchKernelGGL(k_normal_wave, dim3((unsigned)(wave_blocks < 2048 ? wave_blocks : 2048)),
-                     dim3(kWaveThreads), 0, s, grids, cell_start, pts, cloud_of_sorted, k,
-                     (const int2*)list, (const int*)count, n, mom, nsel, deferred);
-  hipLaunchKernelGGL(k_normal_rescan<kMoments>, dim3(1024), dim3(256), 0, s, grids, cell_start, pts,
-                     cloud_of_sorted, k, deferred, (double*)nullptr, nbr);
+  launch_selection<kMoments>(grids, cell_start, pts, cloud_of_sorted, n, k, nbr, mom, nsel, work, s);
   hipLaunchKernelGGL(k_normal_solve, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, pts,
                      cloud_of_sorted, raw, cloud_off, nbr, k, (const double*)mom, nsel, n, vp,
                      flip_all, nrm_sorted);

@@ -117,3 +117,47 @@ def test_depth_fuse_matches_oracle(lcr, k, h, w, factor):
     out = lcr.depth_fuse(frames, factor)
     np.testing.assert_array_equal(out, oracle.depth_fuse(frames, factor))
     assert (out > 0).mean() > 0.05
+
+
+def small_cloud(kind, n):
+    rng = np.random.default_rng(n)
+    if kind == "same":  # one point n times: every distance equal
+        return np.tile(rng.normal(size=(1, 3)), (n, 1)).astype(np.float32)
+    if kind == "line":  # a grid one cell wide along two axes
+        return np.c_[np.linspace(0, 1, n), np.zeros((n, 2))].astype(np.float32)
+    if kind == "far":  # a plane and points far from it: blocks grow over many cells
+        p = np.c_[rng.uniform(-0.5, 0.5, size=(n, 2)), rng.normal(scale=1e-3, size=n)]
+        p[::97, 2] += rng.uniform(0.2, 5.0, size=len(p[::97]))
+        return p.astype(np.float32)
+    return rng.normal(size=(n, 3)).astype(np.float32)
+
+
+@pytest.mark.parametrize("kind,n,k", [("blob", 1, 1), ("blob", 2, 1), ("blob", 3, 8), ("blob", 40, 50),
+                                      ("blob", 65, 20), ("blob", 1000, 50), ("line", 300, 10),
+                                      ("same", 200, 20), ("far", 3000, 12), ("far", 3000, 1)])
+def test_outlier_distances_on_small_and_odd_clouds(lcr, kind, n, k):
+    """Clouds whose candidate blocks cover the whole grid, hold fewer points than
+    asked for, equal distances only, or points far from all others: every pass of
+    the selection.  Distances are FP64 sums of square roots rounded to float (one
+    float ulp against the oracle's order of adding)."""
+    pts = small_cloud(kind, n)
+    print_case(test="outliers_small", kind=kind, n=n, k=k)
+    keep, dist, stats = lcr.outlier_removal(pts, k, 1.0)
+    rkeep, rdist, rstats = oracle.sor(pts, k, 1.0)
+    np.testing.assert_allclose(dist, rdist, rtol=1.2e-7, atol=0)
+    np.testing.assert_allclose(stats, rstats, rtol=1e-6, atol=1e-9)
+    near = np.abs(rdist.astype(np.float64) - rstats[2]) <= 1e-6 * abs(rstats[2]) + 1e-9
+    np.testing.assert_array_equal(keep[~near], rkeep[~near])
+
+
+@pytest.mark.parametrize("kind,n,k", [("blob", 31, 30), ("blob", 120, 50), ("far", 3000, 12)])
+def test_normals_on_small_clouds(lcr, kind, n, k):
+    """The same passes for the normals: blocks that cover the grid, and points far
+    from the rest."""
+    pts = small_cloud(kind, n)
+    print_case(test="normals_small_clouds", kind=kind, n=n, k=k)
+    nrm, curv = lcr.normals(pts, k)
+    rn, rc = oracle.normals(pts, k)
+    dots = np.sum(nrm.astype(np.float64) * rn, axis=1)
+    assert np.all(dots > 1 - 1e-6), np.sort(dots)[:5]
+    np.testing.assert_allclose(curv, rc, rtol=2e-6, atol=1e-9)
