@@ -711,9 +711,9 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
     cs.upload(st.s, {xyz}, {nrm}, {n}, 3 * sizeof(float));
     DevBuf part, box;
     part.reserve((size_t)kBBoxChunks * 7 * sizeof(float));
-    box.reserve(7 * sizeof(float));
+    box.reserve(kGeomWords * sizeof(float));
     launch_bbox(cs.d_raw.as<float4>(), cs.d_cloud_off.as<int64_t>(), 1, part.as<float>(),
-                box.as<float>(), st.s);
+                box.as<float>(), nullptr, nullptr, st.s);
     float b[7];
     LCR_HIP(hipMemcpyAsync(b, box.p, sizeof b, hipMemcpyDeviceToHost, st.s));
     LCR_HIP(hipStreamSynchronize(st.s));

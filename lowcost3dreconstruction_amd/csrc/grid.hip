@@ -24,10 +24,15 @@ __device__ __forceinline__ bool finite3(const float4& p) {
 
 // One block per (cloud, chunk): partial min/max of finite points.
 __global__ void __launch_bounds__(kBBoxThreads)
-k_bbox_partial(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off, int nclouds,
-               int chunks_per_cloud, float* __restrict__ part) {
+k_bbox_partial(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off,
+               float* __restrict__ part, uint32_t* __restrict__ probe_bits) {
+  constexpr int chunks_per_cloud = kBBoxChunks;
   const int cloud = blockIdx.x / chunks_per_cloud;
   const int chunk = blockIdx.x % chunks_per_cloud;
+  // the cloud's probe bits start clear (a share per chunk)
+  if (probe_bits)
+    for (int i = chunk * kBBoxThreads + threadIdx.x; i < kProbeWords; i += chunks_per_cloud * kBBoxThreads)
+      probe_bits[(int64_t)cloud * kProbeWords + i] = 0u;
   const int64_t b = cloud_off[cloud], e = cloud_off[cloud + 1];
   float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
   float cnt = 0.0f;
@@ -77,22 +82,30 @@ k_bbox_partial(const float4* __restrict__ raw, const int64_t* __restrict__ cloud
   }
 }
 
-// One thread per cloud: fold the chunk partials.  Output per cloud: min xyz,
-// max xyz, finite count.
-__global__ void k_bbox_final(const float* __restrict__ part, int nclouds, int chunks_per_cloud,
-                             float* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nclouds) return;
-  float r[7] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0f};
-  for (int k = 0; k < chunks_per_cloud; ++k) {
-    const float* p = part + ((int64_t)c * chunks_per_cloud + k) * 7;
+// One wavefront per cloud: fold the kBBoxChunks (64) chunk partials, a lane each.
+// Output per cloud: min xyz, max xyz, finite count (kGeomWords floats apart), and
+// the probe grid of the box.  (A thread per cloud read the partials one after the
+// other: 10 us a call; this 2.)
+__global__ void __launch_bounds__(64)
+k_bbox_final(const float* __restrict__ part, float* __restrict__ out, GridDesc* __restrict__ probe) {
+  static_assert(kBBoxChunks == 64, "a lane per chunk");
+  const int c = blockIdx.x, lane = threadIdx.x;
+  const float* p = part + ((int64_t)c * kBBoxChunks + lane) * 7;
+  float r[7];
+#pragma unroll
+  for (int a = 0; a < 7; ++a) r[a] = p[a];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
     for (int a = 0; a < 3; ++a) {
-      r[a] = fminf(r[a], p[a]);
-      r[3 + a] = fmaxf(r[3 + a], p[3 + a]);
+      r[a] = fminf(r[a], __shfl_xor(r[a], off, 64));
+      r[3 + a] = fmaxf(r[3 + a], __shfl_xor(r[3 + a], off, 64));
     }
-    r[6] += p[6];
+    r[6] += __shfl_xor(r[6], off, 64);  // counts below 2^24: exact in any order
   }
-  for (int a = 0; a < 7; ++a) out[c * 7 + a] = r[a];
+  if (lane != 0) return;
+  for (int a = 0; a < 7; ++a) out[c * kGeomWords + a] = r[a];
+  if (probe) probe[c] = probe_grid(r);
 }
 
 __device__ __forceinline__ int cell_of(const GridDesc& g, const float4& p) {
@@ -105,33 +118,42 @@ __device__ __forceinline__ int cell_of(const GridDesc& g, const float4& p) {
   return (z * g.ny + y) * g.nx + x;
 }
 
-// Per point: global cell index (or -1 for non-finite points) and per-cell counts.
-// counter[key] += 1 for every calling lane, one atomic per distinct key in the
-// wavefront (raw points in image order share cells, so a wavefront holds a few
-// keys); returns the counter's value before the lane's own increment.  It
-// ballots: every lane of the wavefront that is still running must call it.
+// counter[key] += 1 for every calling lane; returns the counter's value before the
+// lane's own increment.  Raw points in image order share cells, so the lanes of
+// one key add together: kShareRounds keys per wavefront are found by ballots, then
+// every key's first lane (and every lane whose key was not reached) issues its
+// atomic, all in one instruction.  Waiting for one atomic per key in turn made this
+// the longest kernel of a small build (2003 scattered points: 30 -> 4 us); each
+// round of ballots costs about 20 ns of a wavefront, and scattered points share
+// no keys, hence the limit.  Every lane of the wavefront that is still running
+// must call it.
+constexpr int kShareRounds = 8;
+
 __device__ __forceinline__ int wave_counter_add(int* __restrict__ counter, int key) {
   const int lane = (int)(threadIdx.x & 63);
   uint64_t todo = __ballot(true);
-  int result = 0;
-  while (todo) {
+  int first = lane, before = 0, share = 1;
+  for (int round = 0; round < kShareRounds && todo; ++round) {
     const int lead = __ffsll((unsigned long long)todo) - 1;
-    const int k = __shfl(key, lead, 64);
-    const uint64_t same = __ballot(key == k) & todo;
-    int base = 0;
-    if (lane == lead) base = atomicAdd(&counter[k], __popcll(same));
-    base = __shfl(base, lead, 64);
-    if ((same >> lane) & 1ull)
-      result = base + __popcll(same & ((1ull << lane) - 1ull));
+    const uint64_t same = __ballot(key == __shfl(key, lead, 64)) & todo;
+    if ((same >> lane) & 1ull) {
+      first = lead;
+      before = __popcll(same & ((1ull << lane) - 1ull));
+      share = __popcll(same);
+    }
     todo &= ~same;
   }
-  return result;
+  int base = 0;
+  if (first == lane) base = atomicAdd(&counter[key], share);
+  return __shfl(base, first, 64) + before;
 }
 
+// Per point: global cell index (-1 for non-finite points), per-cell counts, and the
+// point's place among its cell's points in the order the atomics came.
 __global__ void k_cell_count(const float4* __restrict__ raw, const int* __restrict__ point_cloud,
                              const GridDesc* __restrict__ grids, int64_t n,
                              int* __restrict__ cid, int* __restrict__ counts,
-                             int* __restrict__ occupied) {
+                             int* __restrict__ place) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float4 p = raw[i];
@@ -143,26 +165,55 @@ __global__ void k_cell_count(const float4* __restrict__ raw, const int* __restri
   const GridDesc g = grids[c];
   const int gc = (int)g.cell_off + cell_of(g, p);
   cid[i] = gc;
-  wave_counter_add(counts, gc);
+  place[i] = wave_counter_add(counts, gc);
 }
 
-// occupied[cloud] = number of non-empty cells of the cloud's grid (one atomic per
-// block after a block reduction)
-__global__ void k_occupancy(const GridDesc* __restrict__ grids, const int* __restrict__ counts,
-                            int* __restrict__ occupied) {
-  __shared__ int s[256];
-  const GridDesc g = grids[blockIdx.y];
-  const int64_t ncells = (int64_t)g.nx * g.ny * g.nz;
-  int a = 0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ncells; i += (int64_t)gridDim.x * 256)
-    a += counts[g.cell_off + i] > 0 ? 1 : 0;
-  s[threadIdx.x] = a;
+// The probe: one bit per cell of each cloud's probe grid (at most 65^3) that holds
+// a point.  A block collects the bits of kBBoxChunks-th part of a cloud, consecutive
+// points, in LDS, then ORs its words that hold any into the cloud's: points in image
+// order touch few words (113k points: 5 us; with an atomic per point that finds
+// its bit clear 74, one per wavefront and cell 17).
+__global__ void __launch_bounds__(1024)
+k_probe(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off,
+        const GridDesc* __restrict__ probe, uint32_t* __restrict__ bits) {
+  __shared__ uint32_t lds[kProbeWords];
+  const int cloud = blockIdx.x / kBBoxChunks, chunk = blockIdx.x % kBBoxChunks;
+  const int64_t b = cloud_off[cloud], n = cloud_off[cloud + 1] - b;
+  const int64_t i0 = b + n * chunk / kBBoxChunks, i1 = b + n * (chunk + 1) / kBBoxChunks;
+  if (i0 >= i1) return;  // uniform across the block
+  for (int i = threadIdx.x; i < kProbeWords; i += 1024) lds[i] = 0u;
+  const GridDesc g = probe[cloud];
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-    __syncthreads();
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += 1024) {
+    const float4 p = raw[i];
+    if (!finite3(p)) continue;
+    const int cell = cell_of(g, p);
+    atomicOr(&lds[cell >> 5], 1u << (cell & 31));
   }
-  if (threadIdx.x == 0 && s[0] > 0) atomicAdd(&occupied[blockIdx.y], s[0]);
+  __syncthreads();
+  uint32_t* out = bits + (int64_t)cloud * kProbeWords;
+  for (int i = threadIdx.x; i < kProbeWords; i += 1024)
+    if (lds[i]) atomicOr(&out[i], lds[i]);
+}
+
+// Occupied probe cells of each cloud, after its box and count (an int's bits).
+__global__ void __launch_bounds__(1024)
+k_probe_count(const uint32_t* __restrict__ bits, float* __restrict__ geom) {
+  __shared__ int s[1024 / 64];
+  const uint32_t* b = bits + (int64_t)blockIdx.x * kProbeWords;
+  int a = 0;
+#pragma unroll
+  for (int i = 0; i < (kProbeWords + 1023) / 1024; ++i) {
+    const int k = i * 1024 + threadIdx.x;
+    a += k < kProbeWords ? __popc(b[k]) : 0;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = a;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int k = 1; k < 1024 / 64; ++k) a += s[k];
+  geom[blockIdx.x * kGeomWords + 7] = __int_as_float(a);
 }
 
 constexpr int kScanThreads = 1024;
@@ -203,29 +254,35 @@ __global__ void __launch_bounds__(kScanThreads)
 k_scan_tiles(int* __restrict__ in, int* __restrict__ out, int64_t n, int* __restrict__ sums) {
   __shared__ int lds[kScanThreads / 64];
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPerThread;
-  int v[kScanPerThread];
-  int s = 0;
+  const bool whole = base + kScanPerThread <= n;  // in and out start on 16 bytes
+  int4 v = make_int4(0, 0, 0, 0);
+  if (whole) {
+    v = *reinterpret_cast<const int4*>(in + base);
+    if constexpr (CONSUME) *reinterpret_cast<int4*>(in + base) = make_int4(0, 0, 0, 0);
+  } else {
+    int* e[3] = {&v.x, &v.y, &v.z};
 #pragma unroll
-  for (int k = 0; k < kScanPerThread; ++k) {
-    v[k] = (base + k < n) ? in[base + k] : 0;
-    s += v[k];
-  }
-  if constexpr (CONSUME) {
-#pragma unroll
-    for (int k = 0; k < kScanPerThread; ++k)
-      if (base + k < n) in[base + k] = 0;
+    for (int k = 0; k < kScanPerThread - 1; ++k)
+      if (base + k < n) {
+        *e[k] = in[base + k];
+        if constexpr (CONSUME) in[base + k] = 0;
+      }
   }
   int total;
-  int run = block_excl_scan(s, lds, total);
-#pragma unroll
-  for (int k = 0; k < kScanPerThread; ++k) {
-    if (base + k < n) out[base + k] = run;
-    run += v[k];
+  const int run = block_excl_scan(v.x + v.y + v.z + v.w, lds, total);
+  const int4 o = make_int4(run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z);
+  if (whole) {
+    *reinterpret_cast<int4*>(out + base) = o;
+  } else {
+    if (base < n) out[base] = o.x;
+    if (base + 1 < n) out[base + 1] = o.y;
+    if (base + 2 < n) out[base + 2] = o.z;
   }
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// Single block: exclusive scan of the tile sums, in chunks with a carry.
+// Single block: exclusive scan of the tile sums, in chunks with a carry (scans of
+// more than kScanInlineTiles tiles).
 __global__ void __launch_bounds__(kScanThreads) k_scan_sums(int* __restrict__ sums, int n) {
   __shared__ int lds[kScanThreads / 64];
   int carry = 0;
@@ -239,22 +296,43 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_sums(int* __restrict__ su
   }
 }
 
-__global__ void k_scan_add(int* __restrict__ out, int64_t n, const int* __restrict__ sums) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  out[i] += sums[i / kScanTile];
+// Adds the sum of the tiles before it to every tile.  scanned: sums holds their
+// exclusive scan; else each block adds the tile sums before its own up.
+__global__ void __launch_bounds__(kScanThreads)
+k_scan_add(int* __restrict__ out, int64_t n, const int* __restrict__ sums, int scanned) {
+  __shared__ int lds[kScanThreads / 64];
+  const int tile = blockIdx.x + 1;  // the first tile's prefix is zero
+  int before;
+  if (scanned) {
+    before = sums[tile];
+  } else {
+    int a = 0;
+    for (int k = threadIdx.x; k < tile; k += kScanThreads) a += sums[k];
+    (void)block_excl_scan(a, lds, before);
+  }
+  const int64_t base = (int64_t)tile * kScanTile + (int64_t)threadIdx.x * kScanPerThread;
+  if (base + kScanPerThread <= n) {
+    int4 v = *reinterpret_cast<int4*>(out + base);
+    v.x += before;
+    v.y += before;
+    v.z += before;
+    v.w += before;
+    *reinterpret_cast<int4*>(out + base) = v;
+  } else {
+    for (int64_t i = base; i < n; ++i) out[i] += before;
+  }
 }
 
-// Cell-sorted placement, step 1: each finite point takes a slot of its cell in
-// arbitrary (atomic) order and leaves its raw index and cell there.
-__global__ void k_scatter(const int* __restrict__ cid, int64_t n, const int* __restrict__ cell_start,
-                          int* __restrict__ fill, int* __restrict__ slot_raw,
+// Cell-sorted placement, step 1: each finite point leaves its raw index and cell at
+// the slot of its cell that its place in the count names (arbitrary, atomic order).
+__global__ void k_scatter(const int* __restrict__ cid, const int* __restrict__ place, int64_t n,
+                          const int* __restrict__ cell_start, int* __restrict__ slot_raw,
                           int* __restrict__ slot_cell) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int c = cid[i];
   if (c < 0) return;
-  const int pos = cell_start[c] + wave_counter_add(fill, c);
+  const int pos = cell_start[c] + place[i];
   slot_raw[pos] = (int)i;
   slot_cell[pos] = c;
 }
@@ -262,21 +340,17 @@ __global__ void k_scatter(const int* __restrict__ cid, int64_t n, const int* __r
 // Step 2, one thread per slot: the point's final position is its cell's start plus
 // the number of the cell's points with a smaller raw index (raw order within a
 // cloud is original-index order), so points of a cell end up sorted by original
-// index whatever order step 1 produced.  The thread of a cell's first slot sets
-// the cell's step-1 counter back to zero (empty cells were never counted), so the
-// counters are all zero again for the next build.  keep_w: the input points
-// already carry their original index in w (an earlier build's sorted points).
+// index whatever order step 1 produced.  keep_w: the input points already carry
+// their original index in w (an earlier build's sorted points).
 __global__ void k_place(const float4* __restrict__ raw, const float4* __restrict__ raw_nrm,
                         const int* __restrict__ slot_raw, const int* __restrict__ slot_cell,
                         int64_t n_sorted, const int* __restrict__ cell_start,
                         const int64_t* __restrict__ cloud_off, const int* __restrict__ point_cloud,
-                        float4* __restrict__ pts, float4* __restrict__ nrm, int* __restrict__ fill,
-                        int keep_w) {
+                        float4* __restrict__ pts, float4* __restrict__ nrm, int keep_w) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n_sorted) return;
   const int c = slot_cell[j], key = slot_raw[j];
   const int b = cell_start[c], e = cell_start[c + 1];
-  if (j == b) fill[c] = 0;
   int rank = 0;
   for (int k = b; k < e; ++k) rank += slot_raw[k] < key ? 1 : 0;
   float4 p = raw[key];
@@ -486,13 +560,19 @@ inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t
 
 }  // namespace
 
-void launch_bbox(const float4* raw, const int64_t* cloud_off, int nclouds, float* part,
-                 float* out, hipStream_t s) {
-  constexpr int chunks = 64;
-  hipLaunchKernelGGL(k_bbox_partial, dim3(nclouds * chunks), dim3(kBBoxThreads), 0, s, raw,
-                     cloud_off, nclouds, chunks, part);
-  hipLaunchKernelGGL(k_bbox_final, dim3(blocks_for(nclouds, 64)), dim3(64), 0, s, part, nclouds,
-                     chunks, out);
+void launch_bbox(const float4* raw, const int64_t* cloud_off, int nclouds, float* part, float* geom,
+                 GridDesc* probe, uint32_t* probe_bits, hipStream_t s) {
+  hipLaunchKernelGGL(k_bbox_partial, dim3(nclouds * kBBoxChunks), dim3(kBBoxThreads), 0, s, raw,
+                     cloud_off, part, probe_bits);
+  hipLaunchKernelGGL(k_bbox_final, dim3(nclouds), dim3(64), 0, s, part, geom, probe);
+}
+
+void launch_probe(const float4* raw, const int64_t* cloud_off, const GridDesc* probe, int nclouds,
+                  uint32_t* probe_bits, float* geom, hipStream_t s) {
+  if (nclouds <= 0) return;
+  hipLaunchKernelGGL(k_probe, dim3(nclouds * kBBoxChunks), dim3(1024), 0, s, raw, cloud_off, probe,
+                     probe_bits);
+  hipLaunchKernelGGL(k_probe_count, dim3(nclouds), dim3(1024), 0, s, (const uint32_t*)probe_bits, geom);
 }
 
 void launch_bvh_build(const GridDesc* grids, int nclouds, int max_depth, const float4* pts,
@@ -543,49 +623,52 @@ void launch_fill_i32(int* p, int64_t n, int v, hipStream_t s) {
 }
 
 void launch_cell_count(const float4* raw, const int* point_cloud, const GridDesc* grids,
-                       int64_t n, int* cid, int* counts, int* occupied, hipStream_t s) {
+                       int64_t n, int* cid, int* counts, int* place, hipStream_t s) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_cell_count, dim3(blocks_for(n, 256)), dim3(256), 0, s, raw, point_cloud,
-                     grids, n, cid, counts, occupied);
-}
-
-void launch_occupancy(const GridDesc* grids, int nclouds, const int* counts, int* occupied,
-                      hipStream_t s) {
-  if (nclouds <= 0) return;
-  hipLaunchKernelGGL(k_occupancy, dim3(64, nclouds), dim3(256), 0, s, grids, counts, occupied);
+                     grids, n, cid, counts, place);
 }
 
 int64_t scan_tmp_ints(int64_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
 
-void launch_exclusive_scan(const int* in, int* out, int64_t n, int* tmp, hipStream_t s) {
+// Up to this many tiles (33 M elements) the last pass adds up the tile sums itself:
+// one launch less, and a block reads at most 32 KB of them; past it that would grow
+// with the square of the size.
+constexpr int64_t kScanInlineTiles = 8192;
+
+template <bool CONSUME>
+static void exclusive_scan(int* in, int* out, int64_t n, int* tmp, hipStream_t s) {
   if (n <= 0) return;
   const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL(k_scan_tiles<false>, dim3((unsigned)tiles), dim3(kScanThreads), 0, s,
-                     const_cast<int*>(in), out, n, tmp);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanThreads), 0, s, tmp, (int)tiles);
-  hipLaunchKernelGGL(k_scan_add, dim3(blocks_for(n, 256)), dim3(256), 0, s, out, n, tmp);
+  hipLaunchKernelGGL(k_scan_tiles<CONSUME>, dim3((unsigned)tiles), dim3(kScanThreads), 0, s, in, out, n,
+                     tmp);
+  if (tiles == 1) return;
+  const bool scanned = tiles > kScanInlineTiles;
+  if (scanned)
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanThreads), 0, s, tmp, (int)tiles);
+  hipLaunchKernelGGL(k_scan_add, dim3((unsigned)(tiles - 1)), dim3(kScanThreads), 0, s, out, n, tmp,
+                     scanned ? 1 : 0);
+}
+
+void launch_exclusive_scan(const int* in, int* out, int64_t n, int* tmp, hipStream_t s) {
+  exclusive_scan<false>(const_cast<int*>(in), out, n, tmp, s);
 }
 
 void launch_exclusive_scan_consume(int* in, int* out, int64_t n, int* tmp, hipStream_t s) {
-  if (n <= 0) return;
-  const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL(k_scan_tiles<true>, dim3((unsigned)tiles), dim3(kScanThreads), 0, s, in, out,
-                     n, tmp);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanThreads), 0, s, tmp, (int)tiles);
-  hipLaunchKernelGGL(k_scan_add, dim3(blocks_for(n, 256)), dim3(256), 0, s, out, n, tmp);
+  exclusive_scan<true>(in, out, n, tmp, s);
 }
 
-void launch_place_points(const float4* raw, const float4* raw_nrm, const int* cid, int64_t n_raw,
-                         int64_t n_sorted, const int* cell_start, int* fill, int* slot_raw,
+void launch_place_points(const float4* raw, const float4* raw_nrm, const int* cid, const int* place,
+                         int64_t n_raw, int64_t n_sorted, const int* cell_start, int* slot_raw,
                          int* slot_cell, const int64_t* cloud_off, const int* point_cloud,
                          float4* pts, float4* nrm, bool keep_w, hipStream_t s) {
   if (n_raw <= 0) return;
-  hipLaunchKernelGGL(k_scatter, dim3(blocks_for(n_raw, 256)), dim3(256), 0, s, cid, n_raw,
-                     cell_start, fill, slot_raw, slot_cell);
+  hipLaunchKernelGGL(k_scatter, dim3(blocks_for(n_raw, 256)), dim3(256), 0, s, cid, place, n_raw,
+                     cell_start, slot_raw, slot_cell);
   if (n_sorted <= 0) return;
   hipLaunchKernelGGL(k_place, dim3(blocks_for(n_sorted, 256)), dim3(256), 0, s, raw, raw_nrm,
                      slot_raw, slot_cell, n_sorted, cell_start, cloud_off, point_cloud, pts, nrm,
-                     fill, keep_w ? 1 : 0);
+                     keep_w ? 1 : 0);
 }
 
 }  // namespace lcr

@@ -8,6 +8,7 @@
 //   * per source tile: FP64 partial sums written by the tile's block.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 namespace lcr {
@@ -42,6 +43,37 @@ struct GridDesc {
 
 // 32-bit words per x-row of a grid's cell mask: bit x & 31 of word x >> 5.
 __host__ __device__ inline int near_row_words(int nx) { return (nx + 31) >> 5; }
+
+// Per cloud what a build measures first: box min xyz, max xyz, finite count, occupied
+// probe cells (an int's bits).
+constexpr int kGeomWords = 8;
+// The probe grid (at most 65 cells per axis) as one bit per cell.
+constexpr int kProbeWords = (65 * 65 * 65 + 31) / 32;
+
+// The probe grid over a cloud's box b (kGeomWords layout): 64 cells on the longest
+// axis, to measure how many cells the points occupy.  The same on host and device.
+__host__ __device__ inline GridDesc probe_grid(const float* b) {
+  GridDesc g{};
+  g.npts = (int)b[6];
+  if (g.npts == 0) {
+    g.ox = g.oy = g.oz = 0.f;
+    g.h = 1.f;
+    g.inv_h = 1.f;
+    g.nx = g.ny = g.nz = 1;
+    return g;
+  }
+  const double ex = (double)b[3] - b[0], ey = (double)b[4] - b[1], ez = (double)b[5] - b[2];
+  const double h0 = fmax(fmax(ex, fmax(ey, ez)) / 64.0, 1e-6);
+  g.ox = b[0];
+  g.oy = b[1];
+  g.oz = b[2];
+  g.h = (float)h0;
+  g.inv_h = (float)(1.0 / h0);
+  g.nx = (int)fmin(floor(ex / h0) + 1, 65.0);
+  g.ny = (int)fmin(floor(ey / h0) + 1, 65.0);
+  g.nz = (int)fmin(floor(ez / h0) + 1, 65.0);
+  return g;
+}
 
 // Points per leaf of the bounding-volume tree over a cloud's points.
 constexpr int kLeaf = 16;

@@ -9,25 +9,31 @@
 namespace lcr {
 
 // ---- K1 grid build (grid.hip)
-void launch_bbox(const float4* raw, const int64_t* cloud_off, int nclouds, float* part,
-                 float* out, hipStream_t s);
-constexpr int kBBoxChunks = 64;  // partial boxes per cloud (part holds 7 floats each)
+// Per cloud its box and finite count (geom: kGeomWords floats each; part holds
+// kBBoxChunks * 7 floats each); with probe and probe_bits (nullable, kProbeWords
+// words each) also its probe grid and that grid's bits, clear.
+void launch_bbox(const float4* raw, const int64_t* cloud_off, int nclouds, float* part, float* geom,
+                 GridDesc* probe, uint32_t* probe_bits, hipStream_t s);
+constexpr int kBBoxChunks = 64;  // partial boxes per cloud
+// After launch_bbox: the occupied cells of every cloud's probe grid, into geom.
+void launch_probe(const float4* raw, const int64_t* cloud_off, const GridDesc* probe, int nclouds,
+                  uint32_t* probe_bits, float* geom, hipStream_t s);
 void launch_fill_i32(int* p, int64_t n, int v, hipStream_t s);
+// Per point its global cell (cid, -1: not finite) and its place among the cell's
+// points (atomic order); counts, zero on entry, holds the points per cell after.
 void launch_cell_count(const float4* raw, const int* point_cloud, const GridDesc* grids,
-                       int64_t n, int* cid, int* counts, int* occupied, hipStream_t s);
-void launch_occupancy(const GridDesc* grids, int nclouds, const int* counts, int* occupied,
-                      hipStream_t s);
+                       int64_t n, int* cid, int* counts, int* place, hipStream_t s);
+// Exclusive scans of n ints; in and out start on 16 bytes, tmp holds scan_tmp_ints(n).
 int64_t scan_tmp_ints(int64_t n);
 void launch_exclusive_scan(const int* in, int* out, int64_t n, int* tmp, hipStream_t s);
 // The same, setting the input to zero as it is read.
 void launch_exclusive_scan_consume(int* in, int* out, int64_t n, int* tmp, hipStream_t s);
 // Places every finite input point at its cell-sorted position (cells in order,
-// points of a cell by input index); fill must be zero on entry and is zero again
-// on exit, slot_* hold n_sorted ints.  The input is the raw upload (w set to the
-// point's index in its cloud) or, with keep_w, an earlier build's sorted points
-// (w already holds it).
-void launch_place_points(const float4* raw, const float4* raw_nrm, const int* cid, int64_t n_raw,
-                         int64_t n_sorted, const int* cell_start, int* fill, int* slot_raw,
+// points of a cell by input index) from launch_cell_count's cid and place; slot_*
+// hold n_sorted ints.  The input is the raw upload (w set to the point's index in
+// its cloud) or, with keep_w, an earlier build's sorted points (w already holds it).
+void launch_place_points(const float4* raw, const float4* raw_nrm, const int* cid, const int* place,
+                         int64_t n_raw, int64_t n_sorted, const int* cell_start, int* slot_raw,
                          int* slot_cell, const int64_t* cloud_off, const int* point_cloud,
                          float4* pts, float4* nrm, bool keep_w, hipStream_t s);
 // Dilated occupancy per cell, one bit (set: some point within r of the cell):

@@ -189,12 +189,11 @@ namespace {
 // Disjoint regions of the pinned scratch used by one grid build (async copies of
 // different regions may be in flight together).
 struct BuildRegions {
-  size_t bbox, occ, grids, poff, total;
+  size_t geom, grids, poff, total;
   explicit BuildRegions(int n) {
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
-    bbox = 0;
-    occ = al(bbox + (size_t)n * 7 * sizeof(float));
-    grids = al(occ + (size_t)n * sizeof(int));
+    geom = 0;
+    grids = al(geom + (size_t)n * kGeomWords * sizeof(float));
     poff = al(grids + (size_t)n * sizeof(GridDesc));
     total = al(poff + (size_t)(n + 1) * sizeof(int64_t));
   }
@@ -221,87 +220,52 @@ void CloudSet::build(hipStream_t s, double factor, std::vector<Profiler::Span>* 
   const BuildRegions R(n);
   h_build.reserve(R.total);
   char* hb = h_build.as<char>();
-  float* bb = reinterpret_cast<float*>(hb + R.bbox);
-  int* occ = reinterpret_cast<int*>(hb + R.occ);
   GridDesc* hg = reinterpret_cast<GridDesc*>(hb + R.grids);
   int64_t* hpoff = reinterpret_cast<int64_t*>(hb + R.poff);
   const int span = prof.begin("grid_build", s, spans);
-  // 1. bounding boxes and finite counts (and 2.'s probe occupancy) depend only on
-  //    the uploaded points: measured once per upload
+  // 1. bounding boxes, finite counts and the probe grids' (<= 65 cells on the longest
+  //    axis) occupied cells depend only on the uploaded points: measured once per
+  //    upload, in one go
+  d_grids.reserve((size_t)n * sizeof(GridDesc));
   if (!geom_valid) {
     d_bbox_part.reserve((size_t)n * kBBoxChunks * 7 * sizeof(float));
-    d_bbox.reserve((size_t)n * 7 * sizeof(float));
+    d_geom.reserve((size_t)n * kGeomWords * sizeof(float));
+    d_probe.reserve((size_t)n * kProbeWords * sizeof(uint32_t));
     launch_bbox(d_raw.as<float4>(), d_cloud_off.as<int64_t>(), n, d_bbox_part.as<float>(),
-                d_bbox.as<float>(), s);
-    LCR_HIP(hipMemcpyAsync(bb, d_bbox.p, (size_t)n * 7 * sizeof(float), hipMemcpyDeviceToHost, s));
+                d_geom.as<float>(), d_grids.as<GridDesc>(), d_probe.as<uint32_t>(), s);
+    launch_probe(d_raw.as<float4>(), d_cloud_off.as<int64_t>(), d_grids.as<GridDesc>(), n,
+                 d_probe.as<uint32_t>(), d_geom.as<float>(), s);
+    float* hgeom = reinterpret_cast<float*>(hb + R.geom);
+    LCR_HIP(hipMemcpyAsync(hgeom, d_geom.p, (size_t)n * kGeomWords * sizeof(float),
+                           hipMemcpyDeviceToHost, s));
     LCR_HIP(hipStreamSynchronize(s));
-    geom_box.assign(bb, bb + (size_t)n * 7);
-  }
-  const std::vector<float>& box = geom_box;
-
-  // 2. probe grid (<= 65 cells on the longest axis) to measure occupancy
-  grids.assign(n, GridDesc{});
-  int64_t cells = 0;
-  for (int c = 0; c < n; ++c) {
-    GridDesc& g = grids[c];
-    const float* b = &box[(size_t)c * 7];
-    g.npts = (int)b[6];
-    g.nraw = (int)nraw[c];
-    if (g.npts == 0) {
-      g.ox = g.oy = g.oz = 0.f;
-      g.h = 1.f;
-      g.inv_h = 1.f;
-      g.nx = g.ny = g.nz = 1;
-    } else {
-      const double ext = std::max({(double)b[3] - b[0], (double)b[4] - b[1], (double)b[5] - b[2]});
-      const double h0 = std::max(ext / 64.0, 1e-6);
-      g.ox = b[0];
-      g.oy = b[1];
-      g.oz = b[2];
-      g.h = (float)h0;
-      g.inv_h = (float)(1.0 / h0);
-      g.nx = (int)std::min<double>(floor(((double)b[3] - b[0]) / h0) + 1, 65);
-      g.ny = (int)std::min<double>(floor(((double)b[4] - b[1]) / h0) + 1, 65);
-      g.nz = (int)std::min<double>(floor(((double)b[5] - b[2]) / h0) + 1, 65);
-    }
-    g.cell_off = cells;
-    g.near_r = 0.0f;
-    g.near_off = 0;
-    cells += (int64_t)g.nx * g.ny * g.nz + 1;
-  }
-  d_grids.reserve((size_t)n * sizeof(GridDesc));
-  d_cid.reserve((size_t)std::max<int64_t>(total_raw, 1) * sizeof(int));
-  if (!geom_valid) {
-    d_counts.reserve((size_t)cells * sizeof(int));
-    counts_zero = false;  // the probe counts below stay in the array
-    d_occ.reserve((size_t)n * sizeof(int));
-    memcpy(hg, grids.data(), (size_t)n * sizeof(GridDesc));
-    LCR_HIP(hipMemcpyAsync(d_grids.p, hg, (size_t)n * sizeof(GridDesc), hipMemcpyHostToDevice, s));
-    launch_fill_i32(d_counts.as<int>(), cells, 0, s);
-    launch_fill_i32(d_occ.as<int>(), n, 0, s);
-    launch_cell_count(d_raw.as<float4>(), d_point_cloud.as<int>(), d_grids.as<GridDesc>(),
-                      total_raw, d_cid.as<int>(), d_counts.as<int>(), nullptr, s);
-    launch_occupancy(d_grids.as<GridDesc>(), n, d_counts.as<int>(), d_occ.as<int>(), s);
-    LCR_HIP(hipMemcpyAsync(occ, d_occ.p, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, s));
-    LCR_HIP(hipStreamSynchronize(s));
-    geom_occ.assign(occ, occ + n);
+    geom.assign(hgeom, hgeom + (size_t)n * kGeomWords);
     geom_valid = true;
-  } else {
-    memcpy(occ, geom_occ.data(), (size_t)n * sizeof(int));
   }
+
+  // 2. the probe grids
+  grids.assign(n, GridDesc{});
+  for (int c = 0; c < n; ++c) {
+    grids[c] = probe_grid(&geom[(size_t)c * kGeomWords]);
+    grids[c].nraw = (int)nraw[c];
+  }
+  d_cid.reserve((size_t)std::max<int64_t>(total_raw, 1) * sizeof(int));
+  d_place.reserve((size_t)std::max<int64_t>(total_raw, 1) * sizeof(int));
 
   // 3. final cell edge: factor * spacing, spacing ~ h0 / sqrt(points per occupied
   //    probe cell) for surface-sampled clouds; capped cell count and extent
-  cells = 0;
+  int64_t cells = 0;
   total_pts = 0;
   for (int c = 0; c < n; ++c) {
     GridDesc& g = grids[c];
-    const float* b = &box[(size_t)c * 7];
+    const float* b = &geom[(size_t)c * kGeomWords];
+    int occ;
+    memcpy(&occ, b + 7, sizeof occ);
     g.pt_off = total_pts;
     total_pts += g.npts;
     if (g.npts > 0) {
       const double h0 = g.h;
-      const double per_cell = (double)g.npts / std::max(occ[c], 1);
+      const double per_cell = (double)g.npts / std::max(occ, 1);
       const double spacing = h0 / sqrt(std::max(per_cell, 1.0));
       double h = std::max(factor * spacing, 1e-6);
       const double ex = (double)b[3] - b[0], ey = (double)b[4] - b[1], ez = (double)b[5] - b[2];
@@ -342,9 +306,8 @@ void CloudSet::build(hipStream_t s, double factor, std::vector<Profiler::Span>* 
   LCR_HIP(hipMemcpyAsync(d_grids.p, hg, (size_t)n * sizeof(GridDesc), hipMemcpyHostToDevice, s));
 
   // 4. count, scan, scatter, per-cell sort.  The counters are zero over the whole
-  // allocation between builds (the scan consumes the counts, the placement
-  // clears its slot counters), so they are filled only after a reallocation or
-  // the geometry probe.
+  // allocation between builds (the scan consumes the counts), so they are filled
+  // only after a reallocation.
   const void* counts_before = d_counts.p;
   d_counts.reserve((size_t)cells * sizeof(int));
   if (d_counts.p != counts_before) counts_zero = false;
@@ -366,13 +329,13 @@ void CloudSet::build(hipStream_t s, double factor, std::vector<Profiler::Span>* 
   if (!counts_zero) launch_fill_i32(d_counts.as<int>(), (int64_t)(d_counts.bytes / sizeof(int)), 0, s);
   counts_zero = false;
   launch_cell_count(in_pts, in_cloud, d_grids.as<GridDesc>(), n_in, d_cid.as<int>(),
-                    d_counts.as<int>(), nullptr, s);
+                    d_counts.as<int>(), d_place.as<int>(), s);
   launch_exclusive_scan_consume(d_counts.as<int>(), d_cell_start.as<int>(), cells,
                                 d_scan_tmp.as<int>(), s);
   d_slot_raw.reserve(npts * sizeof(int));
   d_slot_cell.reserve(npts * sizeof(int));
-  launch_place_points(in_pts, in_nrm, d_cid.as<int>(), n_in, total_pts, d_cell_start.as<int>(),
-                      d_counts.as<int>(), d_slot_raw.as<int>(), d_slot_cell.as<int>(),
+  launch_place_points(in_pts, in_nrm, d_cid.as<int>(), d_place.as<int>(), n_in, total_pts,
+                      d_cell_start.as<int>(), d_slot_raw.as<int>(), d_slot_cell.as<int>(),
                       d_cloud_off.as<int64_t>(), d_point_cloud.as<int>(), out_pts.as<float4>(),
                       out_nrm.as<float4>(), from_normals, s);
   if (from_normals) has_nrm = true;

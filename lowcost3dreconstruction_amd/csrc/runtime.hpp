@@ -117,10 +117,9 @@ struct CloudSet {
   bool has_nrm = false;
   std::vector<GridDesc> grids;
   int64_t total_pts = 0, total_cells = 0, total_nodes = 0;
-  // per cloud: bounding box + finite count (7 floats) and occupied probe cells,
+  // per cloud: bounding box, finite count and occupied probe cells (kGeomWords),
   // measured by the first build after an upload
-  std::vector<float> geom_box;
-  std::vector<int> geom_occ;
+  std::vector<float> geom;
   bool geom_valid = false;
   // recorded after the last copy out of the pinned build region / viewpoint
   // buffer: the next build or normals pass waits on it before rewriting them
@@ -137,9 +136,9 @@ struct CloudSet {
   int max_depth = 0;
 
   DevBuf d_raw, d_raw_nrm, d_point_cloud, d_cloud_off;
-  DevBuf d_grids, d_counts, d_cell_start, d_cid, d_scan_tmp, d_bbox_part, d_bbox, d_occ;
+  DevBuf d_grids, d_counts, d_cell_start, d_cid, d_place, d_scan_tmp, d_bbox_part, d_geom, d_probe;
   // d_counts is zero over its whole allocation once the stream has run the work
-  // issued so far (each build leaves it so; the geometry probe does not)
+  // issued so far (each build leaves it so)
   bool counts_zero = false;
   DevBuf d_pts, d_nrm, d_cloud_of_sorted, d_vp, d_poff, d_nodes, d_nbr, d_nsel;
   DevBuf d_npts, d_nnrm;  // the normals stage's sorted points and normals

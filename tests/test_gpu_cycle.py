@@ -216,3 +216,25 @@ def test_hypothesis_gate_keeps_the_seed_and_the_best_initial_pose(lcr, small_cyc
             np.testing.assert_array_equal(inst["T"][i * H + h], icp.getFinalTransformation())
             assert inst["fitness"][i * H + h] == icp.getFitnessScore()
         np.testing.assert_array_equal(c.initial_poses()[i * H:(i + 1) * H], guesses[i * H:(i + 1) * H])
+
+
+def test_batch_of_more_than_33m_cells_equals_single_pairs(lcr):
+    """Thin diagonal clouds whose boxes take the capped cell count: five of them hold
+    more cells than one scan adds up without its extra pass (8192 tiles of 4096); a
+    pair's own build stays below.  Bitwise the same transforms."""
+    rng = np.random.default_rng(21)
+    clouds = []
+    for i in range(5):
+        t = rng.uniform(0, 1, size=(830_000, 1))
+        clouds.append((t * np.array([[1.0, 0.9, 0.8]]) + rng.normal(scale=2e-3, size=(len(t), 3))
+                       + 1e-4 * i).astype(np.float32))
+    print_case(test="large_scan")
+    kw = dict(max_corr_dist=0.002, max_iterations=2, point_to_plane=False)
+    c = lcr.Cycle(clouds, [(1, 0), (4, 3)], **kw)
+    c.run()
+    T = c.results()["T"]
+    del c
+    for p, (s, t) in enumerate([(1, 0), (4, 3)]):
+        one = lcr.Cycle([clouds[s], clouds[t]], [(0, 1)], **kw)
+        one.run()
+        np.testing.assert_array_equal(one.results()["T"][0], T[p])
