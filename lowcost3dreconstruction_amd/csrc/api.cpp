@@ -742,11 +742,11 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
       nvox *= L.div[a];
     }
     if (nvox > ((int64_t)1 << 30)) return fail(LCR_E_LIMIT, "voxel lattice larger than 2^30");
-    DevBuf skey, skey_sorted, idx, sorted_raw, counts, start, flags, outidx, scan_tmp, sort_tmp,
-        dcurv, drgb, ox, on, oc, orgb;
-    for (DevBuf* v : {&skey, &skey_sorted, &idx, &sorted_raw}) v->reserve((size_t)n * sizeof(int));
-    for (DevBuf* v : {&counts, &start, &flags, &outidx}) v->reserve((size_t)nvox * sizeof(int));
-    scan_tmp.reserve((size_t)scan_tmp_ints(nvox) * sizeof(int));
+    DevBuf skey, skey_sorted, idx, sorted_raw, heads, outidx, scan_tmp, sort_tmp, dcurv, drgb, ox, on,
+        oc, orgb;
+    for (DevBuf* v : {&skey, &skey_sorted, &idx, &sorted_raw, &heads, &outidx})
+      v->reserve((size_t)n * sizeof(int));
+    scan_tmp.reserve((size_t)scan_tmp_ints(n) * sizeof(int));
     const size_t sort_bytes = voxel_sort_tmp_bytes(n, nvox);
     if (sort_bytes == 0) return fail(LCR_E_HIP, "voxel sort: no temporary size");
     sort_tmp.reserve(sort_bytes);
@@ -763,8 +763,7 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
     if (curv && out_curv) oc.reserve((size_t)nfin * sizeof(float));
     if (rgb && out_rgb) orgb.reserve((size_t)nfin * 3);
     VoxScratch w{skey.as<uint32_t>(), skey_sorted.as<uint32_t>(), idx.as<int>(), sorted_raw.as<int>(),
-                 counts.as<int>(), start.as<int>(), flags.as<int>(), outidx.as<int>(),
-                 scan_tmp.as<int>(), sort_tmp.p, sort_bytes};
+                 heads.as<int>(), outidx.as<int>(), scan_tmp.as<int>(), sort_tmp.p, sort_bytes};
     LCR_HIP(launch_voxel_grid(cs.d_raw.as<float4>(),
                               (nrm && cs.has_nrm) ? cs.d_raw_nrm.as<float4>() : nullptr,
                               curv ? dcurv.as<float>() : nullptr, rgb ? drgb.as<uint8_t>() : nullptr,
@@ -772,12 +771,12 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
                               oc.p ? oc.as<float>() : nullptr, orgb.p ? orgb.as<uint8_t>() : nullptr,
                               st.s));
     int last[2];
-    LCR_HIP(hipMemcpyAsync(&last[0], outidx.as<int>() + nvox - 1, sizeof(int), hipMemcpyDeviceToHost,
+    LCR_HIP(hipMemcpyAsync(&last[0], outidx.as<int>() + n - 1, sizeof(int), hipMemcpyDeviceToHost,
                            st.s));
-    LCR_HIP(hipMemcpyAsync(&last[1], counts.as<int>() + nvox - 1, sizeof(int), hipMemcpyDeviceToHost,
+    LCR_HIP(hipMemcpyAsync(&last[1], heads.as<int>() + n - 1, sizeof(int), hipMemcpyDeviceToHost,
                            st.s));
     LCR_HIP(hipStreamSynchronize(st.s));
-    const int64_t nocc = (int64_t)last[0] + (last[1] > 0 ? 1 : 0);
+    const int64_t nocc = (int64_t)last[0] + last[1];
     LCR_HIP(hipMemcpyAsync(out_xyz, ox.p, (size_t)nocc * 3 * sizeof(float), hipMemcpyDeviceToHost,
                            st.s));
     if (on.p)

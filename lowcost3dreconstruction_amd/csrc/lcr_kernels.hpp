@@ -172,11 +172,9 @@ struct VoxScratch {
   uint32_t* skey_sorted;   // n
   int* idx;                // n: input index per point
   int* sorted_raw;         // n: input indices in (voxel, input index) order
-  int* counts;             // nvox
-  int* start;              // nvox
-  int* flags;              // nvox
-  int* outidx;             // nvox
-  int* scan_tmp;           // scan_tmp_ints(nvox)
+  int* heads;              // n: 1 at the first sorted point of each occupied voxel
+  int* outidx;             // n: their prefix sum (the voxel's output)
+  int* scan_tmp;           // scan_tmp_ints(n)
   void* sort_tmp;          // voxel_sort_tmp_bytes(n, nvox)
   size_t sort_tmp_bytes;
 };

@@ -161,3 +161,26 @@ def test_normals_on_small_clouds(lcr, kind, n, k):
     dots = np.sum(nrm.astype(np.float64) * rn, axis=1)
     assert np.all(dots > 1 - 1e-6), np.sort(dots)[:5]
     np.testing.assert_allclose(curv, rc, rtol=2e-6, atol=1e-9)
+
+
+@pytest.mark.parametrize("sizes", [(1, 15, 16, 17, 2, 63, 64, 65, 1, 128, 129, 3), (16,) * 9 + (1,),
+                                   (17,) * 30, (1, 1, 61, 2, 700, 1)])
+def test_voxel_grid_run_lengths(lcr, sizes):
+    """Voxels of chosen point counts, shuffled, with non-finite points in between:
+    runs that end inside a wavefront's 64 sorted points, cross into the next ones or
+    span several, on both sides of the lane sums' limit of 16.  Bitwise equal to the
+    oracle (the same order of additions)."""
+    rng = np.random.default_rng(len(sizes))
+    pts = np.concatenate([rng.uniform(0.05, 0.95, size=(s, 3)) + [v % 5, (v // 5) % 4, v // 20]
+                          for v, s in enumerate(sizes)])
+    pts = pts[rng.permutation(len(pts))].astype(np.float32)
+    pts = np.insert(pts, [0, len(pts) // 2, len(pts)], np.nan, axis=0)
+    nrm = rng.normal(size=pts.shape).astype(np.float32)
+    curv = rng.uniform(0, 0.3, size=len(pts)).astype(np.float32)
+    rgb = rng.integers(0, 256, size=pts.shape).astype(np.uint8)
+    print_case(test="voxel_runs", n=len(pts))
+    got = lcr.voxel_grid(pts, 1.0, nrm=nrm, curv=curv, rgb=rgb)
+    ref = oracle.voxel_grid(pts, 1.0, nrm=nrm, curv=curv, rgb=rgb)
+    assert len(got["xyz"]) == len(ref["xyz"]) == len(sizes)
+    for k in ("xyz", "nrm", "curv", "rgb"):
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
