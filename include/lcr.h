@@ -287,7 +287,7 @@ int lcr_depth_fuse(const uint16_t *frames, int32_t n_frames, int32_t width, int3
  * out_nrm and out_rgb nullable), *out_n is written on the device (one int64), and
  * the work is enqueued on `stream` (a hipStream_t; NULL = the null stream)
  * without waiting for it; intrinsics and crop stay host arrays.  Nothing is
- * allocated: the kernels' scratch is a fixed array of 8 MiB per device, taken by
+ * allocated: the kernels' scratch is a fixed array of 4 KiB per device, taken by
  * lcr_init or on the first call on a device.  width * height must be at most
  * LCR_NOALLOC_MAX_PIXELS (else LCR_E_LIMIT).  Every call on a device shares its
  * scratch, so calls that overlap on one device (other streams, other threads)

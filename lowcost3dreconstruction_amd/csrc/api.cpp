@@ -863,30 +863,24 @@ int lcr_depth_to_cloud(const uint16_t* depth, int32_t width, int32_t height, con
     P.left = crop ? crop[2] : 0;
     P.right = crop ? crop[3] : width - 1;
     Stream st;
-    DevBuf dd, dc, flags, pos, tmp, ox, on, orgb;
+    DevBuf dd, dc, scratch, dn, ox, on, orgb;
     dd.reserve((size_t)np * sizeof(uint16_t));
     LCR_HIP(hipMemcpyAsync(dd.p, depth, (size_t)np * sizeof(uint16_t), hipMemcpyHostToDevice, st.s));
     if (color) {
       dc.reserve((size_t)np * 3);
       LCR_HIP(hipMemcpyAsync(dc.p, color, (size_t)np * 3, hipMemcpyHostToDevice, st.s));
     }
-    flags.reserve((size_t)np * sizeof(int));
-    pos.reserve((size_t)np * sizeof(int));
-    tmp.reserve((size_t)scan_tmp_ints(np) * sizeof(int));
-    launch_depth_flags(dd.as<uint16_t>(), width, height, P, flags.as<int>(), st.s);
-    launch_exclusive_scan(flags.as<int>(), pos.as<int>(), np, tmp.as<int>(), st.s);
-    int last[2];
-    LCR_HIP(hipMemcpyAsync(&last[0], pos.as<int>() + np - 1, sizeof(int), hipMemcpyDeviceToHost, st.s));
-    LCR_HIP(hipMemcpyAsync(&last[1], flags.as<int>() + np - 1, sizeof(int), hipMemcpyDeviceToHost,
-                           st.s));
+    scratch.reserve((size_t)depth_scratch_ints(np) * sizeof(int));
+    dn.reserve(sizeof(int64_t));
+    ox.reserve((size_t)np * 3 * sizeof(float));
+    if (out_nrm) on.reserve((size_t)np * 3 * sizeof(float));
+    if (out_rgb && color) orgb.reserve((size_t)np * 3);
+    launch_depth_cloud(dd.as<uint16_t>(), width, height, color ? dc.as<uint8_t>() : nullptr, P,
+                       scratch.as<int>(), ox.as<float>(), on.p ? on.as<float>() : nullptr,
+                       orgb.p ? orgb.as<uint8_t>() : nullptr, dn.as<int64_t>(), st.s);
+    int64_t m = 0;
+    LCR_HIP(hipMemcpyAsync(&m, dn.p, sizeof m, hipMemcpyDeviceToHost, st.s));
     LCR_HIP(hipStreamSynchronize(st.s));
-    const int64_t m = (int64_t)last[0] + last[1];
-    ox.reserve((size_t)std::max<int64_t>(m, 1) * 3 * sizeof(float));
-    if (out_nrm) on.reserve((size_t)std::max<int64_t>(m, 1) * 3 * sizeof(float));
-    if (out_rgb && color) orgb.reserve((size_t)std::max<int64_t>(m, 1) * 3);
-    launch_depth_points(dd.as<uint16_t>(), width, height, color ? dc.as<uint8_t>() : nullptr, P,
-                        pos.as<int>(), ox.as<float>(), on.p ? on.as<float>() : nullptr,
-                        orgb.p ? orgb.as<uint8_t>() : nullptr, st.s);
     if (m > 0) {
       LCR_HIP(hipMemcpyAsync(out_xyz, ox.p, (size_t)m * 3 * sizeof(float), hipMemcpyDeviceToHost, st.s));
       if (on.p)

@@ -18,9 +18,10 @@
 // two-level reduction) and the keep flags.
 //
 // K13 replaces the depth tool's cross-product normals and back-projection
-// (capture/depth_capture/depth_capture.cpp:230-305) for a 16-bit depth map:
-// per-pixel validity, a prefix sum for row-major output positions, then the
-// points, normals and colours.
+// (capture/depth_capture/depth_capture.cpp:230-305) for a 16-bit depth map: the
+// valid pixels of each 1024-pixel tile are counted, then a block per tile adds the
+// counts before its own up, ranks its pixels (row-major output positions) and
+// writes points, normals and colours.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -255,23 +256,80 @@ __device__ __forceinline__ bool depth_valid(const DepthParams& P, int z, int i, 
          j >= P.left && j <= P.right;
 }
 
-__global__ void k_depth_flags(const uint16_t* __restrict__ depth, int w, int h, DepthParams P,
-                              int* __restrict__ flags) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= (int64_t)w * h) return;
-  const int i = (int)(p / w), j = (int)(p % w);
-  flags[p] = depth_valid(P, depth[p], i, j) ? 1 : 0;
+// Valid pixels per tile of kDepthTile pixels: four pixels per thread.  vec: the map
+// starts on 8 bytes, so four depths come in one load.
+constexpr int kDepthTile = 1024;
+
+__global__ void __launch_bounds__(kDepthTile / 4)
+k_depth_count(const uint16_t* __restrict__ depth, int w, int h, DepthParams P, int vec,
+              int* __restrict__ counts) {
+  __shared__ int s[kDepthTile / 256];
+  const int64_t np = (int64_t)w * h;
+  const int64_t p = (int64_t)blockIdx.x * kDepthTile + 4 * threadIdx.x;
+  int z[4] = {0, 0, 0, 0};
+  if (vec && p + 4 <= np) {
+    const ushort4 v = *reinterpret_cast<const ushort4*>(depth + p);
+    z[0] = v.x;
+    z[1] = v.y;
+    z[2] = v.z;
+    z[3] = v.w;
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (p + u < np) z[u] = depth[p + u];
+  }
+  int i = (int)(p / w), j = (int)(p % w), c = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    c += __popcll(__ballot(depth_valid(P, z[u], i, j)));  // z = 0 past the end: not valid
+    if (++j == w) {
+      j = 0;
+      ++i;
+    }
+  }
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) counts[blockIdx.x] = s[0] + s[1] + s[2] + s[3];
 }
 
-__global__ void k_depth_points(const uint16_t* __restrict__ depth, int w, int h,
-                               const uint8_t* __restrict__ color, DepthParams P,
-                               const int* __restrict__ pos, float* __restrict__ out_xyz,
-                               float* __restrict__ out_nrm, uint8_t* __restrict__ out_rgb) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= (int64_t)w * h) return;
+// One pixel per thread, a block per tile.  scanned: counts holds the tiles'
+// exclusive scan (then its last entry and the last tile's own count give *out_n);
+// else each block adds the counts before its own.
+__global__ void __launch_bounds__(kDepthTile)
+k_depth_points(const uint16_t* __restrict__ depth, int w, int h, const uint8_t* __restrict__ color,
+               DepthParams P, const int* __restrict__ counts, int scanned,
+               float* __restrict__ out_xyz, float* __restrict__ out_nrm,
+               uint8_t* __restrict__ out_rgb, int64_t* __restrict__ out_n) {
+  constexpr int kW = kDepthTile / 64;
+  __shared__ int s_before[kW], s_valid[kW];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int64_t np = (int64_t)w * h;
+  const int64_t p = (int64_t)blockIdx.x * kDepthTile + t;
   const int i = (int)(p / w), j = (int)(p % w);
-  const int z = depth[p];
-  if (!depth_valid(P, z, i, j)) return;
+  const int z = p < np ? depth[p] : 0;
+  const bool valid = depth_valid(P, z, i, j);
+  const uint64_t m = __ballot(valid);
+  int a = 0;
+  if (!scanned)
+    for (int k = t; k < (int)blockIdx.x; k += kDepthTile) a += counts[k];
+  else if (t == 0)
+    a = counts[blockIdx.x];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+  if (lane == 0) {
+    s_before[wv] = a;
+    s_valid[wv] = __popcll(m);
+  }
+  __syncthreads();
+  int o = 0, total = 0;
+#pragma unroll
+  for (int k = 0; k < kW; ++k) {
+    total += s_before[k] + s_valid[k];
+    o += s_before[k] + (k < wv ? s_valid[k] : 0);
+  }
+  if (t == 0 && blockIdx.x == gridDim.x - 1) *out_n = total;
+  if (!valid) return;
+  o += __popcll(m & ((1ull << lane) - 1ull));
   int rt = 0, lf = 0, dn = 0, up = 0;
   if (i > 0 && j > 0 && i < h - 1 && j < w - 1) {
     rt = depth[p + w];
@@ -288,25 +346,20 @@ __global__ void k_depth_points(const uint16_t* __restrict__ depth, int w, int h,
   const double inv = 1.0 / sqrt(vx * vx + vy * vy + vz * vz);
   const double px = (double)z * (j - P.cx) * (1 / P.fx);
   const double py = -(double)z * (i - P.cy) * (1 / P.fy);
-  const int64_t m = pos[p];
-  out_xyz[3 * m] = (float)px;
-  out_xyz[3 * m + 1] = (float)py;
-  out_xyz[3 * m + 2] = (float)(-z);
+  const int64_t q = 3 * (int64_t)o;
+  out_xyz[q] = (float)px;
+  out_xyz[q + 1] = (float)py;
+  out_xyz[q + 2] = (float)(-z);
   if (out_nrm) {
-    out_nrm[3 * m] = (float)(vx * inv);
-    out_nrm[3 * m + 1] = (float)(vy * inv);
-    out_nrm[3 * m + 2] = (float)(vz * inv);
+    out_nrm[q] = (float)(vx * inv);
+    out_nrm[q + 1] = (float)(vy * inv);
+    out_nrm[q + 2] = (float)(vz * inv);
   }
   if (out_rgb && color) {
-    out_rgb[3 * m] = color[3 * p];
-    out_rgb[3 * m + 1] = color[3 * p + 1];
-    out_rgb[3 * m + 2] = color[3 * p + 2];
+    out_rgb[q] = color[3 * p];
+    out_rgb[q + 1] = color[3 * p + 1];
+    out_rgb[q + 2] = color[3 * p + 2];
   }
-}
-
-__global__ void k_depth_count(const int* __restrict__ pos, const int* __restrict__ flags, int64_t n,
-                              int64_t* __restrict__ out_n) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *out_n = (int64_t)pos[n - 1] + flags[n - 1];
 }
 
 }  // namespace
@@ -365,26 +418,34 @@ void launch_sor_stats(const float* dist, const uint8_t* finite, int64_t n, doubl
     hipLaunchKernelGGL(k_sor_keep, dim3(blocks_of(n, 256)), dim3(256), 0, s, dist, n, stats, keep);
 }
 
-void launch_depth_flags(const uint16_t* depth, int w, int h, const DepthParams& P, int* flags,
-                        hipStream_t s) {
-  const int64_t np = (int64_t)w * h;
-  if (np <= 0) return;
-  hipLaunchKernelGGL(k_depth_flags, dim3(blocks_of(np, 256)), dim3(256), 0, s, depth, w, h, P,
-                     flags);
+// Up to this many tiles (4 M pixels) a block adds the counts before its own itself:
+// at most four per thread; past it they are scanned first.
+constexpr int64_t kDepthInlineTiles = 4096;
+
+int64_t depth_tiles(int64_t pixels) { return (pixels + kDepthTile - 1) / kDepthTile; }
+
+int64_t depth_scratch_ints(int64_t pixels) {
+  const int64_t t = depth_tiles(pixels);
+  return t <= kDepthInlineTiles ? t : ((t + 3) & ~(int64_t)3) * 2 + scan_tmp_ints(t);
 }
 
-void launch_depth_points(const uint16_t* depth, int w, int h, const uint8_t* color,
-                         const DepthParams& P, const int* pos, float* out_xyz, float* out_nrm,
-                         uint8_t* out_rgb, hipStream_t s) {
+void launch_depth_cloud(const uint16_t* depth, int w, int h, const uint8_t* color,
+                        const DepthParams& P, int* scratch, float* out_xyz, float* out_nrm,
+                        uint8_t* out_rgb, int64_t* out_n, hipStream_t s) {
   const int64_t np = (int64_t)w * h;
   if (np <= 0) return;
-  hipLaunchKernelGGL(k_depth_points, dim3(blocks_of(np, 256)), dim3(256), 0, s, depth, w, h, color,
-                     P, pos, out_xyz, out_nrm, out_rgb);
-}
-
-void launch_depth_count(const int* pos, const int* flags, int64_t n, int64_t* out_n, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_depth_count, dim3(1), dim3(64), 0, s, pos, flags, n, out_n);
+  const int64_t tiles = depth_tiles(np), pad = (tiles + 3) & ~(int64_t)3;
+  const int vec = (reinterpret_cast<uintptr_t>(depth) & 7) == 0 ? 1 : 0;
+  hipLaunchKernelGGL(k_depth_count, dim3((unsigned)tiles), dim3(kDepthTile / 4), 0, s, depth, w, h, P,
+                     vec, scratch);
+  const bool scanned = tiles > kDepthInlineTiles;
+  int* counts = scratch;
+  if (scanned) {
+    counts = scratch + pad;
+    launch_exclusive_scan(scratch, counts, tiles, scratch + 2 * pad, s);
+  }
+  hipLaunchKernelGGL(k_depth_points, dim3((unsigned)tiles), dim3(kDepthTile), 0, s, depth, w, h, color,
+                     P, counts, scanned ? 1 : 0, out_xyz, out_nrm, out_rgb, out_n);
 }
 
 }  // namespace lcr

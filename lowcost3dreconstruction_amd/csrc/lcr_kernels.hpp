@@ -194,13 +194,13 @@ struct DepthParams {
   double fx, fy, cx, cy;
   int depth_min, depth_max, top, bottom, left, right;
 };
-void launch_depth_flags(const uint16_t* depth, int w, int h, const DepthParams& P, int* flags,
-                        hipStream_t s);
-void launch_depth_points(const uint16_t* depth, int w, int h, const uint8_t* color,
-                         const DepthParams& P, const int* pos, float* out_xyz, float* out_nrm,
-                         uint8_t* out_rgb, hipStream_t s);
-// *out_n = pos[n - 1] + flags[n - 1]: the number of points (n = w * h > 0)
-void launch_depth_count(const int* pos, const int* flags, int64_t n, int64_t* out_n, hipStream_t s);
+// The points of the valid pixels in row-major order and their number (*out_n, on
+// the device); color, out_nrm and out_rgb nullable; scratch holds
+// depth_scratch_ints(w * h) ints, starting on 16 bytes.
+int64_t depth_scratch_ints(int64_t pixels);
+void launch_depth_cloud(const uint16_t* depth, int w, int h, const uint8_t* color,
+                        const DepthParams& P, int* scratch, float* out_xyz, float* out_nrm,
+                        uint8_t* out_rgb, int64_t* out_n, hipStream_t s);
 
 // StatisticalOutlierRemoval distances (normals.hip's selection with mean_k + 1
 // neighbours): dist / finite per input point (the caller zeroes both first);

@@ -184,3 +184,23 @@ def test_voxel_grid_run_lengths(lcr, sizes):
     assert len(got["xyz"]) == len(ref["xyz"]) == len(sizes)
     for k in ("xyz", "nrm", "curv", "rgb"):
         np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 341), (1023, 1), (64, 16), (5, 205), (37, 1001),
+                                 (2099, 2003)])
+def test_depth_to_cloud_tiles(lcr, w, h):
+    """Maps of one pixel, just under, at and over a 1024-pixel tile, rows that cross
+    tiles, and one of more tiles than a block adds up itself (4106 against 4096).
+    Bitwise equal to the oracle."""
+    rng = np.random.default_rng(w * h)
+    depth = (900 + 15 * rng.normal(size=(h, w))).astype(np.uint16)
+    depth[rng.random((h, w)) < 0.3] = 0
+    color = rng.integers(0, 256, size=(h, w, 3)).astype(np.uint8)
+    intr = (500.0, 510.0, w / 2, h / 2)
+    print_case(test="depth_tiles", w=w, h=h)
+    xyz, nrm, rgb = lcr.depth_to_cloud(depth, intr, 700, 1100, color=color)
+    rxyz, rnrm, rrgb = oracle.depth_to_cloud(depth, intr, 700, 1100, color=color)
+    assert len(xyz) == len(rxyz)
+    np.testing.assert_array_equal(xyz, rxyz)
+    np.testing.assert_array_equal(nrm, rnrm)
+    np.testing.assert_array_equal(rgb, rrgb)
