@@ -124,43 +124,30 @@ IcpConst make_const(const lcr_icp_params& p) {
   return c;
 }
 
-struct Stream {
-  hipStream_t s = nullptr;
-  int device = 0;
-  Stream() {
-    device = g_device;
-    LCR_HIP(hipSetDevice(device));
-    LCR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-  }
-  ~Stream() {
-    if (s) (void)hipStreamDestroy(s);
-  }
-  void bind() const { LCR_HIP(hipSetDevice(device)); }
-};
-
+// The caller's copy of a cloud, packed, in pinned memory (uploaded at the next
+// align).
 struct HostCloud {
-  std::vector<float> xyz, nrm;  // packed
+  HostBuf xyz, nrm;
   int64_t n = 0;
   bool has_nrm = false;
   void set(const float* p, const float* q, int64_t count, int64_t stride) {
     n = count;
-    xyz.resize((size_t)std::max<int64_t>(count, 0) * 3);
     has_nrm = q != nullptr;
-    nrm.resize(has_nrm ? xyz.size() : 0);
-    const char* pb = reinterpret_cast<const char*>(p);
-    const char* qb = reinterpret_cast<const char*>(q);
-    for (int64_t i = 0; i < count; ++i) {
-      const float* a = reinterpret_cast<const float*>(pb + i * stride);
-      xyz[3 * i] = a[0];
-      xyz[3 * i + 1] = a[1];
-      xyz[3 * i + 2] = a[2];
-      if (has_nrm) {
-        const float* b = reinterpret_cast<const float*>(qb + i * stride);
-        nrm[3 * i] = b[0];
-        nrm[3 * i + 1] = b[1];
-        nrm[3 * i + 2] = b[2];
-      }
+    pack(xyz, p, stride);
+    if (has_nrm) pack(nrm, q, stride);
+  }
+
+ private:
+  void pack(HostBuf& to, const float* p, int64_t stride) {
+    to.reserve((size_t)std::max<int64_t>(n, 1) * 3 * sizeof(float));
+    float* o = to.as<float>();
+    if (n == 0) return;
+    if (stride == 3 * (int64_t)sizeof(float)) {
+      memcpy(o, p, (size_t)n * 3 * sizeof(float));
+      return;
     }
+    const char* b = reinterpret_cast<const char*>(p);
+    for (int64_t i = 0; i < n; ++i) memcpy(o + 3 * i, b + i * stride, 3 * sizeof(float));
   }
 };
 
@@ -170,7 +157,8 @@ constexpr int64_t kMaxCloudPoints = (int64_t)1 << 24;
 
 struct lcr_icp {
   lcr_icp_params params;
-  Stream stream;
+  Stream stream{g_device};
+  ~lcr_icp() { (void)stream.idle(); }  // before the buffers go back to the pool
   HostCloud src, tgt;
   bool have_src = false, have_tgt = false, dirty = true;
   CloudSet cs;  // cloud 0 = source, cloud 1 = target
@@ -184,7 +172,8 @@ struct lcr_icp {
 
 struct lcr_cycle {
   lcr_cycle_desc desc;
-  Stream stream;
+  Stream stream{g_device};
+  ~lcr_cycle() { (void)stream.idle(); }  // before the buffers go back to the pool
   std::vector<int32_t> src, tgt;
   std::vector<double> guesses;
   std::vector<float> vps;
@@ -287,36 +276,25 @@ static void prepare(lcr_icp* h) {
   h->stream.bind();
   h->eng.c = make_const(h->params);
   if (h->dirty) {
-    std::vector<const float*> xyz = {h->src.xyz.data(), h->tgt.xyz.data()};
-    std::vector<const float*> nrm = {h->src.has_nrm ? h->src.nrm.data() : nullptr,
-                                     h->tgt.has_nrm ? h->tgt.nrm.data() : nullptr};
     // normals travel with the target (point-to-plane); the source's are only
-    // transformed for the output, from the host copy
+    // transformed for the output, from the host copy.  A cloud set has normals for
+    // every cloud or none: without its own the source gets zeros.
     const bool tn = h->tgt.has_nrm;
-    std::vector<const float*> nrm_up = {tn ? (h->src.has_nrm ? h->src.nrm.data() : nullptr)
-                                           : nullptr,
-                                        tn ? h->tgt.nrm.data() : nullptr};
-    (void)nrm;
-    std::vector<int64_t> cnt = {h->src.n, h->tgt.n};
-    // a cloud set has normals only when every cloud has them; give the source
-    // zeros if only the target has normals
-    std::vector<float> zeros;
-    if (tn && !h->src.has_nrm) {
-      zeros.assign(h->src.xyz.size(), 0.0f);
-      nrm_up[0] = zeros.data();
-    }
-    h->cs.upload(h->stream.s, xyz, nrm_up, cnt, 3 * sizeof(float));
+    const std::vector<const float*> xyz = {h->src.xyz.as<float>(), h->tgt.xyz.as<float>()};
+    const std::vector<const float*> nrm = {tn && h->src.has_nrm ? h->src.nrm.as<float>() : nullptr,
+                                           tn ? h->tgt.nrm.as<float>() : nullptr};
+    h->cs.upload(h->stream.s, xyz, nrm, {h->src.n, h->tgt.n}, 3 * sizeof(float), true, true);
     h->cs.build(h->stream.s, h->params.cell_factor, nullptr);
     const double r = h->params.max_corr_dist;
     h->cs.build_near_mask(h->stream.s, r);
-    h->eng.setup(h->cs, {0}, {1}, {r * r}, (h->params.tile && !h->params.precision_mode) ? h->params.tile : 64);
+    h->eng.setup(h->stream.s, h->cs, {0}, {1}, {r * r}, (h->params.tile && !h->params.precision_mode) ? h->params.tile : 64);
     h->dirty = false;
   } else {
     // parameters may have changed: refresh the instance radius
     const double r = h->params.max_corr_dist;
     if (h->eng.hp.size() == 1 && h->eng.hp[0].max_corr_d2 != r * r) {
       h->cs.build_near_mask(h->stream.s, r);
-      h->eng.setup(h->cs, {0}, {1}, {r * r}, (h->params.tile && !h->params.precision_mode) ? h->params.tile : 64);
+      h->eng.setup(h->stream.s, h->cs, {0}, {1}, {r * r}, (h->params.tile && !h->params.precision_mode) ? h->params.tile : 64);
     }
   }
 }
@@ -340,30 +318,27 @@ int lcr_icp_align(lcr_icp* h, const double* guess, float* out_xyz, float* out_nr
       float* dn = dx + 3 * std::max<int64_t>(n, 1);
       DevBuf rawn;
       const float4* raw_nrm = nullptr;
-      if (out_nrm && h->src.has_nrm) {
-        rawn.reserve((size_t)std::max<int64_t>(n, 1) * sizeof(float4));
-        std::vector<float4> tmp((size_t)n);
-        for (int64_t i = 0; i < n; ++i)
-          tmp[i] = make_float4(h->src.nrm[3 * i], h->src.nrm[3 * i + 1], h->src.nrm[3 * i + 2], 0.f);
-        LCR_HIP(hipMemcpyAsync(rawn.p, tmp.data(), n * sizeof(float4), hipMemcpyHostToDevice,
-                               h->stream.s));
-        LCR_HIP(hipStreamSynchronize(h->stream.s));
+      DevBuf packed;
+      if (out_nrm && h->src.has_nrm && n > 0) {
+        rawn.reserve((size_t)n * sizeof(float4));
+        packed.reserve((size_t)n * 3 * sizeof(float));
+        LCR_HIP(hipMemcpyAsync(packed.p, h->src.nrm.p, (size_t)n * 3 * sizeof(float),
+                               hipMemcpyHostToDevice, h->stream.s));
+        launch_widen(nullptr, packed.as<float>(), n, nullptr, rawn.as<float4>(), h->stream.s);
         raw_nrm = rawn.as<float4>();
       }
       launch_transform_output(h->cs.d_raw.as<float4>(), raw_nrm, n, h->eng.d_state.as<PairState>(),
                               0, dx, raw_nrm ? dn : nullptr, h->stream.s);
-      if (out_xyz && n > 0)
-        LCR_HIP(hipMemcpyAsync(out_xyz, dx, n * 3 * sizeof(float), hipMemcpyDeviceToHost,
-                               h->stream.s));
-      if (out_nrm && n > 0) {
+      CopyOut res(h->stream.s, (size_t)n * 6 * sizeof(float));
+      if (out_xyz) res.add(out_xyz, dx, (size_t)n * 3 * sizeof(float));
+      if (out_nrm) {
         if (raw_nrm) {
-          LCR_HIP(hipMemcpyAsync(out_nrm, dn, n * 3 * sizeof(float), hipMemcpyDeviceToHost,
-                                 h->stream.s));
+          res.add(out_nrm, dn, (size_t)n * 3 * sizeof(float));
         } else {
           for (int64_t i = 0; i < 3 * n; ++i) out_nrm[i] = NAN;
         }
       }
-      LCR_HIP(hipStreamSynchronize(h->stream.s));
+      res.finish();
     }
     return LCR_OK;
   });
@@ -461,7 +436,7 @@ int lcr_normals(const float* xyz, int64_t n, int64_t stride_bytes, int32_t k, co
     if (stride_bytes == 0) stride_bytes = 3 * sizeof(float);
     if (stride_bytes < 12 || stride_bytes % 4 != 0) return fail(LCR_E_ARG, "bad stride_bytes");
     if (n == 0) return LCR_OK;
-    Stream st;
+    Stream st(g_device);
     CloudSet cs;
     cs.upload(st.s, {xyz}, {nullptr}, {n}, stride_bytes);
     // cells sized for a k-neighbourhood: ~sqrt(k) point spacings.  0.70 sqrt(k)
@@ -472,17 +447,14 @@ int lcr_normals(const float* xyz, int64_t n, int64_t stride_bytes, int32_t k, co
     cs.build(st.s, factor, nullptr, false);
     const float v[3] = {vp ? vp[0] : 0.f, vp ? vp[1] : 0.f, vp ? vp[2] : 0.f};
     cs.compute_normals(st.s, k, v, flip_all, nullptr);
-    cs.normals_to_raw(st.s);  // input order; NaN for non-finite points
-    std::vector<float4> out((size_t)n);
-    LCR_HIP(hipMemcpyAsync(out.data(), cs.d_raw_nrm.p, n * sizeof(float4), hipMemcpyDeviceToHost,
-                           st.s));
-    LCR_HIP(hipStreamSynchronize(st.s));
-    for (int64_t i = 0; i < n; ++i) {
-      nrm[3 * i] = out[i].x;
-      nrm[3 * i + 1] = out[i].y;
-      nrm[3 * i + 2] = out[i].z;
-      if (curv) curv[i] = out[i].w;
-    }
+    DevBuf out;
+    out.reserve((size_t)n * 4 * sizeof(float));
+    float* d3 = out.as<float>();
+    cs.normals_to_input_order(st.s, d3, d3 + 3 * n);  // NaN for non-finite points
+    CopyOut res(st.s, (size_t)n * 4 * sizeof(float));
+    res.add(nrm, d3, (size_t)n * 3 * sizeof(float));
+    if (curv) res.add(curv, d3 + 3 * n, (size_t)n * sizeof(float));
+    res.finish();
     return LCR_OK;
   });
 }
@@ -597,7 +569,7 @@ int lcr_cycle_run(lcr_cycle* c) {
       for (int i = 0; i < ninst && same; ++i)
         same = c->eng.hp[i].ntiles == (c->cs.grids[src[i]].npts + tile - 1) / tile;
     }
-    if (!same) c->eng.setup(c->cs, src, tgt, r2, tile);
+    if (!same) c->eng.setup(c->stream.s, c->cs, src, tgt, r2, tile);
     if (!spans.empty()) prof.collect(spans, false);
     std::function<void()> pre;
     if (d.proposal && d.n_pairs > 0) {
@@ -680,7 +652,7 @@ int lcr_transform_points(const float* xyz, const float* nrm, int64_t n, int64_t 
     if (stride_bytes == 0) stride_bytes = 3 * sizeof(float);
     if (stride_bytes < 12 || stride_bytes % 4 != 0) return fail(LCR_E_ARG, "bad stride_bytes");
     if (n == 0) return LCR_OK;
-    Stream st;
+    Stream st(g_device);
     CloudSet cs;
     cs.upload(st.s, {xyz}, {nrm}, {n}, stride_bytes);
     DevBuf d_out;
@@ -689,10 +661,10 @@ int lcr_transform_points(const float* xyz, const float* nrm, int64_t n, int64_t 
     float* dn = dx + 3 * n;
     launch_transform_points(cs.d_raw.as<float4>(), (nrm && cs.has_nrm) ? cs.d_raw_nrm.as<float4>() : nullptr,
                             n, T, dx, (nrm && out_nrm) ? dn : nullptr, st.s);
-    LCR_HIP(hipMemcpyAsync(out_xyz, dx, n * 3 * sizeof(float), hipMemcpyDeviceToHost, st.s));
-    if (nrm && out_nrm)
-      LCR_HIP(hipMemcpyAsync(out_nrm, dn, n * 3 * sizeof(float), hipMemcpyDeviceToHost, st.s));
-    LCR_HIP(hipStreamSynchronize(st.s));
+    CopyOut res(st.s, (size_t)n * 6 * sizeof(float));
+    res.add(out_xyz, dx, (size_t)n * 3 * sizeof(float));
+    if (nrm && out_nrm) res.add(out_nrm, dn, (size_t)n * 3 * sizeof(float));
+    res.finish();
     return LCR_OK;
   });
 }
@@ -706,7 +678,7 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
     if (n > kMaxCloudPoints) return fail(LCR_E_LIMIT, "cloud larger than 2^24 points");
     *out_n = 0;
     if (n == 0) return LCR_OK;
-    Stream st;
+    Stream st(g_device);
     CloudSet cs;
     cs.upload(st.s, {xyz}, {nrm}, {n}, 3 * sizeof(float));
     DevBuf part, box;
@@ -714,8 +686,10 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
     box.reserve(kGeomWords * sizeof(float));
     launch_bbox(cs.d_raw.as<float4>(), cs.d_cloud_off.as<int64_t>(), 1, part.as<float>(),
                 box.as<float>(), nullptr, nullptr, st.s);
-    float b[7];
-    LCR_HIP(hipMemcpyAsync(b, box.p, sizeof b, hipMemcpyDeviceToHost, st.s));
+    HostBuf h_box;
+    h_box.reserve(kGeomWords * sizeof(float));
+    const float* b = h_box.as<float>();
+    LCR_HIP(hipMemcpyAsync(h_box.p, box.p, 7 * sizeof(float), hipMemcpyDeviceToHost, st.s));
     LCR_HIP(hipStreamSynchronize(st.s));
     const int64_t nfin = (int64_t)b[6];
     if (nfin == 0) return LCR_OK;
@@ -744,6 +718,7 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
     if (nvox > ((int64_t)1 << 30)) return fail(LCR_E_LIMIT, "voxel lattice larger than 2^30");
     DevBuf skey, skey_sorted, idx, sorted_raw, heads, outidx, scan_tmp, sort_tmp, dcurv, drgb, ox, on,
         oc, orgb;
+    HostBuf h_curv, h_rgb, h_last;
     for (DevBuf* v : {&skey, &skey_sorted, &idx, &sorted_raw, &heads, &outidx})
       v->reserve((size_t)n * sizeof(int));
     scan_tmp.reserve((size_t)scan_tmp_ints(n) * sizeof(int));
@@ -752,11 +727,11 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
     sort_tmp.reserve(sort_bytes);
     if (curv) {
       dcurv.reserve((size_t)n * sizeof(float));
-      LCR_HIP(hipMemcpyAsync(dcurv.p, curv, (size_t)n * sizeof(float), hipMemcpyHostToDevice, st.s));
+      copy_in(st.s, dcurv.p, curv, (size_t)n * sizeof(float), h_curv);
     }
     if (rgb) {
       drgb.reserve((size_t)n * 3);
-      LCR_HIP(hipMemcpyAsync(drgb.p, rgb, (size_t)n * 3, hipMemcpyHostToDevice, st.s));
+      copy_in(st.s, drgb.p, rgb, (size_t)n * 3, h_rgb);
     }
     ox.reserve((size_t)nfin * 3 * sizeof(float));
     if (nrm && out_nrm) on.reserve((size_t)nfin * 3 * sizeof(float));
@@ -770,24 +745,20 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
                               n, L, nvox, w, ox.as<float>(), on.p ? on.as<float>() : nullptr,
                               oc.p ? oc.as<float>() : nullptr, orgb.p ? orgb.as<uint8_t>() : nullptr,
                               st.s));
-    int last[2];
+    h_last.reserve(2 * sizeof(int));
+    int* last = h_last.as<int>();
     LCR_HIP(hipMemcpyAsync(&last[0], outidx.as<int>() + n - 1, sizeof(int), hipMemcpyDeviceToHost,
                            st.s));
     LCR_HIP(hipMemcpyAsync(&last[1], heads.as<int>() + n - 1, sizeof(int), hipMemcpyDeviceToHost,
                            st.s));
     LCR_HIP(hipStreamSynchronize(st.s));
     const int64_t nocc = (int64_t)last[0] + last[1];
-    LCR_HIP(hipMemcpyAsync(out_xyz, ox.p, (size_t)nocc * 3 * sizeof(float), hipMemcpyDeviceToHost,
-                           st.s));
-    if (on.p)
-      LCR_HIP(hipMemcpyAsync(out_nrm, on.p, (size_t)nocc * 3 * sizeof(float), hipMemcpyDeviceToHost,
-                             st.s));
-    if (oc.p)
-      LCR_HIP(hipMemcpyAsync(out_curv, oc.p, (size_t)nocc * sizeof(float), hipMemcpyDeviceToHost,
-                             st.s));
-    if (orgb.p)
-      LCR_HIP(hipMemcpyAsync(out_rgb, orgb.p, (size_t)nocc * 3, hipMemcpyDeviceToHost, st.s));
-    LCR_HIP(hipStreamSynchronize(st.s));
+    CopyOut res(st.s, (size_t)nocc * (7 * sizeof(float) + 3));
+    res.add(out_xyz, ox.p, (size_t)nocc * 3 * sizeof(float));
+    if (on.p) res.add(out_nrm, on.p, (size_t)nocc * 3 * sizeof(float));
+    if (oc.p) res.add(out_curv, oc.p, (size_t)nocc * sizeof(float));
+    if (orgb.p) res.add(out_rgb, orgb.p, (size_t)nocc * 3);
+    res.finish();
     *out_n = nocc;
     return LCR_OK;
   });
@@ -801,7 +772,7 @@ int lcr_outlier_removal(const float* xyz, int64_t n, int32_t mean_k, double stdd
     if (n > kMaxCloudPoints) return fail(LCR_E_LIMIT, "cloud larger than 2^24 points");
     if (kept) *kept = 0;
     if (n == 0) return LCR_OK;
-    Stream st;
+    Stream st(g_device);
     CloudSet cs;
     cs.upload(st.s, {xyz}, {nullptr}, {n}, 3 * sizeof(float));
     cs.build(st.s, std::max(2.5, 0.70 * sqrt((double)mean_k + 1.0)), nullptr, false);
@@ -822,13 +793,12 @@ int lcr_outlier_removal(const float* xyz, int64_t n, int32_t mean_k, double stdd
                          dist.as<float>(), fin.as<uint8_t>(), st.s);
     launch_sor_stats(dist.as<float>(), fin.as<uint8_t>(), n, stddev_mult, part.as<double>(),
                      dstats.as<double>(), dkeep.as<uint8_t>(), st.s);
-    LCR_HIP(hipMemcpyAsync(keep, dkeep.p, (size_t)n, hipMemcpyDeviceToHost, st.s));
-    if (mean_dist)
-      LCR_HIP(hipMemcpyAsync(mean_dist, dist.p, (size_t)n * sizeof(float), hipMemcpyDeviceToHost,
-                             st.s));
     double hs[3];
-    LCR_HIP(hipMemcpyAsync(hs, dstats.p, sizeof hs, hipMemcpyDeviceToHost, st.s));
-    LCR_HIP(hipStreamSynchronize(st.s));
+    CopyOut res(st.s, (size_t)n * (1 + sizeof(float)) + sizeof hs);
+    res.add(keep, dkeep.p, (size_t)n);
+    if (mean_dist) res.add(mean_dist, dist.p, (size_t)n * sizeof(float));
+    res.add(hs, dstats.p, sizeof hs);
+    res.finish();
     if (stats) memcpy(stats, hs, sizeof hs);
     if (kept) {
       int64_t k = 0;
@@ -862,13 +832,14 @@ int lcr_depth_to_cloud(const uint16_t* depth, int32_t width, int32_t height, con
     P.bottom = crop ? crop[1] : height - 1;
     P.left = crop ? crop[2] : 0;
     P.right = crop ? crop[3] : width - 1;
-    Stream st;
+    Stream st(g_device);
     DevBuf dd, dc, scratch, dn, ox, on, orgb;
     dd.reserve((size_t)np * sizeof(uint16_t));
-    LCR_HIP(hipMemcpyAsync(dd.p, depth, (size_t)np * sizeof(uint16_t), hipMemcpyHostToDevice, st.s));
+    HostBuf h_depth, h_color, h_m;
+    copy_in(st.s, dd.p, depth, (size_t)np * sizeof(uint16_t), h_depth);
     if (color) {
       dc.reserve((size_t)np * 3);
-      LCR_HIP(hipMemcpyAsync(dc.p, color, (size_t)np * 3, hipMemcpyHostToDevice, st.s));
+      copy_in(st.s, dc.p, color, (size_t)np * 3, h_color);
     }
     scratch.reserve((size_t)depth_scratch_ints(np) * sizeof(int));
     dn.reserve(sizeof(int64_t));
@@ -878,17 +849,15 @@ int lcr_depth_to_cloud(const uint16_t* depth, int32_t width, int32_t height, con
     launch_depth_cloud(dd.as<uint16_t>(), width, height, color ? dc.as<uint8_t>() : nullptr, P,
                        scratch.as<int>(), ox.as<float>(), on.p ? on.as<float>() : nullptr,
                        orgb.p ? orgb.as<uint8_t>() : nullptr, dn.as<int64_t>(), st.s);
-    int64_t m = 0;
-    LCR_HIP(hipMemcpyAsync(&m, dn.p, sizeof m, hipMemcpyDeviceToHost, st.s));
+    h_m.reserve(sizeof(int64_t));
+    LCR_HIP(hipMemcpyAsync(h_m.p, dn.p, sizeof(int64_t), hipMemcpyDeviceToHost, st.s));
     LCR_HIP(hipStreamSynchronize(st.s));
-    if (m > 0) {
-      LCR_HIP(hipMemcpyAsync(out_xyz, ox.p, (size_t)m * 3 * sizeof(float), hipMemcpyDeviceToHost, st.s));
-      if (on.p)
-        LCR_HIP(hipMemcpyAsync(out_nrm, on.p, (size_t)m * 3 * sizeof(float), hipMemcpyDeviceToHost,
-                               st.s));
-      if (orgb.p) LCR_HIP(hipMemcpyAsync(out_rgb, orgb.p, (size_t)m * 3, hipMemcpyDeviceToHost, st.s));
-    }
-    LCR_HIP(hipStreamSynchronize(st.s));
+    const int64_t m = *h_m.as<int64_t>();
+    CopyOut res(st.s, (size_t)m * (6 * sizeof(float) + 3));
+    res.add(out_xyz, ox.p, (size_t)m * 3 * sizeof(float));
+    if (on.p) res.add(out_nrm, on.p, (size_t)m * 3 * sizeof(float));
+    if (orgb.p) res.add(out_rgb, orgb.p, (size_t)m * 3);
+    res.finish();
     *out_n = m;
     return LCR_OK;
   });

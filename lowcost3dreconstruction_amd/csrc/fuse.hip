@@ -22,8 +22,6 @@
 #include <math.h>
 #include <stdint.h>
 
-#include <memory>
-
 #include "../../include/lcr.h"
 #include "runtime.hpp"
 
@@ -120,17 +118,14 @@ extern "C" int lcr_depth_fuse(const uint16_t* frames, int32_t n_frames, int32_t 
     if (np == 0) return LCR_OK;
     int dev = 0;
     LCR_HIP(hipGetDevice(&dev));
-    hipStream_t s = nullptr;
-    LCR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    std::unique_ptr<ihipStream_t, void (*)(hipStream_t)> guard(s, [](hipStream_t q) {
-      (void)hipStreamDestroy(q);
-    });
+    const Stream st(dev);
+    const hipStream_t s = st.s;
     DevBuf d_frames, d_mean, d_out;
     d_frames.reserve((size_t)(n_frames * np) * sizeof(uint16_t));
     d_mean.reserve((size_t)np * sizeof(float));
     d_out.reserve((size_t)np * sizeof(uint16_t));
-    LCR_HIP(hipMemcpyAsync(d_frames.p, frames, (size_t)(n_frames * np) * sizeof(uint16_t),
-                           hipMemcpyHostToDevice, s));
+    HostBuf h_frames;
+    copy_in(s, d_frames.p, frames, (size_t)(n_frames * np) * sizeof(uint16_t), h_frames);
     hipLaunchKernelGGL(k_fuse_mean, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s,
                        d_frames.as<uint16_t>(), (int)n_frames, np, d_mean.as<float>());
     // output x samples (x + 0.5) factor - 0.5 = factor x + (factor - 1) / 2
@@ -141,8 +136,9 @@ extern "C" int lcr_depth_fuse(const uint16_t* frames, int32_t n_frames, int32_t 
                        dim3(128), 0, s, d_mean.as<float>(), (int)width, (int)height, (int)factor,
                        base, taps, d_out.as<uint16_t>());
     LCR_HIP(hipGetLastError());
-    LCR_HIP(hipMemcpyAsync(out, d_out.p, (size_t)np * sizeof(uint16_t), hipMemcpyDeviceToHost, s));
-    LCR_HIP(hipStreamSynchronize(s));
+    CopyOut res(s, (size_t)np * sizeof(uint16_t));
+    res.add(out, d_out.p, (size_t)np * sizeof(uint16_t));
+    res.finish();
     return LCR_OK;
   } catch (const Error& e) {
     return set_last_error(e.code, e.msg);

@@ -535,20 +535,37 @@ __global__ void k_set_near(GridDesc* grids, int n, float r) {
   }
 }
 
-// sorted-order normals back to input order: raw[cloud_off[c] + id] = nrm[j]
+// Sorted-order normals to input order, split into packed normals and curvatures.
 __global__ void k_unsort_normals(const float4* __restrict__ pts, const float4* __restrict__ nrm,
                                  const int* __restrict__ cloud_of_sorted,
                                  const int64_t* __restrict__ cloud_off, int64_t n,
-                                 float4* __restrict__ raw_nrm) {
+                                 float* __restrict__ out3, float* __restrict__ curv) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  const int id = __float_as_int(pts[j].w);
-  raw_nrm[cloud_off[cloud_of_sorted[j]] + id] = nrm[j];
+  const int64_t i = cloud_off[cloud_of_sorted[j]] + __float_as_int(pts[j].w);
+  const float4 v = nrm[j];
+  out3[3 * i] = v.x;
+  out3[3 * i + 1] = v.y;
+  out3[3 * i + 2] = v.z;
+  curv[i] = v.w;
 }
 
-__global__ void k_fill_f4(float4* __restrict__ p, int64_t n, float4 v) {
+__global__ void k_fill_f32(float* __restrict__ p, int64_t n, float v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
+}
+
+// Packed x, y, z to one 16-byte record a point.
+__device__ __forceinline__ float4 widen(const float* in, int64_t i) {
+  return make_float4(in[3 * i], in[3 * i + 1], in[3 * i + 2], 0.0f);
+}
+
+__global__ void k_widen(const float* __restrict__ xyz, const float* __restrict__ nrm, int64_t n,
+                        float4* __restrict__ out, float4* __restrict__ out_nrm) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (out) out[i] = widen(xyz, i);
+  if (nrm) out_nrm[i] = widen(nrm, i);
 }
 
 __global__ void k_fill_i32(int* __restrict__ p, int64_t n, int v) {
@@ -586,14 +603,23 @@ void launch_bvh_build(const GridDesc* grids, int nclouds, int max_depth, const f
 }
 
 void launch_unsort_normals(const float4* pts, const float4* nrm, const int* cloud_of_sorted,
-                           const int64_t* cloud_off, int64_t n_sorted, float4* raw_nrm,
-                           int64_t n_raw, hipStream_t s) {
-  if (n_raw > 0)
-    hipLaunchKernelGGL(k_fill_f4, dim3(blocks_for(n_raw, 256)), dim3(256), 0, s, raw_nrm, n_raw,
-                       make_float4(NAN, NAN, NAN, NAN));
+                           const int64_t* cloud_off, int64_t n_sorted, int64_t n_raw, float* out3,
+                           float* curv, hipStream_t s) {
+  // non-finite points are not in the sorted order: NaN
+  if (n_raw > n_sorted) {
+    hipLaunchKernelGGL(k_fill_f32, dim3(blocks_for(3 * n_raw, 256)), dim3(256), 0, s, out3, 3 * n_raw,
+                       NAN);
+    hipLaunchKernelGGL(k_fill_f32, dim3(blocks_for(n_raw, 256)), dim3(256), 0, s, curv, n_raw, NAN);
+  }
   if (n_sorted > 0)
     hipLaunchKernelGGL(k_unsort_normals, dim3(blocks_for(n_sorted, 256)), dim3(256), 0, s, pts, nrm,
-                       cloud_of_sorted, cloud_off, n_sorted, raw_nrm);
+                       cloud_of_sorted, cloud_off, n_sorted, out3, curv);
+}
+
+void launch_widen(const float* xyz, const float* nrm, int64_t n, float4* out, float4* out_nrm,
+                  hipStream_t s) {
+  if (n > 0)
+    hipLaunchKernelGGL(k_widen, dim3(blocks_for(n, 256)), dim3(256), 0, s, xyz, nrm, n, out, out_nrm);
 }
 
 void launch_near_mask(const GridDesc* grids, int ngrids, const int* cell_start, int64_t total_words,

@@ -43,9 +43,13 @@ void launch_near_mask(const GridDesc* grids, int ngrids, const int* cell_start, 
                       float r, uint32_t* out, uint32_t* tmp, hipStream_t s);
 // Sets every grid's near_r and its mask's first word (near_off).
 void launch_set_near(GridDesc* grids, int ngrids, float r, hipStream_t s);
+// Cell-sorted normals (and curvatures, w) in input order: packed normals, curvatures.
 void launch_unsort_normals(const float4* pts, const float4* nrm, const int* cloud_of_sorted,
-                           const int64_t* cloud_off, int64_t n_sorted, float4* raw_nrm,
-                           int64_t n_raw, hipStream_t s);
+                           const int64_t* cloud_off, int64_t n_sorted, int64_t n_raw, float* out3,
+                           float* curv, hipStream_t s);
+// Packed x, y, z (and normals, nullable) to 16-byte records; out nullable.
+void launch_widen(const float* xyz, const float* nrm, int64_t n, float4* out, float4* out_nrm,
+                  hipStream_t s);
 // bounding-volume trees (GridDesc::node_off / depth set by the host)
 // Tree order (Tree): Morton keys of the cell-sorted points, a radix sort of
 // (cloud, key) carrying each point's cell-sorted position into tpos, then the

@@ -1,0 +1,161 @@
+// pool.cpp -- see pool.hpp.
+#include "pool.hpp"
+
+#include <string>
+
+#include "runtime.hpp"
+
+namespace lcr {
+
+Pool& Pool::get() {
+  static Pool* p = new Pool();
+  return *p;
+}
+
+size_t Pool::size_class(size_t n) {
+  constexpr size_t kLeast = 4096;
+  if (n <= kLeast) return kLeast;
+  size_t top = kLeast;
+  while (top <= (n - 1) / 2) top *= 2;  // top < n <= 2 top
+  const size_t step = top / 4;
+  return (n + step - 1) / step * step;
+}
+
+void* Pool::take(const Key& k) {
+  std::vector<std::pair<int, void*>> old;
+  void* p = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    auto it = blocks_.find(k);
+    if (it != blocks_.end()) {
+      p = it->second.back().p;
+      it->second.pop_back();
+      if (it->second.empty()) blocks_.erase(it);
+      kept_[k.first] -= k.second;
+    }
+    trim(k.first, &old);
+  }
+  release(old);
+  return p;
+}
+
+void Pool::give(const Key& k, void* p) noexcept {
+  std::vector<std::pair<int, void*>> old;
+  try {
+    std::lock_guard<std::mutex> lock(mu_);
+    blocks_[k].push_back(Block{p, Clock::now()});
+    kept_[k.first] += k.second;
+    trim(k.first, &old);
+  } catch (...) {  // no memory for the bookkeeping
+    old.emplace_back(k.first, p);
+  }
+  release(old);
+}
+
+void Pool::trim(int owner, std::vector<std::pair<int, void*>>* out) {
+  const size_t keep = owner == kPinned ? kPinnedKeep : kDeviceKeep;
+  const Clock::time_point now = Clock::now();
+  // a walk over every class: when over the limit, else once a second
+  Clock::time_point& last = trimmed_[owner];
+  if (kept_[owner] <= keep && now - last < std::chrono::seconds(1)) return;
+  last = now;
+  const Clock::time_point stale = now - std::chrono::seconds(kIdleSeconds);
+  for (;;) {
+    // the block of this owner unused for longest (the first of its class's vector)
+    auto oldest = blocks_.end();
+    for (auto it = blocks_.lower_bound(Key(owner, 0)); it != blocks_.end() && it->first.first == owner;
+         ++it)
+      if (oldest == blocks_.end() || it->second.front().since < oldest->second.front().since) oldest = it;
+    if (oldest == blocks_.end()) return;
+    if (kept_[owner] <= keep && oldest->second.front().since > stale) return;
+    out->emplace_back(owner, oldest->second.front().p);
+    kept_[owner] -= oldest->first.second;
+    oldest->second.erase(oldest->second.begin());
+    if (oldest->second.empty()) blocks_.erase(oldest);
+  }
+}
+
+void Pool::release(const std::vector<std::pair<int, void*>>& blocks) noexcept {
+  for (const auto& b : blocks) {
+    if (b.first == kPinned)
+      (void)hipHostFree(b.second);
+    else
+      (void)hipFree(b.second);
+  }
+}
+
+bool Pool::flush(int owner) {
+  std::vector<std::pair<int, void*>> old;
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    for (auto it = blocks_.lower_bound(Key(owner, 0));
+         it != blocks_.end() && it->first.first == owner;) {
+      for (const Block& b : it->second) old.emplace_back(owner, b.p);
+      it = blocks_.erase(it);
+    }
+    kept_[owner] = 0;
+  }
+  release(old);
+  return !old.empty();
+}
+
+void* Pool::take_device(size_t* bytes, int* device) {
+  LCR_HIP(hipGetDevice(device));
+  *bytes = size_class(*bytes);
+  void* p = take(Key(*device, *bytes));
+  if (p) return p;
+  hipError_t e = hipMalloc(&p, *bytes);
+  if (e == hipErrorOutOfMemory && flush(*device)) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, *bytes);
+  }
+  if (e != hipSuccess) throw Error{-2, std::string("hipMalloc failed: ") + hipGetErrorString(e)};
+  return p;
+}
+
+void* Pool::take_pinned(size_t* bytes) {
+  *bytes = size_class(*bytes);
+  void* p = take(Key(kPinned, *bytes));
+  if (p) return p;
+  hipError_t e = hipHostMalloc(&p, *bytes, hipHostMallocDefault);
+  if (e != hipSuccess && flush(kPinned)) {
+    (void)hipGetLastError();
+    e = hipHostMalloc(&p, *bytes, hipHostMallocDefault);
+  }
+  if (e != hipSuccess) throw Error{-2, std::string("hipHostMalloc failed: ") + hipGetErrorString(e)};
+  return p;
+}
+
+void Pool::give_device(void* p, size_t bytes, int device) noexcept { give(Key(device, bytes), p); }
+
+void Pool::give_pinned(void* p, size_t bytes) noexcept { give(Key(kPinned, bytes), p); }
+
+hipStream_t Pool::take_stream(int device) {
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    std::vector<hipStream_t>& v = streams_[device];
+    if (!v.empty()) {
+      hipStream_t s = v.back();
+      v.pop_back();
+      return s;
+    }
+  }
+  hipStream_t s = nullptr;
+  LCR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+  return s;
+}
+
+void Pool::give_stream(hipStream_t s, int device) noexcept {
+  try {
+    std::lock_guard<std::mutex> lock(mu_);
+    std::vector<hipStream_t>& v = streams_[device];
+    if (v.size() < kStreamsKeep) {
+      v.push_back(s);
+      return;
+    }
+  } catch (...) {
+  }
+  (void)hipStreamDestroy(s);
+}
+
+}  // namespace lcr

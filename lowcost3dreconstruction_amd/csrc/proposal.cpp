@@ -158,7 +158,8 @@ __global__ void k_prop_guess(const float* __restrict__ out, const float* __restr
 
 struct ProposalImpl {
   int device = 0;
-  hipStream_t s = nullptr;
+  Stream stream;
+  const hipStream_t s;
   int cap_pairs = 0, cap_pts = 0;
   int step = 0;
   DevBuf W, M, V, G, W2t, W3t;
@@ -167,9 +168,12 @@ struct ProposalImpl {
   int ds_pairs = 0, ds_pts = 0;
   HostBuf h_io;
 
-  ProposalImpl() {
-    LCR_HIP(hipGetDevice(&device));
-    LCR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+  static int current_device() {
+    int d = 0;
+    LCR_HIP(hipGetDevice(&d));
+    return d;
+  }
+  ProposalImpl() : device(current_device()), stream(device), s(stream.s) {
     W.reserve(kEncNParam * sizeof(float));
     M.reserve(kEncNParam * sizeof(float));
     V.reserve(kEncNParam * sizeof(float));
@@ -179,9 +183,7 @@ struct ProposalImpl {
     LCR_HIP(hipMemsetAsync(W.p, 0, kEncNParam * sizeof(float), s));
     reset_optimizer();
   }
-  ~ProposalImpl() {
-    if (s) (void)hipStreamDestroy(s);
-  }
+  ~ProposalImpl() { (void)stream.idle(); }  // before the buffers go back to the pool
   void bind() const { LCR_HIP(hipSetDevice(device)); }
   void reset_optimizer() {
     LCR_HIP(hipMemsetAsync(M.p, 0, kEncNParam * sizeof(float), s));

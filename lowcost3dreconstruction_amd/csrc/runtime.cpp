@@ -12,6 +12,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <map>
+#include <mutex>
 
 namespace lcr {
 
@@ -90,6 +92,60 @@ int device_cu_count() {
   return cus > 0 ? cus : 1;
 }
 
+// ------------------------------------------------------------------ copies
+
+CopyOut::CopyOut(hipStream_t s, size_t bytes) : s_(s) { stage_.reserve(bytes); }
+
+CopyOut::~CopyOut() {
+  for (const Piece& p : pieces_)
+    if (p.done) (void)hipEventDestroy(p.done);
+}
+
+void CopyOut::add(void* dst, const void* src, size_t bytes) {
+  for (size_t at = 0; at < bytes;) {
+    const size_t len = std::min(kChunk, bytes - at);
+    Piece p{static_cast<char*>(dst) + at, used_, len, nullptr};
+    LCR_HIP(hipMemcpyAsync(stage_.as<char>() + used_, static_cast<const char*>(src) + at, len,
+                           hipMemcpyDeviceToHost, s_));
+    since_event_ += len;
+    if (since_event_ >= kChunk) {
+      LCR_HIP(hipEventCreateWithFlags(&p.done, hipEventDisableTiming));
+      pieces_.push_back(p);
+      LCR_HIP(hipEventRecord(p.done, s_));
+      since_event_ = 0;
+    } else {
+      pieces_.push_back(p);
+    }
+    used_ += len;
+    at += len;
+  }
+}
+
+void CopyOut::finish() {
+  size_t moved = 0;
+  auto move_to = [&](size_t end) {
+    for (; moved < end; ++moved)
+      memcpy(pieces_[moved].dst, stage_.as<char>() + pieces_[moved].off, pieces_[moved].bytes);
+  };
+  for (size_t k = 0; k < pieces_.size(); ++k) {
+    if (!pieces_[k].done) continue;
+    LCR_HIP(hipEventSynchronize(pieces_[k].done));
+    move_to(k + 1);
+  }
+  LCR_HIP(hipStreamSynchronize(s_));
+  move_to(pieces_.size());
+}
+
+void copy_in(hipStream_t s, void* dst, const void* src, size_t bytes, HostBuf& stage) {
+  if (bytes == 0) return;
+  if (bytes <= kCopyInStage) {
+    stage.reserve(bytes);
+    memcpy(stage.p, src, bytes);
+    src = stage.p;
+  }
+  LCR_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+}
+
 // ------------------------------------------------------------------ clouds
 
 namespace {
@@ -123,66 +179,83 @@ constexpr int64_t kMaxDim = 4096;
 constexpr int kStageThreads = 8;
 constexpr int64_t kStageMinPoints = 1 << 18;
 
+// The records are packed to 12 bytes a point in pinned memory, copied over in one
+// go, and widened on the device (with each point's cloud), so 12 bytes a point
+// cross the bus instead of 20 and the host only copies.
 void CloudSet::upload(hipStream_t s, const std::vector<const float*>& xyz,
                       const std::vector<const float*>& nrm, const std::vector<int64_t>& counts,
-                      int64_t stride_bytes) {
+                      int64_t stride_bytes, bool zero_nrm, bool pinned) {
   n = (int)xyz.size();
   geom_valid = false;
   nraw = counts;
   raw_off.assign(n + 1, 0);
   for (int c = 0; c < n; ++c) raw_off[c + 1] = raw_off[c] + counts[c];
   total_raw = raw_off[n];
-  has_nrm = true;
-  for (int c = 0; c < n; ++c)
-    if (!nrm[c]) has_nrm = false;
+  int with = 0;
+  for (int c = 0; c < n; ++c) with += nrm[c] ? 1 : 0;
+  has_nrm = zero_nrm ? with > 0 : with == n;
   const size_t np = (size_t)std::max<int64_t>(total_raw, 1);
-  h_stage.reserve(np * sizeof(float4));
-  float4* st = h_stage.as<float4>();
-  int* pc = nullptr;
-  h_stage_nrm.reserve(np * (sizeof(float4) + sizeof(int)));
-  float4* sn = h_stage_nrm.as<float4>();
-  pc = reinterpret_cast<int*>(sn + np);
-  // host staging into pinned memory, clouds spread over a few threads
-  auto stage = [&](int c) {
-    const char* base = reinterpret_cast<const char*>(xyz[c]);
-    const char* nb = reinterpret_cast<const char*>(nrm[c]);
-    for (int64_t i = 0; i < counts[c]; ++i) {
-      const float* p = reinterpret_cast<const float*>(base + i * stride_bytes);
-      st[raw_off[c] + i] = make_float4(p[0], p[1], p[2], 0.0f);
-      pc[raw_off[c] + i] = c;
-      if (has_nrm) {
-        const float* m = reinterpret_cast<const float*>(nb + i * stride_bytes);
-        sn[raw_off[c] + i] = make_float4(m[0], m[1], m[2], 0.0f);
-      }
-    }
-  };
-  const int nthreads = (int)std::min<int64_t>(
-      {(int64_t)kStageThreads, (int64_t)n, std::max<int64_t>(total_raw / kStageMinPoints, 1)});
-  if (nthreads <= 1) {
-    for (int c = 0; c < n; ++c) stage(c);
-  } else {
-    std::atomic<int> next{0};
-    std::vector<std::thread> pool;
-    for (int t = 0; t < nthreads; ++t)
-      pool.emplace_back([&] {
-        for (int c = next++; c < n; c = next++) stage(c);
-      });
-    for (std::thread& th : pool) th.join();
-  }
+  const int parts = has_nrm ? 2 : 1;  // points, then normals
+  LCR_HIP(hipStreamSynchronize(s));  // the last upload is done with its buffers
+  d_in.reserve(np * 3 * sizeof(float) * parts);
+  float* din[2] = {d_in.as<float>(), d_in.as<float>() + 3 * np};
   d_raw.reserve(np * sizeof(float4));
   d_point_cloud.reserve(np * sizeof(int));
+  if (has_nrm) d_raw_nrm.reserve(np * sizeof(float4));
   d_cloud_off.reserve((n + 1) * sizeof(int64_t));
-  LCR_HIP(hipMemcpyAsync(d_raw.p, st, total_raw * sizeof(float4), hipMemcpyHostToDevice, s));
-  LCR_HIP(hipMemcpyAsync(d_point_cloud.p, pc, total_raw * sizeof(int), hipMemcpyHostToDevice, s));
   h_small.reserve((n + 1) * sizeof(int64_t) + 4096);
   memcpy(h_small.p, raw_off.data(), (n + 1) * sizeof(int64_t));
   LCR_HIP(hipMemcpyAsync(d_cloud_off.p, h_small.p, (n + 1) * sizeof(int64_t),
                          hipMemcpyHostToDevice, s));
-  if (has_nrm) {
-    d_raw_nrm.reserve(np * sizeof(float4));
-    LCR_HIP(hipMemcpyAsync(d_raw_nrm.p, sn, total_raw * sizeof(float4), hipMemcpyHostToDevice, s));
+  if (pinned) {
+    for (int c = 0; c < n; ++c) {
+      const size_t len = (size_t)counts[c] * 3 * sizeof(float);
+      if (len == 0) continue;
+      LCR_HIP(hipMemcpyAsync(din[0] + 3 * raw_off[c], xyz[c], len, hipMemcpyHostToDevice, s));
+      if (!has_nrm) continue;
+      if (nrm[c])
+        LCR_HIP(hipMemcpyAsync(din[1] + 3 * raw_off[c], nrm[c], len, hipMemcpyHostToDevice, s));
+      else
+        launch_fill_i32(reinterpret_cast<int*>(din[1] + 3 * raw_off[c]), 3 * counts[c], 0, s);
+    }
+  } else {
+    h_stage.reserve(np * 3 * sizeof(float) * parts);
+    float* st[2] = {h_stage.as<float>(), h_stage.as<float>() + 3 * np};
+    auto stage = [&](int c) {
+      for (int q = 0; q < parts; ++q) {
+        const char* in = reinterpret_cast<const char*>(q == 0 ? xyz[c] : nrm[c]);
+        float* o = st[q] + 3 * raw_off[c];
+        if (counts[c] == 0) continue;
+        if (!in) {
+          memset(o, 0, (size_t)counts[c] * 3 * sizeof(float));
+        } else if (stride_bytes == 3 * (int64_t)sizeof(float)) {
+          memcpy(o, in, (size_t)counts[c] * 3 * sizeof(float));
+        } else {
+          for (int64_t i = 0; i < counts[c]; ++i) memcpy(o + 3 * i, in + i * stride_bytes, 3 * sizeof(float));
+        }
+      }
+    };
+    const int nthreads = (int)std::min<int64_t>(
+        {(int64_t)kStageThreads, (int64_t)n, std::max<int64_t>(total_raw / kStageMinPoints, 1)});
+    if (nthreads <= 1) {
+      for (int c = 0; c < n; ++c) stage(c);
+    } else {
+      std::atomic<int> next{0};
+      std::vector<std::thread> pool;
+      for (int t = 0; t < nthreads; ++t)
+        pool.emplace_back([&] {
+          for (int c = next++; c < n; c = next++) stage(c);
+        });
+      for (std::thread& th : pool) th.join();
+    }
+    for (int q = 0; q < parts; ++q)
+      if (total_raw > 0)
+        LCR_HIP(hipMemcpyAsync(din[q], st[q], (size_t)total_raw * 3 * sizeof(float),
+                               hipMemcpyHostToDevice, s));
   }
-  LCR_HIP(hipStreamSynchronize(s));  // staging buffers are reused by the next upload
+  launch_segments(d_cloud_off.as<int64_t>(), n, total_raw, d_point_cloud.as<int>(), s);
+  launch_widen(din[0], has_nrm ? din[1] : nullptr, total_raw, d_raw.as<float4>(),
+               has_nrm ? d_raw_nrm.as<float4>() : nullptr, s);
 }
 
 namespace {
@@ -432,11 +505,9 @@ void CloudSet::build_near_mask(hipStream_t s, double r) {
   }
 }
 
-void CloudSet::normals_to_raw(hipStream_t s) {
-  d_raw_nrm.reserve((size_t)std::max<int64_t>(total_raw, 1) * sizeof(float4));
+void CloudSet::normals_to_input_order(hipStream_t s, float* d_nrm3, float* d_curv) {
   launch_unsort_normals(d_pts.as<float4>(), d_nrm.as<float4>(), d_cloud_of_sorted.as<int>(),
-                        d_cloud_off.as<int64_t>(), total_pts, d_raw_nrm.as<float4>(), total_raw, s);
-  has_nrm = true;
+                        d_cloud_off.as<int64_t>(), total_pts, total_raw, d_nrm3, d_curv, s);
 }
 
 // ------------------------------------------------------------------ engine
@@ -445,6 +516,7 @@ Engine::~Engine() { reset_graph(); }
 
 // Never throws: also runs from the destructor.
 void Engine::reset_graph() {
+  eager_key_set_ = false;
   if (exec) (void)hipGraphExecDestroy(exec);
   if (graph) (void)hipGraphDestroy(graph);
   if (tail_exec) (void)hipGraphExecDestroy(tail_exec);
@@ -467,13 +539,48 @@ static int icp_split_units() {
   return 2048;
 }
 
-void Engine::setup(const CloudSet& cs, const std::vector<int>& src, const std::vector<int>& tgt,
-                   const std::vector<double>& r2, int tile_pts) {
+// The resident blocks of the search, fitness and split kernels per CU: properties
+// of the code and the device type, queried once per kernel (a query takes tens of
+// microseconds).
+static int blocks_per_cu(int which, int tile, bool p2pl, int precision) {
+  static std::mutex mu;
+  static std::map<int, int> known;
+  const int key = ((which * 4 + (tile == 64 ? 0 : (tile == 128 ? 1 : 2))) * 2 + (p2pl ? 1 : 0)) * 8 + precision;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = known.find(key);
+  if (it != known.end()) return it->second;
+  const int v = which == 3   ? icp_split_blocks_per_cu(tile, p2pl)
+                : which == 2 ? fitness_max_blocks_per_cu(tile)
+                             : icp_max_blocks_per_cu(tile, p2pl, precision, which != 0);
+  known[key] = v;
+  return v;
+}
+
+namespace {
+// tile -> its instance (instances in tile order): the last whose first tile is <= t
+__global__ void k_tile_pairs(const PairDesc* __restrict__ pairs, int npairs, int ntiles,
+                             int* __restrict__ out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= ntiles) return;
+  int lo = 0, hi = npairs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (pairs[mid].tile_begin <= t)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  out[t] = lo;
+}
+}  // namespace
+
+void Engine::setup(hipStream_t s, const CloudSet& cs, const std::vector<int>& src,
+                   const std::vector<int>& tgt, const std::vector<double>& r2, int tile_pts) {
   reset_graph();
   tile = (tile_pts == 64 || tile_pts == 128 || tile_pts == 256) ? tile_pts : 256;
   npairs = (int)src.size();
   hp.assign(npairs, PairDesc{});
-  std::vector<int> tp, gt;
+  std::vector<int> gt;
   ntiles = 0;
   for (int p = 0; p < npairs; ++p) {
     PairDesc& d = hp[p];
@@ -482,10 +589,10 @@ void Engine::setup(const CloudSet& cs, const std::vector<int>& src, const std::v
     d.tile_begin = ntiles;
     d.ntiles = (cs.grids[d.src].npts + tile - 1) / tile;
     d.max_corr_d2 = r2[p];
-    for (int t = 0; t < d.ntiles; ++t) tp.push_back(p);
     for (int t = 0; t < d.ntiles; t += gate_stride(d.ntiles)) gt.push_back(ntiles + t);
     ntiles += d.ntiles;
   }
+  ngate_tiles = (int)gt.size();
   d_pairs.reserve(std::max(npairs, 1) * sizeof(PairDesc));
   d_tile_pair.reserve(std::max(ntiles, 1) * sizeof(int));
   d_state.reserve((size_t)(npairs + 1) * sizeof(PairState));
@@ -494,49 +601,48 @@ void Engine::setup(const CloudSet& cs, const std::vector<int>& src, const std::v
   d_guess.reserve((size_t)std::max(npairs, 1) * 16 * sizeof(double));
   h_state.reserve((size_t)(npairs + 1) * sizeof(PairState));
   h_guess.reserve((size_t)std::max(npairs, 1) * 16 * sizeof(double));
-  if (npairs > 0)
-    LCR_HIP(hipMemcpy(d_pairs.p, hp.data(), npairs * sizeof(PairDesc), hipMemcpyHostToDevice));
-  if (ntiles > 0)
-    LCR_HIP(hipMemcpy(d_tile_pair.p, tp.data(), ntiles * sizeof(int), hipMemcpyHostToDevice));
-  // live-tile lists: every tile until a run compacts them
+  // live-tile lists (each run compacts them first)
   d_it_list.reserve((size_t)std::max(ntiles, 1) * sizeof(int2));
   d_fit_list.reserve((size_t)std::max(ntiles, 1) * sizeof(int2));
   d_fit_order.reserve((size_t)std::max(ntiles, 1) * sizeof(int2));
   d_fit_flags.reserve((size_t)std::max(ntiles, 1) * sizeof(int));
   d_list_count.reserve(2 * sizeof(int));
   d_list_off.reserve((size_t)std::max(npairs, 1) * sizeof(int));
+  d_gate_tiles.reserve(std::max<size_t>(gt.size(), 1) * sizeof(int));
   if (!d_fetch.p) {
     d_fetch.reserve(kFetchCounters * sizeof(int));
-    LCR_HIP(hipMemset(d_fetch.p, 0, kFetchCounters * sizeof(int)));
+    launch_fill_i32(d_fetch.as<int>(), kFetchCounters, 0, s);
   }
-  {
-    std::vector<int2> all((size_t)ntiles);
-    for (int t = 0; t < ntiles; ++t) all[t] = make_int2(t, tp[t]);
-    const int counts[2] = {ntiles, ntiles};
-    if (ntiles > 0) {
-      LCR_HIP(hipMemcpy(d_it_list.p, all.data(), all.size() * sizeof(int2), hipMemcpyHostToDevice));
-      LCR_HIP(hipMemcpy(d_fit_list.p, all.data(), all.size() * sizeof(int2), hipMemcpyHostToDevice));
-    }
-    LCR_HIP(hipMemcpy(d_list_count.p, counts, sizeof counts, hipMemcpyHostToDevice));
+  // through pinned memory; every run ends with a wait for the stream, so the last
+  // setup's copies are done before this one rewrites it
+  const size_t pair_bytes = (size_t)npairs * sizeof(PairDesc);
+  h_setup.reserve(pair_bytes + gt.size() * sizeof(int));
+  if (npairs > 0) {
+    memcpy(h_setup.p, hp.data(), pair_bytes);
+    LCR_HIP(hipMemcpyAsync(d_pairs.p, h_setup.p, pair_bytes, hipMemcpyHostToDevice, s));
   }
-  ngate_tiles = (int)gt.size();
-  d_gate_tiles.reserve(std::max<size_t>(gt.size(), 1) * sizeof(int));
-  if (ngate_tiles > 0)
-    LCR_HIP(hipMemcpy(d_gate_tiles.p, gt.data(), gt.size() * sizeof(int), hipMemcpyHostToDevice));
+  if (ngate_tiles > 0) {
+    char* g = h_setup.as<char>() + pair_bytes;
+    memcpy(g, gt.data(), gt.size() * sizeof(int));
+    LCR_HIP(hipMemcpyAsync(d_gate_tiles.p, g, gt.size() * sizeof(int), hipMemcpyHostToDevice, s));
+  }
+  if (ntiles > 0)
+    hipLaunchKernelGGL(k_tile_pairs, dim3((unsigned)((ntiles + 255) / 256)), dim3(256), 0, s,
+                       d_pairs.as<PairDesc>(), npairs, ntiles, d_tile_pair.as<int>());
   const int cus = device_cu_count();
   setup_precision = c.precision;
+  const bool pl = c.point_to_plane != 0;
   for (int ring = 0; ring < 2; ++ring) {
-    const int per_cu = icp_max_blocks_per_cu(tile, c.point_to_plane != 0, c.precision, ring != 0);
-    int nb = std::min(std::max(ntiles, 1), cus * per_cu);
+    int nb = std::min(std::max(ntiles, 1), cus * blocks_per_cu(ring, tile, pl, c.precision));
     nb = std::max(8, (nb + 7) / 8 * 8);
     (ring ? nblocks_ring : nblocks) = nb;
   }
-  int nf = std::min(std::max(ntiles, 1), cus * fitness_max_blocks_per_cu(tile));
+  int nf = std::min(std::max(ntiles, 1), cus * blocks_per_cu(2, tile, false, 0));
   nblocks_fit = std::max(8, (nf + 7) / 8 * 8);
   split_units = icp_split_units();
   if (split_units > 0) {
     int ns = std::min(std::max(std::min(ntiles, split_units / (tile / 64)), 1),
-                      cus * icp_split_blocks_per_cu(tile, c.point_to_plane != 0));
+                      cus * blocks_per_cu(3, tile, pl, 0));
     nblocks_split = std::max(8, (ns + 7) / 8 * 8);
   }
 }
@@ -643,7 +749,17 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
   d_active.reserve(2 * sizeof(int));
   h_active.reserve(2 * sizeof(int));
   const bool split_ok = use_split();
-  const bool eager = !use_graph || prof.on();
+  // A run of a new handle, or of other buffers or parameters than the last, issues
+  // its launches directly; capturing and instantiating its three graphs (about half
+  // a millisecond) waits until the same run comes again.
+  bool eager = !use_graph || prof.on();
+  if (!eager) {
+    const GraphKey key = graph_key(b);
+    const bool captured = exec && tail_exec && (!split_ok || split_exec) && key == graph_key_;
+    eager = !captured && !(eager_key_set_ && key == eager_key_);
+    eager_key_ = key;
+    eager_key_set_ = true;
+  }
   std::vector<Profiler::Span> spans;
   if (gate_h > 1 && ntiles > 0) {
     const int k = prof.begin("gate", s, &spans);

@@ -6,6 +6,7 @@
 
 #include <string.h>
 
+#include <exception>
 #include <functional>
 #include <map>
 #include <mutex>
@@ -14,6 +15,7 @@
 
 #include "lcr_common.hpp"
 #include "lcr_kernels.hpp"
+#include "pool.hpp"
 
 struct lcr_proposal;
 
@@ -31,23 +33,30 @@ struct Error {
       throw ::lcr::Error{-2, std::string(#expr) + " failed: " + hipGetErrorString(e_)};  \
   } while (0)
 
-// Device allocation that only grows.
+// Device allocation that only grows, from the pool and back to it.  Whoever destroys
+// one has waited for the work that used it, unless an exception is unwinding (see
+// pool.hpp).
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  int device = 0;
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf() {
-    if (p) (void)hipFree(p);
+    if (!p) return;
+    if (std::uncaught_exceptions() > 0)
+      (void)hipFree(p);
+    else
+      Pool::get().give_device(p, bytes, device);
   }
   void reserve(size_t n) {
     if (n == 0) n = 256;
     if (n <= bytes) return;
-    if (p) LCR_HIP(hipFree(p));
+    if (p) LCR_HIP(hipFree(p));  // waits for work that may still use it
     p = nullptr;
     bytes = 0;
-    LCR_HIP(hipMalloc(&p, n));
+    p = Pool::get().take_device(&n, &device);
     bytes = n;
   }
   template <class T>
@@ -56,7 +65,7 @@ struct DevBuf {
   }
 };
 
-// Pinned host allocation that only grows.
+// Pinned host allocation that only grows, from the pool and back to it.
 struct HostBuf {
   void* p = nullptr;
   size_t bytes = 0;
@@ -64,7 +73,11 @@ struct HostBuf {
   HostBuf(const HostBuf&) = delete;
   HostBuf& operator=(const HostBuf&) = delete;
   ~HostBuf() {
-    if (p) (void)hipHostFree(p);
+    if (!p) return;
+    if (std::uncaught_exceptions() > 0)
+      (void)hipHostFree(p);
+    else
+      Pool::get().give_pinned(p, bytes);
   }
   void reserve(size_t n) {
     if (n == 0) n = 256;
@@ -72,7 +85,7 @@ struct HostBuf {
     if (p) LCR_HIP(hipHostFree(p));
     p = nullptr;
     bytes = 0;
-    LCR_HIP(hipHostMalloc(&p, n, hipHostMallocDefault));
+    p = Pool::get().take_pinned(&n);
     bytes = n;
   }
   template <class T>
@@ -80,6 +93,63 @@ struct HostBuf {
     return static_cast<T*>(p);
   }
 };
+
+// A stream from the pool, on `device` (made current).  Released after a wait for
+// its work.
+struct Stream {
+  hipStream_t s = nullptr;
+  int device = 0;
+  explicit Stream(int dev) : device(dev) {
+    LCR_HIP(hipSetDevice(device));
+    s = Pool::get().take_stream(device);
+  }
+  Stream(const Stream&) = delete;
+  Stream& operator=(const Stream&) = delete;
+  ~Stream() {
+    if (idle())
+      Pool::get().give_stream(s, device);
+    else
+      (void)hipStreamDestroy(s);
+  }
+  void bind() const { LCR_HIP(hipSetDevice(device)); }
+  // Waits for the stream's work: a handle calls it before its buffers go.
+  bool idle() const noexcept { return hipStreamSynchronize(s) == hipSuccess; }
+};
+
+// Results on their way to a caller's arrays: add() queues a device-to-host copy
+// into pinned memory, finish() waits and moves the bytes on, chunk by chunk while
+// later chunks still arrive.  One wait for all of a call's results, where a copy
+// straight into pageable memory waits for each and runs at 17 GB/s (8 MB of points
+// of a 640 x 480 depth map: the call 549 -> 417 us; a normals call on 2003 points
+// 222 -> 195).
+class CopyOut {
+ public:
+  // bytes: an upper bound of what will be added
+  CopyOut(hipStream_t s, size_t bytes);
+  ~CopyOut();
+  CopyOut(const CopyOut&) = delete;
+  CopyOut& operator=(const CopyOut&) = delete;
+  void add(void* dst, const void* src, size_t bytes);
+  void finish();
+
+ private:
+  static constexpr size_t kChunk = (size_t)1 << 20;
+  struct Piece {
+    void* dst;
+    size_t off, bytes;
+    hipEvent_t done;  // null: covered by a later piece's event or the final wait
+  };
+  hipStream_t s_;
+  HostBuf stage_;
+  size_t used_ = 0, since_event_ = 0;
+  std::vector<Piece> pieces_;
+};
+
+// A host-to-device copy of a caller's array; up to kCopyInStage bytes go through
+// `stage` (pinned, alive until the stream has run the copy): 100 KB 14 us against
+// 53 for a copy from pageable memory, which is as fast from half a megabyte on.
+constexpr size_t kCopyInStage = (size_t)512 << 10;
+void copy_in(hipStream_t s, void* dst, const void* src, size_t bytes, HostBuf& stage);
 
 // Per-kernel GPU time from HIP events recorded around each launch on its stream.
 class Profiler {
@@ -146,13 +216,17 @@ struct CloudSet {
   DevBuf d_slot_raw, d_slot_cell, d_near, d_near_tmp;
   DevBuf d_nwork;  // normals: the query lists of the wavefront and rescan passes
   DevBuf d_nmom;   // normals: FP64 neighbour moments, nine arrays of one per point
-  HostBuf h_stage, h_stage_nrm, h_small, h_build, h_vp;
+  DevBuf d_in;      // the last upload's packed input, and its staging: in use until the
+  HostBuf h_stage;  // stream has run the upload
+  HostBuf h_small, h_build, h_vp;
 
-  // Packs and uploads clouds (x, y, z at the start of each `stride` bytes record;
-  // normals at the same stride from their own pointer).
+  // Uploads clouds (x, y, z at the start of each `stride` bytes record; normals at
+  // the same stride from their own pointer).  Normals are taken when every cloud has
+  // them, or, with zero_nrm, when any has (zeros for the others).  pinned: the
+  // arrays are packed and lie in pinned memory, so they need no staging.
   void upload(hipStream_t s, const std::vector<const float*>& xyz,
               const std::vector<const float*>& nrm, const std::vector<int64_t>& counts,
-              int64_t stride_bytes);
+              int64_t stride_bytes, bool zero_nrm = false, bool pinned = false);
   // Builds every cloud's grid; cell edge = factor * estimated point spacing.
   // with_tree: also the tree order and the bounding-volume tree (the 1-NN searches
   // need them; the k-NN selections of normals and outlier removal do not)
@@ -168,9 +242,9 @@ struct CloudSet {
   // d_npts into d_nnrm (after a kBuildNormals build).
   void compute_normals(hipStream_t s, int k, const float* vp_host, int flip_all,
                        std::vector<Profiler::Span>* spans, bool normals_stage = false);
-  // Copies the cell-sorted normals back to input order (d_raw_nrm), so the next
-  // build() carries them into its own order.
-  void normals_to_raw(hipStream_t s);
+  // The cell-sorted normals and curvatures in input order, packed (NaN where the
+  // point is not finite): xyz of every normal, then every curvature.
+  void normals_to_input_order(hipStream_t s, float* d_nrm3, float* d_curv);
   // Per grid cell: 1 if some point of the cloud may lie within r of a position in
   // the cell (d_near; GridDesc::near_r = r).  Skipped (near_r = 0) for an
   // infinite r or one spanning more than kMaxNearCells cells.
@@ -202,7 +276,7 @@ struct Engine {
   DevBuf d_fit_order;  // IcpBuffers::fit_order
   DevBuf d_fit_flags;  // IcpBuffers::fit_flags
   int ngate_tiles = 0;
-  HostBuf h_state, h_guess;
+  HostBuf h_state, h_guess, h_setup;
   static constexpr int kChunk = 4;  // iterations per captured chunk
   DevBuf d_active;
   HostBuf h_active;
@@ -219,6 +293,9 @@ struct Engine {
     bool operator==(const GraphKey& o) const { return memcmp(this, &o, sizeof *this) == 0; }
   };
   GraphKey graph_key_{};
+  // The last eager run's key: a run is captured when its key comes a second time.
+  GraphKey eager_key_{};
+  bool eager_key_set_ = false;
   GraphKey graph_key(const IcpBuffers& b) const;
   static void capture(hipStream_t s, const std::function<void()>& f, hipGraph_t* g,
                       hipGraphExec_t* e);
@@ -226,8 +303,8 @@ struct Engine {
   ~Engine();
   void reset_graph();
   // (src, tgt) cloud indices per instance; squared radius per instance.
-  void setup(const CloudSet& cs, const std::vector<int>& src, const std::vector<int>& tgt,
-             const std::vector<double>& r2, int tile_pts);
+  void setup(hipStream_t s, const CloudSet& cs, const std::vector<int>& src,
+             const std::vector<int>& tgt, const std::vector<double>& r2, int tile_pts);
   int setup_precision = -1;  // c.precision the launch shape was sized for
   // > 1: instances come in groups of gate_h hypotheses of one pair; before the
   // iterations, each group keeps only its best hypothesis by inliers within r.
