@@ -429,8 +429,8 @@ __global__ void __launch_bounds__(kSolveThreads) k_icp_solve(const IcpBuffers b,
   __shared__ double part[kSolveRows][32];
   __shared__ double tot[32];
   PairState* st = b.state + blockIdx.x;
+  const PairDesc pd = b.pairs[blockIdx.x];  // in flight with the flag
   if (st->active == 0) return;  // uniform across the block
-  const PairDesc pd = b.pairs[blockIdx.x];
   // the state, read now so that its latency hides behind the fold
   PairState ls = *st;
   const int i = threadIdx.x & 31, row = threadIdx.x >> 5;
@@ -456,7 +456,9 @@ __global__ void __launch_bounds__(kSolveThreads) k_icp_solve(const IcpBuffers b,
     tot[threadIdx.x] = sum.value();
   }
   __syncthreads();
-  if (threadIdx.x != 0) return;
+  // the first wavefront solves, every lane the same (the angles' sines are shared
+  // out); lane 0 stores
+  if (threadIdx.x >= 64) return;
   double v[NV];
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = tot[k];
@@ -467,7 +469,7 @@ __global__ void __launch_bounds__(kSolveThreads) k_icp_solve(const IcpBuffers b,
     ls.state = kNoCorrespondences;
     ls.converged = 0;
     ls.active = 0;
-    *st = ls;
+    if (threadIdx.x == 0) *st = ls;
     return;
   }
   double Tinc[16];
@@ -487,7 +489,7 @@ __global__ void __launch_bounds__(kSolveThreads) k_icp_solve(const IcpBuffers b,
     ls.converged = 1;
     ls.active = 0;
   }
-  *st = ls;
+  if (threadIdx.x == 0) *st = ls;
 }
 
 // per_instance: each instance's own max_corr_d2 is the range.  A finite range

@@ -6,7 +6,9 @@
 // Solvers:
 //   * horn_rotation   -- point-to-point: the rotation maximising trace(R^T S) from
 //     the 3x3 cross-covariance S, as the eigenvector of Horn's 4x4 matrix with the
-//     largest eigenvalue (Horn 1987).  Equals Umeyama's U diag(1,1,det) V^T, which
+//     largest eigenvalue (Horn 1987): Newton on the characteristic polynomial and
+//     the adjugate where that eigenvalue is well separated, cyclic Jacobi
+//     otherwise.  Equals Umeyama's U diag(1,1,det) V^T, which
 //     TransformationEstimationSVD computes (pcl/registration/impl/
 //     transformation_estimation_svd.hpp; called via fine_registration.cpp:121).
 //   * chol6_solve     -- point-to-plane: the 6x6 normal equations of
@@ -73,6 +75,89 @@ LCR_HD void jacobi4(double a[4][4], double v[4][4]) {
   }
 }
 
+// The eigenvector of the largest eigenvalue of a symmetric traceless 4x4 matrix a
+// with entries of at most 1 in magnitude.  The eigenvalue is the largest root of
+// l^4 + c2 l^2 + c1 l + c0 (all roots real): Newton from a bound above it descends
+// monotonically.  The adjugate of a - l I is the eigenvector's outer product times
+// the product of the eigenvalue's distances to the others, p'(l); its column of
+// largest diagonal is scaled to unit length.  Rounding enters relative to p'(l), so
+// where that is below kSeparated (elongated or degenerate clouds) this returns
+// false and the caller takes Jacobi.  About 0.6 us of one lane's FP64 latency
+// against 9 for Jacobi's 25-30 rotations of two divisions and two square roots.
+constexpr double kSeparated = 0.05;
+
+LCR_HD bool top_eigvec4(const double a[4][4], double q[4]) {
+  double fro = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) fro += a[i][j] * a[i][j];
+  // power sums of the eigenvalues: p2 = fro, p3 = trace(a^3)
+  double p3 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) s += a[i][k] * a[k][j];
+      p3 += s * a[j][i];
+    }
+  // 2x2 minors of the first and the last two rows: determinant and adjugate
+  auto det = [](const double m[4][4]) {
+    const double s0 = m[0][0] * m[1][1] - m[1][0] * m[0][1], s1 = m[0][0] * m[1][2] - m[1][0] * m[0][2];
+    const double s2 = m[0][0] * m[1][3] - m[1][0] * m[0][3], s3 = m[0][1] * m[1][2] - m[1][1] * m[0][2];
+    const double s4 = m[0][1] * m[1][3] - m[1][1] * m[0][3], s5 = m[0][2] * m[1][3] - m[1][2] * m[0][3];
+    const double c5 = m[2][2] * m[3][3] - m[3][2] * m[2][3], c4 = m[2][1] * m[3][3] - m[3][1] * m[2][3];
+    const double c3 = m[2][1] * m[3][2] - m[3][1] * m[2][2], c2 = m[2][0] * m[3][3] - m[3][0] * m[2][3];
+    const double c1 = m[2][0] * m[3][2] - m[3][0] * m[2][2], c0 = m[2][0] * m[3][1] - m[3][0] * m[2][1];
+    return s0 * c5 - s1 * c4 + s2 * c3 + s3 * c2 - s4 * c1 + s5 * c0;
+  };
+  const double c2 = -0.5 * fro, c1 = -p3 / 3.0, c0 = det(a);
+  // a traceless matrix's largest eigenvalue is at most sqrt(3 / 4) of its norm
+  double l = 0.8660254037844387 * sqrt(fro) * (1.0 + 1e-12);
+  double dp = 0.0;
+  for (int it = 0; it < 40; ++it) {
+    const double l2 = l * l;
+    const double f = (l2 + c2) * l2 + (c1 * l + c0);
+    dp = (4.0 * l2 + 2.0 * c2) * l + c1;
+    if (!(dp > 0.0)) return false;
+    const double step = f / dp;
+    l -= step;
+    if (!(fabs(step) > 4e-16 * l)) break;
+  }
+  if (!(dp > kSeparated)) return false;
+  double m[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) m[i][j] = a[i][j] - (i == j ? l : 0.0);
+  // cofactor of (i, j): symmetric, so the adjugate's column j
+  auto cof = [&](int i, int j) {
+    const int r0 = i == 0 ? 1 : 0, r1 = i <= 1 ? 2 : 1, r2 = i <= 2 ? 3 : 2;
+    const int k0 = j == 0 ? 1 : 0, k1 = j <= 1 ? 2 : 1, k2 = j <= 2 ? 3 : 2;
+    const double d = m[r0][k0] * (m[r1][k1] * m[r2][k2] - m[r1][k2] * m[r2][k1]) -
+                     m[r0][k1] * (m[r1][k0] * m[r2][k2] - m[r1][k2] * m[r2][k0]) +
+                     m[r0][k2] * (m[r1][k0] * m[r2][k1] - m[r1][k1] * m[r2][k0]);
+    return ((i + j) & 1) ? -d : d;
+  };
+  double c[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = i; j < 4; ++j) c[i][j] = c[j][i] = cof(i, j);
+  double best = 0.0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (fabs(c[j][j]) > best) {
+      best = fabs(c[j][j]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[i] = c[i][j];
+    }
+  }
+  return best > 0.0;
+}
+
 // S[a][b] = cross-covariance sum_i (s_i - mu_s)_a (t_i - mu_t)_b / n, source first.
 // Returns the row-major rotation R (3x3) taking the source onto the target.
 LCR_HD void horn_rotation(const double S[3][3], double R[3][3]) {
@@ -95,20 +180,23 @@ LCR_HD void horn_rotation(const double S[3][3], double R[3][3]) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) N[i][j] *= inv;
-  double V[4][4];
-  jacobi4(N, V);
-  double best = N[0][0];
-  double q0 = V[0][0], q1 = V[1][0], q2 = V[2][0], q3 = V[3][0];
+  double q[4];
+  if (!top_eigvec4(N, q)) {
+    double V[4][4];
+    jacobi4(N, V);
+    double best = N[0][0];
 #pragma unroll
-  for (int c = 1; c < 4; ++c) {
-    if (N[c][c] > best) {
-      best = N[c][c];
-      q0 = V[0][c];
-      q1 = V[1][c];
-      q2 = V[2][c];
-      q3 = V[3][c];
+    for (int i = 0; i < 4; ++i) q[i] = V[i][0];
+#pragma unroll
+    for (int c = 1; c < 4; ++c) {
+      if (N[c][c] > best) {
+        best = N[c][c];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = V[i][c];
+      }
     }
   }
+  double q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
   const double nq = sqrt(q0 * q0 + q1 * q1 + q2 * q2 + q3 * q3);
   q0 /= nq;
   q1 /= nq;
@@ -155,9 +243,11 @@ LCR_HD void p2p_increment(const double* v, double T[16]) {
 LCR_HD constexpr int tri6(int i, int j) { return i * 6 - (i * (i - 1)) / 2 + (j - i); }
 
 // Solve M x = b for symmetric positive definite M given as its packed upper
-// triangle.  Returns false when a pivot is not positive.
+// triangle.  Returns false when a pivot is not positive.  One division per pivot
+// (the reciprocal of its root scales the column and both substitutions): divisions
+// and roots are what one lane's latency goes to.
 LCR_HD bool chol6_solve(const double* up, const double* b, double x[6]) {
-  double L[6][6];
+  double L[6][6], inv[6];
 #pragma unroll
   for (int i = 0; i < 6; ++i)
 #pragma unroll
@@ -169,14 +259,13 @@ LCR_HD bool chol6_solve(const double* up, const double* b, double x[6]) {
 #pragma unroll
     for (int k = 0; k < j; ++k) d -= L[j][k] * L[j][k];
     if (!(d > 0.0)) ok = false;
-    const double ljj = sqrt(d > 0.0 ? d : 1.0);
-    L[j][j] = ljj;
+    inv[j] = 1.0 / sqrt(d > 0.0 ? d : 1.0);
 #pragma unroll
     for (int i = j + 1; i < 6; ++i) {
       double s = up[tri6(j, i)];
 #pragma unroll
       for (int k = 0; k < j; ++k) s -= L[i][k] * L[j][k];
-      L[i][j] = s / ljj;
+      L[i][j] = s * inv[j];
     }
   }
   double y[6];
@@ -185,24 +274,24 @@ LCR_HD bool chol6_solve(const double* up, const double* b, double x[6]) {
     double s = b[i];
 #pragma unroll
     for (int k = 0; k < i; ++k) s -= L[i][k] * y[k];
-    y[i] = s / L[i][i];
+    y[i] = s * inv[i];
   }
 #pragma unroll
   for (int i = 5; i >= 0; --i) {
     double s = y[i];
 #pragma unroll
     for (int k = i + 1; k < 6; ++k) s -= L[k][i] * x[k];
-    x[i] = s / L[i][i];
+    x[i] = s * inv[i];
   }
   return ok;
 }
 
 // TransformationEstimationPointToPlaneLLS::constructTransformationMatrix:
 // T = [Rz(g) Ry(b) Rx(a) | t].
-LCR_HD void p2pl_matrix(const double x[6], double T[16]) {
-  const double ca = cos(x[0]), sa = sin(x[0]);
-  const double cb = cos(x[1]), sb = sin(x[1]);
-  const double cg = cos(x[2]), sg = sin(x[2]);
+LCR_HD void p2pl_matrix(const double sn[3], const double cs[3], const double x[6], double T[16]) {
+  const double ca = cs[0], sa = sn[0];
+  const double cb = cs[1], sb = sn[1];
+  const double cg = cs[2], sg = sn[2];
   T[0] = cg * cb;
   T[1] = -sg * ca + cg * sb * sa;
   T[2] = sg * sa + cg * sb * ca;
@@ -222,7 +311,9 @@ LCR_HD void p2pl_matrix(const double x[6], double T[16]) {
 }
 
 // Point-to-plane increment from v[1..21] (packed A^T A) and v[22..27] (A^T b).
-// Returns false if the system is not positive definite (T = identity then).
+// Returns false if the system is not positive definite (T = identity then).  On
+// the device every lane of a wavefront calls it with the same v: lane l takes the
+// sine and cosine of angle l % 3, so the three angles cost one's latency.
 LCR_HD bool p2pl_increment(const double* v, double T[16]) {
   double x[6];
   const bool ok = chol6_solve(v + 1, v + 22, x);
@@ -231,7 +322,23 @@ LCR_HD bool p2pl_increment(const double* v, double T[16]) {
     for (int i = 0; i < 16; ++i) T[i] = (i % 5 == 0) ? 1.0 : 0.0;
     return false;
   }
-  p2pl_matrix(x, T);
+  double sn[3], cs[3];
+#ifdef __HIP_DEVICE_COMPILE__
+  const int l = (int)(threadIdx.x & 63) % 3;
+  double s1, c1;
+  sincos(l == 0 ? x[0] : (l == 1 ? x[1] : x[2]), &s1, &c1);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    sn[i] = __shfl(s1, i, 64);
+    cs[i] = __shfl(c1, i, 64);
+  }
+#else
+  for (int i = 0; i < 3; ++i) {
+    sn[i] = sin(x[i]);
+    cs[i] = cos(x[i]);
+  }
+#endif
+  p2pl_matrix(sn, cs, x, T);
   return true;
 }
 

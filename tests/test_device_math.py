@@ -67,6 +67,28 @@ def test_horn_random_rotations(m):
         np.testing.assert_allclose(T.reshape(4, 4)[:3, :3], R, atol=1e-8)
 
 
+@pytest.mark.parametrize("spec", [(1, .8, .6), (1, .7, .01), (1, .05, .02), (1, .03, 0), (1, .025, .025),
+                                  (1, 0, 0), (1, 1, 1), (1, 1, 0), (1, .5, -.3), (1, 1, -1),
+                                  (1e-9, 5e-10, 1e-10), (3e7, 1e7, 1e6), (0, 0, 0)])
+def test_horn_maximises_the_trace_for_every_spectrum(m, spec):
+    """Separated, elongated, flat, reflected, degenerate and zero covariances: on both
+    sides of the closed form's separation limit the result is a rotation, and its
+    trace is the largest one a rotation reaches (the sum of the singular values, the
+    last with the determinant's sign).  Rounding: a few ulps of the largest."""
+    rng = np.random.default_rng(5)
+    for _ in range(40):
+        U, V = synth.random_rotation(rng), synth.random_rotation(rng)
+        S = np.ascontiguousarray(U @ np.diag(spec) @ V.T)
+        R = np.empty(9)
+        m.lcrm_horn(P(S), P(R))
+        R = R.reshape(3, 3)
+        np.testing.assert_allclose(R @ R.T, np.eye(3), atol=4e-15)
+        assert np.linalg.det(R) > 0.99
+        # S is source x target, so R maximises sum_ab R[b][a] S[a][b]
+        best = spec[0] + spec[1] + spec[2]
+        assert abs(np.trace(R @ S) - best) <= 2e-14 * max(abs(spec[0]), 1e-300)
+
+
 def test_p2pl_cholesky_matches_lstsq_golden(m):
     g = golden("p2pl.npz")
     off = 0
