@@ -213,7 +213,8 @@ __global__ void __launch_bounds__(TILE, 7) k_icp_iter(const IcpBuffers b, const 
     const bool empty = own && bounded && b.near && gt.near_r >= r &&
                        !near_cell(gt, b.near, qx, qy, qz);
     bool search = own && !empty;  // lanes that still need the scalar search
-    int seed = (search && b.prev) ? b.prev[slot] : -1;
+    // an instance's first iteration has no matches yet
+    int seed = (search && b.prev && st->iterations > 0) ? b.prev[slot] : -1;
     if constexpr (PREC != 0) {
       __shared__ TileLds tl;
       const bool q_ok = search && isfinite(qx) && isfinite(qy) && isfinite(qz);
@@ -350,7 +351,7 @@ __global__ void __launch_bounds__(64 * kSplitLanes) k_icp_iter_split(const IcpBu
       if (own) xform(st->T, point_of(base + qi), qx, qy, qz);
       const bool empty = own && b.near && gt.near_r >= r && !near_cell(gt, b.near, qx, qy, qz);
       if (own && !empty) {
-        const int seed = b.prev ? b.prev[(int64_t)tile * TILE + qi] : -1;
+        const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + qi] : -1;
         nn = nn_ring_split<S>(gt, b.cell_start + gt.cell_off, b.pts, qx, qy, qz, r, seed, sub);
       }
       if (sub == 0) {
@@ -550,7 +551,7 @@ __global__ void __launch_bounds__(TILE, 6) k_fitness(const IcpBuffers b, double 
       const bool empty = bounded && b.near && gt.near_r >= rq && !near_cell(gt, b.near, qx, qy, qz);
       // the lane's previous match: the iterations take the same points in the same
       // lanes as the final pass (the gate's pass runs before any match exists)
-      const int seed = b.prev ? b.prev[(int64_t)tile * TILE + threadIdx.x] : -1;
+      const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + threadIdx.x] : -1;
       // the final pass over refined instances: a point without a match within r in
       // the last iteration (seed -1) is farther than about r from the target; a
       // ring search would scan two unpruned rings before handing it to the tree,
@@ -712,52 +713,77 @@ __global__ void k_gate(PairState* st, int npairs, int H) {
   }
 }
 
-// The (tile, instance) lists of the tiles whose instance takes part: mode 0 --
-// active instances (the search), mode 1 -- instances the gate kept (the final
-// fitness pass).  With the gate setting most hypotheses aside, a launch over
-// every tile left each block a different number of live tiles and waited for the
-// fullest; over the list the live tiles are dealt out evenly.  Two launches: one
-// block places each instance's run of tiles (a block scan over runs of
-// instances per thread, into off[]), then one thread per tile writes its entry.
+// The (tile, instance) lists of the tiles whose instance takes part: the active
+// instances' (the search) and, with fit_list, those of the instances the gate kept
+// (the final fitness pass), both in tile order.  With the gate setting most
+// hypotheses aside, a launch over every tile left each block a different number of
+// live tiles and waited for the fullest; over the list the live tiles are dealt
+// out evenly.  One launch: a block places its 1024 tiles after the live tiles of
+// the instances before its first one, which it adds up itself (a flag and a count
+// per instance), by ballot ranks.  The last block also leaves the number of active
+// instances and of live tiles in host memory, then a flag the host waits for: a
+// chunk's end costs the host this launch, not three, a copy and a wait for the
+// stream (about 40 us of a chunk of four iterations, now about 15).
 constexpr int kCompactThreads = 1024;
 
 __device__ __forceinline__ bool takes_part(const PairState& st, int mode) {
   return mode == 0 ? st.active != 0 : st.gated == 0;
 }
 
-__global__ void __launch_bounds__(kCompactThreads)
-k_compact_offsets(const IcpBuffers b, int mode, int* __restrict__ off, int* __restrict__ count) {
-  __shared__ int s_off[kCompactThreads];
-  const int t = threadIdx.x;
-  const int per = (b.npairs + kCompactThreads - 1) / kCompactThreads;
-  const int p0 = min(t * per, b.npairs), p1 = min(p0 + per, b.npairs);
-  int n = 0;
-  for (int p = p0; p < p1; ++p)
-    if (takes_part(b.state[p], mode)) n += b.pairs[p].ntiles;
-  s_off[t] = n;
+__device__ __forceinline__ int block_total(int v, int* lds) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  __syncthreads();  // lds may still be read from before
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int o = 1; o < kCompactThreads; o <<= 1) {
-    const int v = t >= o ? s_off[t - o] : 0;
-    __syncthreads();
-    s_off[t] += v;
-    __syncthreads();
-  }
-  if (t == kCompactThreads - 1) *count = s_off[t];
-  int at = s_off[t] - n;
-  for (int p = p0; p < p1; ++p) {
-    const bool on = takes_part(b.state[p], mode);
-    off[p] = on ? at : -1;
-    if (on) at += b.pairs[p].ntiles;
-  }
+  int s = 0;
+#pragma unroll
+  for (int k = 0; k < kCompactThreads / 64; ++k) s += lds[k];
+  return s;
 }
 
-__global__ void k_compact_write(const IcpBuffers b, const int* __restrict__ off,
-                                int2* __restrict__ list) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= b.ntiles) return;
-  const int p = b.tile_pair[t];
-  const int o = off[p];
-  if (o >= 0) list[o + (t - b.pairs[p].tile_begin)] = make_int2(t, p);
+__global__ void __launch_bounds__(kCompactThreads)
+k_compact(const IcpBuffers b, int2* __restrict__ it_list, int* __restrict__ it_count,
+          int2* __restrict__ fit_list, int* __restrict__ fit_count, int* host) {
+  constexpr int kW = kCompactThreads / 64;
+  __shared__ int lds[kW];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int first = blockIdx.x * kCompactThreads, t = first + (int)threadIdx.x;
+  const bool valid = t < b.ntiles;
+  const int p = valid ? b.tile_pair[t] : 0;
+  const int p0 = b.tile_pair[first];  // the grid covers ntiles > 0: first is a tile
+  const bool last = blockIdx.x == gridDim.x - 1;
+  for (int mode = 0; mode < (fit_list ? 2 : 1); ++mode) {
+    const bool on = valid && takes_part(b.state[p], mode);
+    const uint64_t m = __ballot(on);
+    int before = 0;
+    for (int k = threadIdx.x; k <= p0; k += kCompactThreads)
+      if (takes_part(b.state[k], mode))
+        before += k < p0 ? b.pairs[k].ntiles : first - b.pairs[k].tile_begin;
+    const int base = block_total(before, lds);
+    __syncthreads();
+    if (lane == 0) lds[w] = __popcll(m);
+    __syncthreads();
+    int at = base, total = base;
+#pragma unroll
+    for (int k = 0; k < kW; ++k) {
+      at += k < w ? lds[k] : 0;
+      total += lds[k];
+    }
+    int2* list = mode == 0 ? it_list : fit_list;
+    if (on) list[at + __popcll(m & ((1ull << lane) - 1ull))] = make_int2(t, p);
+    if (last && threadIdx.x == 0) *(mode == 0 ? it_count : fit_count) = total;
+    if (mode == 0 && last && host) {  // uniform across the block
+      int active = 0;
+      for (int k = threadIdx.x; k < b.npairs; k += kCompactThreads) active += b.state[k].active ? 1 : 0;
+      active = block_total(active, lds);
+      if (threadIdx.x == 0) {
+        host[0] = active;
+        host[1] = total;
+        __hip_atomic_store(&host[2], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+    }
+  }
 }
 
 __global__ void k_state_init(PairState* st, const double* guesses, const PairDesc* pairs,
@@ -1012,16 +1038,11 @@ void launch_fitness(const IcpBuffers& b, double max_range, int nblocks, hipStrea
   hipLaunchKernelGGL(k_fitness_fold, dim3(b.npairs), dim3(kFoldThreads), 0, s, b, pi);
 }
 
-void launch_compact_tiles(const IcpBuffers& b, int* off, int2* it_list, int* it_count,
-                          int2* fit_list, int* fit_count, bool fit, hipStream_t s) {
+void launch_compact_tiles(const IcpBuffers& b, int2* it_list, int* it_count, int2* fit_list,
+                          int* fit_count, int* host, hipStream_t s) {
   if (b.npairs <= 0 || b.ntiles <= 0) return;
-  const unsigned blocks = (unsigned)((b.ntiles + 255) / 256);
-  hipLaunchKernelGGL(k_compact_offsets, dim3(1), dim3(kCompactThreads), 0, s, b, 0, off, it_count);
-  hipLaunchKernelGGL(k_compact_write, dim3(blocks), dim3(256), 0, s, b, off, it_list);
-  if (!fit) return;
-  hipLaunchKernelGGL(k_compact_offsets, dim3(1), dim3(kCompactThreads), 0, s, b, 1, off,
-                     fit_count);
-  hipLaunchKernelGGL(k_compact_write, dim3(blocks), dim3(256), 0, s, b, off, fit_list);
+  hipLaunchKernelGGL(k_compact, dim3((b.ntiles + kCompactThreads - 1) / kCompactThreads),
+                     dim3(kCompactThreads), 0, s, b, it_list, it_count, fit_list, fit_count, host);
 }
 
 void launch_gate(PairState* st, int npairs, int H, hipStream_t s) {

@@ -117,10 +117,12 @@ void* Pool::take_pinned(size_t* bytes) {
   *bytes = size_class(*bytes);
   void* p = take(Key(kPinned, *bytes));
   if (p) return p;
-  hipError_t e = hipHostMalloc(&p, *bytes, hipHostMallocDefault);
+  // coherent: kernels leave flags there that the host waits for
+  const unsigned flags = hipHostMallocMapped | hipHostMallocCoherent;
+  hipError_t e = hipHostMalloc(&p, *bytes, flags);
   if (e != hipSuccess && flush(kPinned)) {
     (void)hipGetLastError();
-    e = hipHostMalloc(&p, *bytes, hipHostMallocDefault);
+    e = hipHostMalloc(&p, *bytes, flags);
   }
   if (e != hipSuccess) throw Error{-2, std::string("hipHostMalloc failed: ") + hipGetErrorString(e)};
   return p;

@@ -607,7 +607,6 @@ void Engine::setup(hipStream_t s, const CloudSet& cs, const std::vector<int>& sr
   d_fit_order.reserve((size_t)std::max(ntiles, 1) * sizeof(int2));
   d_fit_flags.reserve((size_t)std::max(ntiles, 1) * sizeof(int));
   d_list_count.reserve(2 * sizeof(int));
-  d_list_off.reserve((size_t)std::max(npairs, 1) * sizeof(int));
   d_gate_tiles.reserve(std::max<size_t>(gt.size(), 1) * sizeof(int));
   if (!d_fetch.p) {
     d_fetch.reserve(kFetchCounters * sizeof(int));
@@ -686,29 +685,24 @@ IcpBuffers Engine::buffers(const CloudSet& cs) const {
   return b;
 }
 
-namespace {
-// out[0]: instances still active; out[1]: live tiles (the last compaction's count).
-__global__ void k_count_active(const PairState* __restrict__ st, int n,
-                               const int* __restrict__ live_tiles, int* __restrict__ out) {
-  __shared__ int s[256];
-  int a = 0;
-  for (int i = threadIdx.x; i < n; i += 256) a += st[i].active ? 1 : 0;
-  s[threadIdx.x] = a;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    out[0] = s[0];
-    out[1] = *live_tiles;
+// Waits until a kernel on `s` has set *flag (coherent host memory).  Ends in any
+// case: once the stream has nothing left to run or reports an error.
+static void wait_flag(const int* flag, hipStream_t s) {
+  for (unsigned spins = 1;; ++spins) {
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) return;
+    __builtin_ia32_pause();
+    if (spins % 1024 != 0) continue;
+    const hipError_t e = hipStreamQuery(s);
+    if (e == hipErrorNotReady) continue;
+    LCR_HIP(e);
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) return;
+    throw Error{-2, "the iterations ended without their count"};
   }
 }
-}  // namespace
 
 // The run is: state init -> chunks of kChunk iterations -> fitness.  Each chunk
-// ends with a count of still-active instances copied to pinned memory; the host
-// stops launching chunks once it reads zero, so converged cycles do not replay
+// ends with a count of still-active instances in host memory; the host stops
+// launching chunks once it reads zero, so converged cycles do not replay
 // empty iterations.  With the profiler off each chunk (and the tail) replays a
 // captured hipGraph; HIP events recorded inside a captured graph cannot be timed
 // afterwards, so with the profiler on the same launches are issued eagerly with
@@ -743,11 +737,13 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
   if (pre) pre();
   launch_state_init(d_state.as<PairState>(), d_guess.as<double>(), d_pairs.as<PairDesc>(),
                     cs.d_grids.as<GridDesc>(), npairs, s);
-  launch_fill_i32(d_prev.as<int>(), (int64_t)ntiles * tile, -1, s);  // no previous matches
-  launch_compact_tiles(b, d_list_off.as<int>(), d_it_list.as<int2>(), d_list_count.as<int>(),
-                       d_fit_list.as<int2>(), d_list_count.as<int>() + 1, true, s);
-  d_active.reserve(2 * sizeof(int));
-  h_active.reserve(2 * sizeof(int));
+  auto compact_all = [&] {
+    launch_compact_tiles(b, d_it_list.as<int2>(), d_list_count.as<int>(), d_fit_list.as<int2>(),
+                         d_list_count.as<int>() + 1, nullptr, s);
+  };
+  const bool gated = gate_h > 1 && ntiles > 0;
+  if (!gated) compact_all();
+  h_active.reserve(3 * sizeof(int));
   const bool split_ok = use_split();
   // A run of a new handle, or of other buffers or parameters than the last, issues
   // its launches directly; capturing and instantiating its three graphs (about half
@@ -761,15 +757,14 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
     eager_key_set_ = true;
   }
   std::vector<Profiler::Span> spans;
-  if (gate_h > 1 && ntiles > 0) {
+  if (gated) {
     const int k = prof.begin("gate", s, &spans);
     // XCD-contiguous: the hypotheses of a pair share its target grid in one L2
     // (74 pairs x 15 hypotheses: 21.4 against 21.6 ms per cycle step in grid-stride
     // order)
     launch_fitness(b, 0.0, nblocks_fit, s, true, 0);
     launch_gate(d_state.as<PairState>(), npairs / gate_h, gate_h, s);
-    launch_compact_tiles(b, d_list_off.as<int>(), d_it_list.as<int2>(), d_list_count.as<int>(),
-                         d_fit_list.as<int2>(), d_list_count.as<int>() + 1, true, s);
+    compact_all();
     prof.end(k, s, &spans);
   }
   auto chunk = [&](std::vector<Profiler::Span>* sp, bool split) {
@@ -787,11 +782,8 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
       launch_icp_solve(b, c, s);
       prof.end(k2, s, sp);
     }
-    launch_compact_tiles(b, d_list_off.as<int>(), d_it_list.as<int2>(), d_list_count.as<int>(),
-                         nullptr, nullptr, false, s);
-    hipLaunchKernelGGL(k_count_active, dim3(1), dim3(256), 0, s, d_state.as<PairState>(), npairs,
-                       d_list_count.as<int>(), d_active.as<int>());
-    LCR_HIP(hipMemcpyAsync(h_active.p, d_active.p, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    launch_compact_tiles(b, d_it_list.as<int2>(), d_list_count.as<int>(), nullptr, nullptr,
+                         h_active.as<int>(), s);
   };
   auto tail = [&](std::vector<Profiler::Span>* sp) {
     const int k = prof.begin("fitness", s, sp);
@@ -816,14 +808,16 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
   // when the previous chunk left that few live
   bool split = split_fits(ntiles);
   const int max_chunks = ntiles > 0 ? (c.max_iterations + kChunk - 1) / kChunk : 0;
+  int* const host = h_active.as<int>();
   for (int k = 0; k < max_chunks; ++k) {
+    host[2] = 0;  // the last chunk, if any, has set it
     if (eager)
       chunk(&spans, split);
     else
       LCR_HIP(hipGraphLaunch(split ? split_exec : exec, s));
-    LCR_HIP(hipStreamSynchronize(s));
-    if (h_active.as<int>()[0] == 0) break;
-    split = split_fits(h_active.as<int>()[1]);
+    wait_flag(&host[2], s);
+    if (host[0] == 0) break;
+    split = split_fits(host[1]);
   }
   if (ntiles > 0) {
     if (eager)
@@ -864,7 +858,6 @@ Engine::GraphKey Engine::graph_key(const IcpBuffers& b) const {
   k.nblocks_split = use_split() ? nblocks_split : 0;
   k.guess = d_guess.p;
   k.hstate = h_state.p;
-  k.active = d_active.p;
   k.hactive = h_active.p;
   return k;
 }

@@ -271,15 +271,14 @@ struct Engine {
   IcpConst c{};
   std::vector<PairDesc> hp;
   DevBuf d_pairs, d_tile_pair, d_state, d_partials, d_guess, d_prev, d_gate_tiles;
-  DevBuf d_it_list, d_fit_list, d_list_count, d_list_off;  // live-tile lists (IcpBuffers::it_list)
+  DevBuf d_it_list, d_fit_list, d_list_count;  // live-tile lists (IcpBuffers::it_list)
   DevBuf d_fetch;      // IcpBuffers::fetch
   DevBuf d_fit_order;  // IcpBuffers::fit_order
   DevBuf d_fit_flags;  // IcpBuffers::fit_flags
   int ngate_tiles = 0;
   HostBuf h_state, h_guess, h_setup;
   static constexpr int kChunk = 4;  // iterations per captured chunk
-  DevBuf d_active;
-  HostBuf h_active;
+  HostBuf h_active;  // a chunk's active instances, live tiles and flag (launch_compact_tiles)
   hipGraph_t graph = nullptr, tail_graph = nullptr, split_graph = nullptr;
   hipGraphExec_t exec = nullptr, tail_exec = nullptr, split_exec = nullptr;
   struct GraphKey {
@@ -288,7 +287,6 @@ struct Engine {
     int nblocks = 0, nblocks_fit = 0, nblocks_split = 0;
     const void* guess = nullptr;
     const void* hstate = nullptr;
-    const void* active = nullptr;
     const void* hactive = nullptr;
     bool operator==(const GraphKey& o) const { return memcmp(this, &o, sizeof *this) == 0; }
   };

@@ -72,3 +72,6 @@ def test_repeated_runs_of_a_handle_equal_a_new_one(lcr):
         icp.setMaximumIterations(n)
         np.testing.assert_array_equal(icp.align(), want[n][0])
         work(lcr, 0, n)
+        # waiting for the iterations leaves no error behind for the next call
+        f = np.full((3, 20, 30), 900 + n, np.uint16)
+        np.testing.assert_array_equal(lcr.depth_fuse(f, 2), f[0])
