@@ -485,9 +485,11 @@ void CloudSet::build_near_mask(hipStream_t s, double r) {
   // dilation in cells: a point within r of a query lies at most ceil(r / h) + 1
   // cells away along each axis (the +1 covers positions inside the cells and
   // binning rounding)
-  int kd_max = 0;
+  // (in double: the default radius, sqrt(DBL_MAX), spans more cells than an int
+  // holds, and as one it passed for a small mask whose dilation took minutes)
+  double kd_max = 0.0;
   for (const GridDesc& g : grids)
-    if (g.npts > 0) kd_max = std::max(kd_max, (int)ceil(r * 1.0001 * (double)g.inv_h) + 1);
+    if (g.npts > 0) kd_max = std::max(kd_max, ceil(r * 1.0001 * (double)g.inv_h) + 1.0);
   const bool use = std::isfinite(r) && r > 0.0 && kd_max <= kMaxNearCells && total_cells > 0;
   // the same word offsets launch_set_near gives the device copy
   int64_t words = 0;

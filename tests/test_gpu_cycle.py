@@ -238,3 +238,21 @@ def test_batch_of_more_than_33m_cells_equals_single_pairs(lcr):
         one = lcr.Cycle([clouds[s], clouds[t]], [(0, 1)], **kw)
         one.run()
         np.testing.assert_array_equal(one.results()["T"][0], T[p])
+
+
+def test_default_radius_spans_no_near_mask(lcr):
+    """The radius that the parameters default to, sqrt(DBL_MAX), spans more cells
+    than an int counts: no near mask is built for it, and a pair gets the bits of a
+    radius far beyond every distance."""
+    cyc = synth.turntable_cycle(7, n_captures=2, yaw_step_deg=10.0, scale=1.0,
+                                centre=(0.0, 0.0, -0.8))
+    clouds = [c[:2000] for c in cyc.clouds]
+    res = []
+    for r in (1000.0, 1.3407807929942596e154):
+        print_case(test="default_radius", r=r)
+        c = lcr.Cycle(clouds, [(0, 1)], point_to_plane=False, max_corr_dist=r, max_iterations=6)
+        c.run()
+        res.append(c.results())
+        del c
+    for k in ("T", "iterations", "fitness"):
+        np.testing.assert_array_equal(res[1][k], res[0][k])
