@@ -25,6 +25,8 @@
 #include <hip/hip_runtime.h>
 #include <float.h>
 
+#include <algorithm>
+
 #include "lcr_common.hpp"
 #include "lcr_kernels.hpp"
 #include "lcr_math.hpp"
@@ -264,16 +266,19 @@ __global__ void __launch_bounds__(TILE, 7) k_icp_iter(const IcpBuffers b, const 
   }
 }
 
-// The ring-only search for launches with few live tiles.  Each query gets
-// kSplitLanes lanes; each lane scans every kSplitLanes-th (z, y) row of a ring
-// (ring_rows), and the lanes take the minimum by (d2, id) after every ring, so the
-// result is the one-lane search's.  A block of kSplitLanes wavefronts takes one
-// tile, 64 queries per pass (64 / kSplitLanes per wavefront); the TILE results go
-// through LDS to the first TILE threads, which form the tile's sums exactly as
+// The search for launches with few live tiles.  Each query gets kSplitLanes lanes;
+// each lane scans every kSplitLanes-th (z, y) row of the seed's ball or of a ring,
+// and the lanes take the minimum by (d2, id) after the ball and after every ring,
+// so the result is the one-lane search's.  A block of kSplitLanes wavefronts takes
+// one tile, 64 queries per pass (64 / kSplitLanes per wavefront); the TILE results
+// go through LDS to the first TILE threads, which form the tile's sums exactly as
 // k_icp_iter<TILE> does (query i in lane i % 64 of wavefront i / 64).  With a few
 // hundred tiles live the one-lane kernel leaves most SIMDs idle, and each
 // wavefront waits on its longest chain of row loads; this one runs kSplitLanes
-// times as many wavefronts, each with about 1 / kSplitLanes of the rows.
+// times as many wavefronts, each with about 1 / kSplitLanes of the rows, and a
+// wavefront's tree walk serves a quarter of the queries, whose paths coincide more.
+// A 20k-point pair at a radius of 5 cm (313 tiles): 25 us an iteration with one
+// lane per query, 15.6 with four.
 constexpr int kSplitLanes = 4;
 
 template <int S>
@@ -290,28 +295,44 @@ __device__ __forceinline__ void lanes_min(float& best, int& bid, int& bj) {
   }
 }
 
-// Bounded ring-only 1-NN over S lanes (sub = this lane's index among them).  The S
-// lanes of a query are consecutive and reach every lanes_min together: their
-// early returns and ring loop depend only on the query and the shared best.
-template <int S>
-__device__ __forceinline__ NNResult nn_ring_split(const GridDesc& g, const int* __restrict__ cs,
-                                                  const float4* __restrict__ P, float qx, float qy,
-                                                  float qz, float r, int seed_j, int sub) {
+// nn_query over S lanes (sub = this lane's index among them), the tree part left
+// to the caller (NNResult::tree).  The S lanes of a query are consecutive and
+// reach every lanes_min together: their returns and their ring loop depend only on
+// the query and the shared best.  RING: the radius spans at most kRingOnlyCells
+// cells, so there is no tree part.
+template <int S, bool RING>
+__device__ __forceinline__ NNResult nn_split(const GridDesc& g, const int* __restrict__ cs,
+                                             const float4* __restrict__ P, float qx, float qy,
+                                             float qz, float r, bool bounded, int seed_j, int sub) {
   NNResult res{INFINITY, 0x7fffffff, -1, false};
   if (g.npts == 0 || !(isfinite(qx) && isfinite(qy) && isfinite(qz))) return res;
   const CellPos c = cell_pos(g, qx, qy, qz);
-  const float rlim = r * 1.00001f;
+  const float rlim = bounded ? r * 1.00001f : INFINITY;
   const int k0 = ring_start(g, c, rlim);
   if (k0 < 0) return res;
-  const int kmax = k0 + max(g.nx, max(g.ny, g.nz));
   float best = INFINITY;
   int bid = 0x7fffffff, bj = -1;
   if (seed_j >= 0) scan_points(P, seed_j, seed_j + 1, qx, qy, qz, best, bid, bj);
   const float h2 = g.h * g.h, lim2 = rlim * rlim;
-  for (int k = k0; k <= kmax; ++k) {
-    ring_rows(g, cs, P, c, k, sub, S, h2, lim2, qx, qy, qz, best, bid, bj);
+  SeedBall ball{};
+  if (seed_j >= 0) ball = seed_ball(g, c, best, lim2);
+  if (ball.near) {
+    ball_rows(g, cs, P, c, ball, sub, S, h2, lim2, qx, qy, qz, best, bid, bj);
     lanes_min<S>(best, bid, bj);
-    if (ring_stop(g, c, k, best, rlim)) break;
+  } else if (!RING && !(bounded && rlim * g.inv_h <= kRingOnlyCells) && k0 > kTreeRings) {
+    res.tree = true;  // far outside the grid
+  } else {
+    const bool ring_only = RING || (bounded && rlim * g.inv_h <= kRingOnlyCells);
+    const int kmax = k0 + max(g.nx, max(g.ny, g.nz));
+    for (int k = k0; k <= kmax; ++k) {
+      ring_rows(g, cs, P, c, k, sub, S, h2, lim2, qx, qy, qz, best, bid, bj);
+      lanes_min<S>(best, bid, bj);
+      if (ring_stop(g, c, k, best, rlim)) break;
+      if (!ring_only && (k - k0 >= kTreeRings || best == INFINITY)) {
+        res.tree = true;
+        break;
+      }
+    }
   }
   res.d2 = best;
   res.id = bid;
@@ -319,7 +340,7 @@ __device__ __forceinline__ NNResult nn_ring_split(const GridDesc& g, const int* 
   return res;
 }
 
-template <bool P2PL, int TILE>
+template <bool P2PL, int TILE, bool RING>
 __global__ void __launch_bounds__(64 * kSplitLanes) k_icp_iter_split(const IcpBuffers b,
                                                                      const IcpConst c) {
   constexpr int S = kSplitLanes, NV = P2PL ? kP2LVals : kP2PVals;
@@ -339,8 +360,8 @@ __global__ void __launch_bounds__(64 * kSplitLanes) k_icp_iter_split(const IcpBu
     const GridDesc gs = b.grids[pd.src];
     const GridDesc gt = b.grids[pd.tgt];
     const int base = (tile - pd.tile_begin) * TILE;
-    // every radius is finite here (IcpConst::ring_only)
     const float r = (float)sqrt(pd.max_corr_d2);
+    const bool bounded = RING || isfinite(r);
     // a query's point, in tree or cell order
     auto point_of = [&](int rank) { return b.morton ? b.tpts[gs.pt_off + rank] : b.pts[gs.pt_off + rank]; };
     for (int pass = 0; pass < TILE / 64; ++pass) {
@@ -349,10 +370,17 @@ __global__ void __launch_bounds__(64 * kSplitLanes) k_icp_iter_split(const IcpBu
       float qx = 0.f, qy = 0.f, qz = 0.f;
       NNResult nn{INFINITY, 0x7fffffff, -1, false};
       if (own) xform(st->T, point_of(base + qi), qx, qy, qz);
-      const bool empty = own && b.near && gt.near_r >= r && !near_cell(gt, b.near, qx, qy, qz);
+      const bool empty =
+          own && bounded && b.near && gt.near_r >= r && !near_cell(gt, b.near, qx, qy, qz);
       if (own && !empty) {
         const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + qi] : -1;
-        nn = nn_ring_split<S>(gt, b.cell_start + gt.cell_off, b.pts, qx, qy, qz, r, seed, sub);
+        nn = nn_split<S, RING>(gt, b.cell_start + gt.cell_off, b.pts, qx, qy, qz, r, bounded, seed,
+                               sub);
+      }
+      if constexpr (!RING) {
+        const float rlim = r * 1.00001f;
+        bvh_nn_wave(gt, b.tree(), nn.tree && sub == 0, qx, qy, qz,
+                    bounded ? rlim * rlim : INFINITY, nn.d2, nn.id, nn.j);
       }
       if (sub == 0) {
         s_d2[qi] = nn.d2;
@@ -596,6 +624,64 @@ __global__ void __launch_bounds__(TILE, 6) k_fitness(const IcpBuffers b, double 
   }
 }
 
+// The final pass (every point of the instances the gate kept) when there are few
+// tiles: S lanes per query as in k_icp_iter_split, and a wavefront's tree walk for
+// 64 / S queries.  One tile per block; the sums are k_fitness<TILE>'s.  A
+// 30k-point pair: 250 us with one lane per query, 206 with four (the longest
+// wavefront's walk).
+template <int TILE>
+__global__ void __launch_bounds__(64 * kSplitLanes) k_fitness_split(const IcpBuffers b,
+                                                                    double max_range) {
+  constexpr int S = kSplitLanes;
+  __shared__ double lds[2 * kSplitLanes];
+  __shared__ float s_d2[TILE];
+  const int nt = b.fit_count ? *b.fit_count : b.ntiles;
+  if ((int)blockIdx.x >= nt) return;
+  const int tile = b.fit_count ? b.fit_list[blockIdx.x].x : (int)blockIdx.x;
+  const int p = b.tile_pair[tile];
+  const PairState* st = b.state + p;
+  if (st->gated) return;  // uniform across the block
+  const PairDesc pd = b.pairs[p];
+  const GridDesc gs = b.grids[pd.src];
+  const GridDesc gt = b.grids[pd.tgt];
+  const bool bounded = max_range < DBL_MAX && max_range >= 0.0;
+  const float rq = bounded ? (float)sqrt(max_range) : INFINITY;
+  const float r = rq * 1.00001f;
+  const int q = (int)threadIdx.x / S, sub = (int)threadIdx.x % S;
+  for (int pass = 0; pass < TILE / 64; ++pass) {
+    const int qi = pass * 64 + q;
+    const int rank = (tile - pd.tile_begin) * TILE + qi;
+    const bool own = rank < gs.npts;
+    float qx = 0.f, qy = 0.f, qz = 0.f;
+    NNResult nn{INFINITY, 0x7fffffff, -1, false};
+    if (own) {
+      xform(st->T, b.morton ? b.tpts[gs.pt_off + rank] : b.pts[gs.pt_off + rank], qx, qy, qz);
+      const bool empty = bounded && b.near && gt.near_r >= rq && !near_cell(gt, b.near, qx, qy, qz);
+      const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + qi] : -1;
+      if (!bounded && b.prev && seed < 0)
+        nn.tree = true;  // as in k_fitness
+      else if (!empty)
+        nn = nn_split<S, false>(gt, b.cell_start + gt.cell_off, b.pts, qx, qy, qz, r, bounded, seed,
+                                sub);
+    }
+    bvh_nn_wave(gt, b.tree(), nn.tree && sub == 0, qx, qy, qz, bounded ? r * r : INFINITY, nn.d2,
+                nn.id, nn.j);
+    if (sub == 0) s_d2[qi] = own && nn.j >= 0 && (double)nn.d2 <= max_range ? nn.d2 : -1.0f;
+  }
+  __syncthreads();
+  double v[2] = {0.0, 0.0};
+  if (threadIdx.x < TILE && s_d2[threadIdx.x] >= 0.0f) {
+    v[0] = s_d2[threadIdx.x];
+    v[1] = 1.0;
+  }
+  block_sum<2>(v, lds);
+  if (threadIdx.x == 0) {
+    double* out = b.partials + (int64_t)tile * kMaxVals;
+    out[0] = v[0];
+    out[1] = v[1];
+  }
+}
+
 // The final pass's list of tiles (fit_list) reordered into out: tiles with a
 // point that had no match in its instance's last iteration first (such a point
 // goes straight to the tree walk, tens of times the cost of a seeded one), the
@@ -723,7 +809,7 @@ __global__ void k_gate(PairState* st, int npairs, int H) {
 // per instance), by ballot ranks.  The last block also leaves the number of active
 // instances and of live tiles in host memory, then a flag the host waits for: a
 // chunk's end costs the host this launch, not three, a copy and a wait for the
-// stream (about 40 us of a chunk of four iterations, now about 15).
+// stream (a pair of 20k-point clouds, 13 chunks: 2288 us before, 2114 with it).
 constexpr int kCompactThreads = 1024;
 
 __device__ __forceinline__ bool takes_part(const PairState& st, int mode) {
@@ -958,8 +1044,12 @@ void launch_icp_search(const IcpBuffers& b, const IcpConst& c, int nblocks, hipS
 
 template <bool P2PL, int TILE>
 void launch_split_t(const IcpBuffers& b, const IcpConst& c, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL((k_icp_iter_split<P2PL, TILE>), dim3(nblocks), dim3(64 * kSplitLanes), 0, s, b,
-                     c);
+  if (c.ring_only)
+    hipLaunchKernelGGL((k_icp_iter_split<P2PL, TILE, true>), dim3(nblocks), dim3(64 * kSplitLanes),
+                       0, s, b, c);
+  else
+    hipLaunchKernelGGL((k_icp_iter_split<P2PL, TILE, false>), dim3(nblocks),
+                       dim3(64 * kSplitLanes), 0, s, b, c);
 }
 
 void launch_icp_search_split(const IcpBuffers& b, const IcpConst& c, int nblocks, hipStream_t s) {
@@ -978,21 +1068,24 @@ void launch_icp_search_split(const IcpBuffers& b, const IcpConst& c, int nblocks
 }
 
 template <bool P2PL, int TILE>
-int split_blocks_per_cu_t() {
+int split_blocks_per_cu_t(bool ring) {
   int nb = 0;
-  const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &nb, k_icp_iter_split<P2PL, TILE>, 64 * kSplitLanes, 0);
+  const hipError_t e =
+      ring ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_icp_iter_split<P2PL, TILE, true>,
+                                                          64 * kSplitLanes, 0)
+           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_icp_iter_split<P2PL, TILE, false>,
+                                                          64 * kSplitLanes, 0);
   return (e != hipSuccess || nb < 1) ? 1 : nb;
 }
 
-int icp_split_blocks_per_cu(int tile, bool p2pl) {
+int icp_split_blocks_per_cu(int tile, bool p2pl, bool ring) {
   switch (tile) {
     case 64:
-      return p2pl ? split_blocks_per_cu_t<true, 64>() : split_blocks_per_cu_t<false, 64>();
+      return p2pl ? split_blocks_per_cu_t<true, 64>(ring) : split_blocks_per_cu_t<false, 64>(ring);
     case 128:
-      return p2pl ? split_blocks_per_cu_t<true, 128>() : split_blocks_per_cu_t<false, 128>();
+      return p2pl ? split_blocks_per_cu_t<true, 128>(ring) : split_blocks_per_cu_t<false, 128>(ring);
     default:
-      return p2pl ? split_blocks_per_cu_t<true, 256>() : split_blocks_per_cu_t<false, 256>();
+      return p2pl ? split_blocks_per_cu_t<true, 256>(ring) : split_blocks_per_cu_t<false, 256>(ring);
   }
 }
 
@@ -1005,11 +1098,21 @@ void launch_icp_solve(const IcpBuffers& b, const IcpConst& c, hipStream_t s) {
 }
 
 void launch_fitness(const IcpBuffers& b, double max_range, int nblocks, hipStream_t s,
-                    bool per_instance, int interleave) {
+                    bool per_instance, int interleave, bool split) {
   // (the fold launch below also clears the tile counters, so both run or neither)
   if (b.npairs <= 0) return;
   const int pi = per_instance ? 1 : 0;
-  switch (b.tile) {
+  const dim3 split_grid((unsigned)std::max(b.ntiles, 1)), split_block(64 * kSplitLanes);
+  switch (split && !per_instance ? -b.tile : b.tile) {
+    case -64:
+      hipLaunchKernelGGL(k_fitness_split<64>, split_grid, split_block, 0, s, b, max_range);
+      break;
+    case -128:
+      hipLaunchKernelGGL(k_fitness_split<128>, split_grid, split_block, 0, s, b, max_range);
+      break;
+    case -256:
+      hipLaunchKernelGGL(k_fitness_split<256>, split_grid, split_block, 0, s, b, max_range);
+      break;
     case 64:
       if (!per_instance && b.fetch && b.fit_order && b.fit_flags && b.fit_count && b.prev &&
           b.ntiles > 0) {

@@ -117,15 +117,16 @@ struct IcpBuffers {
 // One ICP iteration for every active instance: the correspondence search with
 // per-tile moment partials, then the per-instance fold, solve and update.
 void launch_icp_search(const IcpBuffers& b, const IcpConst& c, int nblocks, hipStream_t s);
-// The same search with four lanes per query, for ring-only instances
-// (c.ring_only): the launches with few live tiles.
+// The same search with four lanes per query (FP32 scan): the launches with few
+// live tiles.
 void launch_icp_search_split(const IcpBuffers& b, const IcpConst& c, int nblocks, hipStream_t s);
-int icp_split_blocks_per_cu(int tile, bool p2pl);
+int icp_split_blocks_per_cu(int tile, bool p2pl, bool ring_only);
 void launch_icp_solve(const IcpBuffers& b, const IcpConst& c, hipStream_t s);
 // getFitnessScore(max_range) of every instance that is not gated; with
-// per_instance, each instance's own max_corr_d2 replaces max_range.
+// per_instance, each instance's own max_corr_d2 replaces max_range.  split: four
+// lanes per query (not per_instance), for few tiles.
 void launch_fitness(const IcpBuffers& b, double max_range, int nblocks, hipStream_t s,
-                    bool per_instance = false, int interleave = 0);
+                    bool per_instance = false, int interleave = 0, bool split = false);
 // Hypothesis gate over n pairs of H consecutive instances, after a fitness pass
 // with each instance's radius: the best keeps running, the others are set aside.
 void launch_gate(PairState* st, int npairs, int H, hipStream_t s);

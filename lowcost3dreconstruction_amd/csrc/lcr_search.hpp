@@ -309,7 +309,64 @@ LCR_SHD void ring_rows(const GridDesc& g, const int* __restrict__ cs, const floa
 // of the rings.
 constexpr float kSeedBallCells = 3.0f;
 
-// Whether a bounded search (limit rlim) may stop after ring k with `best`: the
+// Rings after which a search without certification goes to the tree.
+constexpr int kTreeRings = 2;
+
+// The cells that the ball around q through `best` (at most the limit) touches.
+// A seed within kSeedBallCells cells, or a limit that close (near): every point at
+// least as close (within the limit) lies in one of them, so the rows of the ball's
+// cell box are scanned instead of the rings.  The rows outside the box's z and y
+// range are those a ring walk prunes (their gap exceeds the ball's radius, slack
+// included), and so are the cells outside its x range; inside a row scan_ring_row
+// prunes and trims by the current best as the rings do.  The result is the same
+// point, in fewer row iterations per wavefront (at most 2 x 2 rows for a radius
+// under one cell, against ring 0 and the nine rows of ring 1; about 16 for a query
+// with no target point within a limit of 1.6 cells, against rings 0-2; the
+// unbounded fitness pass's seeds up to three cells away as well).
+struct SeedBall {
+  bool near;
+  int z0, z1, y0, y1, x0, x1;
+};
+
+LCR_SHD SeedBall seed_ball(const GridDesc& g, const CellPos& c, float best, float lim2) {
+  SeedBall b{};
+  const float thr = fminf(best, lim2) * 1.00002f;
+  const float rho = sqrtf(thr) * g.inv_h * 1.00001f + c.slack;
+  b.near = rho < kSeedBallCells;
+  if (!b.near) return b;
+  b.z0 = max((int)floorf(c.fz - rho), 0);
+  b.z1 = min((int)floorf(c.fz + rho), g.nz - 1);
+  b.y0 = max((int)floorf(c.fy - rho), 0);
+  b.y1 = min((int)floorf(c.fy + rho), g.ny - 1);
+  b.x0 = max((int)floorf(c.fx - rho), 0);
+  b.x1 = min((int)floorf(c.fx + rho), g.nx - 1);
+  return b;
+}
+
+// The ball's rows dealt to `nsub` lanes: rows sub, sub + nsub, ... in row-major
+// order (see ring_rows).
+LCR_SHD void ball_rows(const GridDesc& g, const int* __restrict__ cs, const float4* __restrict__ P,
+                       const CellPos& c, const SeedBall& b, int sub, int nsub, float h2, float lim2,
+                       float qx, float qy, float qz, float& best, int& bid, int& bj) {
+  const int ny = b.y1 - b.y0 + 1;
+  if (ny <= 0 || b.x0 > b.x1) return;
+  int z = b.z0, y = b.y0 + sub;
+  while (y > b.y1) {
+    y -= ny;
+    ++z;
+  }
+  while (z <= b.z1) {
+    const float gz = axis_gap(c.fz, z, c.cz, c.slack);
+    scan_ring_row(g, cs, P, c, 1, z, y, gz, true, b.x0, b.x1, h2, lim2, qx, qy, qz, best, bid, bj);
+    y += nsub;
+    while (y > b.y1) {
+      y -= ny;
+      ++z;
+    }
+  }
+}
+
+// Whether a search (limit rlim, may be +inf) may stop after ring k with `best`: the
 // grid is exhausted, no unvisited cell can hold a point closer than best, or
 // none is within rlim.
 LCR_SHD bool ring_stop(const GridDesc& g, const CellPos& c, int k, float best, float rlim) {
@@ -320,8 +377,8 @@ LCR_SHD bool ring_stop(const GridDesc& g, const CellPos& c, int k, float best, f
   return L > rlim;
 }
 
-// Where a bounded ring-only search starts: k0 = the first ring that can hold a
-// point, -1 if no cell within rlim of q can (the result is then "none").
+// Where a search starts: k0 = the first ring that can hold a point, -1 if no cell
+// within rlim (may be +inf) of q can (the result is then "none").
 LCR_SHD int ring_start(const GridDesc& g, const CellPos& c, float rlim) {
   const int k0 = first_ring(g, c);
   if (k0 > 0 && (block_gap(g, c, k0 - 1) - c.slack) * g.h > rlim) return -1;
@@ -347,7 +404,7 @@ LCR_SHD int ring_start(const GridDesc& g, const CellPos& c, float rlim) {
 // are pruned, and the rings pass r within a few steps.
 LCR_SHD NNResult nn_query(const GridDesc& g, const int* __restrict__ cs,
                           const float4* __restrict__ P, const Tree& tr, float qx, float qy,
-                          float qz, float r, bool bounded, int seed_j = -1, int ring_limit = 2,
+                          float qz, float r, bool bounded, int seed_j = -1, int ring_limit = kTreeRings,
                           bool defer_tree = false) {
   const float4* nodes = tr.nodes;
   NNResult res{INFINITY, 0x7fffffff, -1, false};
@@ -368,30 +425,15 @@ LCR_SHD NNResult nn_query(const GridDesc& g, const int* __restrict__ cs,
   // and the rings reach it within a few steps, so the tree is never needed
   const bool ring_only = bounded && rlim * g.inv_h <= kRingOnlyCells;
   const float lim2 = bounded ? rlim * rlim : INFINITY;
-  // A seed within kSeedBallCells cells, or a limit that close: every point at
-  // least as close (within the limit) lies in a cell that the ball of that radius
-  // around q touches, so the rows of the ball's cell box are scanned instead of
-  // the rings.  The rows outside the box's z and y range are those a ring walk
-  // prunes (their gap exceeds the ball's radius, slack included), and so are the
-  // cells outside its x range; inside a row scan_ring_row prunes and trims by the
-  // current best as the rings do.  The result is the same point, in fewer row
-  // iterations per wavefront (at most 2 x 2 rows for a radius under one cell,
-  // against ring 0 and the nine rows of ring 1; about 16 for a query with no
-  // target point within a limit of 1.6 cells, against rings 0-2; the unbounded
-  // fitness pass's seeds up to three cells away as well).
   if (seed_j >= 0) {
-    const float thr = fminf(best, lim2) * 1.00002f;
-    const float rho = sqrtf(thr) * g.inv_h * 1.00001f + c.slack;
-    if (rho < kSeedBallCells) {
-      const int za = max((int)floorf(c.fz - rho), 0), zb = min((int)floorf(c.fz + rho), g.nz - 1);
-      const int ya = max((int)floorf(c.fy - rho), 0), yb = min((int)floorf(c.fy + rho), g.ny - 1);
-      const int x0 = max((int)floorf(c.fx - rho), 0), x1 = min((int)floorf(c.fx + rho), g.nx - 1);
-      if (x0 <= x1) {
-        for (int z = za; z <= zb; ++z) {
+    const SeedBall b = seed_ball(g, c, best, lim2);
+    if (b.near) {
+      if (b.x0 <= b.x1) {
+        for (int z = b.z0; z <= b.z1; ++z) {
           const float gz = axis_gap(c.fz, z, c.cz, c.slack);
-          for (int y = ya; y <= yb; ++y)
-            scan_ring_row(g, cs, P, c, 1, z, y, gz, true, x0, x1, h2, lim2, qx, qy, qz, best, bid,
-                          bj);
+          for (int y = b.y0; y <= b.y1; ++y)
+            scan_ring_row(g, cs, P, c, 1, z, y, gz, true, b.x0, b.x1, h2, lim2, qx, qy, qz, best,
+                          bid, bj);
         }
       }
       res.d2 = best;

@@ -534,11 +534,13 @@ void Engine::reset_graph() {
 }
 
 // Live 64-point tiles at or below which a chunk runs the four-lanes-per-query
-// search; LCR_SPLIT_TILES (read at every setup) overrides it, 0 turns the split off.
+// search: more fill the chip with one lane per query (a fresh 24-capture cycle's
+// kernels: 7810 us at 2048, 7420 at 4096, 7520 at 8192, 7820 with the split in
+// every launch); LCR_SPLIT_TILES (read at every setup) overrides it, 0 turns the split off.
 static int icp_split_units() {
   const char* e = getenv("LCR_SPLIT_TILES");
   if (e && *e) return std::max(0, atoi(e));
-  return 2048;
+  return 4096;
 }
 
 // The resident blocks of the search, fitness and split kernels per CU: properties
@@ -551,7 +553,7 @@ static int blocks_per_cu(int which, int tile, bool p2pl, int precision) {
   std::lock_guard<std::mutex> lock(mu);
   auto it = known.find(key);
   if (it != known.end()) return it->second;
-  const int v = which == 3   ? icp_split_blocks_per_cu(tile, p2pl)
+  const int v = which >= 3   ? icp_split_blocks_per_cu(tile, p2pl, which == 4)
                 : which == 2 ? fitness_max_blocks_per_cu(tile)
                              : icp_max_blocks_per_cu(tile, p2pl, precision, which != 0);
   known[key] = v;
@@ -642,9 +644,12 @@ void Engine::setup(hipStream_t s, const CloudSet& cs, const std::vector<int>& sr
   nblocks_fit = std::max(8, (nf + 7) / 8 * 8);
   split_units = icp_split_units();
   if (split_units > 0) {
-    int ns = std::min(std::max(std::min(ntiles, split_units / (tile / 64)), 1),
-                      cus * blocks_per_cu(3, tile, pl, 0));
-    nblocks_split = std::max(8, (ns + 7) / 8 * 8);
+    for (int ring = 0; ring < 2; ++ring) {
+      int ns = std::min(std::max(std::min(ntiles, split_units / (tile / 64)), 1),
+                        cus * blocks_per_cu(3 + ring, tile, pl, 0));
+      ns = std::max(8, (ns + 7) / 8 * 8);
+      (ring ? nblocks_split_ring : nblocks_split) = ns;
+    }
   }
 }
 
@@ -726,6 +731,7 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
   Profiler& prof = Profiler::get();
   c.ring_only = ring_only(cs) ? 1 : 0;
   const int nb_search = c.ring_only ? nblocks_ring : nblocks;
+  const int nb_split = c.ring_only ? nblocks_split_ring : nblocks_split;
   const IcpBuffers b = buffers(cs);
   if (guesses) {
     memcpy(h_guess.p, guesses, (size_t)npairs * 16 * sizeof(double));
@@ -775,7 +781,7 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
       const int k = prof.begin("icp_iteration", s, sp);
       const int ks = split ? prof.begin("icp_iteration_split", s, sp) : -1;
       if (split)
-        launch_icp_search_split(b, c, nblocks_split, s);
+        launch_icp_search_split(b, c, nb_split, s);
       else
         launch_icp_search(b, c, nb_search, s);
       prof.end(ks, s, sp);
@@ -791,7 +797,7 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
     const int k = prof.begin("fitness", s, sp);
     // one launch over every instance (with fixed shares, XCD-contiguous tiles keep
     // each target's tree in one L2)
-    launch_fitness(b, DBL_MAX, nblocks_fit, s, false, 0);
+    launch_fitness(b, DBL_MAX, nblocks_fit, s, false, 0, fit_split());
     prof.end(k, s, sp);
     LCR_HIP(hipMemcpyAsync(h_state.p, d_state.p, (size_t)npairs * sizeof(PairState),
                            hipMemcpyDeviceToHost, s));
@@ -857,7 +863,7 @@ Engine::GraphKey Engine::graph_key(const IcpBuffers& b) const {
   k.c = c;
   k.nblocks = c.ring_only ? nblocks_ring : nblocks;
   k.nblocks_fit = nblocks_fit;
-  k.nblocks_split = use_split() ? nblocks_split : 0;
+  k.nblocks_split = use_split() ? (c.ring_only ? nblocks_split_ring : nblocks_split) : 0;
   k.guess = d_guess.p;
   k.hstate = h_state.p;
   k.hactive = h_active.p;
@@ -871,7 +877,7 @@ void Engine::run_fitness(hipStream_t s, const CloudSet& cs, double max_range) {
   const IcpBuffers b = buffers(cs);
   if (ntiles > 0) {
     const int sp = prof.begin("fitness", s, &spans);
-    launch_fitness(b, max_range, nblocks_fit, s, false, c.interleave);
+    launch_fitness(b, max_range, nblocks_fit, s, false, c.interleave, fit_split());
     prof.end(sp, s, &spans);
   }
   LCR_HIP(hipMemcpyAsync(h_state.p, d_state.p, (size_t)npairs * sizeof(PairState),

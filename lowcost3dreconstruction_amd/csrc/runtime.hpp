@@ -256,11 +256,13 @@ struct CloudSet {
 struct Engine {
   int npairs = 0, ntiles = 0, tile = 256, nblocks = 8;
   int nblocks_ring = 8;  // persistent blocks of the ring-only search variant
-  // The four-lanes-per-query search (launch_icp_search_split) runs the chunks of
-  // ring-only instances that start with at most split_units live tiles, counted
-  // in 64-point units, on nblocks_split blocks.
-  int split_units = 0, nblocks_split = 8;
-  bool use_split() const { return c.ring_only && split_units > 0; }
+  // The four-lanes-per-query search (launch_icp_search_split, FP32 scan) runs the
+  // chunks that start with at most split_units live tiles, counted in 64-point
+  // units, on nblocks_split (ring-only instances: nblocks_split_ring) blocks; the
+  // final fitness pass splits when all of the tiles are that few.
+  int split_units = 0, nblocks_split = 8, nblocks_split_ring = 8;
+  bool use_split() const { return c.precision == 0 && split_units > 0; }
+  bool fit_split() const { return (int64_t)ntiles * (tile / 64) <= split_units; }
   bool split_fits(int64_t live_tiles) const {
     return use_split() && live_tiles * (tile / 64) <= split_units;
   }

@@ -296,6 +296,36 @@ def test_split_search_matches_one_lane(lcr, monkeypatch, p2pl, tile):
         np.testing.assert_array_equal(r["fitness"], res[0]["fitness"])
 
 
+@pytest.mark.parametrize("p2pl,tile", [(False, 64), (True, 64), (False, 128), (True, 256)])
+@pytest.mark.parametrize("r,shift", [(0.05, 0.0), (0.3, 0.4), (1.3407807929942596e154, 2.0)])
+def test_split_search_with_tree_walks_matches_one_lane(lcr, monkeypatch, p2pl, tile, r, shift):
+    """Radii of many cells (queries near the target, beside it, and far outside its
+    grid without a limit, the radius that the parameters default to): rings, seeds' balls and tree walks over four lanes per
+    query, in the iterations and in the final fitness pass, give the one-lane
+    search's bits.  The clouds' last tiles and wavefronts are partial."""
+    cyc = synth.turntable_cycle(7, n_captures=2, yaw_step_deg=10.0, scale=1.0,
+                                centre=(0.0, 0.0, -0.8))
+    clouds = [cyc.clouds[0][:4097 + 64], cyc.clouds[1][:5003]]
+    guess = np.eye(4)
+    guess[0, 3] = shift
+    res = []
+    for split in ("0", None, "100000000"):
+        print_case(test="split_tree", p2pl=p2pl, tile=tile, r=r, split=split)
+        if split is None:
+            monkeypatch.delenv("LCR_SPLIT_TILES", raising=False)
+        else:
+            monkeypatch.setenv("LCR_SPLIT_TILES", split)
+        c = lcr.Cycle(clouds, [(0, 1)], guesses=guess[None], point_to_plane=p2pl,
+                      max_corr_dist=r, max_iterations=12, tile=tile)
+        c.run()
+        res.append(c.results())
+        del c
+    for x in res[1:]:
+        np.testing.assert_array_equal(x["T"], res[0]["T"])
+        np.testing.assert_array_equal(x["iterations"], res[0]["iterations"])
+        np.testing.assert_array_equal(x["fitness"], res[0]["fitness"])
+
+
 @pytest.mark.parametrize("p2pl", [False, True])
 def test_fitness_tile_order_does_not_change_results(lcr, monkeypatch, p2pl):
     """The fitness passes' tiles handed out by counters, the tree-walk tiles first,
