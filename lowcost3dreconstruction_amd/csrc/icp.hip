@@ -179,8 +179,8 @@ __device__ __forceinline__ void tile_moments(bool has, float qx, float qy, float
 // dependent loads, and more resident waves hide more of it.
 //
 // RING: every instance's radius spans at most kRingOnlyCells target cells
-// (IcpConst::ring_only), so the bounded search ends inside the ring loop and the
-// tree walk is never needed; this variant carries none of its code or registers.
+// (IcpConst::ring_only): the balls of nn_ball, without the rings' and the tree
+// walk's code and registers.
 template <bool P2PL, int TILE, int PREC, bool RING = false>
 __global__ void __launch_bounds__(TILE, 7) k_icp_iter(const IcpBuffers b, const IcpConst c) {
   constexpr int NV = P2PL ? kP2LVals : kP2PVals;
@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(TILE, 7) k_icp_iter(const IcpBuffers b, const 
                        !near_cell(gt, b.near, qx, qy, qz);
     bool search = own && !empty;  // lanes that still need the scalar search
     // an instance's first iteration has no matches yet
-    int seed = (search && b.prev && st->iterations > 0) ? b.prev[slot] : -1;
+    int seed = (search && b.prev && st->iterations > 0) ? b.prev[slot] : kNoSeed;
     if constexpr (PREC != 0) {
       __shared__ TileLds tl;
       const bool q_ok = search && isfinite(qx) && isfinite(qy) && isfinite(qz);
@@ -233,9 +233,7 @@ __global__ void __launch_bounds__(TILE, 7) k_icp_iter(const IcpBuffers b, const 
       }
     }
     if constexpr (RING) {
-      if (search)
-        nn = nn_query(gt, b.cell_start + gt.cell_off, b.pts, Tree{nullptr, nullptr, nullptr}, qx,
-                      qy, qz, r, bounded, seed, 2, true);
+      if (search) nn = nn_ball<4, 1>(gt, b.cell_start + gt.cell_off, b.pts, qx, qy, qz, r, seed, 0);
     } else {
       if (search)
         nn = nn_query(gt, b.cell_start + gt.cell_off, b.pts, b.tree(), qx, qy, qz, r, bounded,
@@ -281,29 +279,18 @@ __global__ void __launch_bounds__(TILE, 7) k_icp_iter(const IcpBuffers b, const 
 // lane per query, 15.6 with four.
 constexpr int kSplitLanes = 4;
 
-template <int S>
-__device__ __forceinline__ void lanes_min(float& best, int& bid, int& bj) {
-#pragma unroll
-  for (int m = 1; m < S; m <<= 1) {
-    const float ob = __shfl_xor(best, m, 64);
-    const int oid = __shfl_xor(bid, m, 64);
-    const int oj = __shfl_xor(bj, m, 64);
-    const bool take = ob < best || (ob == best && oid < bid);
-    best = take ? ob : best;
-    bid = take ? oid : bid;
-    bj = take ? oj : bj;
-  }
-}
-
 // nn_query over S lanes (sub = this lane's index among them), the tree part left
 // to the caller (NNResult::tree).  The S lanes of a query are consecutive and
 // reach every lanes_min together: their returns and their ring loop depend only on
 // the query and the shared best.  RING: the radius spans at most kRingOnlyCells
-// cells, so there is no tree part.
+// cells.
 template <int S, bool RING>
 __device__ __forceinline__ NNResult nn_split(const GridDesc& g, const int* __restrict__ cs,
                                              const float4* __restrict__ P, float qx, float qy,
                                              float qz, float r, bool bounded, int seed_j, int sub) {
+  if constexpr (RING) {
+    return nn_ball<2, S>(g, cs, P, qx, qy, qz, r, seed_j, sub);
+  }
   NNResult res{INFINITY, 0x7fffffff, -1, false};
   if (g.npts == 0 || !(isfinite(qx) && isfinite(qy) && isfinite(qz))) return res;
   const CellPos c = cell_pos(g, qx, qy, qz);
@@ -314,15 +301,15 @@ __device__ __forceinline__ NNResult nn_split(const GridDesc& g, const int* __res
   int bid = 0x7fffffff, bj = -1;
   if (seed_j >= 0) scan_points(P, seed_j, seed_j + 1, qx, qy, qz, best, bid, bj);
   const float h2 = g.h * g.h, lim2 = rlim * rlim;
+  const bool ring_only = bounded && rlim * g.inv_h <= kRingOnlyCells;
   SeedBall ball{};
-  if (seed_j >= 0) ball = seed_ball(g, c, best, lim2);
+  if (seed_j != kNoSeed) ball = seed_ball(g, c, best, lim2);
   if (ball.near) {
-    ball_rows(g, cs, P, c, ball, sub, S, h2, lim2, qx, qy, qz, best, bid, bj);
+    ball_scan<2, S>(g, cs, P, c, ball, sub, h2, lim2, qx, qy, qz, best, bid, bj);
     lanes_min<S>(best, bid, bj);
-  } else if (!RING && !(bounded && rlim * g.inv_h <= kRingOnlyCells) && k0 > kTreeRings) {
+  } else if (!ring_only && k0 > kTreeRings) {
     res.tree = true;  // far outside the grid
   } else {
-    const bool ring_only = RING || (bounded && rlim * g.inv_h <= kRingOnlyCells);
     const int kmax = k0 + max(g.nx, max(g.ny, g.nz));
     for (int k = k0; k <= kmax; ++k) {
       ring_rows(g, cs, P, c, k, sub, S, h2, lim2, qx, qy, qz, best, bid, bj);
@@ -373,7 +360,7 @@ __global__ void __launch_bounds__(64 * kSplitLanes) k_icp_iter_split(const IcpBu
       const bool empty =
           own && bounded && b.near && gt.near_r >= r && !near_cell(gt, b.near, qx, qy, qz);
       if (own && !empty) {
-        const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + qi] : -1;
+        const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + qi] : kNoSeed;
         nn = nn_split<S, RING>(gt, b.cell_start + gt.cell_off, b.pts, qx, qy, qz, r, bounded, seed,
                                sub);
       }

@@ -296,6 +296,32 @@ def test_split_search_matches_one_lane(lcr, monkeypatch, p2pl, tile):
         np.testing.assert_array_equal(r["fitness"], res[0]["fitness"])
 
 
+@pytest.mark.parametrize("cell_factor", [1.5, 4.0])
+@pytest.mark.parametrize("r", [0.0005, 0.003, 0.01, 0.02, 0.05])
+def test_ball_search_matches_general_search(lcr, monkeypatch, r, cell_factor):
+    """Radii from a fraction of a cell to beyond the ball search's three: an FP32
+    alignment over the balls of seeds, of one cell and of the limit (with one lane and
+    with four lanes per query) gives the bits of the staged tiles, whose uncertified
+    queries take the general search.  Some queries lie outside the target's grid."""
+    base = synth.pair_ellipsoids(11, n_src=3001, n_tgt=2500, angle_deg=4.0, trans=0.01)
+    src = np.concatenate([base.src, base.src[:70] + np.float32(0.7)])
+    ref = None
+    for mode, split in ((3, None), (0, None), (0, "0")):
+        print_case(test="ball_search", r=r, cell_factor=cell_factor, mode=mode, split=split)
+        if split is None:
+            monkeypatch.delenv("LCR_SPLIT_TILES", raising=False)
+        else:
+            monkeypatch.setenv("LCR_SPLIT_TILES", split)
+        icp = make_icp(lcr, src, base.tgt, r=r, iters=8, tile=64, precision_mode=mode,
+                       cell_factor=cell_factor)
+        icp.align()
+        got = (icp.getFinalTransformation(), icp.nr_iterations(), icp.getFitnessScore())
+        if ref is None:
+            ref = got
+        np.testing.assert_array_equal(got[0], ref[0])
+        assert got[1:] == ref[1:]
+
+
 @pytest.mark.parametrize("p2pl,tile", [(False, 64), (True, 64), (False, 128), (True, 256)])
 @pytest.mark.parametrize("r,shift", [(0.05, 0.0), (0.3, 0.4), (1.3407807929942596e154, 2.0)])
 def test_split_search_with_tree_walks_matches_one_lane(lcr, monkeypatch, p2pl, tile, r, shift):
