@@ -212,9 +212,9 @@ __device__ void select_rescan(const GridDesc& g, const int* cs, const float4* pt
 // per-lane histogram of d2 over [0, D2) in NB equal buckets -- on a surface the
 // number of points within a radius grows with its square, so the buckets fill
 // about evenly -- and finds the bucket B that holds the kk-th.  Pass 2 lists
-// every point of a lower bucket and keeps (d2, original index, position) of
-// bucket B's points in LDS; a sorting network orders those by (d2, original
-// index) and the first kk - (count below B) complete the list.  Bucket index =
+// the positions of the points of lower buckets and of bucket B's in LDS; a sorting
+// network orders bucket B's by (d2, original index) and the first kk - (count
+// below B) complete the list.  Bucket index =
 // floor(d2 * scale) is monotone in d2, so the result is exactly the kk smallest
 // (d2, original index).  A query is flagged for the next path when its block
 // covers the grid, holds fewer than kk points under D2 (not certified), more
@@ -293,10 +293,10 @@ __device__ __forceinline__ float4 load_point(__amdgpu_buffer_rsrc_t r, int i) {
 // its next non-empty run as soon as it finishes one.  A loop over one run at a
 // time lasts as long as the wavefront's longest lane in every run; per column,
 // the lanes' long and short runs even out (about 76 against 101 batches per
-// wavefront on the 36-capture cycle's queries).
-template <int K, int NBATCH, class F>
-__device__ __forceinline__ void for_block(const BlockRuns<K>& b, __amdgpu_buffer_rsrc_t rs,
-                                          F&& f) {
+// wavefront on the 36-capture cycle's queries).  after() follows every batch.
+template <int K, int NBATCH, class F, class G>
+__device__ __forceinline__ void for_block(const BlockRuns<K>& b, __amdgpu_buffer_rsrc_t rs, F&& f,
+                                          G&& after) {
   constexpr int S = 2 * K + 1;
 #pragma unroll
   for (int dy = 0; dy < S; ++dy) {
@@ -324,6 +324,7 @@ __device__ __forceinline__ void for_block(const BlockRuns<K>& b, __amdgpu_buffer
       for (int u = 0; u < NBATCH; ++u) p[u] = load_point(rs, i + u);
 #pragma unroll
       for (int u = 0; u < NBATCH; ++u) f(p[u], i + u, i + u < e);
+      after();
       i += NBATCH;
       if (i >= e) {
         i = qs[1];
@@ -383,7 +384,7 @@ __device__ __forceinline__ int xcd_block(int b, int n) {
 
 template <int NB, int NL>
 constexpr int lane_words() {
-  return 3 * NL > NB ? 3 * NL : NB;
+  return 2 * NL > NB ? 2 * NL : NB;
 }
 
 // nsel bit: the query's list holds original indices into the cloud's raw points
@@ -436,7 +437,7 @@ __device__ __forceinline__ int lane_query(const GridDesc* __restrict__ grids,
     const float d = flann_d2(q.x, q.y, q.z, p);
     const int b = (int)fminf(d * scale, (float)(NB - 1));
     atomicAdd(&buf[b][lane], (valid && d < D2) ? 1u : 0u);
-  });
+  }, [] {});
   int B = -1, below = 0, nB = 0, cum = 0;
   // four counts at a time: unrolled whole, the 32 reads would all be in flight
 #pragma unroll 4
@@ -460,31 +461,56 @@ __device__ __forceinline__ int lane_query(const GridDesc* __restrict__ grids,
       B < NB - 1 ? block_runs<K>(g, cs, cp, fminf(D2, D2 * ((float)(B + 1) / (float)NB) * 1.0001f))
                  : blk;
   // the moments of the lower buckets' points in block order, then of bucket B's
-  // picks in (d2, original index) order
+  // picks in (d2, original index) order.  The block's scan only writes positions to
+  // the lane's column: lower buckets' to rows 0 .. kList - 1, bucket B's to the last
+  // NL (at most nB of them).  The moments are then added over the list, where nearly
+  // every lane has a point in every step; added in the scan, each of its steps ran
+  // the FP64 sums for the few lanes whose point was in (62 % of the pass).  A slot
+  // that is not taken leaves its position at the row the next one overwrites.
+  // bucket < B: d2 * scale < B; bucket B: below B + 1, or the last one.
+  constexpr int kList = lane_words<NB, NL>() - NL;
+  static_assert(kList >= 8, "a list of two batches at least");
+  const float fB = (float)B, fB1 = B < NB - 1 ? (float)(B + 1) : INFINITY;
   Moments acc;
 #pragma unroll
   for (int c = 0; c < 9; ++c) acc.v[c] = 0.0;
-  int nl = 0;
-  for_block<K, 4>(sel, rs, [&](const float4& p, int i, bool valid) {
-    const float d = flann_d2(q.x, q.y, q.z, p);
-    if (valid && d < D2) {
-      const int b = min((int)(d * scale), NB - 1);
-      if (b < B) {
-        take<MODE>(acc, q, p, d);
-      } else if (b == B && nl < NL) {
-        buf[3 * nl][lane] = __float_as_uint(d);
-        buf[3 * nl + 1][lane] = (uint32_t)__float_as_int(p.w);
-        buf[3 * nl + 2][lane] = (uint32_t)i;
-        ++nl;
-      }
+  int na = 0, nl = 0;
+  auto flush = [&] {
+    for (int t = 0; t < na; t += 4) {
+      float4 p[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) p[u] = load_point(rs, t + u < na ? (int)buf[t + u][lane] : 0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (t + u < na) take<MODE>(acc, q, p[u], flann_d2(q.x, q.y, q.z, p[u]));
     }
-  });
+    na = 0;
+  };
+  for_block<K, 4>(
+      sel, rs,
+      [&](const float4& p, int i, bool valid) {
+        const float d = flann_d2(q.x, q.y, q.z, p);
+        const float x = d * scale;
+        const bool lower = x < fB;
+        const bool in = valid & (d < D2) & (x < fB1);
+        const int row = in & !lower ? kList + nl : na;
+        buf[row][lane] = (uint32_t)i;
+        na += in & lower ? 1 : 0;
+        nl += in & !lower ? 1 : 0;
+      },
+      [&] {
+        if (__any(na > kList - 4)) flush();
+      });
+  flush();
   uint64_t e[NL];
   int ei[NL];
 #pragma unroll
   for (int t = 0; t < NL; ++t) {
-    e[t] = t < nl ? ((uint64_t)buf[3 * t][lane] << 32) | buf[3 * t + 1][lane] : ~0ull;
-    ei[t] = t < nl ? (int)buf[3 * t + 2][lane] : 0;
+    ei[t] = t < nl ? (int)buf[kList + t][lane] : 0;
+    const float4 p = load_point(rs, ei[t]);
+    const uint64_t key =
+        ((uint64_t)__float_as_uint(flann_d2(q.x, q.y, q.z, p)) << 32) | (uint32_t)__float_as_int(p.w);
+    e[t] = t < nl ? key : ~0ull;
   }
   sort_keys<NL>(e, ei);
   const int need = kk - below;
