@@ -13,8 +13,9 @@
 //     transformation_estimation_svd.hpp; called via fine_registration.cpp:121).
 //   * chol6_solve     -- point-to-plane: the 6x6 normal equations of
 //     TransformationEstimationPointToPlaneLLS, by Cholesky.
-//   * eigh3           -- normals: symmetric 3x3 eigen-decomposition by cyclic
-//     Jacobi (NormalEstimation's solvePlaneParameters, normal_estimation.cpp:108).
+//   * smallest_eigvec3, eigh3 -- normals: the smallest eigenvalue's eigenvector of
+//     the covariance from its characteristic polynomial where that eigenvalue is
+//     well separated, cyclic Jacobi otherwise (NormalEstimation's solvePlaneParameters, normal_estimation.cpp:108).
 //   * conv_step       -- DefaultConvergenceCriteria::hasConverged.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -355,6 +356,64 @@ LCR_HD void mat4_mul(const double* A, const double* B, double* C) {
     }
 #pragma unroll
   for (int i = 0; i < 16; ++i) C[i] = t[i];
+}
+
+// Smallest eigenvalue w and its unit eigenvector v of a symmetric positive
+// semi-definite 3x3 matrix.  With entries scaled to at most 1 and the mean
+// eigenvalue taken off, the smallest root of the characteristic polynomial
+// x^3 - (p2 / 2) x - det by Newton from a bound below it (f is increasing and
+// concave there, so the steps never pass it); the adjugate at that root is
+// v v^T times the product of its distances to the other two, f'(x), and w is v's
+// Rayleigh quotient.  Rounding enters relative to f'(x): below kSeparated3 (points
+// on a line, or one cloud of them) this returns false and the caller takes Jacobi.
+// One division and two square roots plus 4-6 divisions of Newton, against about
+// nine rotations of two divisions and two square roots each.
+constexpr double kSeparated3 = 0.01;
+
+LCR_HD bool smallest_eigvec3(const double C[3][3], double& w, double v[3]) {
+  const double m = fmax(fmax(C[0][0], C[1][1]), C[2][2]);
+  if (!(m > 0.0)) return false;
+  const double inv = 1.0 / m;
+  const double q = (C[0][0] + C[1][1] + C[2][2]) * inv * (1.0 / 3.0);
+  const double d0 = C[0][0] * inv - q, d1 = C[1][1] * inv - q, d2 = C[2][2] * inv - q;
+  const double a01 = C[0][1] * inv, a02 = C[0][2] * inv, a12 = C[1][2] * inv;
+  const double h = 0.5 * (d0 * d0 + d1 * d1 + d2 * d2) + (a01 * a01 + a02 * a02 + a12 * a12);
+  const double det = d0 * (d1 * d2 - a12 * a12) - a01 * (a01 * d2 - a12 * a02) +
+                     a02 * (a01 * a12 - d1 * a02);
+  // the roots lie within 2 sqrt(h / 3) of 0
+  double x = -1.1547005383792517 * sqrt(h) * (1.0 + 1e-12);
+  double dp = 0.0;
+  for (int it = 0; it < 40; ++it) {
+    const double x2 = x * x;
+    dp = 3.0 * x2 - h;
+    if (!(dp > kSeparated3)) return false;
+    const double step = ((x2 - h) * x - det) / dp;
+    x -= step;
+    if (!(fabs(step) > 4e-16)) break;
+  }
+  const double b0 = d0 - x, b1 = d1 - x, b2 = d2 - x;
+  const double c00 = b1 * b2 - a12 * a12, c11 = b0 * b2 - a02 * a02, c22 = b0 * b1 - a01 * a01;
+  const double c01 = a02 * a12 - a01 * b2, c02 = a01 * a12 - a02 * b1, c12 = a01 * a02 - a12 * b0;
+  double v0 = c00, v1 = c01, v2 = c02, best = c00;
+  if (c11 > best) {
+    best = c11;
+    v0 = c01;
+    v1 = c11;
+    v2 = c12;
+  }
+  if (c22 > best) {
+    v0 = c02;
+    v1 = c12;
+    v2 = c22;
+  }
+  const double n = 1.0 / sqrt(v0 * v0 + v1 * v1 + v2 * v2);
+  v[0] = v0 * n;
+  v[1] = v1 * n;
+  v[2] = v2 * n;
+  w = v[0] * (C[0][0] * v[0] + C[0][1] * v[1] + C[0][2] * v[2]) +
+      v[1] * (C[0][1] * v[0] + C[1][1] * v[1] + C[1][2] * v[2]) +
+      v[2] * (C[0][2] * v[0] + C[1][2] * v[1] + C[2][2] * v[2]);
+  return true;
 }
 
 // Symmetric 3x3 eigen-decomposition (cyclic Jacobi, FP64).  a is row-major and

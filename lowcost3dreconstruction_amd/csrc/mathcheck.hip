@@ -43,6 +43,15 @@ void lcrm_eigh3(const double* A, double* w, double* V) {
     for (int j = 0; j < 3; ++j) V[3 * i + j] = v[i][j];
 }
 
+// A: symmetric positive semi-definite 3x3 -> smallest eigenvalue, eigenvector; 0 when
+// it leaves the matrix to eigh3
+int lcrm_smallest_eigvec3(const double* A, double* w, double* v) {
+  double a[3][3];
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) a[i][j] = A[3 * i + j];
+  return smallest_eigvec3(a, *w, v) ? 1 : 0;
+}
+
 // One convergence step.  io[0..3] = iterations, state, similar, converged;
 // dio[0] = prev_mse.  cst: max_iterations, then (rot_thr, trans_thr, rel, abs).
 int lcrm_conv_step(int* io, double* dio, int max_iterations, const double* thr,

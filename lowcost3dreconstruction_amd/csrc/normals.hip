@@ -916,10 +916,11 @@ k_normal_rescan(const GridDesc* __restrict__ grids, const int* __restrict__ cell
 
 // Solve pass, one point per lane: the FP64 moments of its neighbours relative to
 // it (from the lane and wavefront passes, or summed here in list order from the
-// rescan pass's list of original indices, kNselOrig set), covariance, FP64
-// eigen-decomposition, normal (eigenvector of the smallest eigenvalue) oriented
-// towards the viewpoint.
-__global__ void __launch_bounds__(256)
+// rescan pass's list of original indices, kNselOrig set), covariance, normal
+// (eigenvector of the smallest eigenvalue, FP64) oriented towards the viewpoint.
+// Bound by FP64 latency: 36 captures (1 M points) 211 us with Jacobi for every point,
+// 62 with the closed form; four wavefronts a SIMD for it (8 spills) over two.
+__global__ void __launch_bounds__(256, 4)
 k_normal_solve(const float4* __restrict__ pts, const int* __restrict__ cloud_of_sorted,
                const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off,
                const int* __restrict__ nbr, int k, const double* __restrict__ mom,
@@ -958,13 +959,23 @@ k_normal_solve(const float4* __restrict__ pts, const int* __restrict__ cloud_of_
   C[1][0] = C[0][1];
   C[2][0] = C[0][2];
   C[2][1] = C[1][2];
-  double wv[3], V[3][3];
-  eigh3(C, wv, V);
-  double nx = V[0][0], ny = V[1][0], nz = V[2][0];
-  const double sum = wv[0] + wv[1] + wv[2];
-  const double curv = sum != 0.0 ? fabs(wv[0] / sum) : 0.0;
   const float* v = vp + 3 * cloud_of_sorted[jq];
-  const double dot = ((double)v[0] - q.x) * nx + ((double)v[1] - q.y) * ny + ((double)v[2] - q.z) * nz;
+  const double ex = (double)v[0] - q.x, ey = (double)v[1] - q.y, ez = (double)v[2] - q.z;
+  const double sum = C[0][0] + C[1][1] + C[2][2];
+  double w0, e[3];
+  bool ok = smallest_eigvec3(C, w0, e);
+  double dot = ex * e[0] + ey * e[1] + ez * e[2];
+  // (a normal square to the view keeps the sign that Jacobi gives it)
+  if (!ok || !(fabs(dot) > 0.0)) {
+    double wv[3], V[3][3];
+    eigh3(C, wv, V);
+    w0 = wv[0];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) e[i] = V[i][0];
+    dot = ex * e[0] + ey * e[1] + ez * e[2];
+  }
+  double nx = e[0], ny = e[1], nz = e[2];
+  const double curv = sum != 0.0 ? fabs(w0 / sum) : 0.0;
   if (dot < 0.0) {
     nx = -nx;
     ny = -ny;

@@ -24,6 +24,7 @@ def m():
     L.lcrm_p2pl_increment.argtypes = [dp, dp]
     L.lcrm_horn.argtypes = [dp, dp]
     L.lcrm_eigh3.argtypes = [dp, dp, dp]
+    L.lcrm_smallest_eigvec3.argtypes = [dp, dp, dp]
     L.lcrm_conv_step.argtypes = [ip, dp, C.c_int, dp, dp, C.c_double]
     L.lcrm_mat4_mul.argtypes = [dp, dp, dp]
     return L
@@ -124,6 +125,38 @@ def test_eigh3_matches_golden(m):
         V = V.reshape(3, 3)
         np.testing.assert_allclose(w, w_ref, atol=1e-12 * max(1.0, np.abs(w_ref).max()))
         np.testing.assert_allclose(V @ np.diag(w) @ V.T, A, atol=1e-12 * max(1, np.abs(A).max()))
+
+
+@pytest.mark.parametrize("spectrum", [(0.0, 1.0, 1.0), (1e-9, 0.3, 1.0), (0.02, 0.5, 0.9),
+                                      (0.3, 0.33, 1.0), (0.9, 0.95, 1.0), (0.0, 1e-6, 1.0),
+                                      (1e-4, 0.02, 1.0), (1.0, 1.0, 1.0), (0.0, 0.0, 0.0)])
+@pytest.mark.parametrize("scale", [1e-8, 1.0, 1e6])
+def test_smallest_eigenvector_for_every_spectrum(m, spectrum, scale):
+    """A plane's, a volume's, a line's and a point's covariance under random rotations:
+    where the closed form answers, the product of the eigenvalue's distances to the
+    others exceeds 0.01 of the largest entry squared, so rounding (a few tens of 2^-53
+    of the largest entry) moves the vector by less than 100 * 2^-53 / 0.01 and the
+    eigenvalue (a Rayleigh quotient) by less than 20 * 2^-53 of the trace; planes
+    and volumes are answered, lines, points and equal eigenvalues left to Jacobi."""
+    rng = np.random.default_rng(3)
+    w = np.array(spectrum) * scale
+    answered = 0
+    for _ in range(200):
+        Q, _r = np.linalg.qr(rng.normal(size=(3, 3)))
+        A = (Q * w) @ Q.T
+        A = np.ascontiguousarray(0.5 * (A + A.T))
+        got, v = np.empty(1), np.empty(3)
+        if not m.lcrm_smallest_eigvec3(P(A), P(got), P(v)):
+            continue
+        answered += 1
+        assert abs(np.linalg.norm(v) - 1.0) <= 1e-14
+        assert abs(got[0] - w[0]) <= 20 * 2.0 ** -53 * w.sum()
+        assert np.linalg.norm(np.cross(v, Q[:, 0])) <= 100 * 2.0 ** -53 / 0.01
+    separated = (spectrum[1] - spectrum[0]) * (spectrum[2] - spectrum[0])
+    if separated > 0.0101 * max(spectrum) ** 2:
+        assert answered == 200
+    elif separated < 0.003 * max(spectrum) ** 2 or max(spectrum) == 0.0:
+        assert answered == 0
 
 
 def _conv_run(m, seq, max_it=4):
