@@ -104,7 +104,7 @@ __device__ __forceinline__ TileRange xcd_tiles(int ntiles, int interleave) {
 // leaves its totals in LDS and the store adds the rows and the wavefronts in order.
 // The additions are those of one wave_sum_dpp per value, to the bit, in 240
 // instead of 810 instructions of a tile's 3000 (point-to-plane): an iteration of 74
-// pairs over 36 captures 386 -> 347 us, of a 30k-point pair 17 -> 14.
+// pairs over 36 captures 386 -> 347 us, of a 67k-point pair 17 -> 14.
 //
 // tile_moments_emit writes each wavefront's row totals to lds (every lane of the
 // wavefront calls it); tile_moments_store adds them into out.
@@ -663,7 +663,7 @@ __global__ void __launch_bounds__(TILE, 6) k_fitness(const IcpBuffers b, double 
 // The final pass (every point of the instances the gate kept) when there are few
 // tiles: S lanes per query as in k_icp_iter_split, and a wavefront's tree walk for
 // 64 / S queries.  One tile per block; the sums are k_fitness<TILE>'s.  A
-// 30k-point pair: 250 us with one lane per query, 206 with four (the longest
+// 67k-point pair: 250 us with one lane per query, 206 with four (the longest
 // wavefront's walk).
 template <int TILE>
 __global__ void __launch_bounds__(64 * kSplitLanes) k_fitness_split(const IcpBuffers b,

@@ -918,7 +918,7 @@ k_normal_rescan(const GridDesc* __restrict__ grids, const int* __restrict__ cell
 // it (from the lane and wavefront passes, or summed here in list order from the
 // rescan pass's list of original indices, kNselOrig set), covariance, normal
 // (eigenvector of the smallest eigenvalue, FP64) oriented towards the viewpoint.
-// Bound by FP64 latency: 36 captures (1 M points) 211 us with Jacobi for every point,
+// Bound by FP64 latency: 36 captures (37k-113k points each) 211 us with Jacobi for every point,
 // 62 with the closed form; four wavefronts a SIMD for it (8 spills) over two.
 __global__ void __launch_bounds__(256, 4)
 k_normal_solve(const float4* __restrict__ pts, const int* __restrict__ cloud_of_sorted,

@@ -22,8 +22,12 @@ namespace {
 
 // Inputs of the network for every pair of a cycle: n_out points subsampled evenly
 // from each raw cloud, the source moved by the pair's seed T0, both normalised by
-// the target sample's centroid and RMS radius.  One block per pair; the sums are
-// folded by a fixed LDS tree, so the frame does not depend on timing.
+// the target sample's centroid and RMS radius.  k_prop_frame: one block per pair,
+// its first kPrepKeep samples per thread loaded together and kept for both sums,
+// which a fixed LDS tree folds, so the frame does not depend on timing.
+// k_prop_inputs: a thread per sample.  A sample is a cache line of its own, so one
+// block per pair for all of it waited on its CU's loads (36 pairs, 8192 samples:
+// 64 us, now 28 + 9).
 constexpr int kPrepThreads = 1024;
 
 // Sample i of n_out taken evenly from a cloud of n points: floor(i * n / n_out),
@@ -51,40 +55,50 @@ __device__ __forceinline__ void prep_sum(double (&v)[N], double (*red)[N]) {
   __syncthreads();  // red is reused
 }
 
+constexpr int kPrepKeep = 8;
+
 __global__ void __launch_bounds__(kPrepThreads)
-k_prop_prepare(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off,
-               const int* __restrict__ src, const int* __restrict__ tgt,
-               const double* __restrict__ guesses, int guess_stride, int n_out,
-               float4* __restrict__ X, float* __restrict__ frame) {
+k_prop_frame(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off,
+             const int* __restrict__ tgt, int n_out, double* __restrict__ norm,
+             float* __restrict__ frame) {
   __shared__ double red[kPrepThreads][4];
   const int pr = blockIdx.x, t = threadIdx.x;
-  const int64_t s0 = cloud_off[src[pr]], ns = cloud_off[src[pr] + 1] - s0;
   const int64_t t0 = cloud_off[tgt[pr]], nt = cloud_off[tgt[pr] + 1] - t0;
-  float4* Xs = X + (int64_t)pr * 2 * n_out;
-  float4* Xt = Xs + n_out;
+  float4 keep[kPrepKeep];
+#pragma unroll
+  for (int u = 0; u < kPrepKeep; ++u) {
+    const int i = t + u * kPrepThreads;
+    keep[u] = i < n_out ? raw[t0 + sample_at(i, nt, n_out)] : make_float4(NAN, NAN, NAN, NAN);
+  }
   double a[4] = {0, 0, 0, 0};
-  for (int i = t; i < n_out; i += kPrepThreads) {
-    const float4 q = raw[t0 + sample_at(i, nt, n_out)];
+  auto add = [&](const float4& q) {
     if (isfinite(q.x) && isfinite(q.y) && isfinite(q.z)) {
       a[0] += q.x;
       a[1] += q.y;
       a[2] += q.z;
       a[3] += 1.0;
     }
-  }
+  };
+#pragma unroll
+  for (int u = 0; u < kPrepKeep; ++u) add(keep[u]);
+  for (int i = t + kPrepKeep * kPrepThreads; i < n_out; i += kPrepThreads)
+    add(raw[t0 + sample_at(i, nt, n_out)]);
   prep_sum<4>(a, red);
   const double n = a[3] > 0 ? a[3] : 1.0;
   const double cx = a[0] / n, cy = a[1] / n, cz = a[2] / n;
-  double b[4] = {0, 0, 0, 0};
-  for (int i = t; i < n_out; i += kPrepThreads) {
-    const float4 q = raw[t0 + sample_at(i, nt, n_out)];
+  double b[2] = {0, 0};
+  auto spread = [&](const float4& q) {
     if (isfinite(q.x) && isfinite(q.y) && isfinite(q.z)) {
       const double dx = q.x - cx, dy = q.y - cy, dz = q.z - cz;
       b[0] += dx * dx + dy * dy + dz * dz;
       b[1] += 1.0;
     }
-  }
-  prep_sum<4>(b, red);
+  };
+#pragma unroll
+  for (int u = 0; u < kPrepKeep; ++u) spread(keep[u]);
+  for (int i = t + kPrepKeep * kPrepThreads; i < n_out; i += kPrepThreads)
+    spread(raw[t0 + sample_at(i, nt, n_out)]);
+  prep_sum<2>(b, reinterpret_cast<double(*)[2]>(red));
   const double rr = b[1] > 0 ? sqrt(b[0] / b[1]) : 1.0;
   const double rad = rr > 1e-12 ? rr : 1.0;
   if (t == 0) {
@@ -92,25 +106,39 @@ k_prop_prepare(const float4* __restrict__ raw, const int64_t* __restrict__ cloud
     frame[pr * 4 + 1] = (float)cy;
     frame[pr * 4 + 2] = (float)cz;
     frame[pr * 4 + 3] = (float)rad;
+    norm[pr] = 1.0 / rad;
   }
-  const double* T = guesses + (int64_t)pr * guess_stride * 16;
-  const float inv = (float)(1.0 / rad);
-  const float c0 = (float)cx, c1 = (float)cy, c2 = (float)cz;
-  for (int i = t; i < n_out; i += kPrepThreads) {
-    const float4 q = raw[t0 + sample_at(i, nt, n_out)];
-    Xt[i] = (isfinite(q.x) && isfinite(q.y) && isfinite(q.z))
-                ? make_float4((q.x - c0) * inv, (q.y - c1) * inv, (q.z - c2) * inv, 0.f)
-                : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 p = raw[s0 + sample_at(i, ns, n_out)];
-    if (isfinite(p.x) && isfinite(p.y) && isfinite(p.z)) {
-      float m[3];
+}
+
+// `per` blocks for a pair's target sample, then `per` for its source's.
+__global__ void __launch_bounds__(256)
+k_prop_inputs(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off,
+              const int* __restrict__ src, const int* __restrict__ tgt,
+              const double* __restrict__ guesses, int guess_stride, int n_out,
+              const double* __restrict__ norm, const float* __restrict__ frame, int per,
+              float4* __restrict__ X) {
+  const int part = (int)blockIdx.x / per, pr = part >> 1;
+  const int i = ((int)blockIdx.x % per) * 256 + (int)threadIdx.x;
+  if (i >= n_out) return;
+  const bool source = part & 1;
+  const int cloud = source ? src[pr] : tgt[pr];
+  const int64_t o = cloud_off[cloud], n = cloud_off[cloud + 1] - o;
+  const float inv = (float)norm[pr];
+  const float c0 = frame[pr * 4], c1 = frame[pr * 4 + 1], c2 = frame[pr * 4 + 2];
+  float4* out = X + (int64_t)pr * 2 * n_out + (source ? 0 : n_out);
+  const float4 p = raw[o + sample_at(i, n, n_out)];
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (isfinite(p.x) && isfinite(p.y) && isfinite(p.z)) {
+    float m[3] = {p.x, p.y, p.z};
+    if (source) {
+      const double* T = guesses + (int64_t)pr * guess_stride * 16;
+#pragma unroll
       for (int r = 0; r < 3; ++r)
         m[r] = (float)(T[4 * r] * p.x + T[4 * r + 1] * p.y + T[4 * r + 2] * p.z + T[4 * r + 3]);
-      Xs[i] = make_float4((m[0] - c0) * inv, (m[1] - c1) * inv, (m[2] - c2) * inv, 0.f);
-    } else {
-      Xs[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    v = make_float4((m[0] - c0) * inv, (m[1] - c1) * inv, (m[2] - c2) * inv, 0.f);
   }
+  out[i] = v;
 }
 
 // learned guess = [R(omega) | s tau + c - R c] * T0, written to the pair's learned slot
@@ -163,7 +191,7 @@ struct ProposalImpl {
   int cap_pairs = 0, cap_pts = 0;
   int step = 0;
   DevBuf W, M, V, G, W2t, W3t;
-  DevBuf X, part_max, part_arg, F, ARG, Z, OUT, DOUT, loss_part, DZ, DG, part_grad, lab, losses, frame;
+  DevBuf X, part_max, part_arg, F, ARG, Z, OUT, DOUT, loss_part, DZ, DG, part_grad, lab, losses, frame, norm;
   DevBuf ds_X, ds_lab;
   int ds_pairs = 0, ds_pts = 0;
   HostBuf h_io;
@@ -260,9 +288,14 @@ void proposal_guesses(ProposalImpl& P, hipStream_t s, const CloudSet& cs, const 
   P.reserve(npairs, npts);
   P.reserve_points(npairs, npts);
   P.frame.reserve((size_t)npairs * 4 * sizeof(float));
-  hipLaunchKernelGGL(k_prop_prepare, dim3(npairs), dim3(kPrepThreads), 0, s, cs.d_raw.as<float4>(),
-                     cs.d_cloud_off.as<int64_t>(), d_src, d_tgt, d_guess, stride, npts,
-                     P.X.as<float4>(), P.frame.as<float>());
+  P.norm.reserve((size_t)npairs * sizeof(double));
+  hipLaunchKernelGGL(k_prop_frame, dim3(npairs), dim3(kPrepThreads), 0, s, cs.d_raw.as<float4>(),
+                     cs.d_cloud_off.as<int64_t>(), d_tgt, npts, P.norm.as<double>(),
+                     P.frame.as<float>());
+  const int per = (npts + 255) / 256;
+  hipLaunchKernelGGL(k_prop_inputs, dim3((unsigned)npairs * 2 * per), dim3(256), 0, s,
+                     cs.d_raw.as<float4>(), cs.d_cloud_off.as<int64_t>(), d_src, d_tgt, d_guess, stride,
+                     npts, P.norm.as<double>(), P.frame.as<float>(), per, P.X.as<float4>());
   launch_enc_forward(P.bufs(), npairs, npts, nullptr, s);
   hipLaunchKernelGGL(k_prop_guess, dim3((npairs + 63) / 64), dim3(64), 0, s, P.OUT.as<float>(),
                      P.frame.as<float>(), npairs, stride, slot, d_guess);

@@ -536,7 +536,8 @@ void Engine::reset_graph() {
 // Live 64-point tiles at or below which a chunk runs the four-lanes-per-query
 // search: more fill the chip with one lane per query (a fresh 24-capture cycle's
 // kernels, with the seeds' balls walked row by row: 7810 us at 2048, 7420 at 4096,
-// 7520 at 8192, 7820 with the split in every launch); LCR_SPLIT_TILES (read at every setup) overrides it, 0 turns the split off.
+// 7520 at 8192, 7820 with the split in every launch); LCR_SPLIT_TILES (read at every
+// setup) overrides it, 0 turns the split off.
 static int icp_split_units() {
   const char* e = getenv("LCR_SPLIT_TILES");
   if (e && *e) return std::max(0, atoi(e));
