@@ -381,9 +381,7 @@ void CloudSet::build(hipStream_t s, double factor, std::vector<Profiler::Span>* 
   // 4. count, scan, scatter, per-cell sort.  The counters are zero over the whole
   // allocation between builds (the scan consumes the counts), so they are filled
   // only after a reallocation.
-  const void* counts_before = d_counts.p;
-  d_counts.reserve((size_t)cells * sizeof(int));
-  if (d_counts.p != counts_before) counts_zero = false;
+  if (d_counts.reserve((size_t)cells * sizeof(int))) counts_zero = false;
   d_cell_start.reserve((size_t)cells * sizeof(int));
   d_scan_tmp.reserve((size_t)scan_tmp_ints(cells) * sizeof(int));
   const size_t npts = (size_t)std::max<int64_t>(total_pts, 1);

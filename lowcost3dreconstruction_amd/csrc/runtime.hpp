@@ -50,14 +50,16 @@ struct DevBuf {
     else
       Pool::get().give_device(p, bytes, device);
   }
-  void reserve(size_t n) {
+  // true: a new block, its contents lost (its address may be the old one's).
+  bool reserve(size_t n) {
     if (n == 0) n = 256;
-    if (n <= bytes) return;
+    if (n <= bytes) return false;
     if (p) LCR_HIP(hipFree(p));  // waits for work that may still use it
     p = nullptr;
     bytes = 0;
     p = Pool::get().take_device(&n, &device);
     bytes = n;
+    return true;
   }
   template <class T>
   T* as() const {

@@ -1,0 +1,66 @@
+"""The library's host code over tests/fake_hip.cpp (the HIP calls on host memory, no
+kernels): what a call allocates, keeps, waits for and leaves behind when it fails.
+Each case runs in a process of its own, so that the library binds to those calls."""
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import ROOT
+
+HEAD = """
+import ctypes as C, sys
+import numpy as np
+fake = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
+fake.fake_get.restype = fake.fake_pending.restype = fake.fake_streams.restype = C.c_int64
+fake.fake_launches.restype = C.c_int64
+fake.fake_faults.restype = C.c_char_p
+(POINTS, DEVICE_LIMIT, PINNED_LIMIT, FAIL_MALLOC_AT, NO_COMPACT, CLOCK_NS) = range(6)
+(DEVICE_BYTES, DEVICE_PEAK, PINNED_BYTES, PINNED_PEAK, MALLOCS, LARGEST_PINNED, PAGEABLE) = range(7)
+def put(what, v):
+    fake.fake_set(C.c_int(what), C.c_int64(v))
+get = lambda what: fake.fake_get(C.c_int(what))
+sys.path.insert(0, {root!r})
+import lowcost3dreconstruction_amd as lcr
+lcr.init(0)
+def cloud(n):
+    return np.random.default_rng(n).uniform(size=(n, 3)).astype(np.float32)
+def raises(f, *a):
+    try:
+        f(*a)
+    except lcr.LcrError:
+        return True
+    return False
+"""
+TAIL = """
+faults = fake.fake_faults().decode()
+assert not faults, faults
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", ROOT + "/tests/fake_hip.cpp", "-o", lib], check=True)
+
+    def run(code):
+        text = HEAD.format(lib=lib, root=ROOT) + textwrap.dedent(code) + TAIL
+        r = subprocess.run([sys.executable, "-c", text], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+def test_grown_counters_are_cleared_at_the_same_address(host):
+    """A handle whose clouds grow: the larger table of cell counters may get the
+    smaller one's address, and is cleared all the same."""
+    host("""
+    icp = lcr.IterativeClosestPoint()
+    for n in (500, 800, 4000, 3000, 20000):
+        put(POINTS, n)
+        icp.setInputSource(cloud(n))
+        icp.setInputTarget(cloud(n))
+        icp.align()
+    assert fake.fake_launches(b"k_cell_count") == 5
+    """)
