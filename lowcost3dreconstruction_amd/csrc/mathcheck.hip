@@ -33,6 +33,15 @@ void lcrm_horn(const double* S, double* R) {
     for (int j = 0; j < 3; ++j) R[3 * i + j] = r[i][j];
 }
 
+// A: symmetric 4x4 -> eigenvalues on the diagonal of W, V columns (Jacobi)
+void lcrm_jacobi4(const double* A, double* W, double* V) {
+  double a[4][4], v[4][4];
+  memcpy(a, A, sizeof a);
+  jacobi4(a, v);
+  memcpy(W, a, sizeof a);
+  memcpy(V, v, sizeof v);
+}
+
 // A: symmetric 3x3 -> w ascending, V columns
 void lcrm_eigh3(const double* A, double* w, double* V) {
   double a[3][3], v[3][3];

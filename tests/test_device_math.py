@@ -25,6 +25,7 @@ def m():
     L.lcrm_horn.argtypes = [dp, dp]
     L.lcrm_eigh3.argtypes = [dp, dp, dp]
     L.lcrm_smallest_eigvec3.argtypes = [dp, dp, dp]
+    L.lcrm_jacobi4.argtypes = [dp, dp, dp]
     L.lcrm_conv_step.argtypes = [ip, dp, C.c_int, dp, dp, C.c_double]
     L.lcrm_mat4_mul.argtypes = [dp, dp, dp]
     return L
@@ -157,6 +158,65 @@ def test_smallest_eigenvector_for_every_spectrum(m, spectrum, scale):
         assert answered == 200
     elif separated < 0.003 * max(spectrum) ** 2 or max(spectrum) == 0.0:
         assert answered == 0
+
+
+def _eigh_long(A):
+    """Eigenvalues and eigenvectors by cyclic Jacobi in 64-bit-mantissa arithmetic."""
+    a = A.astype(np.longdouble)
+    v = np.eye(len(a), dtype=np.longdouble)
+    for _ in range(12):
+        for p in range(len(a) - 1):
+            for q in range(p + 1, len(a)):
+                if a[p, q] == 0:
+                    continue
+                th = (a[q, q] - a[p, p]) / (2 * a[p, q])
+                t = (1 if th >= 0 else -1) / (abs(th) + np.hypot(th, 1))
+                c = 1 / np.sqrt(t * t + 1)
+                G = np.array([[c, t * c], [-t * c, c]])
+                a[:, [p, q]] = a[:, [p, q]] @ G
+                a[[p, q]] = G.T @ a[[p, q]]
+                v[:, [p, q]] = v[:, [p, q]] @ G
+    return np.diag(a), v
+
+
+def _rms(e):
+    return np.sqrt(np.mean(np.square(np.array(e, np.float64))))
+
+
+# 60 draws: the rms of either side is known to about a tenth
+RMS_RATIO = 1.3
+
+
+@pytest.mark.parametrize("spec", [(1, .8, .6), (1, .2, .1), (1, .08, .02), (1, .04, .01), (1, .006, .004),
+                                  (1, .9, -.5), (1, .95, -.7), (1, 1, -.9)])
+def test_horn_is_as_exact_as_jacobi(m, spec):
+    """The rotation's error against 64-bit-mantissa arithmetic is no larger than that of
+    Horn's matrix solved by Jacobi (FP64), the form that the closed one replaces."""
+    def horn(S):
+        N = np.empty((4, 4), S.dtype)
+        N[0] = [S.trace(), S[1, 2] - S[2, 1], S[2, 0] - S[0, 2], S[0, 1] - S[1, 0]]
+        N[1:, 1:] = S + S.T - S.trace() * np.eye(3, dtype=S.dtype)
+        N[:, 0] = N[0]
+        return N
+
+    def rotation(w, V):
+        a, x, y, z = q = V[:, np.argmax(w)] / np.sqrt(np.sum(V[:, np.argmax(w)] ** 2))
+        return np.array([[a*a+x*x-y*y-z*z, 2*(x*y-a*z), 2*(x*z+a*y)],
+                         [2*(x*y+a*z), a*a-x*x+y*y-z*z, 2*(y*z-a*x)],
+                         [2*(x*z-a*y), 2*(y*z+a*x), a*a-x*x-y*y+z*z]])
+
+    rng = np.random.default_rng(17)
+    got, jac = [], []
+    for _ in range(60):
+        S = np.ascontiguousarray(synth.random_rotation(rng) @ np.diag(spec) @ synth.random_rotation(rng))
+        ref = rotation(*_eigh_long(horn(S.astype(np.longdouble))))
+        R, W, V = np.empty(9), np.empty((4, 4)), np.empty((4, 4))
+        m.lcrm_horn(P(S), P(R))
+        N = horn(S)
+        m.lcrm_jacobi4(P(np.ascontiguousarray(N / np.abs(N).max())), P(W), P(V))
+        got.append(np.max(np.abs(R.reshape(3, 3) - ref)))
+        jac.append(np.max(np.abs(rotation(np.diag(W), V) - ref)))
+    assert _rms(got) <= RMS_RATIO * _rms(jac), (_rms(got), _rms(jac))
 
 
 def _conv_run(m, seq, max_it=4):
