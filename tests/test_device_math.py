@@ -219,6 +219,27 @@ def test_horn_is_as_exact_as_jacobi(m, spec):
     assert _rms(got) <= RMS_RATIO * _rms(jac), (_rms(got), _rms(jac))
 
 
+@pytest.mark.parametrize("spectrum", [(0, 1, 1), (0, .3, 1), (0, .1, 1), (0, .05, 1), (0, .03, 1), (1e-4, .05, 1),
+                                      (.3, .4, 1), (.6, .75, 1), (.3, .33, 1)])
+def test_smallest_eigenvector_is_as_exact_as_jacobi(m, spectrum):
+    """The same for the normals' eigenvector, against eigh3 (Jacobi)."""
+    rng = np.random.default_rng(18)
+    got, jac = [], []
+    for _ in range(60):
+        Q = synth.random_rotation(rng)
+        A = (Q * np.array(spectrum)) @ Q.T
+        A = np.ascontiguousarray(0.5 * (A + A.T))
+        wl, vl = _eigh_long(A)
+        ref = vl[:, np.argmin(wl)]
+        w, v, W, V = np.empty(1), np.empty(3), np.empty(3), np.empty((3, 3))
+        if not m.lcrm_smallest_eigvec3(P(A), P(w), P(v)):
+            continue
+        m.lcrm_eigh3(P(A), P(W), P(V))
+        got.append(np.max(np.abs(v * np.sign(v @ ref) - ref)))
+        jac.append(np.max(np.abs(V[:, 0] * np.sign(V[:, 0] @ ref) - ref)))
+    assert len(got) > 50 and _rms(got) <= RMS_RATIO * _rms(jac), (_rms(got), _rms(jac))
+
+
 def _conv_run(m, seq, max_it=4):
     io = np.array([0, 0, 0, 0], np.int32)
     dio = np.array([np.finfo(np.float64).max])
