@@ -208,7 +208,10 @@ struct ProposalImpl {
     G.reserve(kEncNParam * sizeof(float));
     W2t.reserve(64 * 128 * sizeof(__bf16));
     W3t.reserve(128 * 256 * sizeof(__bf16));
+    // no block is clear when it is taken
     LCR_HIP(hipMemsetAsync(W.p, 0, kEncNParam * sizeof(float), s));
+    LCR_HIP(hipMemsetAsync(W2t.p, 0, 64 * 128 * sizeof(__bf16), s));
+    LCR_HIP(hipMemsetAsync(W3t.p, 0, 128 * 256 * sizeof(__bf16), s));
     reset_optimizer();
   }
   ~ProposalImpl() { (void)stream.idle(); }  // before the buffers go back to the pool

@@ -142,6 +142,13 @@ void launch(const std::string& name, dim3 grid, void** args) {
           break;
         }
     }
+  } else if (is("k_enc_bf16_weights")) {
+    memset(arg<char*>(args, 1), 0, 64 * 128 * 2);
+    memset(arg<char*>(args, 2), 0, 128 * 256 * 2);
+  } else if (is("k_enc_points")) {
+    // both layers' BF16 weights were written
+    for (int i : {5, 6})
+      if (*arg<unsigned char*>(args, i) == kPoison) fault("k_enc_points: weights not written");
   } else if (is("9k_compact")) {
     if (arg<int*>(args, 5)) compact_host = arg<int*>(args, 5);
     compact();

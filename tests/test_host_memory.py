@@ -64,3 +64,13 @@ def test_grown_counters_are_cleared_at_the_same_address(host):
         icp.align()
     assert fake.fake_launches(b"k_cell_count") == 5
     """)
+
+
+def test_new_proposal_has_every_weight_zero(host):
+    """A proposal without set_weights: the BF16 copies that the forward reads are
+    written too, whatever their blocks held."""
+    host("""
+    p = lcr.Proposal()
+    p.forward(np.zeros((2, 40, 3), np.float32), np.zeros((2, 40, 3), np.float32))
+    assert fake.fake_launches(b"k_enc_points") == 1
+    """)
