@@ -213,6 +213,7 @@ struct ProposalImpl {
     LCR_HIP(hipMemsetAsync(W2t.p, 0, 64 * 128 * sizeof(__bf16), s));
     LCR_HIP(hipMemsetAsync(W3t.p, 0, 128 * 256 * sizeof(__bf16), s));
     reset_optimizer();
+    LCR_HIP(hipStreamSynchronize(s));  // a cycle reads the weights on its own stream
   }
   ~ProposalImpl() { (void)stream.idle(); }  // before the buffers go back to the pool
   void bind() const { LCR_HIP(hipSetDevice(device)); }

@@ -74,3 +74,12 @@ def test_new_proposal_has_every_weight_zero(host):
     p.forward(np.zeros((2, 40, 3), np.float32), np.zeros((2, 40, 3), np.float32))
     assert fake.fake_launches(b"k_enc_points") == 1
     """)
+
+
+def test_new_proposal_is_ready_for_any_stream(host):
+    """Cycles read a proposal's weights on their own streams: creating one leaves
+    nothing in flight on its own."""
+    host("""
+    p = lcr.Proposal()
+    assert fake.fake_pending() == 0
+    """)
