@@ -305,6 +305,7 @@ int lcr_icp_align(lcr_icp* h, const double* guess, float* out_xyz, float* out_nr
     if (!h->have_src || !h->have_tgt) return fail(LCR_E_STATE, "source and target must be set");
     if (h->params.point_to_plane && !h->tgt.has_nrm)
       return fail(LCR_E_NORMALS, "point-to-plane ICP needs target normals");
+    const IdleOnError idle(h->stream);
     prepare(h);
     h->eng.run(h->stream.s, h->cs, guess, true);
     h->result = h->eng.states()[0];
@@ -379,6 +380,7 @@ int lcr_icp_fitness(lcr_icp* h, double max_range, double* out) {
       *out = h->result.fitness;  // computed by align with max_range = DBL_MAX
       return LCR_OK;
     }
+    const IdleOnError idle(h->stream);
     h->eng.run_fitness(h->stream.s, h->cs, max_range);
     *out = h->eng.states()[0].fitness;
     return LCR_OK;
@@ -389,6 +391,7 @@ int lcr_icp_correspondences(lcr_icp* h, const double* T, int32_t* idx, float* d2
   return guarded([&] {
     if (!h || !idx || !d2) return fail(LCR_E_ARG, "NULL argument");
     if (!h->have_src || !h->have_tgt) return fail(LCR_E_STATE, "source and target must be set");
+    const IdleOnError idle(h->stream);
     prepare(h);
     const int64_t n = h->src.n;
     for (int64_t i = 0; i < n; ++i) {
@@ -532,6 +535,7 @@ int lcr_cycle_run(lcr_cycle* c) {
   return guarded([&] {
     if (!c) return fail(LCR_E_ARG, "handle is NULL");
     c->stream.bind();
+    const IdleOnError idle(c->stream);
     const lcr_cycle_desc& d = c->desc;
     Profiler& prof = Profiler::get();
     std::vector<Profiler::Span> spans;

@@ -118,6 +118,18 @@ struct Stream {
   bool idle() const noexcept { return hipStreamSynchronize(s) == hipSuccess; }
 };
 
+// Waits for a handle's stream when an exception leaves the scope: what a failed call
+// launched may use the caller's other handles (a cycle the proposal's buffers) and
+// pinned memory that the next call rewrites.
+struct IdleOnError {
+  const Stream& st;
+  int unwinding = std::uncaught_exceptions();
+  explicit IdleOnError(const Stream& stream) : st(stream) {}
+  ~IdleOnError() {
+    if (std::uncaught_exceptions() > unwinding) (void)st.idle();
+  }
+};
+
 // Results on their way to a caller's arrays: add() queues a device-to-host copy
 // into pinned memory, finish() waits and moves the bytes on, chunk by chunk while
 // later chunks still arrive.  One wait for all of a call's results, where a copy

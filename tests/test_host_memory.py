@@ -83,3 +83,30 @@ def test_new_proposal_is_ready_for_any_stream(host):
     p = lcr.Proposal()
     assert fake.fake_pending() == 0
     """)
+
+
+@pytest.mark.parametrize("what", ["cycle", "icp"])
+def test_failed_run_leaves_nothing_in_flight(host, what):
+    """A run that fails midway returns after the device is done with what it launched:
+    the caller may destroy the proposal (whose buffers that work uses) or hand in
+    other clouds next."""
+    host(f"""
+    put(POINTS, 500)
+    clouds = [cloud(500)] * 3
+    if {what!r} == "cycle":
+        p = lcr.Proposal()
+        c = lcr.Cycle(clouds, [(0, 1), (1, 2)], guesses=np.stack([np.eye(4)] * 2), proposal=p,
+                      max_corr_dist=0.1, max_iterations=5)
+        run = c.run
+    else:
+        icp = lcr.IterativeClosestPoint()
+        icp.setInputSource(clouds[0])
+        icp.setInputTarget(clouds[1])
+        run = icp.align
+    run()
+    put(NO_COMPACT, 1)
+    assert raises(run)
+    assert fake.fake_pending() == 0
+    put(NO_COMPACT, 0)
+    run()
+    """)
