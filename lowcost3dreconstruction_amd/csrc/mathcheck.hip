@@ -2,9 +2,11 @@
 // same __host__ __device__ code the ICP and normals kernels run), so the CPU test
 // suite can check them against the oracle without a GPU.  Not part of liblcr's
 // C ABI.
+#include <stddef.h>
 #include <string.h>
 
 #include "lcr_common.hpp"
+#include "lcr_kernels.hpp"
 #include "lcr_math.hpp"
 #include "lcr_search.hpp"
 #include "tune_cache.hpp"
@@ -235,6 +237,11 @@ int lcrm_nn_grid(const float* tgt, int64_t nt, const float* q, int64_t nq, float
     d2[i] = res.d2;
   }
   return 0;
+}
+
+// Where IcpBuffers holds prev (0) and fit_list (1), for the tests that look at launches.
+int lcrm_icp_buffers_at(int what) {
+  return (int)(what == 0 ? offsetof(IcpBuffers, prev) : offsetof(IcpBuffers, fit_list));
 }
 
 // C = A * B (4x4 row-major)

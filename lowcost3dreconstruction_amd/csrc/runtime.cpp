@@ -580,6 +580,7 @@ __global__ void k_tile_pairs(const PairDesc* __restrict__ pairs, int npairs, int
 void Engine::setup(hipStream_t s, const CloudSet& cs, const std::vector<int>& src,
                    const std::vector<int>& tgt, const std::vector<double>& r2, int tile_pts) {
   reset_graph();
+  matched = false;
   tile = (tile_pts == 64 || tile_pts == 128 || tile_pts == 256) ? tile_pts : 256;
   npairs = (int)src.size();
   hp.assign(npairs, PairDesc{});
@@ -727,6 +728,7 @@ bool Engine::ring_only(const CloudSet& cs) const {
 void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool use_graph,
                  const std::function<void()>& pre) {
   if (npairs == 0) return;
+  matched = false;
   Profiler& prof = Profiler::get();
   c.ring_only = ring_only(cs) ? 1 : 0;
   const int nb_search = c.ring_only ? nblocks_ring : nblocks;
@@ -836,6 +838,7 @@ void Engine::run(hipStream_t s, const CloudSet& cs, const double* guesses, bool 
                            hipMemcpyDeviceToHost, s));
   }
   LCR_HIP(hipStreamSynchronize(s));
+  matched = true;
   if (!spans.empty()) prof.collect(spans, false);
 }
 
@@ -873,7 +876,12 @@ void Engine::run_fitness(hipStream_t s, const CloudSet& cs, double max_range) {
   if (npairs == 0) return;
   Profiler& prof = Profiler::get();
   std::vector<Profiler::Span> spans;
-  const IcpBuffers b = buffers(cs);
+  IcpBuffers b = buffers(cs);
+  if (!matched) {  // other tiles since the last run: every tile, no seeds
+    b.prev = nullptr;
+    b.fit_list = nullptr;
+    b.fit_count = nullptr;
+  }
   if (ntiles > 0) {
     const int sp = prof.begin("fitness", s, &spans);
     launch_fitness(b, max_range, nblocks_fit, s, false, c.interleave, fit_split());

@@ -319,6 +319,8 @@ struct Engine {
   // (src, tgt) cloud indices per instance; squared radius per instance.
   void setup(hipStream_t s, const CloudSet& cs, const std::vector<int>& src,
              const std::vector<int>& tgt, const std::vector<double>& r2, int tile_pts);
+  // The tiles' matches and the lists of them are those of a run since the last setup.
+  bool matched = false;
   int setup_precision = -1;  // c.precision the launch shape was sized for
   // > 1: instances come in groups of gate_h hypotheses of one pair; before the
   // iterations, each group keeps only its best hypothesis by inliers within r.

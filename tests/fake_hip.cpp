@@ -46,8 +46,8 @@ int* compact_host = nullptr;         // where the last k_compact reports to
 std::string faults;                  // what a check found, a line each
 int64_t opt[8];                      // see fake_set
 int64_t stat[8];                     // see fake_get
-enum Opt { kPoints, kDeviceLimit, kPinnedLimit, kFailMallocAt, kNoCompact, kClockNs };
-enum Stat { kDeviceBytes, kDevicePeak, kPinnedBytes, kPinnedPeak, kMallocs, kLargestPinned, kPageable };
+enum Opt { kPoints, kDeviceLimit, kPinnedLimit, kFailMallocAt, kNoCompact, kClockNs, kPrevAt, kFitListAt };
+enum Stat { kDeviceBytes, kDevicePeak, kPinnedBytes, kPinnedPeak, kMallocs, kLargestPinned, kPageable, kFitnessOld };
 
 void fault(const std::string& what) { faults += what + "\n"; }
 
@@ -142,6 +142,13 @@ void launch(const std::string& name, dim3 grid, void** args) {
           break;
         }
     }
+  } else if (is("k_fitness") && !is("fold") && opt[kPrevAt]) {
+    // whether the last fitness pass was given previous matches or a list of tiles
+    const char* b = static_cast<const char*>(args[0]);
+    void *prev, *list;
+    memcpy(&prev, b + opt[kPrevAt], sizeof prev);
+    memcpy(&list, b + opt[kFitListAt], sizeof list);
+    stat[kFitnessOld] = (prev ? 1 : 0) + (list ? 2 : 0);
   } else if (is("k_enc_bf16_weights")) {
     memset(arg<char*>(args, 1), 0, 64 * 128 * 2);
     memset(arg<char*>(args, 2), 0, 128 * 256 * 2);

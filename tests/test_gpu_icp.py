@@ -393,3 +393,19 @@ def test_distance_tiles_cycle_matches_exact(lcr):
         np.testing.assert_array_equal(r["T"], res[0]["T"])
         np.testing.assert_array_equal(r["iterations"], res[0]["iterations"])
         np.testing.assert_array_equal(r["fitness"], res[0]["fitness"])
+
+
+def test_fitness_on_tiles_laid_out_since_the_last_align(lcr):
+    """Other tiles and another grid (set_params, then correspondences) between align and
+    the fitness: the same points under the same transform, so the same score up to the
+    order of its FP64 sum."""
+    p = synth.pair_ellipsoids(5, n_src=5001, n_tgt=4800)
+    icp = make_icp(lcr, p.src, p.tgt, r=0.05, iters=6, tile=256)
+    icp.align()
+    want = icp.getFitnessScore(0.0004)
+    for tile, cell_factor in ((64, 0.0), (128, 4.0), (256, 1.5)):
+        print_case(test="fitness_new_tiles", tile=tile, cell_factor=cell_factor)
+        icp._p.tile, icp._p.cell_factor = tile, cell_factor
+        icp._push()
+        icp.correspondences()
+        assert abs(icp.getFitnessScore(0.0004) - want) <= 1e-12 * want

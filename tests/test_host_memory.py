@@ -1,6 +1,7 @@
 """The library's host code over tests/fake_hip.cpp (the HIP calls on host memory, no
 kernels): what a call allocates, keeps, waits for and leaves behind when it fails.
 Each case runs in a process of its own, so that the library binds to those calls."""
+import ctypes as C
 import subprocess
 import sys
 import textwrap
@@ -16,8 +17,8 @@ fake = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
 fake.fake_get.restype = fake.fake_pending.restype = fake.fake_streams.restype = C.c_int64
 fake.fake_launches.restype = C.c_int64
 fake.fake_faults.restype = C.c_char_p
-(POINTS, DEVICE_LIMIT, PINNED_LIMIT, FAIL_MALLOC_AT, NO_COMPACT, CLOCK_NS) = range(6)
-(DEVICE_BYTES, DEVICE_PEAK, PINNED_BYTES, PINNED_PEAK, MALLOCS, LARGEST_PINNED, PAGEABLE) = range(7)
+(POINTS, DEVICE_LIMIT, PINNED_LIMIT, FAIL_MALLOC_AT, NO_COMPACT, CLOCK_NS, PREV_AT, FIT_LIST_AT) = range(8)
+(DEVICE_BYTES, DEVICE_PEAK, PINNED_BYTES, PINNED_PEAK, MALLOCS, LARGEST_PINNED, PAGEABLE, FITNESS_OLD) = range(8)
 def put(what, v):
     fake.fake_set(C.c_int(what), C.c_int64(v))
 get = lambda what: fake.fake_get(C.c_int(what))
@@ -109,4 +110,30 @@ def test_failed_run_leaves_nothing_in_flight(host, what):
     assert fake.fake_pending() == 0
     put(NO_COMPACT, 0)
     run()
+    """)
+
+
+def test_fitness_after_new_parameters_takes_nothing_from_the_old_tiles(host):
+    """A handle whose grid or tiles were laid out anew since its last align (other
+    parameters, then correspondences) has neither matches nor tile lists for them."""
+    m = C.CDLL(ROOT + "/lowcost3dreconstruction_amd/liblcr_mathcheck.so")
+    host(f"""
+    put(PREV_AT, {m.lcrm_icp_buffers_at(0)})
+    put(FIT_LIST_AT, {m.lcrm_icp_buffers_at(1)})
+    put(POINTS, 5000)
+    icp = lcr.IterativeClosestPoint(tile=256)
+    icp.setInputSource(cloud(5000))
+    icp.setInputTarget(cloud(5000))
+    icp.setMaxCorrespondenceDistance(0.1)
+    icp.align()
+    icp.getFitnessScore(0.01)
+    assert get(FITNESS_OLD) == 3
+    icp._p.tile = 64
+    icp._push()
+    icp.correspondences()
+    icp.getFitnessScore(0.01)
+    assert get(FITNESS_OLD) == 0
+    icp.align()
+    icp.getFitnessScore(0.01)
+    assert get(FITNESS_OLD) == 3
     """)
