@@ -224,9 +224,8 @@ struct ProposalImpl {
   }
   void reserve(int npairs, int npts) {
     if (npairs <= cap_pairs && npts <= cap_pts) return;
-    cap_pairs = std::max(cap_pairs, npairs);
-    cap_pts = std::max(cap_pts, npts);
-    const int64_t P = cap_pairs, C = 2 * P, N = cap_pts;
+    const int64_t P = std::max(cap_pairs, npairs), C = 2 * P, N = std::max(cap_pts, npts);
+    cap_pairs = cap_pts = 0;  // until every buffer is there
     const int64_t chunks = enc_forward_chunks((int)N);
     part_max.reserve(C * chunks * 256 * sizeof(float));
     part_arg.reserve(C * chunks * 256 * sizeof(int));
@@ -240,6 +239,8 @@ struct ProposalImpl {
     DG.reserve(P * 512 * sizeof(float));
     part_grad.reserve(enc_part_grad_floats((int)P) * sizeof(float));
     lab.reserve(P * 6 * sizeof(float));
+    cap_pairs = (int)P;
+    cap_pts = (int)N;
   }
   // the batch's own points (training and prediction read the resident set in place)
   void reserve_points(int npairs, int npts) {
@@ -423,6 +424,7 @@ int lcr_proposal_dataset(lcr_proposal* p, const float* src, const float* tgt, co
     ProposalImpl& P = p->impl;
     P.bind();
     const int64_t per = 2 * (int64_t)n_points;
+    P.ds_pairs = 0;  // no set until it is there
     P.ds_X.reserve((size_t)n_pairs * per * sizeof(float4));
     P.ds_lab.reserve((size_t)n_pairs * 6 * sizeof(float));
     // upload in slices through the pinned staging buffer
@@ -461,6 +463,7 @@ int lcr_proposal_synthesize(lcr_proposal* p, const float* shapes, const float* w
     ProposalImpl& P = p->impl;
     P.bind();
     const int64_t per = 2 * (int64_t)n_points;
+    P.ds_pairs = 0;  // no set until it is there
     P.ds_X.reserve((size_t)n_pairs * per * sizeof(float4));
     P.ds_lab.reserve((size_t)n_pairs * 6 * sizeof(float));
     std::vector<double> Pinv((size_t)n_pairs * 16);

@@ -46,7 +46,7 @@ int* compact_host = nullptr;         // where the last k_compact reports to
 std::string faults;                  // what a check found, a line each
 int64_t opt[8];                      // see fake_set
 int64_t stat[8];                     // see fake_get
-enum Opt { kPoints, kDeviceLimit, kPinnedLimit, kFailMallocAt, kNoCompact, kClockNs, kPrevAt, kFitListAt };
+enum Opt { kPoints, kDeviceLimit, kPinnedLimit, kFailMallocFrom, kNoCompact, kClockNs, kPrevAt, kFitListAt };
 enum Stat { kDeviceBytes, kDevicePeak, kPinnedBytes, kPinnedPeak, kMallocs, kLargestPinned, kPageable, kFitnessOld };
 
 void fault(const std::string& what) { faults += what + "\n"; }
@@ -153,7 +153,9 @@ void launch(const std::string& name, dim3 grid, void** args) {
     memset(arg<char*>(args, 1), 0, 64 * 128 * 2);
     memset(arg<char*>(args, 2), 0, 128 * 256 * 2);
   } else if (is("k_enc_points")) {
-    // both layers' BF16 weights were written
+    // every buffer is there and both layers' BF16 weights were written
+    for (int i : {0, 4, 5, 6, 7, 8})
+      if (!arg<char*>(args, i)) return fault("k_enc_points: null buffer");
     for (int i : {5, 6})
       if (*arg<unsigned char*>(args, i) == kPoison) fault("k_enc_points: weights not written");
   } else if (is("9k_compact")) {
@@ -198,7 +200,7 @@ hipError_t hipMalloc(void** p, size_t n) {
   std::lock_guard<std::mutex> g(mu);
   stat[kMallocs] += 1;
   *p = nullptr;
-  if ((opt[kFailMallocAt] && stat[kMallocs] == opt[kFailMallocAt]) ||
+  if ((opt[kFailMallocFrom] && stat[kMallocs] >= opt[kFailMallocFrom]) ||
       (opt[kDeviceLimit] && stat[kDeviceBytes] + (int64_t)n > opt[kDeviceLimit]) || n > kSlot)
     return hipErrorOutOfMemory;
   if (!arena)
