@@ -255,10 +255,11 @@ static int set_cloud(lcr_icp* h, HostCloud& hc, bool& have, const float* xyz, co
   if (stride == 0) stride = 3 * sizeof(float);
   if (stride < (int64_t)(3 * sizeof(float)) || stride % 4 != 0)
     return fail(LCR_E_ARG, "stride_bytes must be a multiple of 4 and >= 12");
-  hc.set(xyz, nrm, n, stride);
-  have = true;
+  have = false;  // until the copy is there
   h->dirty = true;
   h->aligned = false;
+  hc.set(xyz, nrm, n, stride);
+  have = true;
   return LCR_OK;
 }
 

@@ -149,6 +149,14 @@ void launch(const std::string& name, dim3 grid, void** args) {
     memcpy(&prev, b + opt[kPrevAt], sizeof prev);
     memcpy(&list, b + opt[kFitListAt], sizeof list);
     stat[kFitnessOld] = (prev ? 1 : 0) + (list ? 2 : 0);
+  } else if (is("k_icp_iter") && opt[kPrevAt]) {
+    // every buffer up to prev is there (normals: not point-to-point)
+    const char* b = static_cast<const char*>(args[0]);
+    for (int64_t at = 0; at <= opt[kPrevAt]; at += 8) {
+      void* p;
+      memcpy(&p, b + at, sizeof p);
+      if (!p && at != 24) return fault("k_icp_iter: null buffer");
+    }
   } else if (is("k_enc_bf16_weights")) {
     memset(arg<char*>(args, 1), 0, 64 * 128 * 2);
     memset(arg<char*>(args, 2), 0, 128 * 256 * 2);
@@ -159,8 +167,10 @@ void launch(const std::string& name, dim3 grid, void** args) {
     for (int i : {5, 6})
       if (*arg<unsigned char*>(args, i) == kPoison) fault("k_enc_points: weights not written");
   } else if (is("9k_compact")) {
-    if (arg<int*>(args, 5)) compact_host = arg<int*>(args, 5);
-    compact();
+    if (arg<int*>(args, 5)) {
+      compact_host = arg<int*>(args, 5);
+      compact();
+    }
   }
 }
 

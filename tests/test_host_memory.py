@@ -170,3 +170,49 @@ def test_proposal_after_failed_allocations(host):
     assert failing(1, p.dataset, *batch(300, 100), np.zeros((300, 6), np.float32))
     assert raises(p.predict, 0, 3) and raises(p.train, 1, 2)
     """)
+
+
+@pytest.mark.parametrize("what", ["cycle", "icp"])
+def test_run_after_failed_allocations(host, what):
+    """A run whose buffers do not fit is set up again by the next one, whichever of the
+    allocations failed."""
+    m = C.CDLL(ROOT + "/lowcost3dreconstruction_amd/liblcr_mathcheck.so")
+    host(f"""
+    put(PREV_AT, {m.lcrm_icp_buffers_at(0)})
+    put(FIT_LIST_AT, {m.lcrm_icp_buffers_at(1)})
+    failed = 0
+    for j in range(1, 60):
+        put(POINTS, 4000)
+        if {what!r} == "cycle":
+            c = lcr.Cycle([cloud(4000)] * 3, [(0, 1), (1, 2)], max_corr_dist=0.1, max_iterations=5)
+            run = c.run
+        else:
+            icp = lcr.IterativeClosestPoint()
+            icp.setInputSource(cloud(4000))
+            icp.setInputTarget(cloud(4000))
+            icp.setMaxCorrespondenceDistance(0.1)
+            run = icp.align
+        failed += failing(j, run)
+        run()
+    assert failed >= 20, failed
+    """)
+
+
+@pytest.mark.parametrize("which", ["Source", "Target"])
+def test_cloud_that_does_not_fit_is_not_set(host, which):
+    """When the copy of a new cloud cannot be taken the handle has none on that side:
+    the old one is not used under the new one's size."""
+    host(f"""
+    put(POINTS, 4000)
+    icp = lcr.IterativeClosestPoint()
+    icp.setInputSource(cloud(4000))
+    icp.setInputTarget(cloud(4000))
+    icp.align()
+    put(PINNED_LIMIT, get(PINNED_BYTES) + 4096)
+    assert raises(icp.setInput{which}, cloud(50000))
+    put(PINNED_LIMIT, 0)
+    assert raises(icp.align) and raises(icp.correspondences)
+    icp.setInput{which}(cloud(50000))
+    put(POINTS, 50000)
+    icp.align()
+    """)
