@@ -331,7 +331,7 @@ int lcr_icp_align(lcr_icp* h, const double* guess, float* out_xyz, float* out_nr
       }
       launch_transform_output(h->cs.d_raw.as<float4>(), raw_nrm, n, h->eng.d_state.as<PairState>(),
                               0, dx, raw_nrm ? dn : nullptr, h->stream.s);
-      CopyOut res(h->stream.s, (size_t)n * 6 * sizeof(float));
+      CopyOut res(h->stream.s);
       if (out_xyz) res.add(out_xyz, dx, (size_t)n * 3 * sizeof(float));
       if (out_nrm) {
         if (raw_nrm) {
@@ -455,7 +455,7 @@ int lcr_normals(const float* xyz, int64_t n, int64_t stride_bytes, int32_t k, co
     out.reserve((size_t)n * 4 * sizeof(float));
     float* d3 = out.as<float>();
     cs.normals_to_input_order(st.s, d3, d3 + 3 * n);  // NaN for non-finite points
-    CopyOut res(st.s, (size_t)n * 4 * sizeof(float));
+    CopyOut res(st.s);
     res.add(nrm, d3, (size_t)n * 3 * sizeof(float));
     if (curv) res.add(curv, d3 + 3 * n, (size_t)n * sizeof(float));
     res.finish();
@@ -666,7 +666,7 @@ int lcr_transform_points(const float* xyz, const float* nrm, int64_t n, int64_t 
     float* dn = dx + 3 * n;
     launch_transform_points(cs.d_raw.as<float4>(), (nrm && cs.has_nrm) ? cs.d_raw_nrm.as<float4>() : nullptr,
                             n, T, dx, (nrm && out_nrm) ? dn : nullptr, st.s);
-    CopyOut res(st.s, (size_t)n * 6 * sizeof(float));
+    CopyOut res(st.s);
     res.add(out_xyz, dx, (size_t)n * 3 * sizeof(float));
     if (nrm && out_nrm) res.add(out_nrm, dn, (size_t)n * 3 * sizeof(float));
     res.finish();
@@ -758,7 +758,7 @@ int lcr_voxel_grid(const float* xyz, const float* nrm, const float* curv, const 
                            st.s));
     LCR_HIP(hipStreamSynchronize(st.s));
     const int64_t nocc = (int64_t)last[0] + last[1];
-    CopyOut res(st.s, (size_t)nocc * (7 * sizeof(float) + 3));
+    CopyOut res(st.s);
     res.add(out_xyz, ox.p, (size_t)nocc * 3 * sizeof(float));
     if (on.p) res.add(out_nrm, on.p, (size_t)nocc * 3 * sizeof(float));
     if (oc.p) res.add(out_curv, oc.p, (size_t)nocc * sizeof(float));
@@ -799,7 +799,7 @@ int lcr_outlier_removal(const float* xyz, int64_t n, int32_t mean_k, double stdd
     launch_sor_stats(dist.as<float>(), fin.as<uint8_t>(), n, stddev_mult, part.as<double>(),
                      dstats.as<double>(), dkeep.as<uint8_t>(), st.s);
     double hs[3];
-    CopyOut res(st.s, (size_t)n * (1 + sizeof(float)) + sizeof hs);
+    CopyOut res(st.s);
     res.add(keep, dkeep.p, (size_t)n);
     if (mean_dist) res.add(mean_dist, dist.p, (size_t)n * sizeof(float));
     res.add(hs, dstats.p, sizeof hs);
@@ -858,7 +858,7 @@ int lcr_depth_to_cloud(const uint16_t* depth, int32_t width, int32_t height, con
     LCR_HIP(hipMemcpyAsync(h_m.p, dn.p, sizeof(int64_t), hipMemcpyDeviceToHost, st.s));
     LCR_HIP(hipStreamSynchronize(st.s));
     const int64_t m = *h_m.as<int64_t>();
-    CopyOut res(st.s, (size_t)m * (6 * sizeof(float) + 3));
+    CopyOut res(st.s);
     res.add(out_xyz, ox.p, (size_t)m * 3 * sizeof(float));
     if (on.p) res.add(out_nrm, on.p, (size_t)m * 3 * sizeof(float));
     if (orgb.p) res.add(out_rgb, orgb.p, (size_t)m * 3);

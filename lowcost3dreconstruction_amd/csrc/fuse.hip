@@ -136,7 +136,7 @@ extern "C" int lcr_depth_fuse(const uint16_t* frames, int32_t n_frames, int32_t 
                        dim3(128), 0, s, d_mean.as<float>(), (int)width, (int)height, (int)factor,
                        base, taps, d_out.as<uint16_t>());
     LCR_HIP(hipGetLastError());
-    CopyOut res(s, (size_t)np * sizeof(uint16_t));
+    CopyOut res(s);
     res.add(out, d_out.p, (size_t)np * sizeof(uint16_t));
     res.finish();
     return LCR_OK;

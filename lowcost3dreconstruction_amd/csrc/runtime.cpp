@@ -94,46 +94,54 @@ int device_cu_count() {
 
 // ------------------------------------------------------------------ copies
 
-CopyOut::CopyOut(hipStream_t s, size_t bytes) : s_(s) { stage_.reserve(bytes); }
-
 CopyOut::~CopyOut() {
-  for (const Piece& p : pieces_)
-    if (p.done) (void)hipEventDestroy(p.done);
+  for (hipEvent_t e : done_)
+    if (e) (void)hipEventDestroy(e);
 }
 
 void CopyOut::add(void* dst, const void* src, size_t bytes) {
   for (size_t at = 0; at < bytes;) {
-    const size_t len = std::min(kChunk, bytes - at);
-    Piece p{static_cast<char*>(dst) + at, used_, len, nullptr};
-    LCR_HIP(hipMemcpyAsync(stage_.as<char>() + used_, static_cast<const char*>(src) + at, len,
-                           hipMemcpyDeviceToHost, s_));
-    since_event_ += len;
-    if (since_event_ >= kChunk) {
-      LCR_HIP(hipEventCreateWithFlags(&p.done, hipEventDisableTiming));
-      pieces_.push_back(p);
-      LCR_HIP(hipEventRecord(p.done, s_));
-      since_event_ = 0;
-    } else {
-      pieces_.push_back(p);
+    if (filled_ == kChunk) {
+      first_.push_back(pieces_.size());
+      filled_ = 0;
     }
-    used_ += len;
+    const size_t len = std::min(kChunk - filled_, bytes - at);
+    pieces_.push_back(Piece{static_cast<char*>(dst) + at, static_cast<const char*>(src) + at, len, filled_});
+    filled_ += len;
     at += len;
   }
 }
 
+// A chunk that has arrived goes to the caller.
+void CopyOut::move(size_t chunk) {
+  const char* in = stage_.as<char>() + chunk % kSlots * kChunk;
+  const size_t end = chunk + 1 < first_.size() ? first_[chunk + 1] : pieces_.size();
+  for (size_t k = first_[chunk]; k < end; ++k) memcpy(pieces_[k].dst, in + pieces_[k].off, pieces_[k].bytes);
+}
+
 void CopyOut::finish() {
+  const size_t n = first_.size();
+  if (n > 0) stage_.reserve(n == 1 ? filled_ : std::min<size_t>(n, kSlots) * kChunk);
   size_t moved = 0;
-  auto move_to = [&](size_t end) {
-    for (; moved < end; ++moved)
-      memcpy(pieces_[moved].dst, stage_.as<char>() + pieces_[moved].off, pieces_[moved].bytes);
+  auto arrive = [&] {  // the oldest chunk under way
+    LCR_HIP(hipEventSynchronize(done_[moved % kSlots]));
+    move(moved++);
   };
-  for (size_t k = 0; k < pieces_.size(); ++k) {
-    if (!pieces_[k].done) continue;
-    LCR_HIP(hipEventSynchronize(pieces_[k].done));
-    move_to(k + 1);
+  for (size_t c = 0; c < n; ++c) {
+    if (c >= (size_t)kSlots) arrive();  // its place in the ring
+    char* to = stage_.as<char>() + c % kSlots * kChunk;
+    const size_t end = c + 1 < n ? first_[c + 1] : pieces_.size();
+    for (size_t k = first_[c]; k < end; ++k)
+      LCR_HIP(hipMemcpyAsync(to + pieces_[k].off, pieces_[k].src, pieces_[k].bytes, hipMemcpyDeviceToHost,
+                             s_));
+    if (c + 1 == n) break;  // the wait for the stream covers the last one
+    hipEvent_t& e = done_[c % kSlots];
+    if (!e) LCR_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    LCR_HIP(hipEventRecord(e, s_));
   }
+  while (moved + 1 < n) arrive();
   LCR_HIP(hipStreamSynchronize(s_));
-  move_to(pieces_.size());
+  if (moved < n) move(moved);
 }
 
 void copy_in(hipStream_t s, void* dst, const void* src, size_t bytes, HostBuf& stage) {

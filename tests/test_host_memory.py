@@ -216,3 +216,16 @@ def test_cloud_that_does_not_fit_is_not_set(host, which):
     put(POINTS, 50000)
     icp.align()
     """)
+
+
+def test_results_need_no_pinned_memory_of_their_size(host):
+    """The staging of results stays at a few megabytes: beside the upload's copy (24
+    bytes a point, a quarter more at most), a call on 2 M points takes little, and every
+    byte of its results arrives."""
+    host("""
+    n = 2_000_003
+    x = cloud(n)
+    got = lcr.transform_points(x, np.eye(4), nrm=x)
+    assert all((g.view(np.uint8) == 0xA5).all() for g in got)  # what a new block holds
+    assert get(PINNED_PEAK) <= 24 * n * 5 // 4 + (9 << 20), get(PINNED_PEAK)
+    """)
