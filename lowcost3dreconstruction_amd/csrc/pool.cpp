@@ -17,7 +17,8 @@ size_t Pool::size_class(size_t n) {
   if (n <= kLeast) return kLeast;
   size_t top = kLeast;
   while (top <= (n - 1) / 2) top *= 2;  // top < n <= 2 top
-  const size_t step = top / 4;
+  constexpr size_t kMostStep = (size_t)16 << 20;
+  const size_t step = top / 4 < kMostStep ? top / 4 : kMostStep;
   return (n + step - 1) / step * step;
 }
 
@@ -99,33 +100,44 @@ bool Pool::flush(int owner) {
   return !old.empty();
 }
 
-void* Pool::take_device(size_t* bytes, int* device) {
-  LCR_HIP(hipGetDevice(device));
-  *bytes = size_class(*bytes);
-  void* p = take(Key(*device, *bytes));
-  if (p) return p;
-  hipError_t e = hipMalloc(&p, *bytes);
-  if (e == hipErrorOutOfMemory && flush(*device)) {
+// A block that was not kept.  Without room for its class: what is kept goes first,
+// then the bytes asked for have to do.
+template <class F>
+void* Pool::allocate(int owner, size_t asked, size_t* bytes, const char* what, F&& alloc) {
+  void* p = nullptr;
+  hipError_t e = alloc(&p, *bytes);
+  if (e == hipErrorOutOfMemory && flush(owner)) {
     (void)hipGetLastError();
-    e = hipMalloc(&p, *bytes);
+    e = alloc(&p, *bytes);
   }
-  if (e != hipSuccess) throw Error{-2, std::string("hipMalloc failed: ") + hipGetErrorString(e)};
+  const size_t least = (asked + 255) / 256 * 256;
+  if (e == hipErrorOutOfMemory && least < *bytes) {
+    (void)hipGetLastError();
+    *bytes = least;
+    e = alloc(&p, *bytes);
+  }
+  if (e != hipSuccess) throw Error{-2, std::string(what) + " failed: " + hipGetErrorString(e)};
   return p;
 }
 
+void* Pool::take_device(size_t* bytes, int* device) {
+  LCR_HIP(hipGetDevice(device));
+  const size_t asked = *bytes;
+  *bytes = size_class(asked);
+  void* p = take(Key(*device, *bytes));
+  if (p) return p;
+  return allocate(*device, asked, bytes, "hipMalloc", [](void** q, size_t n) { return hipMalloc(q, n); });
+}
+
 void* Pool::take_pinned(size_t* bytes) {
-  *bytes = size_class(*bytes);
+  const size_t asked = *bytes;
+  *bytes = size_class(asked);
   void* p = take(Key(kPinned, *bytes));
   if (p) return p;
   // coherent: kernels leave flags there that the host waits for
-  const unsigned flags = hipHostMallocMapped | hipHostMallocCoherent;
-  hipError_t e = hipHostMalloc(&p, *bytes, flags);
-  if (e != hipSuccess && flush(kPinned)) {
-    (void)hipGetLastError();
-    e = hipHostMalloc(&p, *bytes, flags);
-  }
-  if (e != hipSuccess) throw Error{-2, std::string("hipHostMalloc failed: ") + hipGetErrorString(e)};
-  return p;
+  return allocate(kPinned, asked, bytes, "hipHostMalloc", [](void** q, size_t n) {
+    return hipHostMalloc(q, n, hipHostMallocMapped | hipHostMallocCoherent);
+  });
 }
 
 void Pool::give_device(void* p, size_t bytes, int device) noexcept { give(Key(device, bytes), p); }

@@ -43,7 +43,9 @@ class Pool {
   void give_stream(hipStream_t s, int device) noexcept;  // synchronised by the caller
 
   // Size classes: four per power of two, so a block is at most a quarter larger
-  // than asked for and a slightly different cloud finds the last one's blocks.
+  // than asked for and a slightly different cloud finds the last one's blocks; above
+  // 64 MiB steps of 16 MiB, so that a large call takes little more than it asks for.
+  // Where that does not fit either, a block has the size asked for.
   static size_t size_class(size_t n);
 
  private:
@@ -66,6 +68,8 @@ class Pool {
   void trim(int owner, std::vector<std::pair<int, void*>>* out);
   static void release(const std::vector<std::pair<int, void*>>& blocks) noexcept;
   bool flush(int owner);
+  template <class F>
+  void* allocate(int owner, size_t asked, size_t* bytes, const char* what, F&& alloc);
 
   std::mutex mu_;
   std::map<Key, std::vector<Block>> blocks_;

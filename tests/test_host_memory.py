@@ -229,3 +229,19 @@ def test_results_need_no_pinned_memory_of_their_size(host):
     assert all((g.view(np.uint8) == 0xA5).all() for g in got)  # what a new block holds
     assert get(PINNED_PEAK) <= 24 * n * 5 // 4 + (9 << 20), get(PINNED_PEAK)
     """)
+
+
+@pytest.mark.parametrize("limit", ["DEVICE_LIMIT", "PINNED_LIMIT"])
+def test_a_large_call_takes_little_more_than_it_asks_for(host, limit):
+    """Blocks are rounded up to size classes, by at most 16 MiB and only while there is
+    room for it (12 M points and their normals: 24 bytes each of input and output, 32 of
+    records, 4 of cloud numbers, five blocks; 24 bytes pinned and the results' ring),
+    also where blocks of other sizes are kept."""
+    host(f"""
+    n = 12_000_000
+    x = np.zeros((n, 3), np.float32)
+    lcr.transform_points(x[:500_000], np.eye(4), nrm=x[:500_000])
+    put({limit}, (24 + 24 + 32 + 4) * n + 5 * (16 << 20) if {limit} == DEVICE_LIMIT
+        else 24 * n + (9 << 20))
+    lcr.transform_points(x, np.eye(4), nrm=x)
+    """)
