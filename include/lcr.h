@@ -350,6 +350,12 @@ int lcr_prof_enable(int32_t on);
 int lcr_prof_reset(void);
 int lcr_prof_read(const char *name, int64_t *launches, double *total_ms);
 
+/* Gives back the device memory, pinned host memory and streams that the library keeps
+ * between calls for the next one (at most 1 GiB and 8 streams a device, 256 MiB
+ * pinned; blocks unused for 20 s go at the next call by themselves).  Handles and
+ * calls on other threads are not affected; later calls allocate anew. */
+int lcr_release_memory(void);
+
 const char *lcr_last_error(void);
 const char *lcr_version(void);
 

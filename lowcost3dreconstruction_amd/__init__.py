@@ -49,6 +49,7 @@ EXPORTS = (
     "lcr_proposal_predict", "lcr_cycle_autotune", "lcr_transform_points", "lcr_voxel_grid",
     "lcr_outlier_removal", "lcr_depth_to_cloud", "lcr_depth_to_cloud_noalloc",
     "lcr_chain_poses", "lcr_se3_pow", "lcr_centroid_align", "lcr_depth_fuse",
+    "lcr_release_memory",
 )
 
 
@@ -210,6 +211,12 @@ def version():
 
 def init(device=0):
     _check(lib.lcr_init(device))
+
+
+def release_memory():
+    """Gives back the device memory, pinned memory and streams that the library keeps
+    between calls (for another allocator in the process, or after the last call)."""
+    _check(lib.lcr_release_memory())
 
 
 def default_params():

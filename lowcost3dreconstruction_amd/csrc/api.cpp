@@ -1004,6 +1004,13 @@ int lcr_prof_read(const char* name, int64_t* launches, double* total_ms) {
   return LCR_OK;
 }
 
+int lcr_release_memory(void) {
+  return guarded([&] {
+    Pool::get().release_all();
+    return LCR_OK;
+  });
+}
+
 const char* lcr_last_error(void) { return g_err.c_str(); }
 
 const char* lcr_version(void) { return "lcr 0.1 (gfx950)"; }

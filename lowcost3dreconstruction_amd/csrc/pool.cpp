@@ -34,7 +34,7 @@ void* Pool::take(const Key& k) {
       if (it->second.empty()) blocks_.erase(it);
       kept_[k.first] -= k.second;
     }
-    trim(k.first, &old);
+    trim(&old);
   }
   release(old);
   return p;
@@ -44,45 +44,75 @@ void Pool::give(const Key& k, void* p) noexcept {
   std::vector<std::pair<int, void*>> old;
   try {
     std::lock_guard<std::mutex> lock(mu_);
-    blocks_[k].push_back(Block{p, Clock::now()});
-    kept_[k.first] += k.second;
-    trim(k.first, &old);
+    size_t& kept = kept_[k.first];
+    std::vector<Block>& v = blocks_[k];
+    try {
+      v.push_back(Block{p, Clock::now()});
+    } catch (...) {
+      if (v.empty()) blocks_.erase(k);
+      throw;
+    }
+    kept += k.second;
+    p = nullptr;
+    trim(&old);
   } catch (...) {  // no memory for the bookkeeping
-    old.emplace_back(k.first, p);
   }
+  if (p) free_block(k.first, p);
   release(old);
 }
 
-void Pool::trim(int owner, std::vector<std::pair<int, void*>>* out) {
-  const size_t keep = owner == kPinned ? kPinnedKeep : kDeviceKeep;
+void Pool::trim(std::vector<std::pair<int, void*>>* out) noexcept {
   const Clock::time_point now = Clock::now();
-  // a walk over every class: when over the limit, else once a second
-  Clock::time_point& last = trimmed_[owner];
-  if (kept_[owner] <= keep && now - last < std::chrono::seconds(1)) return;
-  last = now;
+  bool over = false;
+  for (const auto& o : kept_) over = over || o.second > limit(o.first);
+  // a walk over every class: when over a limit, else once a second
+  if (!over && now - trimmed_ < std::chrono::seconds(1)) return;
+  trimmed_ = now;
   const Clock::time_point stale = now - std::chrono::seconds(kIdleSeconds);
-  for (;;) {
-    // the block of this owner unused for longest (the first of its class's vector)
-    auto oldest = blocks_.end();
-    for (auto it = blocks_.lower_bound(Key(owner, 0)); it != blocks_.end() && it->first.first == owner;
-         ++it)
-      if (oldest == blocks_.end() || it->second.front().since < oldest->second.front().since) oldest = it;
-    if (oldest == blocks_.end()) return;
-    if (kept_[owner] <= keep && oldest->second.front().since > stale) return;
-    out->emplace_back(owner, oldest->second.front().p);
-    kept_[owner] -= oldest->first.second;
-    oldest->second.erase(oldest->second.begin());
-    if (oldest->second.empty()) blocks_.erase(oldest);
+  try {
+    for (auto& o : kept_) {
+      for (;;) {
+        // the block of this owner unused for longest (the first of its class's vector)
+        auto oldest = blocks_.end();
+        for (auto it = blocks_.lower_bound(Key(o.first, 0));
+             it != blocks_.end() && it->first.first == o.first; ++it)
+          if (oldest == blocks_.end() || it->second.front().since < oldest->second.front().since) oldest = it;
+        if (oldest == blocks_.end()) break;
+        if (o.second <= limit(o.first) && oldest->second.front().since > stale) break;
+        out->emplace_back(o.first, oldest->second.front().p);
+        o.second -= oldest->first.second;
+        oldest->second.erase(oldest->second.begin());
+        if (oldest->second.empty()) blocks_.erase(oldest);
+      }
+    }
+  } catch (...) {  // no memory for the list: later
   }
 }
 
+void Pool::free_block(int owner, void* p) noexcept {
+  if (owner == kPinned)
+    (void)hipHostFree(p);
+  else
+    (void)hipFree(p);
+}
+
 void Pool::release(const std::vector<std::pair<int, void*>>& blocks) noexcept {
-  for (const auto& b : blocks) {
-    if (b.first == kPinned)
-      (void)hipHostFree(b.second);
-    else
-      (void)hipFree(b.second);
+  for (const auto& b : blocks) free_block(b.first, b.second);
+}
+
+void Pool::release_all() {
+  std::vector<int> owners;
+  std::vector<hipStream_t> streams;
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    for (const auto& o : kept_) owners.push_back(o.first);
+    for (auto& v : streams_) {
+      streams.insert(streams.end(), v.second.begin(), v.second.end());
+      v.second.clear();
+    }
   }
+  for (hipStream_t s : streams) (void)hipStreamDestroy(s);
+  for (int o : owners) (void)flush(o);
 }
 
 bool Pool::flush(int owner) {

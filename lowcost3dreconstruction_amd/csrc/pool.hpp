@@ -10,8 +10,10 @@
 //   * bounded: at most kDeviceKeep bytes per device, kPinnedKeep bytes of pinned
 //     memory and kStreamsKeep streams per device; the blocks unused for longest
 //     are freed first;
-//   * given back: a block unused for kIdleSeconds is freed at the next use of the
-//     pool, and everything kept on a device when an allocation there fails;
+//   * given back: everything by release_all (lcr_release_memory); a block unused for
+//     kIdleSeconds at the next use of the pool (nothing runs between calls: after its
+//     last one a process keeps what the limits allow); everything kept on a device
+//     when an allocation there fails;
 //   * only idle memory enters: an owner synchronises the stream that used its
 //     buffers before it releases them (Stream's release does, and every handle's
 //     destructor and every call's normal end come after such a wait), and buffers
@@ -41,6 +43,7 @@ class Pool {
   void give_device(void* p, size_t bytes, int device) noexcept;
   void give_pinned(void* p, size_t bytes) noexcept;
   void give_stream(hipStream_t s, int device) noexcept;  // synchronised by the caller
+  void release_all();
 
   // Size classes: four per power of two, so a block is at most a quarter larger
   // than asked for and a slightly different cloud finds the last one's blocks; above
@@ -62,10 +65,12 @@ class Pool {
   static constexpr size_t kStreamsKeep = 8;
   static constexpr int kIdleSeconds = 20;
 
+  static size_t limit(int owner) { return owner == kPinned ? kPinnedKeep : kDeviceKeep; }
   void* take(const Key& k);
   void give(const Key& k, void* p) noexcept;
-  // Moves to `out` what is over the owner's limit or idle for too long.
-  void trim(int owner, std::vector<std::pair<int, void*>>* out);
+  // Moves to `out` what is over an owner's limit or idle for too long.
+  void trim(std::vector<std::pair<int, void*>>* out) noexcept;
+  static void free_block(int owner, void* p) noexcept;
   static void release(const std::vector<std::pair<int, void*>>& blocks) noexcept;
   bool flush(int owner);
   template <class F>
@@ -74,7 +79,7 @@ class Pool {
   std::mutex mu_;
   std::map<Key, std::vector<Block>> blocks_;
   std::map<int, size_t> kept_;
-  std::map<int, Clock::time_point> trimmed_;
+  Clock::time_point trimmed_{};
   std::map<int, std::vector<hipStream_t>> streams_;
 };
 

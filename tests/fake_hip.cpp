@@ -21,8 +21,8 @@
 
 namespace {
 
-constexpr size_t kSlot = (size_t)1 << 32;
-constexpr int kSlots = 512;
+constexpr size_t kSlot = (size_t)1 << 31;
+constexpr int kSlots = 2048;
 constexpr int kPoison = 0xA5;
 
 struct Stream {

@@ -245,3 +245,51 @@ def test_a_large_call_takes_little_more_than_it_asks_for(host, limit):
         else 24 * n + (9 << 20))
     lcr.transform_points(x, np.eye(4), nrm=x)
     """)
+
+
+def test_kept_memory_is_given_back(host):
+    """lcr.release_memory() frees every kept block and stream, beside a live handle that
+    goes on; idle blocks go at a later call, whichever kind of memory that one uses."""
+    host("""
+    def kept():
+        return get(DEVICE_BYTES), get(PINNED_BYTES), fake.fake_streams()
+    put(POINTS, 3000)
+    lcr.normals(cloud(3000), 10)
+    lcr.depth_fuse(np.full((4, 64, 64), 900, np.uint16), 2)
+    assert min(kept()) > 0
+    lcr.release_memory()
+    assert kept() == (0, 0, 0)
+    icp = lcr.IterativeClosestPoint()
+    icp.setInputSource(cloud(3000))
+    icp.setInputTarget(cloud(3000))
+    icp.align()
+    live = kept()
+    lcr.normals(cloud(3000), 10)
+    lcr.release_memory()
+    assert all(a <= b for a, b in zip(kept(), live)) and min(kept()) > 0
+    icp.align()
+    del icp
+    lcr.normals(cloud(3000), 10)
+    before = kept()
+    put(CLOCK_NS, 30 * 10**9)
+    c = lcr.IterativeClosestPoint()
+    c.setInputSource(cloud(300))  # takes pinned memory only
+    assert kept()[0] == 0 and kept()[1] <= 8192 < before[1], (kept(), before)
+    """)
+
+
+def test_kept_memory_is_bounded(host):
+    """Blocks that many live handles give back are kept up to a gigabyte on the device
+    and 256 MiB of pinned memory; a call that fails midway keeps none of its own."""
+    host("""
+    put(POINTS, 150_000)
+    cs = [lcr.Cycle([cloud(150_000)] * 2, [(0, 1)], max_corr_dist=0.05) for _ in range(12)]
+    for c in cs:
+        c.run()
+    assert get(DEVICE_BYTES) > 1 << 30
+    del cs, c
+    assert 0 < get(DEVICE_BYTES) <= 1 << 30 and 0 < get(PINNED_BYTES) <= 256 << 20
+    lcr.release_memory()
+    assert failing(6, lcr.normals, cloud(150_000), 10)
+    assert get(DEVICE_BYTES) <= 1 << 16, get(DEVICE_BYTES)
+    """)
