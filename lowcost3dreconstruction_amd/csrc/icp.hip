@@ -264,8 +264,7 @@ __global__ void __launch_bounds__(TILE, 7) k_icp_iter(const IcpBuffers b, const 
     const bool empty = own && bounded && b.near && gt.near_r >= r &&
                        !near_cell(gt, b.near, qx, qy, qz);
     bool search = own && !empty;  // lanes that still need the scalar search
-    // an instance's first iteration has no matches yet
-    int seed = (search && b.prev && st->iterations > 0) ? b.prev[slot] : kNoSeed;
+    int seed = search ? last_match(b.prev, slot, st->iterations) : kNoSeed;
     if constexpr (PREC != 0) {
       __shared__ TileLds tl;
       const bool q_ok = search && isfinite(qx) && isfinite(qy) && isfinite(qz);
@@ -409,7 +408,7 @@ __global__ void __launch_bounds__(64 * kSplitLanes) k_icp_iter_split(const IcpBu
       const bool empty =
           own && bounded && b.near && gt.near_r >= r && !near_cell(gt, b.near, qx, qy, qz);
       if (own && !empty) {
-        const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + qi] : kNoSeed;
+        const int seed = last_match(b.prev, (int64_t)tile * TILE + qi, st->iterations);
         nn = nn_split<S, RING>(gt, b.cell_start + gt.cell_off, b.pts, qx, qy, qz, r, bounded, seed,
                                sub);
       }
@@ -615,7 +614,7 @@ __global__ void __launch_bounds__(TILE, 6) k_fitness(const IcpBuffers b, double 
       const bool empty = bounded && b.near && gt.near_r >= rq && !near_cell(gt, b.near, qx, qy, qz);
       // the lane's previous match: the iterations take the same points in the same
       // lanes as the final pass (the gate's pass runs before any match exists)
-      const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + threadIdx.x] : -1;
+      const int seed = last_match(b.prev, (int64_t)tile * TILE + threadIdx.x, st->iterations);
       // the final pass over refined instances: a point without a match within r in
       // the last iteration (seed -1) is farther than about r from the target; a
       // ring search would scan two unpruned rings before handing it to the tree,
@@ -693,7 +692,7 @@ __global__ void __launch_bounds__(64 * kSplitLanes) k_fitness_split(const IcpBuf
     if (own) {
       xform(st->T, b.morton ? b.tpts[gs.pt_off + rank] : b.pts[gs.pt_off + rank], qx, qy, qz);
       const bool empty = bounded && b.near && gt.near_r >= rq && !near_cell(gt, b.near, qx, qy, qz);
-      const int seed = b.prev && st->iterations > 0 ? b.prev[(int64_t)tile * TILE + qi] : -1;
+      const int seed = last_match(b.prev, (int64_t)tile * TILE + qi, st->iterations);
       if (!bounded && b.prev && seed < 0)
         nn.tree = true;  // as in k_fitness
       else if (!empty)

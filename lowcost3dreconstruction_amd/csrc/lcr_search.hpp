@@ -313,6 +313,14 @@ constexpr float kSeedBallCells = 3.0f;
 // hold points, as a query with a far seed does.
 constexpr int kNoSeed = -2;
 
+// The seed of the source point in `slot` of an instance: its match in the last
+// iteration (-1: none), kNoSeed before the first one or without a list of matches.
+// (With -1 for the gate's queries, which were not searched before, they scanned the
+// whole ball of the limit from its corner: the gate's pass 110 us instead of 97 on 36 captures.)
+LCR_SHD int last_match(const int* prev, int64_t slot, int iterations) {
+  return prev && iterations > 0 ? prev[slot] : kNoSeed;
+}
+
 // Rings after which a search without certification goes to the tree.
 constexpr int kTreeRings = 2;
 

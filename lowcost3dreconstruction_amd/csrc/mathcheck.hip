@@ -239,6 +239,9 @@ int lcrm_nn_grid(const float* tgt, int64_t nt, const float* q, int64_t nq, float
   return 0;
 }
 
+// The search's seed of slot 0 after `iterations` iterations that left `match` there.
+int lcrm_last_match(int match, int iterations) { return last_match(&match, 0, iterations); }
+
 // Where IcpBuffers holds prev (0) and fit_list (1), for the tests that look at launches.
 int lcrm_icp_buffers_at(int what) {
   return (int)(what == 0 ? offsetof(IcpBuffers, prev) : offsetof(IcpBuffers, fit_list));

@@ -352,6 +352,13 @@ def test_grid_ring_search_equals_bruteforce(m, h, r):
                 np.testing.assert_array_equal(d2[idx >= 0], rd2[ridx >= 0])
 
 
+def test_seed_of_a_query_that_was_not_searched(m):
+    """Before an instance's first iteration its points have no seed (-2: rings), which is
+    not the -1 of a point whose last search found nothing (the limit's ball)."""
+    assert [m.lcrm_last_match(7, 0), m.lcrm_last_match(-1, 0)] == [-2, -2]
+    assert [m.lcrm_last_match(7, 1), m.lcrm_last_match(-1, 3)] == [7, -1]
+
+
 def test_tune_cache_key_and_lookup(m, tmp_path):
     """The autotuner's cache: the key carries the workload's real point total, a
     choice of any precision mode (the FP32-staged tiles, mode 3, included) is found
