@@ -918,8 +918,12 @@ int lcr_cycle_autotune(lcr_cycle* c, const char* cache_path, lcr_tune_result* ou
       P.tile = k.tile;
       P.precision_mode = k.prec;
       P.cell_factor = k.cf;
-      rc = lcr_cycle_run(c);  // the first run of a setting captures its graphs
-      if (rc != LCR_OK) return -1.0;
+      // a setting's first run goes direct and its second captures the graphs, which the
+      // runs after them replay
+      for (int warm = 0; warm < 2; ++warm) {
+        rc = lcr_cycle_run(c);
+        if (rc != LCR_OK) return -1.0;
+      }
       const auto t0 = std::chrono::steady_clock::now();
       rc = lcr_cycle_run(c);
       const auto t1 = std::chrono::steady_clock::now();

@@ -13,11 +13,12 @@ namespace lcr {
 
 // The workload's shape: the device (arch and CU count), clouds, pairs, pose
 // hypotheses per pair, points over all clouds, the radius, the estimator and the
-// k of the normals.
+// k of the normals.  v2: choices from before it were timed with the capture of their
+// graphs, and are not used again.
 inline std::string tune_key(const std::string& device, int clouds, int pairs, int hyp,
                             int64_t points, double radius, int point_to_plane, int normals_k) {
   char buf[512];
-  snprintf(buf, sizeof buf, "dev=%s clouds=%d pairs=%d hyp=%d points=%lld r=%.6g p2pl=%d k=%d",
+  snprintf(buf, sizeof buf, "v2 dev=%s clouds=%d pairs=%d hyp=%d points=%lld r=%.6g p2pl=%d k=%d",
            device.c_str(), clouds, pairs, hyp, (long long)points, radius, point_to_plane ? 1 : 0,
            normals_k);
   return buf;

@@ -392,6 +392,7 @@ hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
   return hipSuccess;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+  opt[kClockNs] += 1000000;  // the only call that takes time: a millisecond
   *e = reinterpret_cast<hipGraphExec_t>(1);
   return hipSuccess;
 }

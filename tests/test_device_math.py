@@ -393,3 +393,16 @@ def test_tune_cache_key_and_lookup(m, tmp_path):
                               C.byref(cf)) == 0
     assert m.lcrm_tune_lookup(str(tmp_path / "none.txt").encode(), k, C.byref(t), C.byref(p),
                               C.byref(cf)) == 0
+
+
+def test_tune_cache_leaves_choices_of_the_first_key(m, tmp_path):
+    """Entries written under the key without a version were timed with the capture of
+    their graphs: a lookup does not find them."""
+    buf = C.create_string_buffer(512)
+    m.lcrm_tune_key.argtypes = [C.c_char_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_double,
+                                C.c_int, C.c_int, C.c_char_p, C.c_int]
+    m.lcrm_tune_key(b"gfx950:256", 36, 36, 2, 1000, 0.01, 1, 30, buf, 512)
+    path = tmp_path / "tune.txt"
+    path.write_bytes(b"dev=gfx950:256 clouds=36 pairs=36 hyp=2 points=1000 r=0.01 p2pl=1 k=30\t64 3 2.5 1.0\n")
+    t, p, cf = C.c_int(), C.c_int(), C.c_double()
+    assert m.lcrm_tune_lookup(str(path).encode(), buf.value, C.byref(t), C.byref(p), C.byref(cf)) == 0

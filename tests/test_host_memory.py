@@ -293,3 +293,15 @@ def test_kept_memory_is_bounded(host):
     assert failing(6, lcr.normals, cloud(150_000), 10)
     assert get(DEVICE_BYTES) <= 1 << 16, get(DEVICE_BYTES)
     """)
+
+
+def test_autotune_times_runs_whose_graphs_are_captured(host):
+    """No candidate's time holds the capture and instantiation of its graphs (three for
+    an FP32 scan, two for the tile modes), which a user's later runs do not pay."""
+    host("""
+    put(POINTS, 3000)
+    c = lcr.Cycle([cloud(3000)] * 3, [(0, 1), (1, 2)], max_corr_dist=0.1, max_iterations=5)
+    t = c.autotune()
+    assert t["candidates"] == 30
+    assert t["default_ms"] == 0 and t["best_ms"] == 0, t
+    """)
