@@ -174,7 +174,16 @@ def measured_traffic():
         return json.load(f).get("kernels", {})
 
 
-def timed_steps(cycle, steps):
+def settle(cycle):
+    """A handle's first run of a setting issues its launches directly and its second
+    captures them: the graphs are there from the third on."""
+    for _ in range(2):
+        cycle.run()
+
+
+def timed_steps(cycle, steps, settled=False):
+    if not settled:
+        settle(cycle)
     t0 = time.perf_counter()
     for _ in range(steps):
         cycle.run()
@@ -276,7 +285,7 @@ def main():
         log(f"autotune: {tune}")
     # steady-state hand-over: a second cycle object over the same clouds (the first
     # creation in a process also pays the runtime's warm-up and first allocations),
-    # then its first run (graph capture, per-upload geometry probe): a fresh cycle's
+    # then its first run (issued directly, per-upload geometry probe): a fresh cycle's
     # latency
     t_up = time.perf_counter()
     spare = make_cycle()
@@ -296,7 +305,7 @@ def main():
     # launches eagerly with an event pair around each kernel on its stream.
     lcr.prof_reset()
     lcr.prof_enable(True)
-    prof_step_s = timed_steps(cycle, args.steps)
+    prof_step_s = timed_steps(cycle, args.steps, settled=True)
     lcr.prof_enable(False)
     prof = {k: lcr.prof_read(k) for k in ("icp_iteration", "icp_solve", "fitness", "grid_build",
                                           "normals", "proposal", "gate")}
@@ -313,9 +322,9 @@ def main():
     no_prop = None
     if prop is not None:
         c0 = make_cycle(with_prop=False)
-        c0.run()
+        settle(c0)
         r0 = c0.results()
-        no_prop = {"ms_per_step": timed_steps(c0, max(1, args.steps // 2)) * 1e3,
+        no_prop = {"ms_per_step": timed_steps(c0, max(1, args.steps // 2), settled=True) * 1e3,
                    "iterations_mean": float(r0["iterations"].mean())}
         no_prop_T = r0["T"]
         no_prop_start = c0.initial_poses()[np.arange(len(cyc.pairs)) * c0.n_total_hyp
@@ -330,7 +339,7 @@ def main():
             cm.run()
             lcr.prof_reset()
             lcr.prof_enable(True)
-            ms = timed_steps(cm, args.compare_precisions) * 1e3
+            ms = timed_steps(cm, args.compare_precisions, settled=True) * 1e3
             lcr.prof_enable(False)
             _, it_ms = lcr.prof_read("icp_iteration")
             T = cm.results()["T"]
@@ -384,7 +393,7 @@ def main():
             c1 = lcr.Cycle([cyc.clouds[s], cyc.clouds[t]], [(0, 1)], guesses=prior[i:i + 1],
                            point_to_plane=True, normals_k=30, precision_mode=launch["mode"],
                            tile=launch["tile"], cell_factor=launch["cell_factor"], **icp_kw())
-            c1.run()
+            settle(c1)
             singles.append(c1)
         reps = 3
         t1 = time.perf_counter()
@@ -421,7 +430,6 @@ def main():
         out = {}
         for name, p in (("seed_only", False), ("seed_and_learned", True)):
             cp = make_cycle(with_prop=p, g=seeds, nh=1)
-            cp.run()
             ms = timed_steps(cp, max(1, args.steps // 2)) * 1e3
             rp = cp.results()
             ge = gt_errors(rp["T"], cyc.T_gt)

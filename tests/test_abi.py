@@ -87,3 +87,22 @@ def test_cycle_wrapper_fills_every_descriptor_field():
     for name in re.findall(r"int\(bool\((\w+)\)\)", src):
         assert name in params, name
     assert {"hyp_gate", "precision_mode", "proposal", "n_hyp", "guesses"} <= params
+
+
+def test_bench_times_runs_after_the_capture(monkeypatch):
+    """A handle's second run captures its graphs; what bench.py times comes after it."""
+    import sys
+    sys.path.insert(0, ROOT)
+    import bench
+
+    class Cycle:
+        runs = 0
+
+        def run(self):
+            self.runs += 1
+
+    c = Cycle()
+    ticks = []
+    monkeypatch.setattr(bench.time, "perf_counter", lambda: ticks.append(c.runs) or float(c.runs))
+    assert bench.timed_steps(c, 3) == 1.0
+    assert ticks == [2, 5]
