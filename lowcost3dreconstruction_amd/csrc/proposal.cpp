@@ -30,7 +30,7 @@ namespace {
 // 64 us, now 28 + 9).
 constexpr int kPrepThreads = 1024;
 
-// Sample i of n_out taken evenly from a cloud of n points: floor(i * n / n_out),
+// Sample i of n_out taken evenly from a cloud of n > 0 points: floor(i * n / n_out),
 // in 32-bit arithmetic when the product fits.
 __device__ __forceinline__ int64_t sample_at(int i, int64_t n, int n_out) {
   if (n < ((int64_t)1 << 31) / n_out) return (int64_t)((unsigned)(i * (int)n) / (unsigned)n_out);
@@ -64,11 +64,12 @@ k_prop_frame(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_o
   __shared__ double red[kPrepThreads][4];
   const int pr = blockIdx.x, t = threadIdx.x;
   const int64_t t0 = cloud_off[tgt[pr]], nt = cloud_off[tgt[pr] + 1] - t0;
+  const int taken = nt > 0 ? n_out : 0;  // an empty cloud has nothing to read
   float4 keep[kPrepKeep];
 #pragma unroll
   for (int u = 0; u < kPrepKeep; ++u) {
     const int i = t + u * kPrepThreads;
-    keep[u] = i < n_out ? raw[t0 + sample_at(i, nt, n_out)] : make_float4(NAN, NAN, NAN, NAN);
+    keep[u] = i < taken ? raw[t0 + sample_at(i, nt, n_out)] : make_float4(NAN, NAN, NAN, NAN);
   }
   double a[4] = {0, 0, 0, 0};
   auto add = [&](const float4& q) {
@@ -81,7 +82,7 @@ k_prop_frame(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_o
   };
 #pragma unroll
   for (int u = 0; u < kPrepKeep; ++u) add(keep[u]);
-  for (int i = t + kPrepKeep * kPrepThreads; i < n_out; i += kPrepThreads)
+  for (int i = t + kPrepKeep * kPrepThreads; i < taken; i += kPrepThreads)
     add(raw[t0 + sample_at(i, nt, n_out)]);
   prep_sum<4>(a, red);
   const double n = a[3] > 0 ? a[3] : 1.0;
@@ -96,7 +97,7 @@ k_prop_frame(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_o
   };
 #pragma unroll
   for (int u = 0; u < kPrepKeep; ++u) spread(keep[u]);
-  for (int i = t + kPrepKeep * kPrepThreads; i < n_out; i += kPrepThreads)
+  for (int i = t + kPrepKeep * kPrepThreads; i < taken; i += kPrepThreads)
     spread(raw[t0 + sample_at(i, nt, n_out)]);
   prep_sum<2>(b, reinterpret_cast<double(*)[2]>(red));
   const double rr = b[1] > 0 ? sqrt(b[0] / b[1]) : 1.0;
@@ -126,7 +127,7 @@ k_prop_inputs(const float4* __restrict__ raw, const int64_t* __restrict__ cloud_
   const float inv = (float)norm[pr];
   const float c0 = frame[pr * 4], c1 = frame[pr * 4 + 1], c2 = frame[pr * 4 + 2];
   float4* out = X + (int64_t)pr * 2 * n_out + (source ? 0 : n_out);
-  const float4 p = raw[o + sample_at(i, n, n_out)];
+  const float4 p = n > 0 ? raw[o + sample_at(i, n, n_out)] : make_float4(NAN, NAN, NAN, NAN);
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
   if (isfinite(p.x) && isfinite(p.y) && isfinite(p.z)) {
     float m[3] = {p.x, p.y, p.z};

@@ -10,6 +10,7 @@ import os
 
 import numpy as np
 import pytest
+from scipy.spatial.transform import Rotation
 
 import oracle
 from conftest import ROOT, print_case
@@ -209,3 +210,26 @@ def test_learned_proposal_gains_over_plain_icp(lcr):
     assert learned["success"] >= plain["success"] + 0.15
     assert learned["iterations"].mean() <= 0.8 * plain["iterations"].mean()
     assert np.mean(plain["ok"] & ~learned["ok"]) <= 0.03
+
+
+def test_learned_guess_beside_empty_clouds(lcr):
+    """Pairs with an empty cloud (the last one: nothing lies behind it) read no points
+    of it: their guess is that of samples at the origin, and the other pairs' results
+    are those of a cycle without it."""
+    rng = np.random.default_rng(4)
+    a = rng.normal(size=(700, 3)).astype(np.float32)
+    b = (a[:650] + np.float32(0.01))
+    prop = lcr.Proposal(init_weights(rng))
+    kw = dict(proposal=prop, max_corr_dist=0.2, max_iterations=5, proposal_points=256)
+    print_case(test="proposal_empty_clouds")
+    c = lcr.Cycle([a, b, np.zeros((0, 3), np.float32)], [(0, 1), (2, 1), (0, 2)],
+                  guesses=np.stack([np.eye(4)] * 3), **kw)
+    c.run()
+    one = lcr.Cycle([a, b], [(0, 1)], guesses=np.eye(4)[None], **kw)
+    one.run()
+    np.testing.assert_array_equal(c.results()["T"][0], one.results()["T"][0])
+    np.testing.assert_array_equal(c.initial_poses()[:2], one.initial_poses())
+    learned = c.initial_poses()[5]  # (0, 2): the target's frame is the origin, radius 1
+    out = prop.forward(a[(np.arange(256) * 700) // 256][None], np.zeros((1, 256, 3), np.float32))[0]
+    np.testing.assert_allclose(learned[:3, :3], Rotation.from_rotvec(out[:3]).as_matrix(), atol=1e-6)
+    np.testing.assert_allclose(learned[:3, 3], out[3:], rtol=1e-5, atol=1e-7)
