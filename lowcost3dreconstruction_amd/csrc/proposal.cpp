@@ -507,7 +507,7 @@ int lcr_proposal_predict(lcr_proposal* p, int32_t first, int32_t count, float* o
   return pguard([&]() -> int {
     if (!p || !out || count < 1 || first < 0) return lcr_set_error_(LCR_E_ARG, "invalid arguments");
     ProposalImpl& P = p->impl;
-    if (first + count > P.ds_pairs) return lcr_set_error_(LCR_E_ARG, "range beyond the resident set");
+    if (count > P.ds_pairs - first) return lcr_set_error_(LCR_E_ARG, "range beyond the resident set");
     P.bind();
     const int chunk = 512;
     for (int b0 = 0; b0 < count; b0 += chunk) {

@@ -305,3 +305,15 @@ def test_autotune_times_runs_whose_graphs_are_captured(host):
     assert t["candidates"] == 30
     assert t["default_ms"] == 0 and t["best_ms"] == 0, t
     """)
+
+
+def test_predict_refuses_a_range_whose_end_overflows(host):
+    host("""
+    p = lcr.Proposal()
+    p.dataset(np.zeros((3, 10, 3), np.float32), np.zeros((3, 10, 3), np.float32), np.zeros((3, 6), np.float32))
+    out = np.zeros((512, 6), np.float32)
+    fp = out.ctypes.data_as(C.POINTER(C.c_float))
+    assert lcr.lib.lcr_proposal_predict(p._h, 2, 1, fp, None) == 0
+    for first, count in ((2, 2), (0, 4), (3, 1), (2, 2**31 - 1), (2**31 - 1, 1), (2**31 - 1, 2**31 - 1)):
+        assert lcr.lib.lcr_proposal_predict(p._h, first, count, fp, None) == -1, (first, count)
+    """)
