@@ -322,6 +322,8 @@ void CloudSet::build(hipStream_t s, double factor, std::vector<Profiler::Span>* 
     LCR_HIP(hipStreamSynchronize(s));
     geom.assign(hgeom, hgeom + (size_t)n * kGeomWords);
     geom_valid = true;
+    d_in.release();  // the upload is done with them
+    h_stage.release();
   }
 
   // 2. the probe grids

@@ -43,12 +43,15 @@ struct DevBuf {
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  ~DevBuf() {
+  ~DevBuf() { release(); }
+  void release() {
     if (!p) return;
     if (std::uncaught_exceptions() > 0)
       (void)hipFree(p);
     else
       Pool::get().give_device(p, bytes, device);
+    p = nullptr;
+    bytes = 0;
   }
   // true: a new block, its contents lost (its address may be the old one's).
   bool reserve(size_t n) {
@@ -74,12 +77,15 @@ struct HostBuf {
   HostBuf() = default;
   HostBuf(const HostBuf&) = delete;
   HostBuf& operator=(const HostBuf&) = delete;
-  ~HostBuf() {
+  ~HostBuf() { release(); }
+  void release() {
     if (!p) return;
     if (std::uncaught_exceptions() > 0)
       (void)hipHostFree(p);
     else
       Pool::get().give_pinned(p, bytes);
+    p = nullptr;
+    bytes = 0;
   }
   void reserve(size_t n) {
     if (n == 0) n = 256;
@@ -234,8 +240,8 @@ struct CloudSet {
   DevBuf d_slot_raw, d_slot_cell, d_near, d_near_tmp;
   DevBuf d_nwork;  // normals: the query lists of the wavefront and rescan passes
   DevBuf d_nmom;   // normals: FP64 neighbour moments, nine arrays of one per point
-  DevBuf d_in;      // the last upload's packed input, and its staging: in use until the
-  HostBuf h_stage;  // stream has run the upload
+  DevBuf d_in;      // an upload's packed input, and its staging: until the first build
+  HostBuf h_stage;  // after it has waited for the stream
   HostBuf h_small, h_build, h_vp;
 
   // Uploads clouds (x, y, z at the start of each `stride` bytes record; normals at

@@ -317,3 +317,19 @@ def test_predict_refuses_a_range_whose_end_overflows(host):
     for first, count in ((2, 2), (0, 4), (3, 1), (2, 2**31 - 1), (2**31 - 1, 1), (2**31 - 1, 2**31 - 1)):
         assert lcr.lib.lcr_proposal_predict(p._h, first, count, fp, None) == -1, (first, count)
     """)
+
+
+def test_resident_cycle_keeps_no_copy_of_its_upload(host):
+    """Once a cycle's clouds are on the device in their own layout, the packed copies
+    they came in (12 bytes a point pinned, as many on the device) go back."""
+    host("""
+    n = 100_000
+    put(POINTS, n)
+    c = lcr.Cycle([cloud(n)] * 2, [(0, 1)], max_corr_dist=0.05)
+    c.run()
+    held = get(DEVICE_BYTES)
+    lcr.release_memory()
+    assert get(PINNED_BYTES) < 12 * n, get(PINNED_BYTES)
+    assert get(DEVICE_BYTES) <= held - 2 * 12 * n, (held, get(DEVICE_BYTES))
+    c.run()
+    """)
