@@ -443,10 +443,11 @@ int lcr_normals(const float* xyz, int64_t n, int64_t stride_bytes, int32_t k, co
     Stream st(g_device);
     CloudSet cs;
     cs.upload(st.s, {xyz}, {nullptr}, {n}, stride_bytes);
-    // cells sized for a k-neighbourhood: ~sqrt(k) point spacings.  0.70 sqrt(k)
-    // (3.8 spacings at k = 30) keeps the 3x3x3 blocks of dense capture regions
-    // inside LDS more often than 0.75 (Kinect-v2 cycle 20.2 -> 19.5 ms per step, no
-    // change on the Kinect-v1 cycle); certification rarely needs a larger block.
+    // cells sized for a k-neighbourhood: ~sqrt(k) point spacings.  A wider cell gives
+    // the lane pass more candidates and fuller buckets, a narrower one leaves more
+    // queries to the wavefront pass.  The passes at 0.60, 0.70 and 0.80 sqrt(k): 36
+    // Kinect-v1 captures 1.50, 1.54 and 1.92 ms, 24 Kinect-v2 captures 0.91, 1.07 and
+    // 1.41, one capture of 113k points 126, 132 and 146 us.
     const double factor = std::max(2.5, 0.70 * sqrt((double)k));
     cs.build(st.s, factor, nullptr, false);
     const float v[3] = {vp ? vp[0] : 0.f, vp ? vp[1] : 0.f, vp ? vp[2] : 0.f};

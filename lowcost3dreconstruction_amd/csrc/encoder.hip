@@ -16,7 +16,7 @@
 // the chip.  At 128 rows a block holds 53 KB of LDS and three blocks share a CU, so
 // one block's MFMA work overlaps another's vector work.  Bound by the vector
 // instructions around the MFMAs (per value of layer 3: bias, compare, select, max).
-// 256 pairs x 8192 points: 682 -> 342 us (1.01 PFLOP/s; a large bf16 matrix product
+// 256 pairs x 8192 points: 682 -> 347 us (0.99 PFLOP/s; a large bf16 matrix product
 // reaches 1.18 here) from one pass per block, weights loaded each time, two-byte
 // stores of h2 and a bounds test per value.
 //

@@ -588,9 +588,9 @@ k_normal_lane(const GridDesc* __restrict__ grids, const int* __restrict__ cell_s
 // original index, position) in LDS, where each one's rank among them picks the
 // first kk - (count below); a wavefront sum in a fixed order then gives the
 // query's moments.  The selected set is exactly the kk smallest (d2, original
-// index).  A block that covers the
-// grid, a radius above kWaveMaxK, or more than 64 equal keys sends the query to
-// the rescan pass.
+// index).  A block that covers the grid holds every point and certifies itself;
+// a radius above kWaveMaxK or more than 64 equal keys sends the query to the
+// rescan pass.
 constexpr int kWaveBuckets = 256;
 constexpr int kWaveMaxK = 48;
 constexpr int kWaveThreads = 256;
@@ -919,7 +919,7 @@ k_normal_rescan(const GridDesc* __restrict__ grids, const int* __restrict__ cell
 // rescan pass's list of original indices, kNselOrig set), covariance, normal
 // (eigenvector of the smallest eigenvalue, FP64) oriented towards the viewpoint.
 // Bound by FP64 latency: 36 captures (37k-113k points each) 211 us with Jacobi for every point,
-// 62 with the closed form; four wavefronts a SIMD for it (8 spills) over two.
+// 64 with the closed form; four wavefronts a SIMD for it (8 spills) over two.
 __global__ void __launch_bounds__(256, 4)
 k_normal_solve(const float4* __restrict__ pts, const int* __restrict__ cloud_of_sorted,
                const float4* __restrict__ raw, const int64_t* __restrict__ cloud_off,

@@ -75,3 +75,29 @@ def test_repeated_runs_of_a_handle_equal_a_new_one(lcr):
         # waiting for the iterations leaves no error behind for the next call
         f = np.full((3, 20, 30), 900 + n, np.uint16)
         np.testing.assert_array_equal(lcr.depth_fuse(f, 2), f[0])
+
+
+def test_handle_made_beside_a_live_one_shares_nothing_with_it(lcr):
+    """Two handles of the same sizes, made and run in turn, and memory given back while
+    both live: each keeps giving what it gives alone."""
+    p = [synth.pair_ellipsoids(s, n_src=4000, n_tgt=4100) for s in (3, 4)]
+    print_case(test="pool_live_handles")
+
+    def make(q):
+        return lcr.Cycle([q.src, q.tgt], [(0, 1)], max_corr_dist=0.05, max_iterations=9)
+
+    def run(c):
+        c.run()
+        r = c.results()
+        return r["T"], r["fitness"]
+
+    alone = [run(make(q)) for q in p]
+    a = make(p[0])
+    first = run(a)
+    b = make(p[1])
+    for _ in range(3):
+        got = run(b), run(a)
+        lcr.release_memory()
+        for x, y in zip((first, *got), (alone[0], alone[1], alone[0])):
+            np.testing.assert_array_equal(x[0], y[0])
+            np.testing.assert_array_equal(x[1], y[1])
