@@ -184,7 +184,8 @@ void lcr_cycle_destroy(lcr_cycle *c);
 /* Autotuner (no counterpart in the reference, which has no launch shape to
  * choose).  Times repeat runs of the cycle under candidate launch settings --
  * tile (64/128/256), cell_factor (1.5..4) and precision_mode (FP32 scan or
- * FP16/BF16 distance tiles) -- and keeps the fastest in the cycle's parameters.
+ * FP16/BF16 distance tiles) -- and keeps the fastest in the cycle's parameters; of
+ * those within the noise of it, the one nearest to the cycle's own setting.
  * Every candidate gives the same correspondences; only speed differs.  With a
  * cache_path (nullable) the choice is looked up first and appended after
  * tuning; entries are keyed by the device and the workload's shape

@@ -902,68 +902,56 @@ int lcr_cycle_autotune(lcr_cycle* c, const char* cache_path, lcr_tune_result* ou
       if (out) *out = r;
       return LCR_OK;
     }
-    struct Cand {
-      int tile, prec;
-      double cf;
-    };
-    std::vector<Cand> cands;
+    std::vector<TuneSetting> cands;
     for (double cf : {1.5, 2.0, 2.5, 3.0, 4.0}) {
-      for (int tile : {64, 128, 256}) cands.push_back({tile, LCR_PREC_FP32, cf});
-      cands.push_back({64, LCR_PREC_FP16, cf});
-      cands.push_back({64, LCR_PREC_BF16, cf});
-      cands.push_back({64, LCR_PREC_FP32_TILES, cf});
+      for (int tile : {64, 128, 256}) cands.push_back({tile, LCR_PREC_FP32, cf, 0.0});
+      cands.push_back({64, LCR_PREC_FP16, cf, 0.0});
+      cands.push_back({64, LCR_PREC_BF16, cf, 0.0});
+      cands.push_back({64, LCR_PREC_FP32_TILES, cf, 0.0});
     }
     const lcr_icp_params saved = P;
-    int rc = LCR_OK;
-    auto time_run = [&](const Cand& k) -> double {
+    // The least of three runs; a setting's first run goes direct and its second
+    // captures the graphs, which the runs after them replay.
+    auto time_run = [&](TuneSetting& k) -> int {
       P.tile = k.tile;
       P.precision_mode = k.prec;
-      P.cell_factor = k.cf;
-      // a setting's first run goes direct and its second captures the graphs, which the
-      // runs after them replay
-      for (int warm = 0; warm < 2; ++warm) {
-        rc = lcr_cycle_run(c);
-        if (rc != LCR_OK) return -1.0;
+      P.cell_factor = k.cell_factor;
+      for (int run = 0; run < 5; ++run) {
+        const auto t0 = std::chrono::steady_clock::now();
+        const int rc = lcr_cycle_run(c);
+        const auto t1 = std::chrono::steady_clock::now();
+        if (rc != LCR_OK) {
+          P = saved;
+          return rc;
+        }
+        const double ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
+        if (run == 2 || (run > 2 && ms < k.ms)) k.ms = ms;
       }
-      const auto t0 = std::chrono::steady_clock::now();
-      rc = lcr_cycle_run(c);
-      const auto t1 = std::chrono::steady_clock::now();
-      if (rc != LCR_OK) return -1.0;
-      return std::chrono::duration<double, std::milli>(t1 - t0).count();
+      return LCR_OK;
     };
-    const double dms = time_run({saved.tile ? saved.tile : 64, saved.precision_mode,
-                                 saved.cell_factor > 0.0 ? saved.cell_factor : 2.5});
-    if (dms < 0.0) {
-      P = saved;
-      return rc;
-    }
-    r.default_ms = dms;
-    double best = 1e300;
-    Cand bc{64, 0, 2.5};
-    for (const Cand& k : cands) {
-      const double ms = time_run(k);
-      if (ms < 0.0) {
-        P = saved;
-        return rc;
-      }
+    TuneSetting own{saved.tile ? saved.tile : 64, saved.precision_mode,
+                    saved.cell_factor > 0.0 ? saved.cell_factor : 2.5, 0.0};
+    int rc = time_run(own);
+    if (rc != LCR_OK) return rc;
+    r.default_ms = own.ms;
+    for (TuneSetting& k : cands) {
+      rc = time_run(k);
+      if (rc != LCR_OK) return rc;
       ++r.candidates;
-      if (ms < best) {
-        best = ms;
-        bc = k;
-      }
     }
+    const TuneSetting bc = cands[tune_pick(cands, own)];
     P = saved;
     P.tile = bc.tile;
     P.precision_mode = bc.prec;
-    P.cell_factor = bc.cf;
+    P.cell_factor = bc.cell_factor;
     r.tile = bc.tile;
     r.precision_mode = bc.prec;
-    r.cell_factor = bc.cf;
-    r.best_ms = best;
+    r.cell_factor = bc.cell_factor;
+    r.best_ms = bc.ms;
     if (cache_path) {
       FILE* f = fopen(cache_path, "a");
       if (f) {
-        fprintf(f, "%s\t%d %d %.17g %.6f\n", key.c_str(), bc.tile, bc.prec, bc.cf, best);
+        fprintf(f, "%s\t%d %d %.17g %.6f\n", key.c_str(), bc.tile, bc.prec, bc.cell_factor, bc.ms);
         fclose(f);
       }
     }

@@ -259,6 +259,14 @@ int lcrm_tune_key(const char* device, int clouds, int pairs, int hyp, int64_t po
   return (int)s.size();
 }
 
+// The index that tune_pick takes of n settings (tile, precision_mode, cell_factor, ms
+// each) for a cycle whose own setting is own.
+int lcrm_tune_pick(const double* v, int n, const double* own) {
+  std::vector<TuneSetting> s;
+  for (int i = 0; i < n; ++i) s.push_back({(int)v[4 * i], (int)v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]});
+  return (int)tune_pick(s, TuneSetting{(int)own[0], (int)own[1], own[2], own[3]});
+}
+
 // 1 and the entry's (tile, precision_mode, cell_factor) when `key` is cached in
 // the file at `path` (the last valid entry wins), else 0.
 int lcrm_tune_lookup(const char* path, const char* key, int* tile, int* prec, double* cf) {

@@ -3,11 +3,14 @@
 // winning.  Host-only and free of HIP calls, so the CPU tests exercise the same
 // code through liblcr_mathcheck.so.
 #pragma once
+#include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <string.h>
 
 #include <string>
+#include <tuple>
+#include <vector>
 
 namespace lcr {
 
@@ -32,6 +35,33 @@ inline bool tune_entry_valid(int tile, int prec, double cell_factor) {
   if (prec < 0 || prec > 3) return false;
   if (prec != 0 && tile != 64) return false;
   return cell_factor > 0.0;
+}
+
+// A launch setting and the time of a run with it.
+struct TuneSetting {
+  int tile, prec;
+  double cell_factor, ms;
+};
+
+// The setting to take: of those within the noise of the fastest (2 % of its time, and
+// 15 us of the host's part of a run whatever its length) the one nearest to the
+// cycle's own -- the same precision mode, the same tile, the nearest cell factor, the
+// faster.  Another setting adds the FP64 sums in another order, and a match that
+// flips with their last bits moves a transform by up to 5e-9 m: no gain beyond the
+// noise, no other order.
+constexpr double kTuneNoise = 0.02, kTuneNoiseMs = 0.015;
+
+inline size_t tune_pick(const std::vector<TuneSetting>& v, const TuneSetting& own) {
+  double best = v[0].ms;
+  for (const TuneSetting& c : v) best = c.ms < best ? c.ms : best;
+  auto far = [&](const TuneSetting& c) {
+    return std::make_tuple(c.prec != own.prec, c.tile != own.tile,
+                           fabs(log(c.cell_factor / own.cell_factor)), c.ms);
+  };
+  size_t at = v.size();
+  for (size_t i = 0; i < v.size(); ++i)
+    if (v[i].ms <= best * (1.0 + kTuneNoise) + kTuneNoiseMs && (at == v.size() || far(v[i]) < far(v[at]))) at = i;
+  return at;
 }
 
 // Parses one cache line; true when it is a valid entry for `key`.

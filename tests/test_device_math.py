@@ -406,3 +406,25 @@ def test_tune_cache_leaves_choices_of_the_first_key(m, tmp_path):
     path.write_bytes(b"dev=gfx950:256 clouds=36 pairs=36 hyp=2 points=1000 r=0.01 p2pl=1 k=30\t64 3 2.5 1.0\n")
     t, p, cf = C.c_int(), C.c_int(), C.c_double()
     assert m.lcrm_tune_lookup(str(path).encode(), buf.value, C.byref(t), C.byref(p), C.byref(cf)) == 0
+
+
+def test_tuner_leaves_the_own_setting_only_for_a_gain_beyond_the_noise(m):
+    """Of the settings within two percent and 15 us of the fastest the one nearest to
+    the cycle's own is taken; a setting that is faster by more wins from anywhere."""
+    m.lcrm_tune_pick.argtypes = [C.POINTER(C.c_double), C.c_int, C.POINTER(C.c_double)]
+    own = np.array([64, 0, 2.5, 1.0])
+
+    def pick(*rows):
+        v = np.array(rows, np.float64)
+        return m.lcrm_tune_pick(P(v), len(v), P(own))
+
+    near = [(64, 0, 1.5, 9.90), (64, 0, 2.0, 9.99), (64, 0, 2.5, 10.00), (128, 0, 2.5, 9.85)]
+    assert pick(*near) == 2
+    assert pick(*near[:2], near[3]) == 1
+    assert pick((64, 3, 2.5, 10.0), (128, 0, 4.0, 10.1)) == 1
+    assert pick(*near, (256, 2, 4.0, 9.0)) == 4
+    assert pick((64, 0, 3.0, 10.21), (64, 0, 1.5, 10.0)) == 0
+    assert pick((64, 0, 3.0, 10.22), (64, 0, 1.5, 10.0)) == 1
+    assert pick((64, 0, 3.0, 0.516), (64, 0, 1.5, 0.5)) == 0
+    assert pick((64, 0, 3.0, 0.526), (64, 0, 1.5, 0.5)) == 1
+    assert pick((64, 0, 2.5, 5.0)) == 0
