@@ -1,7 +1,7 @@
 // fake_hip.cpp -- the HIP calls that liblcr.so makes, over host memory and without
 // kernels, for CPU tests of its host code: what is allocated, kept and given back,
 // what is in flight when, and what a failing call leaves.  Loaded before liblcr.so
-// with RTLD_GLOBAL, so that liblcr.so's calls bind here.
+// (preloaded), so that liblcr.so's calls bind here.
 //
 // Device blocks come from slots of address space, the lowest free one first: a block
 // freed and one allocated next share an address, whatever their sizes.  Every new

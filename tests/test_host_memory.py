@@ -2,6 +2,7 @@
 kernels): what a call allocates, keeps, waits for and leaves behind when it fails.
 Each case runs in a process of its own, so that the library binds to those calls."""
 import ctypes as C
+import os
 import subprocess
 import sys
 import textwrap
@@ -59,7 +60,10 @@ def host(tmp_path_factory):
 
     def run(code):
         text = HEAD.format(lib=lib, root=ROOT) + textwrap.dedent(code) + TAIL
-        r = subprocess.run([sys.executable, "-c", text], capture_output=True, text=True, timeout=120)
+        # preloaded, it also stands before a C++ library that the interpreter brings in
+        env = dict(os.environ, LD_PRELOAD=" ".join(filter(None, [os.environ.get("LD_PRELOAD"), lib])))
+        r = subprocess.run([sys.executable, "-c", text], capture_output=True, text=True, timeout=120,
+                           env=env)
         assert r.returncode == 0, r.stdout + r.stderr
     return run
 
